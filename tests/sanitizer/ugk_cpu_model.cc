@@ -391,7 +391,8 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
   if (n == 0) return 0;
   REQUIRE(keys && out && status, "ugk_extract_mix: null keys, output or status");
   if (check_table(t, "ugk_extract_mix")) return 1;
-  REQUIRE(rb > 0 && rb % 16 == 0, "ugk_extract_mix: rows must be multiples of 16 bytes (row_bytes=%zu)", rb);
+  REQUIRE(rb > 0 && (rb % 16 == 0 || (!stage && rb % 4 == 0 && rb >= 20)),
+          "ugk_extract_mix: rows must be multiples of 16 bytes, or without a stage of 4 bytes (row_bytes=%zu)", rb);
   uint64_t local = 0, others = 0;
   for (size_t i = 0; i < n; ++i) {
     const uint64_t key = k64(keys[i]);

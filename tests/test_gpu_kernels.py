@@ -50,6 +50,47 @@ def test_gather_direct_matches_oracle(row_bytes, kdtype):
         assert got.tobytes() == ORC.gather(table, keys).tobytes(), (row_bytes, n)
 
 
+# rows that are no 2^k vectors of 16 bytes: lengths around the limits of the flat copy (20 bytes, 4-byte multiples) and of
+# the kernel that deals the output out (256 and 1024 bytes, a part of 4096), one and several rounds per wavefront
+@pytest.mark.parametrize("row_bytes", [20, 28, 36, 52, 100, 204, 256 + 16, 404, 800, 1020, 1024 + 4, 1204, 4092, 4096 + 4,
+                                       4096 + 48, 16384 + 4, 40004, 131072 + 4])
+@pytest.mark.parametrize("shift", [0, 4, 8])
+def test_gather_of_rows_that_are_no_whole_vectors(row_bytes, shift):
+    """table and output `shift` bytes off a 16-byte boundary, a tenth of the keys without a row: their rows, and the bytes
+    around the output, stay as they were"""
+    rng = np.random.default_rng(row_bytes + shift)
+    rows = max(7, 600_000 // row_bytes)
+    table = _rand_table(rng, rows, row_bytes)
+    d_table = to_dev(np.concatenate([np.zeros(shift, np.uint8), table.reshape(-1)]))
+    for n in (1, 2, 61, 64, 65, 2049):
+        if n * row_bytes > 20_000_000:
+            continue
+        keys = rng.integers(0, rows, size=n)
+        bad = rng.random(n) < (0.1 if n > 2 else 0.0)
+        keys[0] = keys[-1] = rows - 1
+        q = np.where(bad, rows + 3, keys)
+        want = table[keys]
+        want[bad] = 0xEE
+        for capped in (0, 2):
+            out, st = dev_bytes(n * row_bytes + 64, fill=0xEE), dev_zeros_u32(1)
+            at = ptr(out) + 16 + shift
+            d_q = to_dev(q.astype(np.int64))
+            hip.call("ugk_gather_direct_i64", ptr(d_table) + shift, rows, ptr(d_q), n, at, row_bytes, capped, ptr(st),
+                     None, None)
+            assert status_value(st) == (hip.ST_KEY_OUT_OF_RANGE if bad.any() else 0)
+            got = to_np(out)
+            assert got[16 + shift : 16 + shift + n * row_bytes].tobytes() == want.tobytes(), n
+            assert (got[: 16 + shift] == 0xEE).all() and (got[16 + shift + n * row_bytes :] == 0xEE).all()
+        # the same rows through destinations in another order
+        dst = rng.permutation(n).astype(np.uint32)
+        out, st = dev_bytes(n * row_bytes + 64, fill=0xEE), dev_zeros_u32(1)
+        d_q, d_dst = to_dev(q.astype(np.uint32)), to_dev(dst)
+        hip.call("ugk_gather_scatter_u32", ptr(d_table) + shift, rows, ptr(d_q), ptr(d_dst), n, ptr(out) + shift, n,
+                 row_bytes, 0, ptr(st), None, None)
+        got = to_np(out)[shift : shift + n * row_bytes].reshape(n, row_bytes)
+        assert got[dst].tobytes() == want.tobytes(), n
+
+
 def test_gather_direct_empty_and_capped_grid():
     rng = np.random.default_rng(1)
     table = _rand_table(rng, 100, 512)
@@ -1292,6 +1333,46 @@ def test_extract_mix_other_row_sizes(row_bytes):
                  nkeys, ptr(out), row_bytes, ptr(st), None, None, None, hip.HINT_UNKNOWN, None)
         assert status_value(st) == 0
         assert to_np(out)[: len(keys) * row_bytes].tobytes() == host[keys].tobytes()
+    finally:
+        sync()
+        pin.free()
+
+
+@pytest.mark.parametrize("row_bytes", [20, 36, 100, 128 + 4, 404, 1204, 4096 + 4, 131072 + 4])
+@pytest.mark.parametrize("kind", ["flat", "hash", "hash32"])
+def test_extract_mix_of_rows_that_are_no_whole_vectors(row_bytes, kind):
+    """cached, host and missing rows of 4-byte multiples; batches that end inside, on and behind a wavefront's keys"""
+    rng = np.random.default_rng(row_bytes)
+    nkeys = max(40, min(3000, 2_000_000 // row_bytes))
+    host = _rand_table(rng, nkeys, row_bytes)
+    cached = rng.choice(nkeys, nkeys // 3, replace=False).astype(np.uint32)
+    cache = host[cached].copy()
+    if kind == "flat":
+        mem, tb = _make_flat(nkeys)
+    elif kind == "hash":
+        mem, tb, _ = _make_hash(len(cached))
+    else:
+        mem, tb, _ = _make_hash32(len(cached))
+    assert _insert(tb, cached) == 0
+    pin = pinned_from(host)
+    try:
+        d_cache = to_dev(cache)
+        for n in (1, 7, 8, 33, 64, 1025, 9000):
+            if n * row_bytes > 40_000_000:
+                continue
+            keys = rng.integers(0, nkeys, size=n).astype(np.int64)
+            bad = rng.random(n) < (0.05 if n > 8 else 0.0)
+            q = np.where(bad, nkeys + 1, keys)
+            want = host[keys]
+            want[bad] = 0xEE
+            out, st = dev_bytes(n * row_bytes + 32, fill=0xEE), dev_zeros_u32(1)
+            d_q = to_dev(q)
+            hip.call("ugk_extract_mix_i64", tb, ptr(d_q), n, ptr(d_cache), len(cached), pin.ptr, nkeys, ptr(out),
+                     row_bytes, ptr(st), None, None, None, hip.HINT_UNKNOWN, None)
+            assert status_value(st) == (hip.ST_KEY_OUT_OF_RANGE if bad.any() else 0)
+            got = to_np(out)
+            assert got[: n * row_bytes].tobytes() == want.tobytes(), n
+            assert (got[n * row_bytes :] == 0xEE).all()
     finally:
         sync()
         pin.free()

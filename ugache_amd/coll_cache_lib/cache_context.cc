@@ -708,6 +708,18 @@ static int ExtractMix(ugk_table_t t, const Id64Type *keys, size_t n, const void 
                              s);
 }
 
+// What the fused kernel can take: rows and buffers of whole 16-byte vectors, or of 4-byte words with rows of more than
+// one vector.  The rest (rows of 4 to 16 bytes that are no vector) takes the factored path, whose gathers fall back to
+// narrower lanes.
+static bool FusedTakes(const void *cache, const void *host, const void *output, size_t rb) {
+  const uintptr_t align = (uintptr_t)cache | (uintptr_t)host | (uintptr_t)output | (uintptr_t)rb;
+  return align % 16 == 0 || (align % 4 == 0 && rb >= 20);
+}
+
+// Rows are filed in the stage next to their copy into the output by the kernels of whole 16-byte vectors only (a stage
+// exists only for such rows; the output is the caller's).
+static bool StageTakes(const void *output) { return (uintptr_t)output % 16 == 0; }
+
 static int ExtractPool(ugk_table_t t, const IdType *ids, const int64_t *seg_off, const float *w, size_t n_rows,
                        uint64_t nnz, int combiner, int elem_bytes, float max_norm, const void *cache,
                        uint64_t cache_rows, const void *host, uint64_t host_rows, void *out, size_t rb, uint32_t *st,
@@ -926,10 +938,7 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
   }
   const size_t nbytes_extracted = skip_local ? num_nodes * rb : nbytes;
 
-  // the fused kernel moves 16-byte vectors; rows or buffers that are not multiples of 16 bytes take the factored
-  // path, whose gathers fall back to narrower lanes
-  const bool vec16 = (((uintptr_t)cache | (uintptr_t)host | (uintptr_t)output | (uintptr_t)rb) & 15u) == 0;
-  if (RunConfig::concurrent_link_impl == kDirectNoGroup && dst_map == nullptr && vec16) {
+  if (RunConfig::concurrent_link_impl == kDirectNoGroup && dst_map == nullptr && FusedTakes(cache, host, output, rb)) {
     // one fused lookup + gather kernel, source chosen per row (cache_context.cu:1295-1329).  The default here: the
     // host link is busy from the first wavefront on, with no classify pass and no cross-stream hand-off in front of
     // it, and since the link bounds a mixed batch it does not matter that host loads spread over the chip slow the
@@ -943,7 +952,8 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
     // from outside the cache), not guessed from the previous batch.
     const uint32_t hint = skip_local ? (uint32_t)num_nodes : UGK_HINT_UNKNOWN;
     UGK_CALL(ExtractMix(table, nodes, num_nodes, cache, cache_rows, host, host_rows, output, rb, _status,
-                        _host_mirror, _mix_counts->ptr<uint64_t>(), &_mix_groups, hint, NextStage(stream, false), stream));
+                        _host_mirror, _mix_counts->ptr<uint64_t>(), &_mix_groups, hint,
+                        StageTakes(output) ? NextStage(stream, false) : nullptr, stream));
     if (events) UGK_CALL(ugk_event_record(_ev_t[1], stream));
     RecordLaunch(input_nodes, num_input, keys_ready);
     WaitForBatch(stream);
@@ -1091,15 +1101,14 @@ void ExtractSession::ExtractFeatAsyncImpl(const KeyT *nodes, size_t num_nodes, v
     _host_mirror[kMirGroupSizes + UGK_LOC_LOCAL] = from_host ? 0 : (uint32_t)num_nodes;
     _host_mirror[kMirGroupSizes + UGK_LOC_HOST] = from_host ? (uint32_t)num_nodes : 0;
   } else if (!ctx->IsDirectMapping() && !dedup && RunConfig::concurrent_link_impl == kDirectNoGroup &&
-             (((uintptr_t)ctx->_device_cache_data[ctx->_local_location_id] |
-               (uintptr_t)ctx->_device_cache_data[ctx->_cpu_location_id] | (uintptr_t)output | (uintptr_t)rb) &
-              15u) == 0) {
+             FusedTakes(ctx->_device_cache_data[ctx->_local_location_id],
+                        ctx->_device_cache_data[ctx->_cpu_location_id], output, rb)) {
     const RecordPlan keys_ready = RecordBegin(stream);
     UGK_CALL(ExtractMix(ctx->_new_hash_table->Table(), nodes, num_nodes,
                         ctx->_device_cache_data[ctx->_local_location_id], ctx->_cache_space_capacity,
                         ctx->_device_cache_data[ctx->_cpu_location_id], ctx->_num_total_nodes, output, rb, _status,
                         _host_mirror, _mix_counts->ptr<uint64_t>(), &_mix_groups, UGK_HINT_UNKNOWN,
-                        NextStage(stream, true), stream));
+                        StageTakes(output) ? NextStage(stream, true) : nullptr, stream));
     RecordLaunch(nodes, num_nodes, keys_ready);
     JoinRecord(stream);
     _async_last_fused = true;

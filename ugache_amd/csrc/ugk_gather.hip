@@ -12,11 +12,14 @@
 //     beyond that or when the caller says its outputs do not stay there (ugk_set_output_hint);
 //   * the grid has one workgroup per pass of rows, or is capped by the caller so a host-link gather occupies
 //     only a few CUs while the HBM gather runs next to it (then the workgroups stride over the batch);
+//   * rows of other lengths have two more kernels: gather_flat_kernel (any multiple of 4 bytes, see flat_copy) and
+//     gather_stream_kernel (long ones that come out in the order of the keys);
 //   * keys / index records are range-checked against the source's row count: a bad key sets a status bit
 //     and its row is skipped instead of faulting.
 #include <cstdlib>
 
 #include "ugk_internal.h"
+#include "ugk_mix.cuh"
 #include "ugk_table.cuh"
 
 namespace ugk {
@@ -26,6 +29,7 @@ constexpr uint64_t kNoLimit = ~0ull;
 
 // ---- index functors (what the reference calls IdxStore*) -------------------------------------------
 struct DirectU32 {
+  static constexpr bool kDense = true;  // row i goes to output row i
   const uint32_t *keys;
   __device__ __forceinline__ void get(size_t i, uint64_t &s, uint64_t &d) const {
     s = keys[i];
@@ -33,6 +37,7 @@ struct DirectU32 {
   }
 };
 struct DirectI64 {
+  static constexpr bool kDense = true;
   const int64_t *keys;
   __device__ __forceinline__ void get(size_t i, uint64_t &s, uint64_t &d) const {
     s = (uint64_t)keys[i];  // negative keys become huge and fail the range check
@@ -40,6 +45,7 @@ struct DirectI64 {
   }
 };
 struct ScatterU32 {
+  static constexpr bool kDense = false;
   const uint32_t *keys;
   const uint32_t *dst;
   __device__ __forceinline__ void get(size_t i, uint64_t &s, uint64_t &d) const {
@@ -48,6 +54,7 @@ struct ScatterU32 {
   }
 };
 struct ScatterI64 {
+  static constexpr bool kDense = false;
   const int64_t *keys;
   const uint32_t *dst;
   __device__ __forceinline__ void get(size_t i, uint64_t &s, uint64_t &d) const {
@@ -56,6 +63,7 @@ struct ScatterI64 {
   }
 };
 struct IdxList {
+  static constexpr bool kDense = false;
   const ugk_idx_t *idx;
   __device__ __forceinline__ void get(size_t i, uint64_t &s, uint64_t &d) const {
     const uint2 e = *reinterpret_cast<const uint2 *>(idx + i);  // one 8-byte load
@@ -126,6 +134,163 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
             if constexpr (NT_STORE) st_stream(out + d[u] * vpr + col, v[u]);
             else out[d[u] * vpr + col] = v[u];
           }
+      }
+    }
+  }
+}
+
+// The same for rows the lanes of gather_kernel do not fit (see flat_copy): a wavefront takes f.tile rows, one index
+// word per lane, and copies their vectors numbered through.
+template <typename Idx>
+__global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
+                                                             char *__restrict__ out, uint64_t out_rows, FlatRow f,
+                                                             const uint32_t *__restrict__ counts, uint32_t group,
+                                                             size_t n, uint32_t *status, uint32_t *host_mirror) {
+  size_t begin = 0, count = n;
+  if (counts) {
+    const uint32_t c = counts[group];
+    count = c;
+    begin = (group == UGK_LOC_LOCAL) ? 0 : n - c;
+    if (host_mirror && blockIdx.x == 0 && threadIdx.x == 0) host_mirror[1 + group] = c;
+  }
+  const size_t wave = (size_t)blockIdx.x * kWavesPerBlock + wave_in_block();
+  const size_t stride = (size_t)gridDim.x * kWavesPerBlock * f.tile;
+  for (size_t base = wave * f.tile; base < count; base += stride) {
+    const uint32_t rows = (uint32_t)min((size_t)f.tile, count - base);
+    uint64_t s = 0, d = 0;
+    bool ok = lane_id() < rows;
+    if (ok) ix.get(begin + base + lane_id(), s, d);
+    if (ok && (s >= src_rows || d >= out_rows)) {
+      ok = false;
+      atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
+      if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
+    }
+    const unsigned long long good = __ballot(ok);
+    if (good == 0ull) continue;
+    // a row that is skipped is read where the tile's first good row is
+    const uint64_t at = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
+    const uint64_t dummy = shfl64(at, __ffsll(good) - 1);
+    flat_copy<Idx::kDense>(ok ? at : dummy | kNoRowBit, (uint32_t)d, out, base, 0, rows, f);
+  }
+}
+
+// ... and with the output dealt out instead of the rows, for batches whose row i becomes output row i: a wavefront owns
+// kStreamPart aligned bytes of it, whichever rows those are.  Its stores are whole aligned vectors and lines, where the
+// edges of flat_copy's rows are lines written in two pieces; a vector that two rows share (SHARE: rows that are no
+// multiple of 16 bytes) is put together from the last vector of the one and the first vector of the other.  Bound by
+// HBM: 262,144 rows of 1204 bytes 122 us (231.6 us with 4-byte lanes) for 664 MB of lines read and rows written.
+constexpr uint32_t kStreamPart = kWave * 16 * 4;  // 4 vectors per lane
+constexpr uint32_t kStreamMinBytes = 256;         // a part is in at most 17 rows then
+
+struct StreamRow {
+  uint32_t row_bytes;
+  uint32_t magic;  // floor(2^32 / row_bytes) + 1 for rows below kStreamPart: x / row_bytes = mulhi(x, magic) for
+                   // x < row_bytes + kStreamPart; 0 for longer ones, of which a part is in two at most
+  uint64_t total;  // bytes of the output
+};
+StreamRow stream_row(size_t row_bytes, size_t n) {
+  return StreamRow{(uint32_t)row_bytes, row_bytes < kStreamPart ? (uint32_t)(0x100000000ull / row_bytes) + 1u : 0u,
+                   (uint64_t)n * row_bytes};
+}
+
+template <bool NT_STORE, bool SHARE, typename Idx>
+__global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
+                                                               char *__restrict__ out, StreamRow f, uint32_t *status,
+                                                               uint32_t *host_mirror) {
+  static_assert(Idx::kDense, "row i goes to output row i");
+  typedef __attribute__((address_space(1))) uint32_t *gword_t;
+  constexpr int U = (int)(kStreamPart / (kWave * 16));
+  const uint32_t lane = lane_id();
+  const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock * kStreamPart;
+  for (uint64_t begin = ((uint64_t)blockIdx.x * kWavesPerBlock + wave_in_block()) * kStreamPart; begin < f.total;
+       begin += stride) {
+    const uint64_t row0 = begin / f.row_bytes;
+    const uint32_t off0 = (uint32_t)(begin - row0 * f.row_bytes);  // the part begins at byte off0 of row row0
+    const uint32_t bytes = (uint32_t)min((uint64_t)kStreamPart, f.total - begin);
+    const uint64_t to = reinterpret_cast<uint64_t>(out) + begin;
+    // lane l: where row row0 + l is read
+    uint64_t s = 0, d = 0;
+    const bool active = (uint64_t)lane * f.row_bytes < (uint64_t)off0 + bytes;
+    bool ok = active;
+    if (ok) ix.get(row0 + lane, s, d);
+    if (ok && s >= src_rows) {
+      ok = false;
+      atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
+      if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
+    }
+    const unsigned long long good = __ballot(ok);
+    if (good == 0ull) continue;
+    // a row that is skipped is read where the first good one is (all lanes take part in the shuffle)
+    const uint64_t mine = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
+    const uint64_t dummy = shfl64(mine, __ffsll(good) - 1);
+    const uint64_t at = ok ? mine : dummy;
+    const uint32_t lo = (uint32_t)at | (ok ? 0u : kNoRowBit), hi = (uint32_t)(at >> 32);
+    // the vector that row l shares with the next one is lane l's: `end` is where row l ends in the part, its last `head`
+    // bytes lie in that vector (no branch around the two loads: the ones that follow would wait for them at its end)
+    u32x4 sa{}, sb{};
+    uint32_t head = 0, end = 0, nlo = kNoRowBit;
+    if constexpr (SHARE) {
+      nlo = __shfl_down(lo, 1);
+      const uint32_t nhi = __shfl_down(hi, 1);
+      end = (lane + 1) * f.row_bytes - off0;
+      if (active && end < bytes) head = end % 16;
+      sa = __builtin_nontemporal_load(reinterpret_cast<grow_by4_t>(at + f.row_bytes - 16));
+      sb = __builtin_nontemporal_load(reinterpret_cast<grow_by4_t>(((uint64_t)nhi << 32) | (nlo & ~kNoRowBit)));
+    }
+    grow_by4_t p[U];
+    bool copy[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t i = (u * kWave + lane) * 16;
+      const bool in = i + 16 <= bytes;
+      const uint32_t x = off0 + (in ? i : 0u);  // a lane past the end reads the part's first vector
+      const uint32_t r = max(__umulhi(x, f.magic), x >= f.row_bytes ? 1u : 0u);
+      const uint32_t off = x - r * f.row_bytes;
+      const uint32_t rlo = __shfl(lo, (int)r), rhi = __shfl(hi, (int)r);
+      copy[u] = in && (rlo & kNoRowBit) == 0 && (!SHARE || off + 16 <= f.row_bytes);
+      p[u] = reinterpret_cast<grow_by4_t>((((uint64_t)rhi << 32) | (rlo & ~kNoRowBit)) +
+                                          (SHARE ? min(off, f.row_bytes - 16) : off));
+    }
+    u32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
+    if constexpr (SHARE) {
+      if (head) {
+        const gout_t q = reinterpret_cast<gout_t>(to + end - head);
+        const bool row_a = (lo & kNoRowBit) == 0, row_b = (nlo & kNoRowBit) == 0;
+        u32x4 w;  // the last words of sa, then the first of sb
+        w.x = head == 12 ? sa.y : head == 8 ? sa.z : sa.w;
+        w.y = head == 12 ? sa.z : head == 8 ? sa.w : sb.x;
+        w.z = head == 12 ? sa.w : head == 8 ? sb.x : sb.y;
+        w.w = head == 12 ? sb.x : head == 8 ? sb.y : sb.z;
+        if (row_a && row_b) {
+          if constexpr (NT_STORE) __builtin_nontemporal_store(w, q);
+          else *q = w;
+        } else {  // a skipped row leaves its words of the output alone
+          const gword_t q1 = reinterpret_cast<gword_t>(q);
+          if (row_a) q1[0] = w.x;
+          if (head > 4 ? row_a : row_b) q1[1] = w.y;
+          if (head > 8 ? row_a : row_b) q1[2] = w.z;
+          if (row_b) q1[3] = w.w;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (copy[u]) {
+        const gout_t q = reinterpret_cast<gout_t>(to + (u * kWave + lane) * 16);
+        if constexpr (NT_STORE) __builtin_nontemporal_store(v[u], q);
+        else *q = v[u];
+      }
+    if constexpr (SHARE) {
+      const uint32_t rest = bytes % 16;  // the words behind the last whole vector of the output: the end of its last row
+      if (rest) {
+        const uint32_t r = (uint32_t)((f.total - 1) / f.row_bytes - row0);
+        const uint32_t rlo = __shfl(lo, (int)r), rhi = __shfl(hi, (int)r);
+        if (lane < rest / 4 && (rlo & kNoRowBit) == 0) {
+          const uint64_t from = (((uint64_t)rhi << 32) | rlo) + f.row_bytes - rest;
+          reinterpret_cast<gword_t>(to + bytes - rest)[lane] = reinterpret_cast<gword_t>(from)[lane];
+        }
       }
     }
   }
@@ -270,7 +435,7 @@ int launch_one(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t o
                                          host_mirror, nt_store_for(n * (size_t)vpr * sizeof(V)), stream);
 }
 
-template <typename V, typename Idx, bool ALL_LPR>
+template <typename V, typename Idx>
 int launch_vec(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, size_t row_bytes,
                const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
                uint32_t *host_mirror, hipStream_t stream) {
@@ -278,7 +443,7 @@ int launch_vec(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t o
 #define UGK_GO(L) \
   return launch_one<V, L, Idx>(ix, src, src_rows, out, out_rows, vpr, counts, group, n, max_blocks, status, host_mirror, \
                                stream)
-  if (ALL_LPR) {
+  if constexpr (sizeof(V) == 16) {
     if (vpr <= 1) UGK_GO(1);
     if (vpr <= 2) UGK_GO(2);
     if (vpr <= 4) UGK_GO(4);
@@ -286,12 +451,78 @@ int launch_vec(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t o
     if (vpr <= 16) UGK_GO(16);
     if (vpr <= 32) UGK_GO(32);
     UGK_GO(64);
+  } else if constexpr (sizeof(V) == 4) {  // rows of up to 16 bytes: the longer ones are copied flat
+    if (vpr <= 1) UGK_GO(1);
+    UGK_GO(4);
   } else {
     if (vpr <= 1) UGK_GO(1);
     if (vpr <= 16) UGK_GO(16);
     UGK_GO(64);
   }
 #undef UGK_GO
+}
+
+// Rows per wavefront of a flat copy: the fewest that fill nine tenths of the last round of 4 vectors per lane, or the
+// number that fills it best.  Few, because wavefronts that start in order keep the rows being written in one window
+// (see gather_grid).
+uint32_t flat_tile(size_t row_bytes) {
+  const size_t chunks = (row_bytes + 15) / 16, round = 4 * kWave;
+  uint32_t best = 1;
+  double best_fill = 0;
+  for (uint32_t t = 1; t <= (uint32_t)kWave && t * chunks <= 4 * round; ++t) {
+    const double fill = (double)(t * chunks) / (double)((t * chunks + round - 1) / round * round);
+    if (fill > best_fill) best = t, best_fill = fill;
+    if (fill >= 0.9) break;
+  }
+  return best;
+}
+
+// Which dense gathers deal the output out instead of the rows.  Measured, us per launch, rows out of 4 GiB of HBM:
+//   rows of whole vectors, against gather_kernel's 2^k lanes per row, which idle unless the row is 2^k vectors:
+//     160 bytes: 65,536 keys 7.4 -> 8.2, 262,144 keys 23.4 -> 22.1, 1 M keys 73.0 -> 70.8; 400 bytes: 13.9 -> 13.7, 42.6 ->
+//     40.8, 165.1 -> 165.4; 640 bytes: 18.4 -> 18.0, 58.6 -> 53.4; 800 bytes: 23.1 -> 22.0, 78.6 -> 79.3; 1600 bytes: 38.0 ->
+//     36.4, 153.6 -> 148.3; rows of 2^k vectors from 256 to 2048 bytes are level or up to 3 % slower
+//   other rows, against gather_flat_kernel: 404 bytes: 65,536 keys 13.4 -> 14.4, 262,144 keys 42.5 -> 44.6; 804 bytes: 21.9
+//     -> 22.3, 71.6 -> 74.3; 1204 bytes: 32.3 -> 30.5, 137.6 -> 124.4; 2404 bytes: 55.1 -> 52.3; 3000 bytes: 66.1 -> 62.6
+//     (the vectors that two rows share cost two loads and a store per row, which short rows have too many of)
+bool stream_pays(uintptr_t align, const void *out, size_t row_bytes) {
+  if (align % 16 == 0) return row_bytes >= kStreamMinBytes && (row_bytes & (row_bytes - 1)) != 0;
+  return align % 4 == 0 && (uintptr_t)out % 16 == 0 && row_bytes >= 1024;
+}
+
+template <typename Idx>
+int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, size_t row_bytes,
+                const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
+                uint32_t *host_mirror, hipStream_t stream) {
+  const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes));
+  const size_t per_block = (size_t)f.tile * kWavesPerBlock;
+  const unsigned grid = gather_grid((n + per_block - 1) / per_block, max_blocks);
+  hipLaunchKernelGGL((gather_flat_kernel<Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src, src_rows,
+                     (char *)out, out_rows, f, counts, group, n, status, host_mirror);
+  UGK_HIP(hipGetLastError());
+  return 0;
+}
+
+template <typename Idx>
+int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t row_bytes, size_t n,
+                  unsigned max_blocks, uint32_t *status, uint32_t *host_mirror, hipStream_t stream) {
+  const StreamRow f = stream_row(row_bytes, n);
+  const uint64_t per_block = (uint64_t)kStreamPart * kWavesPerBlock;
+  const unsigned grid = gather_grid((f.total + per_block - 1) / per_block, max_blocks);
+  const bool nt = nt_store_for(n * row_bytes);
+#define UGK_GO(NT, SHARE)                                                                                             \
+  hipLaunchKernelGGL((gather_stream_kernel<NT, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,                \
+                     (const char *)src, src_rows, (char *)out, f, status, host_mirror)
+  if (row_bytes % 16 == 0) {
+    if (nt) UGK_GO(true, false);
+    else UGK_GO(false, false);
+  } else {
+    if (nt) UGK_GO(true, true);
+    else UGK_GO(false, true);
+  }
+#undef UGK_GO
+  UGK_HIP(hipGetLastError());
+  return 0;
 }
 
 template <typename Idx>
@@ -305,23 +536,21 @@ int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_
   UGK_REQUIRE(n <= 0xffffffffull, "gather: batch of %zu rows exceeds 2^32", n);
   const uintptr_t align = (uintptr_t)src | (uintptr_t)out | (uintptr_t)row_bytes;
   hipStream_t st = as_stream(stream);
-  if (align % 16 == 0)
-    return launch_vec<u32x4, Idx, true>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks,
-                                            status, host_mirror, st);
-  if (align % 8 == 0)
-    return launch_vec<unsigned long long, Idx, false>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n,
-                                                      max_blocks,
-                                            status, host_mirror, st);
-  if (align % 4 == 0)
-    return launch_vec<uint32_t, Idx, false>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n,
-                                            max_blocks,
-                                            status, host_mirror, st);
-  if (align % 2 == 0)
-    return launch_vec<uint16_t, Idx, false>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n,
-                                            max_blocks,
-                                            status, host_mirror, st);
-  return launch_vec<uint8_t, Idx, false>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks,
-                                            status, host_mirror, st);
+#define UGK_VEC(V)                                                                                                  \
+  return launch_vec<V, Idx>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks, status,      \
+                            host_mirror, st)
+  if constexpr (Idx::kDense) {
+    if (stream_pays(align, out, row_bytes))
+      return launch_stream<Idx>(ix, src, src_rows, out, row_bytes, n, max_blocks, status, host_mirror, st);
+  }
+  if (align % 16 == 0) UGK_VEC(u32x4);
+  if (flat_row_ok(align, row_bytes))
+    return launch_flat<Idx>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks, status,
+                            host_mirror, st);
+  if (align % 4 == 0) UGK_VEC(uint32_t);
+  if (align % 2 == 0) UGK_VEC(uint16_t);
+  UGK_VEC(uint8_t);
+#undef UGK_VEC
 }
 
 }  // namespace

@@ -52,6 +52,8 @@ static inline unsigned clamp_grid(size_t want, unsigned max_blocks) {
 bool nt_store_for(size_t out_bytes);
 
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
+// number of the wavefront in its workgroup, in a scalar register: what is computed from it stays scalar
+__device__ __forceinline__ unsigned wave_in_block() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }
 
 // one per source file with kernels: launches an empty kernel of that file on `stream`
 void preload_gather(hipStream_t stream);

@@ -1,5 +1,7 @@
 // What the kernels that look a key up and read its row in one go have in common (the fused extraction and the pooled
-// one): where a key's row lives, and how a launch hands its per-source row counts to the host.
+// one): where a key's row lives, and how a launch hands its per-source row counts to the host.  And the copy of rows
+// that are no power of two of 16-byte vectors, or start at 4-byte boundaries only, which the gathers share with the
+// fused extraction.
 #pragma once
 
 #include "ugk_internal.h"
@@ -13,6 +15,78 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 typedef const __attribute__((address_space(1))) u32x4 *grow_t;  // a row in global memory (HBM, or mapped host memory)
 typedef __attribute__((address_space(1))) u32x4 *gout_t;
 
+// ---- flat row copy -------------------------------------------------------------------------------------------------
+// Rows of any multiple of 4 bytes above 16, as 16-byte vectors all the same: a vector load or store of global memory
+// needs 4-byte alignment only, and the last vector of a row is moved back so that it ends with the row (it overlaps
+// the one before it; both write the same bytes).  The vectors of a wavefront's rows are numbered through and dealt
+// to the 64 lanes in order, so that no lane is idle whatever the row's length.  Bound by HBM, whose unit is a line of 128
+// bytes: a row of R bytes at a random multiple of 4 touches (R + 124) / 128 of them.  What it replaced were lanes of 4 or
+// 8 bytes, 16 or 64 to a row; gathers of 262,144 rows out of 4 GiB of HBM, before -> after: 36 bytes 14.6 -> 10.6 us,
+// 100 bytes 38.0 -> 17.0 us (5.0 TB/s of lines read and rows written), 200 bytes 44.3 -> 25.7, 404 bytes 64.3 -> 42.7,
+// 804 bytes 137.8 -> 71.6.  The stores are ordinary ones whatever the size of the output: rows that end inside a line
+// leave it in two pieces, which non-temporal stores write out apart (804 bytes: 71.6 us, non-temporal 89.3).
+typedef u32x4 u32x4_by4 __attribute__((aligned(4)));
+typedef const __attribute__((address_space(1))) u32x4_by4 *grow_by4_t;
+typedef __attribute__((address_space(1))) u32x4_by4 *gout_by4_t;
+
+struct FlatRow {
+  uint32_t row_bytes;
+  uint32_t chunks;  // 16-byte vectors of a row, the last one overlapping
+  uint32_t magic;   // floor(2^32 / chunks) + 1: idx / chunks = mulhi(idx, magic) for every idx < 64 * chunks
+  uint32_t tile;    // rows numbered through together, at most 64
+};
+constexpr uint32_t kFlatMinBytes = 20;        // shorter rows are one vector or none
+constexpr uint32_t kFlatMaxTiled = 8192;      // chunks up to which mulhi divides exactly (idx * chunks < 2^32)
+constexpr uint32_t kNoRowBit = 1;             // in a row's address: nothing is copied for it
+
+static inline bool flat_row_ok(uintptr_t align, size_t row_bytes) { return align % 4 == 0 && row_bytes >= kFlatMinBytes; }
+
+// tile: how many rows a wavefront numbers through (a row too long to divide by is a tile of its own)
+static inline FlatRow flat_row(size_t row_bytes, uint32_t tile) {
+  FlatRow f;
+  f.row_bytes = (uint32_t)row_bytes;
+  f.chunks = (uint32_t)((row_bytes + 15) / 16);
+  const bool tiled = f.chunks < kFlatMaxTiled;
+  f.magic = tiled ? (uint32_t)(0x100000000ull / f.chunks) + 1u : 0u;
+  f.tile = tiled ? tile : 1u;
+  return f;
+}
+
+// Copies the rows r0 .. r0 + count - 1 of the wavefront, count <= f.tile: lane r holds where row r is read (kNoRowBit:
+// not at all) and, with DENSE false, which output row it becomes; with DENSE row r becomes output row d0 + r.  All
+// lanes call it with the same r0 and count.
+template <bool DENSE>
+__device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, char *out, size_t d0, uint32_t r0,
+                                          uint32_t count, const FlatRow &f) {
+  constexpr int U = 4;  // vectors in flight per lane
+  const uint32_t total = count * f.chunks;
+  const uint32_t tail = f.row_bytes - 16;
+  for (uint32_t i0 = 0; i0 < total; i0 += kWave * U) {
+    grow_by4_t p[U];
+    gout_by4_t q[U];
+    bool ok[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t want = i0 + u * kWave + lane_id();
+      // a lane past the end reads the last vector again instead of branching around its load
+      const uint32_t idx = want < total ? want : total - 1;
+      const uint32_t r = __umulhi(idx, f.magic);
+      const uint32_t at = min((idx - r * f.chunks) * 16, tail);
+      const uint32_t lo = __shfl((uint32_t)src_bits, (int)(r0 + r)), hi = __shfl((uint32_t)(src_bits >> 32), (int)(r0 + r));
+      ok[u] = want < total && (lo & kNoRowBit) == 0;
+      p[u] = reinterpret_cast<grow_by4_t>((((uint64_t)hi << 32) | (lo & ~kNoRowBit)) + at);
+      const size_t d = DENSE ? d0 + r0 + r : (size_t)__shfl(dst_row, (int)(r0 + r));
+      q[u] = reinterpret_cast<gout_by4_t>(reinterpret_cast<uint64_t>(out) + d * f.row_bytes + at);
+    }
+    u32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (ok[u]) *q[u] = v[u];
+  }
+}
+
 // where a key's row lives, as an integer address (the head of the output for a key without a row, see below)
 struct MixRow {
   uint64_t bits;
@@ -21,13 +95,13 @@ struct MixRow {
 };
 
 __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key, bool active, const Found &f,
-                                              const u32x4 *cache, uint64_t cache_rows, const u32x4 *host,
-                                              uint64_t host_rows, const u32x4 *out, uint32_t vpr, uint32_t *status,
-                                              uint32_t *host_mirror) {
-  const u32x4 *rowp = nullptr;
+                                              const void *cache, uint64_t cache_rows, const void *host,
+                                              uint64_t host_rows, const void *out, uint32_t row_bytes,
+                                              uint32_t *status, uint32_t *host_mirror) {
+  const char *rowp = nullptr;
   uint64_t host_row = ~0ull;
   if (active) {
-    if (f.hit && f.loc == UGK_LOC_LOCAL && f.off < cache_rows) rowp = cache + (uint64_t)f.off * vpr;
+    if (f.hit && f.loc == UGK_LOC_LOCAL && f.off < cache_rows) rowp = static_cast<const char *>(cache) + (uint64_t)f.off * row_bytes;
     else if (f.hit && f.loc == UGK_LOC_HOST && f.off < host_rows) host_row = f.off;
     else if (!f.hit && fallback_row(t, key) < host_rows) host_row = fallback_row(t, key);
     else {
@@ -37,7 +111,7 @@ __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key
   }
   // A key without a row copies nothing; its lanes read the head of the output instead (mapped whatever the key), so
   // that the loads of the copy carry no branch: behind a branch each of them waits for the one before.
-  if (host_row != ~0ull) rowp = host + host_row * vpr;
+  if (host_row != ~0ull) rowp = static_cast<const char *>(host) + host_row * row_bytes;
   MixRow r;
   r.host_row = host_row;
   r.has_row = rowp != nullptr;

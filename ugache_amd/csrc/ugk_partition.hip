@@ -222,11 +222,12 @@ __device__ __forceinline__ uint64_t stage_claim(const ugk_stage_t &stage, const 
   return reinterpret_cast<uint64_t>(reinterpret_cast<u32x4 *>(stage.rows_dev) + h * vpr);
 }
 
+// LPR: lanes per row, or 0 for rows that are copied flat (flat_copy; f.tile rows at a time)
 template <typename K, int KIND, int LPR, int KPW, bool NT_STORE, bool STAGE>
 __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, const K *__restrict__ keys, size_t n,
-                                                             const u32x4 *__restrict__ cache, uint64_t cache_rows,
-                                                             const u32x4 *__restrict__ host, uint64_t host_rows,
-                                                             u32x4 *__restrict__ out, uint32_t vpr,
+                                                             const void *__restrict__ cache, uint64_t cache_rows,
+                                                             const void *__restrict__ host, uint64_t host_rows,
+                                                             void *__restrict__ out, FlatRow f_row,
                                                              uint32_t *status, uint32_t *host_mirror,
                                                              unsigned long long *counts, ugk_stage_t stage) {
   __shared__ uint32_t block_tot[2];
@@ -244,16 +245,25 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
     // (fewer keys: their home lines in one go as well, and only the rounds of the probe that have keys to serve)
     constexpr int ROUNDS = KPW >= 8 ? KPW / 8 : 1;
     const Found f = table_lookup<KIND, (KPW == kWave || ROUNDS < 8) ? 1 : 2, ROUNDS>(t, key, active);
-    const MixRow row = mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
+    const MixRow row =
+        mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, f_row.row_bytes, status, host_mirror);
     if (counts) {
       // rows from the cache, and all others (host rows, and rows skipped for a key without a row: the launch is
       // flagged then and its group sizes mean nothing, but the two sums still add up to n)
       wave_local += __popcll(__ballot(row.from_cache));
       wave_host += __popcll(__ballot(active && !row.from_cache));
     }
-    uint64_t stage_bits = 0;
-    if constexpr (STAGE) stage_bits = stage_claim(stage, row, vpr);
-    mix_copy<LPR, KPW, NT_STORE, STAGE>(row, stage_bits, out, b0, vpr);
+    if constexpr (LPR == 0) {
+      const uint64_t bits = row.has_row ? row.bits : row.bits | kNoRowBit;
+      const uint32_t here = (uint32_t)min((size_t)KPW, n - b0);
+      for (uint32_t r0 = 0; r0 < here; r0 += f_row.tile)
+        flat_copy<true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
+    } else {
+      const uint32_t vpr = f_row.row_bytes / 16;
+      uint64_t stage_bits = 0;
+      if constexpr (STAGE) stage_bits = stage_claim(stage, row, vpr);
+      mix_copy<LPR, KPW, NT_STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
+    }
   }
   if (counts) mix_leave_counts(block_tot, wave_local, wave_host, counts);
 }
@@ -490,12 +500,13 @@ int select_keys(const K *keys, const uint32_t *sel, size_t m, K *out, void *stre
 
 template <typename K, int KIND>
 int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, uint64_t cache_rows, const void *host,
-                    uint64_t host_rows, void *out, uint32_t vpr, uint32_t *status, uint32_t *host_mirror,
-                    uint64_t *counts, uint32_t *num_groups, uint32_t others_hint, const ugk_stage_t *stage,
+                    uint64_t host_rows, void *out, size_t row_bytes, bool flat, uint32_t *status,
+                    uint32_t *host_mirror, uint64_t *counts, uint32_t *num_groups, uint32_t others_hint, const ugk_stage_t *stage,
                     hipStream_t st) {
   // ordinary write-back stores while the output fits the memory-side cache (the consumer finds it there),
   // non-temporal beyond, or as the caller's hint says
-  const bool nt = nt_store_for(n * (size_t)vpr * 16);
+  const bool nt = nt_store_for(n * row_bytes);
+  const uint32_t vpr = (uint32_t)((row_bytes + 15) / 16);
   // Keys per wavefront.  A wavefront resolves its keys together and then copies their rows a few at a time; once its
   // first stores are out, every later load of the wavefront returns behind them, so wavefronts of one round of rows
   // (8 keys of 512 bytes) keep memory busier than long ones, and short ones also fill a chip that a small batch
@@ -537,15 +548,17 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
     const int v = atoi(forced);
     if (v == 8 || v == 16 || v == 32 || v == 64) kpw = v;
   }
-  if (kpw < kWave / lpr) kpw = kWave / lpr;  // one wavefront instruction copies 64 / lpr rows
+  if (!flat && kpw < kWave / lpr) kpw = kWave / lpr;  // one wavefront instruction copies 64 / lpr rows
+  // a wavefront copies all its rows as one run of vectors, or a row at a time where they are too long to divide by
+  const FlatRow f_row = flat_row(row_bytes, (uint32_t)kpw);
   const size_t keys_per_group = (size_t)kpw * kWavesPerBlock;
   const unsigned grid = clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u);
   if (num_groups) *num_groups = grid;
   const ugk_stage_t no_stage{};
 #define UGK_GO4(L, W, NT, ST)                                                                                       \
   hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, NT, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
-                     (const u32x4 *)cache, cache_rows, (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, status,  \
-                     host_mirror, reinterpret_cast<unsigned long long *>(counts), ST ? *stage : no_stage)
+                     cache, cache_rows, host, host_rows, out, f_row, status, host_mirror,                          \
+                     reinterpret_cast<unsigned long long *>(counts), ST ? *stage : no_stage)
 #define UGK_GO3(L, W, NT)               \
   do {                                  \
     if (stage) UGK_GO4(L, W, NT, true); \
@@ -578,13 +591,24 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
     }                                               \
     UGK_GO2(L, kWave);                              \
   } while (0)
-  if (vpr <= 1) UGK_GO2(1, kWave);
+#define UGK_FLAT(W)                 \
+  do {                              \
+    if (nt) UGK_GO4(0, W, true, false); \
+    else UGK_GO4(0, W, false, false);   \
+  } while (0)
+  if (flat) {
+    if (kpw == 8) UGK_FLAT(8);
+    else if (kpw == 16) UGK_FLAT(16);
+    else if (kpw == 32) UGK_FLAT(32);
+    else UGK_FLAT(kWave);
+  } else if (vpr <= 1) UGK_GO2(1, kWave);
   else if (vpr <= 2) UGK_GO(2);
   else if (vpr <= 4) UGK_GO(4);
   else if (vpr <= 8) UGK_GO(8);
   else if (vpr <= 16) UGK_GO(16);
   else if (vpr <= 32) UGK_GO(32);
   else UGK_GO(64);
+#undef UGK_FLAT
 #undef UGK_GO
 #undef UGK_GO2
 #undef UGK_GO3
@@ -611,9 +635,12 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
   UGK_REQUIRE(host_rows == 0 || host, "ugk_extract_mix: null host table with %llu rows",
               (unsigned long long)host_rows);
   const uintptr_t align = (uintptr_t)cache | (uintptr_t)host | (uintptr_t)out | (uintptr_t)row_bytes;
-  UGK_REQUIRE(row_bytes > 0 && align % 16 == 0,
-              "ugk_extract_mix: rows and buffers must be multiples of 16 bytes (row_bytes=%zu)", row_bytes);
-  const uint32_t vpr = (uint32_t)(row_bytes / 16);
+  UGK_REQUIRE(row_bytes > 0 && row_bytes <= (1u << 30), "ugk_extract_mix: row_bytes %zu out of range", row_bytes);
+  const bool flat = align % 16 != 0;
+  UGK_REQUIRE(!flat || (flat_row_ok(align, row_bytes) && !stage),
+              "ugk_extract_mix: rows and buffers must be multiples of 16 bytes, or without a stage of 4 bytes with rows "
+              "of at least %u (row_bytes=%zu)",
+              kFlatMinBytes, row_bytes);
   if (stage) {
     UGK_REQUIRE(stage->rows_dev && stage->owner_dev, "ugk_extract_mix_staged: null stage");
     UGK_REQUIRE(((stage->mask + 1) & stage->mask) == 0, "ugk_extract_mix_staged: the stage needs a power of two of entries");
@@ -622,13 +649,13 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
                 "ugk_extract_mix_staged: misaligned stage");
   }
   if (t.kind == 1)
-    return extract_mix_lpr<K, 1>(t, keys, n, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror,
-                                 counts, num_groups, others_hint, stage, as_stream(stream));
+    return extract_mix_lpr<K, 1>(t, keys, n, cache, cache_rows, host, host_rows, out, row_bytes, flat, status,
+                                 host_mirror, counts, num_groups, others_hint, stage, as_stream(stream));
   if (t.kind == 2)
-    return extract_mix_lpr<K, 2>(t, keys, n, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror,
-                                 counts, num_groups, others_hint, stage, as_stream(stream));
-  return extract_mix_lpr<K, 3>(t, keys, n, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror,
-                               counts, num_groups, others_hint, stage, as_stream(stream));
+    return extract_mix_lpr<K, 2>(t, keys, n, cache, cache_rows, host, host_rows, out, row_bytes, flat, status,
+                                 host_mirror, counts, num_groups, others_hint, stage, as_stream(stream));
+  return extract_mix_lpr<K, 3>(t, keys, n, cache, cache_rows, host, host_rows, out, row_bytes, flat, status,
+                               host_mirror, counts, num_groups, others_hint, stage, as_stream(stream));
 }
 
 // The workspace is laid out by its own size, not by the batch's: `cap` slot words, then cap / 2 words of unique ids by
