@@ -172,8 +172,8 @@ int ugk_copy_rows(void *dst_dev, const void *src_dev, size_t nbytes, void *strea
  * out[dst(i), :] = src[srcrow(i), :] for row_bytes bytes.  max_blocks = 0 lets the kernel fill the
  * chip; a non-zero value caps the grid (the reference's limit_block / per-source SM budget). */
 /* Where the rows an extraction writes go next, for the launches the calling thread makes from now on (the gathers and
- * ugk_extract_mix_*).  UGK_OUTPUT_AUTO: decided by size — an output of up to 192 MB is written with ordinary stores and
- * stays in the 256 MB memory-side cache for its consumer, a larger one with non-temporal stores.  UGK_OUTPUT_STREAMS:
+ * ugk_extract_mix_*).  UGK_OUTPUT_AUTO: decided by size — an output of up to 256 MiB is written with ordinary stores and
+ * stays in the 256 MiB memory-side cache for its consumer, a larger one with non-temporal stores.  UGK_OUTPUT_STREAMS:
  * non-temporal stores whatever the size (a caller that rotates its outputs over more buffers than the cache holds: the
  * rows of one launch are evicted by the next anyway, and evicting them costs more than streaming them, 51.4 us against
  * 47.5 us for 262,144 rows of 512 bytes).  UGK_OUTPUT_STAYS: ordinary stores whatever the size.  Never a byte of the

@@ -793,7 +793,7 @@ void ExtractSession::NoteOutput(const void *output, size_t nbytes) {
       for (int j = 0; j < i && !seen; j++) seen = _out_ptr[j] == _out_ptr[i];
       if (!seen) distinct += _out_bytes[i];
     }
-    hint = distinct > ((size_t)192 << 20) ? UGK_OUTPUT_STREAMS : UGK_OUTPUT_AUTO;
+    hint = distinct > ((size_t)256 << 20) ? UGK_OUTPUT_STREAMS : UGK_OUTPUT_AUTO;
   }
   // the hint is a thread's own in the kernel library: set it on every call that may come from another thread than
   // the last one did, which costs a store

@@ -8,7 +8,7 @@
 //     launch uses many small workgroups of one pass each:
 //     measured on MI355X this beats deeper unrolling with fewer, longer-lived workgroups by ~15 %;
 //   * loads carry the non-temporal hint (table rows are touched once); stores are ordinary write-back stores
-//     while the output fits the 256 MB memory-side cache, so the consumer finds it there, and non-temporal
+//     while the output fits the 256 MiB memory-side cache, so the consumer finds it there, and non-temporal
 //     beyond that or when the caller says its outputs do not stay there (ugk_set_output_hint);
 //   * the grid has one workgroup per pass of rows, or is capped by the caller so a host-link gather occupies
 //     only a few CUs while the HBM gather runs next to it (then the workgroups stride over the batch);
@@ -566,7 +566,7 @@ bool nt_store_for(size_t out_bytes) {
   if (forced >= 0) return forced != 0;
   if (g_output_hint == UGK_OUTPUT_STREAMS) return true;
   if (g_output_hint == UGK_OUTPUT_STAYS) return false;
-  return out_bytes > ((size_t)192 << 20);
+  return out_bytes > kMemorySideCacheBytes;
 }
 // an empty launch: what it costs is the load of this file's code object onto the device (see ugk_preload_kernels)
 namespace {

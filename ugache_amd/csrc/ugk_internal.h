@@ -46,9 +46,13 @@ static inline unsigned clamp_grid(size_t want, unsigned max_blocks) {
   return (unsigned)want;
 }
 
-// Non-temporal stores for an extraction whose output of `out_bytes` will not stay in the 256 MB memory-side cache
+// Non-temporal stores for an extraction whose output of `out_bytes` will not stay in the 256 MiB memory-side cache
 // anyway; ordinary write-back stores otherwise, so that the consumer finds the rows there.  The caller's hint
-// (ugk_set_output_hint) and UGK_GATHER_NT_STORE=0/1 override the size rule.
+// (ugk_set_output_hint) and UGK_GATHER_NT_STORE=0/1 override the size rule.  The line is the cache's size to the megabyte;
+// gathers into one buffer, ordinary / non-temporal stores, us: 512-byte rows, output of 192 MiB 63.9 / 70.2, 224 MiB 72.8 /
+// 81.2, 256 MiB 83.7 / 92.0, 288 MiB 112.5 / 103.4; 128-byte rows 256 MiB 89.3 / 94.0, 288 MiB 114.1 / 105.1; 1204-byte
+// rows 256 MiB 89.5 / 105.5, 288 MiB 120.9 / 118.0.
+constexpr size_t kMemorySideCacheBytes = (size_t)256 << 20;
 bool nt_store_for(size_t out_bytes);
 
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
