@@ -977,6 +977,58 @@ def test_pooled_extraction_matches_a_float64_segment_sum(kind, dim, etype, rows_
         words.free()
 
 
+@pytest.mark.parametrize("kind", ["none", "flat"])
+@pytest.mark.parametrize("vpr", [1, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256])
+def test_pooled_extraction_at_the_edges_of_its_shapes(kind, vpr):
+    """Rows of vpr 16-byte vectors around the sizes where the lanes per row and the chunks per lane change, with 1, 2, 5,
+    9 and 40 ids per sample on average (the rows in flight change between them), fp32 and fp16: mean over weights in
+    [0.5, 1.5], against the float64 segment mean.  n terms added in fp32 are off by at most (n + 2) 2^-24 of their
+    magnitudes, twice that with the sum of weights, n <= 80: 1e-5; an fp16 result is rounded to 2^-11 on top."""
+    rng = np.random.default_rng(vpr)
+    nkeys, rb = 3_000, vpr * 16
+    cached = rng.choice(nkeys, nkeys // 2, replace=False).astype(np.int64)
+    for dt in (np.float32, np.float16):
+        dim = rb // np.dtype(dt).itemsize
+        host = rng.standard_normal((nkeys, dim)).astype(dt)
+        pin = pinned_from(host.view(np.uint8).reshape(nkeys, rb))
+        try:
+            if kind == "none":
+                mem, tb, cache = None, hip.table(0, None, 0), np.zeros((1, rb), np.uint8)
+            else:
+                mem, tb = _make_flat(nkeys)
+                slots = rng.permutation(len(cached)).astype(np.uint32)
+                cache = np.zeros((len(cached), rb), np.uint8)
+                cache[slots] = host.view(np.uint8).reshape(nkeys, rb)[cached]
+                assert _insert(tb, cached, slots) == 0
+            st, d_cache = dev_zeros_u32(1), to_dev(cache)
+            for most in (1, 3, 9, 17, 80):
+                n_rows = 259
+                lens = rng.integers(1 if most < 80 else 0, most + 1, size=n_rows)
+                seg_off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+                nnz = int(seg_off[-1])
+                ids = rng.integers(0, nkeys, size=nnz).astype(np.int64)
+                wts = (rng.random(nnz) + 0.5).astype(np.float32)
+                d_ids, d_off, d_w = to_dev(ids), to_dev(seg_off), to_dev(wts)
+                out = dev_bytes(n_rows * rb + 64, fill=0x7F)
+                hip.call("ugk_extract_pool_i64", tb, ptr(d_ids), ptr(d_off), ptr(d_w), n_rows, nnz, 1,
+                         np.dtype(dt).itemsize, ptr(d_cache), 0 if kind == "none" else len(cached), pin.ptr, nkeys,
+                         ptr(out), rb, ptr(st), None, None, None, None)
+                sync()
+                assert status_value(st) == 0
+                raw = to_np(out)
+                assert (raw[n_rows * rb:n_rows * rb + 64] == 0x7F).all()
+                got = raw[: n_rows * rb].view(dt).reshape(n_rows, dim).astype(np.float64)
+                f64 = host.astype(np.float64)
+                want = _pool_reference(f64, ids, seg_off, wts, 1)
+                bound = 1e-5 * _pool_reference(np.abs(f64), ids, seg_off, wts, 1) + 1e-30
+                if dt == np.float16:
+                    bound = bound + 2.0 ** -11 * np.abs(want) + 2.0 ** -25
+                assert (np.abs(got - want) <= bound).all(), (dt, most)
+        finally:
+            sync()
+            pin.free()
+
+
 @pytest.mark.parametrize("rows_per_group", ["", "2", "8"])
 def test_pooled_extraction_hand_worked(rows_per_group, monkeypatch):
     if rows_per_group:

@@ -72,13 +72,20 @@ struct PoolElem<__half> {
   }
 };
 
-constexpr int kPoolChunks = 4;  // 16-byte chunks of a row a lane may own: rows of up to LPR x 64 bytes
+constexpr int kPoolChunks = 4;  // 16-byte chunks of a row a lane may own at most: rows of up to LPR x 64 bytes
 
+// Bound by the host link where rows are missing from the cache (65,536 samples of 16 ids over rows of 512 bytes, 2.6 %
+// of them over the link: 280 us, 51 GB/s of link; 398 us before), else by the lines of the rows.  What decides is how
+// many rows are on their way at once and that no load waits for another: a lane reads its CH chunks of U ids before it
+// adds the first of them (a row of the host table whose chunks were read one after the other cost its wavefront CH
+// round trips over the link), and CH and U are template parameters so that short rows do not pay for the registers of
+// long ones.  The loads are ordinary ones: ids repeat in real batches, and the hot rows stay in L2 (1 M ids, Zipf 1.2,
+// all in HBM: 87 us with non-temporal loads, 66 with ordinary ones; uniform ids 121 / 122).
 // CLIP: every looked-up row is clipped to the l2 norm max_norm before it is weighted (clip_by_norm over the row:
 // x * max_norm / max(||x||, max_norm)).  The whole row has to be seen before any of it can be added, so the chunks of
 // the U rows in flight are held in registers (up to 64 more than without), the squares summed per row over the lanes
 // of the group, and the row's weight scaled; a kernel of its own, so that the plain combination keeps its registers.
-template <typename K, int KIND, int LPR, typename E, bool CLIP>
+template <typename K, int KIND, int LPR, int CH, int U, typename E, bool CLIP>
 __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, const K *__restrict__ ids,
                                                               const long long *__restrict__ seg_off,
                                                               const float *__restrict__ weights, size_t n_rows,
@@ -90,7 +97,6 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
                                                               unsigned long long *counts) {
   constexpr int RPW = kWave / LPR;  // output rows per wavefront and pass
   constexpr int EPC = PoolElem<E>::kPerChunk;
-  constexpr int U = 4;  // rows in flight per lane group
   static_assert(LPR % U == 0, "ids are taken in rounds of U");
   __shared__ uint32_t block_tot[2];
   if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
@@ -116,12 +122,15 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
       atomicOr(status, UGK_ST_BAD_SEGMENT);
       if (host_mirror) host_mirror[0] = UGK_ST_BAD_SEGMENT;
     }
-    float acc[kPoolChunks][EPC];
+    float acc[CH][EPC];
 #pragma unroll
-    for (int c = 0; c < kPoolChunks; ++c)
+    for (int c = 0; c < CH; ++c)
 #pragma unroll
       for (int e = 0; e < EPC; ++e) acc[c][e] = 0.f;
-    float wsum = 0.f;  // this lane's share of the row's sum of weights (or of their squares)
+    // this lane's share of the row's sum of weights (or of their squares); with four lanes the rounds alternate between
+    // two sums, so that the weights are added in the order in which eight lanes add them
+    float wsum = 0.f, wsum_odd = 0.f;
+    bool odd = false;
     for (long long j0 = beg; __ballot(j0 < end) != 0ull; j0 += LPR) {  // until every group of the wavefront is through
       const long long j = j0 + sub;
       const bool active = j < end;
@@ -134,7 +143,10 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
       }
       const bool use = active && row.has_row;  // a key without a row adds nothing (the launch is flagged)
       const float w = use ? (weights ? weights[j] : 1.f) : 0.f;
-      wsum += combiner == 2 ? w * w : w;
+      const float wterm = combiner == 2 ? w * w : w;
+      if (LPR == 4 && odd) wsum_odd += wterm;
+      else wsum += wterm;
+      odd = !odd;
       for (int s0 = 0; s0 < LPR; s0 += U) {
         if (__ballot(active && sub >= s0) == 0ull) break;  // no group has an id left in this round
         grow_t p[U];
@@ -148,18 +160,18 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
           ok[u] = __shfl((int)use, src) != 0;
         }
         if constexpr (CLIP) {
-          u32x4 v[kPoolChunks][U];
+          u32x4 v[CH][U];
           float ss[U];
 #pragma unroll
           for (int u = 0; u < U; ++u) ss[u] = 0.f;
 #pragma unroll
-          for (int c = 0; c < kPoolChunks; ++c) {
+          for (int c = 0; c < CH; ++c) {
             const uint32_t col = (uint32_t)c * LPR + sub;
 #pragma unroll
             for (int u = 0; u < U; ++u) v[c][u] = col < vpr ? __builtin_nontemporal_load(p[u] + col) : u32x4{0, 0, 0, 0};
           }
 #pragma unroll
-          for (int c = 0; c < kPoolChunks; ++c) {
+          for (int c = 0; c < CH; ++c) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
               float x[EPC];
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
             wv[u] *= max_norm / fmaxf(sqrtf(ss[u]), max_norm);
           }
 #pragma unroll
-          for (int c = 0; c < kPoolChunks; ++c) {
+          for (int c = 0; c < CH; ++c) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
               float x[EPC];
@@ -187,17 +199,23 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
             }
           }
         } else {
+          u32x4 v[CH][U];
 #pragma unroll
-          for (int c = 0; c < kPoolChunks; ++c) {
+          for (int c = 0; c < CH; ++c) {
             const uint32_t col = (uint32_t)c * LPR + sub;
             if (col < vpr) {
-              u32x4 v[U];
 #pragma unroll
-              for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u] + col);
+              for (int u = 0; u < U; ++u) v[c][u] = p[u][col];
+            }
+          }
+#pragma unroll
+          for (int c = 0; c < CH; ++c) {
+            const uint32_t col = (uint32_t)c * LPR + sub;
+            if (col < vpr) {
 #pragma unroll
               for (int u = 0; u < U; ++u) {
                 float x[EPC];
-                PoolElem<E>::unpack(v[u], x, bf16);
+                PoolElem<E>::unpack(v[c][u], x, bf16);
                 if (ok[u]) {
 #pragma unroll
                   for (int e = 0; e < EPC; ++e) acc[c][e] = fmaf(wv[u], x[e], acc[c][e]);
@@ -209,12 +227,13 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
       }
     }
     // the row's denominator: every lane of the group holds a share
+    if (LPR == 4) wsum += wsum_odd;
 #pragma unroll
     for (int d = LPR / 2; d > 0; d >>= 1) wsum += __shfl_xor(wsum, d);
     const float denom = combiner == 1 ? wsum : combiner == 2 ? sqrtf(wsum) : 1.f;
     if (row_ok) {
 #pragma unroll
-      for (int c = 0; c < kPoolChunks; ++c) {
+      for (int c = 0; c < CH; ++c) {
         const uint32_t col = (uint32_t)c * LPR + sub;
         if (col < vpr) {
           float y[EPC];
@@ -235,10 +254,11 @@ constexpr int kPoolMaxRows = 8;  // output rows a lane group may own per pass
 // seg_start is <= f.  The lanes resolve LPR positions at a time; the rows behind them are then read U at a time
 // whatever segments they belong to and added in the order of the list, an output row being written when the list
 // moves on to a later one.  What keeps memory busy is then the number of ids, not the shape of the segments: with one
-// row per group a sample of one or two ids leaves most of the group's lookups and loads unused (262,144 samples of
-// one id: 84 us per call with one row per group, 70 us with four).  The bookkeeping costs registers (three
-// wavefronts per SIMD instead of four), which is why samples of more ids stay with the kernel above (65,536 samples
-// of 16 ids: 121 us here, 114 us there).
+// row per group a sample of one id leaves most of the group's lookups and loads unused.  The bookkeeping costs
+// registers (three wavefronts per SIMD instead of four) and a lane's chunks are read one after the other, so this is
+// for ids without a table only, where no row comes over the host link: samples of one id over rows of 512 bytes, all in
+// HBM, 115 us for 390,625 of them against 124 with one row per group; 60 % of the table uncached, 262,144 of them, 123
+// against 98 us.
 template <typename K, int KIND, int LPR, typename E>
 __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t, const K *__restrict__ ids,
                                                               const long long *__restrict__ seg_off,
@@ -349,7 +369,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
           if (col < vpr) {
             u32x4 v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u] + col);
+            for (int u = 0; u < U; ++u) v[u] = p[u][col];
             int cc = cur;  // every chunk walks the same ids from the same state
             float ws = wsum;
 #pragma unroll
@@ -396,54 +416,96 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
                      const void *cache, uint64_t cache_rows, const void *host, uint64_t host_rows, void *out,
                      uint32_t vpr, uint64_t nnz, int combiner, bool bf16, float max_norm, uint32_t *status,
                      uint32_t *host_mirror, uint64_t *counts, uint32_t *num_groups, hipStream_t st) {
-  // Lanes per output row: rows of up to 512 bytes go to 8 lanes of up to four chunks each (eight lane groups per
-  // wavefront; with 32 lanes and two groups 65,536 samples of 16 ids took 123 us instead of 112 us), rows of up to
-  // 2 KB to 32 lanes, longer ones to 64.
-  int lpr = vpr <= 8 * kPoolChunks ? 8 : vpr <= 32 * kPoolChunks ? 32 : 64;
+  // Lanes per output row, chunks per lane and ids in flight (LPR, CH, U).  The fewest lanes that hold a row with the
+  // fewest registers are best for few ids per sample (a lane group resolves LPR ids at a time and keeps U rows on
+  // their way, and both are wasted on a sample that has fewer), more lanes and more rows in flight for many.  us per
+  // call, rows in HBM, Zipf 1.05, about 400,000 ids (200,000 of 1 KB, 100,000 of 2 KB), by ids per sample:
+  //   64 B    (8,4,4) / (4,1,2) / (4,1,4):              2 ids 76 / 34 / 38,  4: 65 / 33 / 35,  8: 41 / 29 / 29,
+  //                                                     40: 37 / 41 / 37;  1 id 43 with (4,1,2), 51 with (4,1,4)
+  //   128 B   (8,4,4) / (8,1,2) / (8,1,4):              2 ids 68 / 41 / 42,  4: 58 / 40 / 38,  40: 34 / 41 / 33
+  //   256 B   (8,4,4) / (8,2,2) / (16,2,4):             2 ids 73 / 45 / 82,  8: 42 / 36 / 43,  40: 39 / 42 / 34
+  //   512 B   (8,4,4) / (8,4,2) / (16,2,2) / (16,2,4):  2 ids 93 / 74 / 82 / 100,  4: 80 / 75 / 77 / 84,
+  //                                                     8: 49 / 46 / 47 / 49,  40: 48 / 57 / 44 / 40
+  //   512 B of two-byte elements, the same:             2 ids 68 / 61 / 54 / 67,  8: 43 / 45 / 38 / 39,
+  //                                                     40: 53 / 63 / 45 / 41
+  //   1 KB    (32,4,4) / (16,4,2) / (32,2,4):           2 ids 130 / 72 / 97,  8: 57 / 47 / 49,  40: 49 / 56 / 39
+  //   2 KB    (32,4,4) / (32,4,2):                      2 ids 91 / 68,  8: 49 / 44,  40: 46 / 41
+  // and with 512-byte rows over the host link among them, (8,4,4) / (8,4,2) / (16,2,4): 4 ids 115 / 110 / 89, 16 ids
+  // 394 / 387 / 279.
+  const uint64_t rows64 = n_rows;
+  const bool upto2 = nnz <= rows64 * 5 / 2, upto6 = nnz <= rows64 * 6, upto12 = nnz <= rows64 * 12;
+  const bool clip = max_norm > 0.f;
+  int shape;
+  if (clip) shape = vpr <= 32 ? 844 : vpr <= 128 ? 3244 : 6444;
+  else if (vpr <= 4) shape = upto6 ? 412 : 414;
+  else if (vpr <= 8) shape = 814;
+  else if (vpr <= 16) shape = upto12 ? 822 : 1624;
+  else if (vpr <= 32) shape = upto2 && sizeof(E) == 4 ? 842 : upto12 ? 1622 : 1624;
+  else if (vpr <= 64) shape = upto12 ? 1642 : 3224;
+  else if (vpr <= 128) shape = 3242;
+  else shape = 6442;
   if (const char *forced = getenv("UGK_POOL_LPR")) {  // for sweeps; never a byte of the result depends on it
     const int v = atoi(forced);
-    if ((v == 8 || v == 32 || v == 64) && vpr <= (uint32_t)v * kPoolChunks) lpr = v;
+    if (!clip && (v == 8 || v == 32 || v == 64) && vpr <= (uint32_t)v * kPoolChunks) shape = v * 100 + 42;
   }
-  // Output rows per lane group and pass.  One row each (extract_pool_kernel) is the faster kernel from two ids per
-  // sample on (it needs fewer registers: four wavefronts per SIMD instead of three; at two ids the two are level);
-  // for samples of mostly one id a group takes four rows as one list (extract_pool_rows_kernel), as long as the
-  // launch still has wavefronts for every CU.
-  const int groups_per_wave = kWave / lpr;
-  int rows = n_rows && nnz <= (uint64_t)n_rows + n_rows / 2 ? 4 : 1;
-  const size_t enough_waves = (size_t)cu_count() * 8;
-  while (rows > 1 && n_rows / ((size_t)rows * groups_per_wave) < enough_waves) rows /= 2;
-  if (const char *forced = getenv("UGK_POOL_ROWS")) {  // for sweeps, like the one above
-    const int v = atoi(forced);
-    if (v >= 1 && v <= kPoolMaxRows) rows = v;
+  // Output rows per lane group and pass: one, but four as one list (extract_pool_rows_kernel) for samples of mostly one
+  // id that need no table, as long as the launch still has wavefronts for every CU.  Rows of up to 64 and of 129 to 256
+  // bytes are faster with one all the same (43 / 60 and 68 / 74 us for 400,000 samples).
+  int rows = 1;
+  if constexpr (KIND == 0) {
+    const int lanes = vpr <= 32 ? 8 : vpr <= 128 ? 32 : 64;
+    const int groups = kWave / lanes;
+    if (n_rows && nnz <= rows64 + rows64 / 2 && vpr > 4 && (vpr <= 8 || vpr > 16)) rows = 4;
+    const size_t enough_waves = (size_t)cu_count() * 8;
+    while (rows > 1 && n_rows / ((size_t)rows * groups) < enough_waves) rows /= 2;
+    if (const char *forced = getenv("UGK_POOL_ROWS")) {  // for sweeps, like the one above
+      const int v = atoi(forced);
+      if (v >= 1 && v <= kPoolMaxRows) rows = v;
+    }
+    if (nnz >= ((uint64_t)1 << 28) || clip) rows = 1;  // the list is counted in 32 bits; clipping lives in the other kernel
+    if (rows > 1) {
+      const size_t rows_per_block = (size_t)rows * groups * kWavesPerBlock;
+      const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
+      if (num_groups) *num_groups = grid;
+#define UGK_POOL_ROWS_GO(L)                                                                                            \
+  hipLaunchKernelGGL((extract_pool_rows_kernel<K, KIND, L, E>), dim3(grid), dim3(kBlock), 0, st, t, ids, seg_off,      \
+                     weights, n_rows, (long long)nnz, rows, (const u32x4 *)cache, cache_rows, (const u32x4 *)host,     \
+                     host_rows, (u32x4 *)out, vpr, combiner, bf16, status, host_mirror,                                \
+                     reinterpret_cast<unsigned long long *>(counts))
+      if (lanes == 8) UGK_POOL_ROWS_GO(8);
+      else if (lanes == 32) UGK_POOL_ROWS_GO(32);
+      else UGK_POOL_ROWS_GO(64);
+#undef UGK_POOL_ROWS_GO
+      UGK_HIP(hipGetLastError());
+      return 0;
+    }
   }
-  if (nnz >= ((uint64_t)1 << 28)) rows = 1;  // the list of a group is counted in 32 bits
-  const bool clip = max_norm > 0.f;
-  if (clip) rows = 1;  // clipping lives in the kernel of one output row per lane group
-  const size_t rows_per_block = (size_t)rows * groups_per_wave * kWavesPerBlock;
+  const size_t rows_per_block = (size_t)(kWave / (shape / 100)) * kWavesPerBlock;
   const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
   if (num_groups) *num_groups = grid;
-#define UGK_POOL(L)                                                                                                    \
-  if (clip)                                                                                                            \
-    hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, E, true>), dim3(grid), dim3(kBlock), 0, st, t, ids, seg_off,   \
-                       weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows, (const u32x4 *)host,         \
-                       host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status, host_mirror,                    \
-                       reinterpret_cast<unsigned long long *>(counts));                                                \
-  else if (rows == 1)                                                                                                  \
-    hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, E, false>), dim3(grid), dim3(kBlock), 0, st, t, ids, seg_off,  \
-                       weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows, (const u32x4 *)host,         \
-                       host_rows, (u32x4 *)out, vpr, combiner, bf16, 0.f, status, host_mirror,                         \
-                       reinterpret_cast<unsigned long long *>(counts));                                                \
-  else                                                                                                                 \
-    hipLaunchKernelGGL((extract_pool_rows_kernel<K, KIND, L, E>), dim3(grid), dim3(kBlock), 0, st, t, ids, seg_off,    \
-                       weights, n_rows, (long long)nnz, rows, (const u32x4 *)cache, cache_rows, (const u32x4 *)host,   \
-                       host_rows, (u32x4 *)out, vpr, combiner, bf16, status, host_mirror,                              \
-                       reinterpret_cast<unsigned long long *>(counts))
-  if (lpr == 8) {
-    UGK_POOL(8);
-  } else if (lpr == 32) {
-    UGK_POOL(32);
-  } else {
-    UGK_POOL(64);
+#define UGK_POOL(L, CH, U, CLIP)                                                                                       \
+  case L * 100 + CH * 10 + U:                                                                                          \
+    hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, CH, U, E, CLIP>), dim3(grid), dim3(kBlock), 0, st, t, ids,     \
+                       seg_off, weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows,                     \
+                       (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status,            \
+                       host_mirror, reinterpret_cast<unsigned long long *>(counts));                                   \
+    break
+  switch (shape) {
+    UGK_POOL(4, 1, 2, false);
+    UGK_POOL(4, 1, 4, false);
+    UGK_POOL(8, 1, 4, false);
+    UGK_POOL(8, 2, 2, false);
+    UGK_POOL(8, 4, 2, false);
+    UGK_POOL(16, 2, 2, false);
+    UGK_POOL(16, 2, 4, false);
+    UGK_POOL(16, 4, 2, false);
+    UGK_POOL(32, 2, 4, false);
+    UGK_POOL(32, 4, 2, false);
+    UGK_POOL(64, 4, 2, false);
+    UGK_POOL(8, 4, 4, true);
+    UGK_POOL(32, 4, 4, true);
+    UGK_POOL(64, 4, 4, true);
+    default: return ugk_set_error("ugk_extract_pool: no kernel of shape %d", shape);
   }
 #undef UGK_POOL
   UGK_HIP(hipGetLastError());
