@@ -79,8 +79,10 @@ constexpr int kPoolChunks = 4;  // 16-byte chunks of a row a lane may own at mos
 // many rows are on their way at once and that no load waits for another: a lane reads its CH chunks of U ids before it
 // adds the first of them (a row of the host table whose chunks were read one after the other cost its wavefront CH
 // round trips over the link), and CH and U are template parameters so that short rows do not pay for the registers of
-// long ones.  The loads are ordinary ones: ids repeat in real batches, and the hot rows stay in L2 (1 M ids, Zipf 1.2,
-// all in HBM: 87 us with non-temporal loads, 66 with ordinary ones; uniform ids 121 / 122).
+// long ones.  The loads are ordinary ones: ids repeat
+// in real batches, and the hot rows stay in L2.  800,000 ids over rows of 512 bytes, all in HBM, us before / now, 4, 8 and
+// 16 ids per sample: Zipf 1.05 104 / 86, 88 / 66, 81 / 61; uniform ids, which reuse nothing, 113 / 125, 105 / 111, 98 /
+// 105; rows of 800 bytes 184 / 129, 147 / 95, 130 / 92 and uniform 197 / 181, 180 / 162, 170 / 152.
 // CLIP: every looked-up row is clipped to the l2 norm max_norm before it is weighted (clip_by_norm over the row:
 // x * max_norm / max(||x||, max_norm)).  The whole row has to be seen before any of it can be added, so the chunks of
 // the U rows in flight are held in registers (up to 64 more than without), the squares summed per row over the lanes
@@ -199,27 +201,24 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
             }
           }
         } else {
+          // No branch around the loads (behind one they would wait for each other): a lane past the end of the row
+          // reads the row's last chunk again, and what it adds up is never written.
           u32x4 v[CH][U];
 #pragma unroll
           for (int c = 0; c < CH; ++c) {
-            const uint32_t col = (uint32_t)c * LPR + sub;
-            if (col < vpr) {
+            const uint32_t col = min((uint32_t)c * LPR + sub, vpr - 1);
 #pragma unroll
-              for (int u = 0; u < U; ++u) v[c][u] = p[u][col];
-            }
+            for (int u = 0; u < U; ++u) v[c][u] = p[u][col];
           }
 #pragma unroll
           for (int c = 0; c < CH; ++c) {
-            const uint32_t col = (uint32_t)c * LPR + sub;
-            if (col < vpr) {
 #pragma unroll
-              for (int u = 0; u < U; ++u) {
-                float x[EPC];
-                PoolElem<E>::unpack(v[c][u], x, bf16);
-                if (ok[u]) {
+            for (int u = 0; u < U; ++u) {
+              float x[EPC];
+              PoolElem<E>::unpack(v[c][u], x, bf16);
+              if (ok[u]) {
 #pragma unroll
-                  for (int e = 0; e < EPC; ++e) acc[c][e] = fmaf(wv[u], x[e], acc[c][e]);
-                }
+                for (int e = 0; e < EPC; ++e) acc[c][e] = fmaf(wv[u], x[e], acc[c][e]);
               }
             }
           }
@@ -255,10 +254,11 @@ constexpr int kPoolMaxRows = 8;  // output rows a lane group may own per pass
 // whatever segments they belong to and added in the order of the list, an output row being written when the list
 // moves on to a later one.  What keeps memory busy is then the number of ids, not the shape of the segments: with one
 // row per group a sample of one id leaves most of the group's lookups and loads unused.  The bookkeeping costs
-// registers (three wavefronts per SIMD instead of four) and a lane's chunks are read one after the other, so this is
-// for ids without a table only, where no row comes over the host link: samples of one id over rows of 512 bytes, all in
-// HBM, 115 us for 390,625 of them against 124 with one row per group; 60 % of the table uncached, 262,144 of them, 123
-// against 98 us.
+// registers (three wavefronts per SIMD instead of four) and a lane's chunks are read one after the other, so it is not
+// for flat tables, behind which rows come over the host link: samples of one id over rows of 512 bytes, all in HBM, 115
+// us for 390,625 of them against 124 with one row per group; 60 % of the table uncached behind a flat table, 262,144 of
+// them, 123 against 98 us; behind a hash table, whose lookup works on all lanes of a wavefront at once and wants them
+// to hold ids, 195,312 of them 107 against 128 us.
 template <typename K, int KIND, int LPR, typename E>
 __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t, const K *__restrict__ ids,
                                                               const long long *__restrict__ seg_off,
@@ -432,6 +432,9 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   //   2 KB    (32,4,4) / (32,4,2):                      2 ids 91 / 68,  8: 49 / 44,  40: 46 / 41
   // and with 512-byte rows over the host link among them, (8,4,4) / (8,4,2) / (16,2,4): 4 ids 115 / 110 / 89, 16 ids
   // 394 / 387 / 279.
+  // (These were taken with a branch around the loads of each chunk; without it the chosen shapes gained another 5 to 25 %,
+  // and (8,4,4) with its chunks one after the other stayed behind them: 64-byte rows aside, it ran at 0.81 to 1.31 of the speed
+  // of the kernel this replaces, the chosen shapes at 0.79 to 1.60, the low ends for uniform ids.)
   const uint64_t rows64 = n_rows;
   const bool upto2 = nnz <= rows64 * 5 / 2, upto6 = nnz <= rows64 * 6, upto12 = nnz <= rows64 * 12;
   const bool clip = max_norm > 0.f;
@@ -449,13 +452,13 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
     if (!clip && (v == 8 || v == 32 || v == 64) && vpr <= (uint32_t)v * kPoolChunks) shape = v * 100 + 42;
   }
   // Output rows per lane group and pass: one, but four as one list (extract_pool_rows_kernel) for samples of mostly one
-  // id that need no table, as long as the launch still has wavefronts for every CU.  Rows of up to 64 and of 129 to 256
-  // bytes are faster with one all the same (43 / 60 and 68 / 74 us for 400,000 samples).
+  // id without a flat table (see there), as long as the launch still has wavefronts for every CU.  Rows of up to 64 bytes
+  // without any table are faster with one all the same (43 / 60 us for 400,000 samples).
   int rows = 1;
-  if constexpr (KIND == 0) {
+  if constexpr (KIND != 1) {
     const int lanes = vpr <= 32 ? 8 : vpr <= 128 ? 32 : 64;
     const int groups = kWave / lanes;
-    if (n_rows && nnz <= rows64 + rows64 / 2 && vpr > 4 && (vpr <= 8 || vpr > 16)) rows = 4;
+    if (n_rows && nnz <= rows64 + rows64 / 2 && (KIND != 0 || vpr > 4)) rows = 4;
     const size_t enough_waves = (size_t)cu_count() * 8;
     while (rows > 1 && n_rows / ((size_t)rows * groups) < enough_waves) rows /= 2;
     if (const char *forced = getenv("UGK_POOL_ROWS")) {  // for sweeps, like the one above
@@ -483,31 +486,31 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   const size_t rows_per_block = (size_t)(kWave / (shape / 100)) * kWavesPerBlock;
   const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
   if (num_groups) *num_groups = grid;
+  bool launched = false;
 #define UGK_POOL(L, CH, U, CLIP)                                                                                       \
-  case L * 100 + CH * 10 + U:                                                                                          \
-    hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, CH, U, E, CLIP>), dim3(grid), dim3(kBlock), 0, st, t, ids,     \
-                       seg_off, weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows,                     \
-                       (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status,            \
-                       host_mirror, reinterpret_cast<unsigned long long *>(counts));                                   \
-    break
-  switch (shape) {
-    UGK_POOL(4, 1, 2, false);
-    UGK_POOL(4, 1, 4, false);
-    UGK_POOL(8, 1, 4, false);
-    UGK_POOL(8, 2, 2, false);
-    UGK_POOL(8, 4, 2, false);
-    UGK_POOL(16, 2, 2, false);
-    UGK_POOL(16, 2, 4, false);
-    UGK_POOL(16, 4, 2, false);
-    UGK_POOL(32, 2, 4, false);
-    UGK_POOL(32, 4, 2, false);
-    UGK_POOL(64, 4, 2, false);
-    UGK_POOL(8, 4, 4, true);
-    UGK_POOL(32, 4, 4, true);
-    UGK_POOL(64, 4, 4, true);
-    default: return ugk_set_error("ugk_extract_pool: no kernel of shape %d", shape);
+  if (shape == L * 100 + CH * 10 + U && clip == CLIP) {                                                                \
+    launched = true;                                                                                                   \
+    hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, CH, U, E, CLIP>), dim3(grid), dim3(kBlock), 0, st, t, ids,       \
+                     seg_off, weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows, (const u32x4 *)host,  \
+                     host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status, host_mirror,                      \
+                     reinterpret_cast<unsigned long long *>(counts));                                                \
   }
+  UGK_POOL(4, 1, 2, false)
+  UGK_POOL(4, 1, 4, false)
+  UGK_POOL(8, 1, 4, false)
+  UGK_POOL(8, 2, 2, false)
+  UGK_POOL(16, 2, 4, false)
+  UGK_POOL(8, 4, 4, true)
+  UGK_POOL(32, 4, 4, true)
+  UGK_POOL(64, 4, 4, true)
+  UGK_POOL(8, 4, 2, false)
+  UGK_POOL(16, 2, 2, false)
+  UGK_POOL(16, 4, 2, false)
+  UGK_POOL(32, 2, 4, false)
+  UGK_POOL(32, 4, 2, false)
+  UGK_POOL(64, 4, 2, false)
 #undef UGK_POOL
+  UGK_REQUIRE(launched, "ugk_extract_pool: no kernel of shape %d", shape);
   UGK_HIP(hipGetLastError());
   return 0;
 }
