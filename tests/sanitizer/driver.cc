@@ -12,6 +12,8 @@
 // host table, so a refresh that reused a slot too early is also seen as a wrong row.
 //
 // usage: driver <FLAT|HASH> <host|device> [lookup steps per phase, default 150]
+// DRIVER_TABLE_SHIFT=n: the host table begins n bytes behind a 64-byte boundary (pooled lookups, which want whole 16-byte
+// vectors, are left out where n is no multiple of 16)
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
@@ -66,10 +68,14 @@ int main(int argc, char **argv) {
   const char *keys[] = {"cache_percentage", "_cache_policy", "num_device", "num_global_step_per_epoch", "num_epoch",
                         "num_total_item",   "omp_thread_num"};
   const char *vals[] = {"0.25", "13", "1", "10", "1", "20000", "4"};
+  const char *shift_text = getenv("DRIVER_TABLE_SHIFT");
+  const size_t table_shift = shift_text ? (size_t)atoi(shift_text) : 0;
+  const bool pooled_too = table_shift % 16 == 0;
   long bad_rows = 0;
   for (int round = 0; round < 2; ++round) {
     coll_cache_config(keys, vals, 7);
-    float *table = static_cast<float *>(coll_cache_alloc_host_table(kRows * kDim * sizeof(float)));
+    char *table_mem = static_cast<char *>(coll_cache_alloc_host_table(kRows * kDim * sizeof(float) + table_shift));
+    float *table = reinterpret_cast<float *>(table_mem + table_shift);
     for (size_t r = 0; r < kRows; ++r)
       for (size_t c = 0; c < kDim; ++c) table[r * kDim + c] = cell(r, c);
     std::mt19937_64 g(17 + round);
@@ -90,12 +96,13 @@ int main(int argc, char **argv) {
         std::this_thread::sleep_for(std::chrono::milliseconds(2));
       }
     });
-    std::vector<float> out(4096 * kDim);
+    std::vector<float> out(4096 * kDim + 1);
     for (int step = 0; step < steps || refreshes.load() < 3; ++step) {
       auto k = skewed_keys(g, 1 + g() % 4096, (uint64_t)step * 97);
       if (!on_device) coll_cache_record(0, k.data(), k.size());
-      coll_cache_lookup(0, k.data(), k.size(), out.data(), nullptr);
-      bad_rows += check_rows(table, out.data(), k.data(), k.size());
+      float *to = out.data() + (step & 1);  // every other output starts at a 4-byte boundary only
+      coll_cache_lookup(0, k.data(), k.size(), to, nullptr);
+      bad_rows += check_rows(table, to, k.data(), k.size());
       if (step > 100 * steps) break;
     }
     stop.store(true);
@@ -108,13 +115,13 @@ int main(int argc, char **argv) {
       std::vector<std::vector<float>> outs;
       for (int b = 0; b < 8; ++b) {
         batches.push_back(skewed_keys(g, 2048, 5000 + b));
-        outs.emplace_back(2048 * kDim);
+        outs.emplace_back(2048 * kDim + 1);
       }
       for (int b = 0; b < 8; ++b)
-        coll_cache_lookup_async(0, batches[b].data(), batches[b].size(), outs[b].data(), nullptr);
+        coll_cache_lookup_async(0, batches[b].data(), batches[b].size(), outs[b].data() + (b & 1), nullptr);
       coll_cache_lookup_wait(0, nullptr);
       one_refresh.join();
-      for (int b = 0; b < 8; ++b) bad_rows += check_rows(table, outs[b].data(), batches[b].data(), batches[b].size());
+      for (int b = 0; b < 8; ++b) bad_rows += check_rows(table, outs[b].data() + (b & 1), batches[b].data(), batches[b].size());
     }
 
     // 3. wide keys, the distinct-keys lookup, a foreground refresh
@@ -146,7 +153,7 @@ int main(int argc, char **argv) {
       bad_rows += check_rows(table, out.data(), k.data(), k.size());
     }
     // 5. pooled lookups (segments of ids combined per sample): plain, as steps of the serving loop, stream-ordered
-    for (int step = 0; step < 8; ++step) {
+    for (int step = 0; pooled_too && step < 8; ++step) {
       auto k = skewed_keys(g, 2000, 20000 + (uint64_t)step * 31);
       std::vector<int64_t> off(1, 0);
       while ((size_t)off.back() < k.size()) off.push_back(std::min<int64_t>((int64_t)k.size(), off.back() + (int64_t)(g() % 6)));
@@ -201,14 +208,15 @@ int main(int argc, char **argv) {
       coll_cache_forward_join();  // the foreground refresh below must not meet one of the serving loop's
       if (ugk_model_capture_begin(caller_stream) != 0) return 1;
       coll_cache_lookup_async(0, k.data(), k.size(), plain.data(), caller_stream);
-      coll_cache_lookup_pooled_async(0, k.data(), off.data(), nullptr, off.size() - 1, k.size(), 0, 4, pooled.data(),
-                                     caller_stream);
+      if (pooled_too)
+        coll_cache_lookup_pooled_async(0, k.data(), off.data(), nullptr, off.size() - 1, k.size(), 0, 4, pooled.data(),
+                                       caller_stream);
       coll_cache_forward_async(0, k.data(), k.size(), step_out.data(), caller_stream);
       if (ugk_model_capture_end(caller_stream, &graph) != 0) return 1;
       coll_cache_lookup_wait(0, caller_stream);
       bad_rows += check_rows(table, plain.data(), k.data(), k.size());
       bad_rows += check_rows(table, step_out.data(), k.data(), k.size());
-      for (size_t r = 0; r + 1 < off.size(); ++r)
+      for (size_t r = 0; pooled_too && r + 1 < off.size(); ++r)
         for (size_t c = 0; c < kDim; ++c) {
           double sum = 0;
           for (int64_t j = off[r]; j < off[r + 1]; ++j) sum += table[(size_t)k[j] * kDim + c];
@@ -261,7 +269,7 @@ int main(int argc, char **argv) {
       return 1;
     }
     coll_cache_shutdown();
-    coll_cache_free_host_table(table);
+    coll_cache_free_host_table(table_mem);
     ugk_model_graph_destroy(graph);
     ugk_stream_destroy(caller_stream);
     for (void *st : extra_streams) ugk_stream_destroy(st);

@@ -391,8 +391,10 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
   if (n == 0) return 0;
   REQUIRE(keys && out && status, "ugk_extract_mix: null keys, output or status");
   if (check_table(t, "ugk_extract_mix")) return 1;
-  REQUIRE(rb > 0 && (rb % 16 == 0 || (!stage && rb % 4 == 0 && rb >= 20)),
-          "ugk_extract_mix: rows must be multiples of 16 bytes, or without a stage of 4 bytes (row_bytes=%zu)", rb);
+  const uintptr_t align = (uintptr_t)cache | (uintptr_t)host | (uintptr_t)out | (uintptr_t)rb;
+  REQUIRE(rb > 0 && (align % 16 == 0 || (!stage && align % 4 == 0 && rb >= 20)),
+          "ugk_extract_mix: rows and buffers must be multiples of 16 bytes, or without a stage of 4 bytes (row_bytes=%zu)",
+          rb);
   uint64_t local = 0, others = 0;
   for (size_t i = 0; i < n; ++i) {
     const uint64_t key = k64(keys[i]);
@@ -1193,6 +1195,8 @@ int ugk_gather_scatter_staged_u32(const void *host, uint64_t host_rows, const ui
   if (n == 0) return 0;
   REQUIRE(host && rows && dst && out && status && stage.rows_dev && stage.owner_dev, "staged gather: null pointer");
   REQUIRE(done_count == nullptr || rest_count, "staged gather: a done count without rest lists");
+  const uintptr_t align = (uintptr_t)host | (uintptr_t)out | (uintptr_t)stage.rows_dev | (uintptr_t)rb;
+  REQUIRE(rb > 0 && align % 16 == 0, "staged gather: rows and buffers must be multiples of 16 bytes (row_bytes=%zu)", rb);
   for (size_t i = 0; i < n; ++i) {
     const uint64_t r = rows[i];
     if (r >= host_rows || dst[i] >= out_rows) {

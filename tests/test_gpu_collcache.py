@@ -468,6 +468,44 @@ def test_rows_that_are_not_multiples_of_16_bytes(dim, dtype, pct):
         assert out.cpu().numpy().tobytes() == ORC.gather(table, q.astype(np.int64)).tobytes()
 
 
+@pytest.mark.parametrize("on_device", [False, True])
+@pytest.mark.parametrize("table_shift,out_shift", [(4, 0), (8, 4), (0, 4), (0, 0)])
+def test_miss_stage_with_a_table_or_output_between_two_vectors(table_shift, out_shift, on_device, monkeypatch):
+    """COLL_MISS_STAGE_ROWS with rows of whole 16-byte vectors in a host table, or looked up into an output, that starts
+    `shift` bytes off a 16-byte boundary: blocking and stream-ordered lookups before and behind foreground refreshes"""
+    monkeypatch.setenv("COLL_MISS_STAGE_ROWS", "2048")
+    if on_device:
+        monkeypatch.setenv("COLL_GPU_RECORD", "1")
+        monkeypatch.setenv("COLL_GPU_REFRESH", "1")
+    rng = np.random.default_rng(41)
+    n_item, dim, pct, n = 20_000, 32, 0.25, 3_001
+    co.config(make_config(n_item, pct))
+    co.coll_cache_record_init(0)
+    co.coll_torch_record(0, torch.from_numpy(zipf_ranks(rng, 40_000, n_item, 1.1)).to(torch.int32))
+    whole = co.coll_torch_create_emb_shm(0, n_item * dim + 16, 1, torch.float32).view(-1)
+    emb = whole[table_shift // 4 :][: n_item * dim].view(n_item, dim)
+    assert emb.data_ptr() % 16 == table_shift
+    table = fill_table(emb, rng)
+    co.coll_torch_init_t(0, 0, emb, pct)
+    out = torch.empty(n * dim + 4, dtype=torch.float32, device="cuda")
+    to = out.data_ptr() + out_shift
+    lib = _basics.C_LIB_CTYPES
+    for step in range(3):
+        for blocking in (True, False):
+            q = ((zipf_ranks(rng, n, n_item, 1.1) + step * 4_000) % n_item).astype(np.int64)
+            keys = torch.from_numpy(q).to(torch.int32).cuda()
+            if not on_device:
+                co.coll_torch_record(0, keys.cpu())
+            out.fill_(0)
+            torch.cuda.synchronize()
+            (lib.coll_cache_lookup if blocking else lib.coll_cache_lookup_async)(0, keys.data_ptr(), n, to, None)
+            lib.coll_cache_lookup_wait(0, None)
+            torch.cuda.synchronize()
+            got = out[out_shift // 4 :][: n * dim].cpu().numpy()
+            assert got.tobytes() == ORC.gather(table, q).tobytes()
+        co.coll_torch_refresh(0, True)
+
+
 def test_key_tensors_are_checked_and_strided_ones_accepted():
     rng = np.random.default_rng(3)
     n_item, dim = 5_000, 32

@@ -23,8 +23,9 @@ def drivers():
     return {"asan": os.path.join(BUILD, "driver_asan"), "tsan": os.path.join(BUILD, "driver_tsan")}
 
 
-def _run(exe, table, refresh, steps):
+def _run(exe, table, refresh, steps, **more):
     env = dict(os.environ)
+    env.update(more)
     env["COLL_HASH_REBUILD_FRAC"] = "0.02"  # a few hundred evictions already rebuild the open-addressing table
     env["COLL_MISS_STAGE_ROWS"] = "4096"  # lookups file the rows they fetch from the host, foreground refreshes read them
     if table.startswith("HASH"):  # refreshes on the device keep cached rows that tie (the second placement path)
@@ -53,6 +54,16 @@ def test_host_library_under_asan_and_ubsan(drivers, table, refresh):
     if table.startswith("HASH"):  # the table swap of a rebuild ran beside the lookups
         rebuilds = [int(l.split(" table rebuilds")[0].split()[-1]) for l in out.splitlines() if " table rebuilds" in l]
         assert rebuilds and max(rebuilds) > 0, out[-3000:]
+
+
+@pytest.mark.parametrize("refresh", ["host", "device"])
+@pytest.mark.parametrize("table,shift", [("FLAT", 4), ("HASH", 8)])
+def test_host_table_between_two_vectors(drivers, table, refresh, shift):
+    """COLL_MISS_STAGE_ROWS with rows of whole 16-byte vectors in a host table (a view of a larger tensor) that starts at a
+    4- or 8-byte boundary: looked up, blocking and stream-ordered, refreshed and served like any other"""
+    rc, out = _run(drivers["asan"], table, refresh, 60, DRIVER_TABLE_SHIFT=str(shift))
+    assert "AddressSanitizer" not in out and "runtime error" not in out and "LeakSanitizer" not in out, out[-6000:]
+    assert rc == 0 and out.rstrip().endswith("OK"), out[-3000:]
 
 
 @pytest.mark.parametrize("refresh", ["host", "device"])

@@ -333,7 +333,15 @@ ExtractSession::ExtractSession(std::shared_ptr<CacheContext> cache_ctx) : _cache
   memset(_host_mirror, 0, 256);
   const auto &desc = RunConfig::coll_cache_link_desc;
   if (!desc.cpu_sm.empty()) _cpu_blocks = (unsigned)desc.cpu_sm[0];
-  if (RunConfig::miss_stage_rows > 0 && !_cache_ctx->IsDirectMapping() && _cache_ctx->_row_bytes % 16 == 0 &&
+  // Rows are filed in the stage next to their copy into the output, and read from it by a refresh, by the kernels of whole
+  // 16-byte vectors only: a stage exists only where the rows, the cache and the host table (the caller's, perhaps a view
+  // that starts anywhere) are made of such vectors.
+  const auto whole_vectors = [&] {
+    return ((uintptr_t)_cache_ctx->_device_cache_data[_cache_ctx->_local_location_id] |
+            (uintptr_t)_cache_ctx->_device_cache_data[_cache_ctx->_cpu_location_id] |
+            (uintptr_t)_cache_ctx->_row_bytes) % 16 == 0;
+  };
+  if (RunConfig::miss_stage_rows > 0 && !_cache_ctx->IsDirectMapping() && whole_vectors() &&
       _cache_ctx->_num_total_nodes <= 0x100000000ull) {
     size_t entries = 1024;
     while (entries < RunConfig::miss_stage_rows) entries <<= 1;
@@ -716,8 +724,7 @@ static bool FusedTakes(const void *cache, const void *host, const void *output, 
   return align % 16 == 0 || (align % 4 == 0 && rb >= 20);
 }
 
-// Rows are filed in the stage next to their copy into the output by the kernels of whole 16-byte vectors only (a stage
-// exists only for such rows; the output is the caller's).
+// Nor does a lookup file rows whose output (the caller's) is not made of such vectors.
 static bool StageTakes(const void *output) { return (uintptr_t)output % 16 == 0; }
 
 static int ExtractPool(ugk_table_t t, const IdType *ids, const int64_t *seg_off, const float *w, size_t n_rows,
