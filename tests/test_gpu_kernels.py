@@ -1390,6 +1390,24 @@ def test_extract_mix_other_row_sizes(row_bytes):
         pin.free()
 
 
+def test_extract_mix_rows_beyond_a_gigabyte():
+    """rows of 2^30 + 16 bytes, 16-byte vectors behind a flat table: taken as any others, the last ones more than 2^32
+    bytes into the buffers"""
+    rb, nkeys = (1 << 30) + 16, 6
+    words = rb // 8
+    host = torch.arange(nkeys * words, dtype=torch.int64, device="cuda").view(nkeys, words)
+    cache = host[[5, 1]] + (1 << 40)  # told apart from the host rows
+    mem, tb = _make_flat(nkeys)
+    assert _insert(tb, np.array([5, 1], np.uint32)) == 0
+    keys = to_dev(np.array([5, 3, 1, 4, 0], np.uint32))
+    out, st = torch.zeros((5, words), dtype=torch.int64, device="cuda"), dev_zeros_u32(1)
+    hip.call("ugk_extract_mix_u32", tb, ptr(keys), 5, ptr(cache), 2, ptr(host), nkeys, ptr(out), rb, ptr(st), None, None,
+             None, hip.HINT_UNKNOWN, None)
+    assert status_value(st) == 0
+    for at, want in enumerate((cache[0], host[3], cache[1], host[4], host[0])):
+        assert torch.equal(out[at], want), at
+
+
 @pytest.mark.parametrize("row_bytes", [20, 36, 100, 128 + 4, 404, 1204, 4096 + 4, 131072 + 4])
 @pytest.mark.parametrize("kind", ["flat", "hash", "hash32"])
 def test_extract_mix_of_rows_that_are_no_whole_vectors(row_bytes, kind):

@@ -36,6 +36,7 @@ struct FlatRow {
   uint32_t tile;    // rows numbered through together, at most 64
 };
 constexpr uint32_t kFlatMinBytes = 20;        // shorter rows are one vector or none
+constexpr uint32_t kFlatMaxBytes = 1u << 30;  // lengths and offsets in a row are counted in 32 bits
 constexpr uint32_t kFlatMaxTiled = 8192;      // chunks up to which mulhi divides exactly (idx * chunks < 2^32)
 constexpr uint32_t kNoRowBit = 1;             // in a row's address: nothing is copied for it
 
@@ -94,14 +95,16 @@ struct MixRow {
   bool has_row, from_cache;
 };
 
+// row_units: length of a row in units of T (a row of 16-byte vectors may be longer than 32 bits of bytes)
+template <typename T>
 __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key, bool active, const Found &f,
-                                              const void *cache, uint64_t cache_rows, const void *host,
-                                              uint64_t host_rows, const void *out, uint32_t row_bytes,
-                                              uint32_t *status, uint32_t *host_mirror) {
-  const char *rowp = nullptr;
+                                              const T *cache, uint64_t cache_rows, const T *host, uint64_t host_rows,
+                                              const void *out, uint32_t row_units, uint32_t *status,
+                                              uint32_t *host_mirror) {
+  const T *rowp = nullptr;
   uint64_t host_row = ~0ull;
   if (active) {
-    if (f.hit && f.loc == UGK_LOC_LOCAL && f.off < cache_rows) rowp = static_cast<const char *>(cache) + (uint64_t)f.off * row_bytes;
+    if (f.hit && f.loc == UGK_LOC_LOCAL && f.off < cache_rows) rowp = cache + (uint64_t)f.off * row_units;
     else if (f.hit && f.loc == UGK_LOC_HOST && f.off < host_rows) host_row = f.off;
     else if (!f.hit && fallback_row(t, key) < host_rows) host_row = fallback_row(t, key);
     else {
@@ -111,7 +114,7 @@ __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key
   }
   // A key without a row copies nothing; its lanes read the head of the output instead (mapped whatever the key), so
   // that the loads of the copy carry no branch: behind a branch each of them waits for the one before.
-  if (host_row != ~0ull) rowp = static_cast<const char *>(host) + host_row * row_bytes;
+  if (host_row != ~0ull) rowp = host + host_row * row_units;
   MixRow r;
   r.host_row = host_row;
   r.has_row = rowp != nullptr;

@@ -10,6 +10,7 @@
 #include <cstdlib>
 
 #include <mutex>
+#include <type_traits>
 
 #include "ugk_internal.h"
 #include "ugk_mix.cuh"
@@ -245,8 +246,10 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
     // (fewer keys: their home lines in one go as well, and only the rounds of the probe that have keys to serve)
     constexpr int ROUNDS = KPW >= 8 ? KPW / 8 : 1;
     const Found f = table_lookup<KIND, (KPW == kWave || ROUNDS < 8) ? 1 : 2, ROUNDS>(t, key, active);
-    const MixRow row =
-        mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, f_row.row_bytes, status, host_mirror);
+    typedef typename std::conditional<LPR == 0, char, u32x4>::type unit_t;
+    const MixRow row = mix_resolve(t, key, active, f, static_cast<const unit_t *>(cache), cache_rows,
+                                   static_cast<const unit_t *>(host), host_rows, out,
+                                   LPR == 0 ? f_row.row_bytes : f_row.chunks, status, host_mirror);
     if (counts) {
       // rows from the cache, and all others (host rows, and rows skipped for a key without a row: the launch is
       // flagged then and its group sizes mean nothing, but the two sums still add up to n)
@@ -259,7 +262,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       for (uint32_t r0 = 0; r0 < here; r0 += f_row.tile)
         flat_copy<true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
     } else {
-      const uint32_t vpr = f_row.row_bytes / 16;
+      const uint32_t vpr = f_row.chunks;
       uint64_t stage_bits = 0;
       if constexpr (STAGE) stage_bits = stage_claim(stage, row, vpr);
       mix_copy<LPR, KPW, NT_STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
@@ -635,8 +638,9 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
   UGK_REQUIRE(host_rows == 0 || host, "ugk_extract_mix: null host table with %llu rows",
               (unsigned long long)host_rows);
   const uintptr_t align = (uintptr_t)cache | (uintptr_t)host | (uintptr_t)out | (uintptr_t)row_bytes;
-  UGK_REQUIRE(row_bytes > 0 && row_bytes <= (1u << 30), "ugk_extract_mix: row_bytes %zu out of range", row_bytes);
   const bool flat = align % 16 != 0;
+  UGK_REQUIRE(row_bytes > 0 && (!flat || row_bytes <= kFlatMaxBytes), "ugk_extract_mix: row_bytes %zu out of range",
+              row_bytes);
   UGK_REQUIRE(!flat || (flat_row_ok(align, row_bytes) && !stage),
               "ugk_extract_mix: rows and buffers must be multiples of 16 bytes, or without a stage of 4 bytes with rows "
               "of at least %u (row_bytes=%zu)",

@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
       const bool active = j < end;
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
       const Found f = table_lookup<KIND>(t, key, active);
-      const MixRow row = mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, vpr * 16u, status, host_mirror);
+      const MixRow row = mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
       if (counts) {
         wave_local += __popcll(__ballot(row.from_cache));
         wave_host += __popcll(__ballot(active && !row.from_cache));
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
       const long long j = active ? my_beg[k] + (long long)(f - my_start[k]) : 0;
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
       const Found fd = table_lookup<KIND>(t, key, active);
-      const MixRow row = mix_resolve(t, key, active, fd, cache, cache_rows, host, host_rows, out, vpr * 16u, status, host_mirror);
+      const MixRow row = mix_resolve(t, key, active, fd, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
       if (counts) {
         wave_local += __popcll(__ballot(row.from_cache));
         wave_host += __popcll(__ballot(active && !row.from_cache));
