@@ -424,6 +424,10 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   //                                                     40: 37 / 41 / 37;  1 id 43 with (4,1,2), 51 with (4,1,4)
   //   128 B   (8,4,4) / (8,1,2) / (8,1,4):              2 ids 68 / 41 / 42,  4: 58 / 40 / 38,  40: 34 / 41 / 33
   //   256 B   (8,4,4) / (8,2,2) / (16,2,4):             2 ids 73 / 45 / 82,  8: 42 / 36 / 43,  40: 39 / 42 / 34
+  //           many ids, 800,000 of them, Zipf / uniform, no branch around the loads: (16,2,4), whose second chunk is past the
+  //           end of these rows (their last chunk again, for nothing), then (16,1,4), then (16,1,2): 16 ids 29 / 45, 24 / 42,
+  //           26 / 46; 40 ids 31 / 45, 20 / 40, 22 / 40; of two-byte elements 16 ids 35 / 48, 26 / 45, 24 / 43; 40 ids
+  //           32 / 44, 27 / 44, 24 / 40.  Where rows come over the host link (16,1,4) keeps more of them on their way
   //   512 B   (8,4,4) / (8,4,2) / (16,2,2) / (16,2,4):  2 ids 93 / 74 / 82 / 100,  4: 80 / 75 / 77 / 84,
   //                                                     8: 49 / 46 / 47 / 49,  40: 48 / 57 / 44 / 40
   //   512 B of two-byte elements, the same:             2 ids 68 / 61 / 54 / 67,  8: 43 / 45 / 38 / 39,
@@ -442,7 +446,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   if (clip) shape = vpr <= 32 ? 844 : vpr <= 128 ? 3244 : 6444;
   else if (vpr <= 4) shape = upto6 ? 412 : 414;
   else if (vpr <= 8) shape = 814;
-  else if (vpr <= 16) shape = upto12 ? 822 : 1624;
+  else if (vpr <= 16) shape = upto12 ? 822 : KIND == 0 && sizeof(E) == 2 ? 1612 : 1614;
   else if (vpr <= 32) shape = upto2 && sizeof(E) == 4 ? 842 : upto12 ? 1622 : 1624;
   else if (vpr <= 64) shape = upto12 ? 1642 : 3224;
   else if (vpr <= 128) shape = 3242;
@@ -499,6 +503,11 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   UGK_POOL(4, 1, 4, false)
   UGK_POOL(8, 1, 4, false)
   UGK_POOL(8, 2, 2, false)
+  if constexpr (KIND == 0 && sizeof(E) == 2) {
+    UGK_POOL(16, 1, 2, false)
+  } else {
+    UGK_POOL(16, 1, 4, false)
+  }
   UGK_POOL(16, 2, 4, false)
   UGK_POOL(8, 4, 4, true)
   UGK_POOL(32, 4, 4, true)
