@@ -978,7 +978,7 @@ def test_pooled_extraction_matches_a_float64_segment_sum(kind, dim, etype, rows_
 
 
 @pytest.mark.parametrize("kind", ["none", "flat"])
-@pytest.mark.parametrize("vpr", [1, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("vpr", [1, 4, 5, 8, 9, 16, 17, 24, 32, 33, 64, 65, 128, 129, 256])
 def test_pooled_extraction_at_the_edges_of_its_shapes(kind, vpr):
     """Rows of vpr 16-byte vectors around the sizes where the lanes per row and the chunks per lane change, with 1, 2, 5,
     9 and 40 ids per sample on average (the rows in flight change between them), fp32 and fp16: mean over weights in

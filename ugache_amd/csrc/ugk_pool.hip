@@ -79,31 +79,30 @@ constexpr int kPoolChunks = 4;  // 16-byte chunks of a row a lane may own at mos
 // many rows are on their way at once and that no load waits for another: a lane reads its CH chunks of U ids before it
 // adds the first of them (a row of the host table whose chunks were read one after the other cost its wavefront CH
 // round trips over the link), and CH and U are template parameters so that short rows do not pay for the registers of
-// long ones.  The loads are ordinary ones: ids repeat
-// in real batches, and the hot rows stay in L2.  800,000 ids over rows of 512 bytes, all in HBM, us before / now, 4, 8 and
-// 16 ids per sample: Zipf 1.05 104 / 86, 88 / 66, 81 / 61; uniform ids, which reuse nothing, 113 / 125, 105 / 111, 98 /
-// 105; rows of 800 bytes 184 / 129, 147 / 95, 130 / 92 and uniform 197 / 181, 180 / 162, 170 / 152.
+// long ones.
+// KEEP: the loads are ordinary ones: ids repeat in real batches, and the hot rows stay in L2.  Uniform ids, which reuse
+// nothing, are up to a tenth faster with non-temporal ones where rows are whole lines, and which law its ids follow a launch
+// does not know.  Where that matters (MIXED) keep_waves of a workgroup's four wavefronts load ordinarily: a row that many
+// wavefronts read comes by one of those soon and stays in L2 for all of them, and rows read once mostly pass through.  Two
+// bodies and not a branch around the loads: of two loads that differ in the hint only the compiler makes one.  800,000 ids
+// over rows of 512 bytes, all in HBM, 4 ids per sample, none / one / two / three / all four ordinary: uniform 90 / 88 / 92 / 97 /
+// 100 us, Zipf 1.05 76 / 62 / 60 / 58 / 56.
 // CLIP: every looked-up row is clipped to the l2 norm max_norm before it is weighted (clip_by_norm over the row:
 // x * max_norm / max(||x||, max_norm)).  The whole row has to be seen before any of it can be added, so the chunks of
 // the U rows in flight are held in registers (up to 64 more than without), the squares summed per row over the lanes
 // of the group, and the row's weight scaled; a kernel of its own, so that the plain combination keeps its registers.
-template <typename K, int KIND, int LPR, int CH, int U, typename E, bool CLIP>
-__global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, const K *__restrict__ ids,
-                                                              const long long *__restrict__ seg_off,
-                                                              const float *__restrict__ weights, size_t n_rows,
-                                                              long long nnz, const u32x4 *__restrict__ cache,
-                                                              uint64_t cache_rows,
-                                                              const u32x4 *__restrict__ host, uint64_t host_rows,
-                                                              u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
-                                                              float max_norm, uint32_t *status, uint32_t *host_mirror,
-                                                              unsigned long long *counts) {
+template <typename K, int KIND, int LPR, int CH, int U, typename E, bool CLIP, bool KEEP>
+__device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__restrict__ ids,
+                                             const long long *__restrict__ seg_off, const float *__restrict__ weights,
+                                             size_t n_rows, long long nnz, const u32x4 *__restrict__ cache,
+                                             uint64_t cache_rows, const u32x4 *__restrict__ host, uint64_t host_rows,
+                                             u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
+                                             float max_norm, uint32_t *status, uint32_t *host_mirror,
+                                             const unsigned long long *counts, uint32_t &wave_local,
+                                             uint32_t &wave_host) {
   constexpr int RPW = kWave / LPR;  // output rows per wavefront and pass
   constexpr int EPC = PoolElem<E>::kPerChunk;
   static_assert(LPR % U == 0, "ids are taken in rounds of U");
-  __shared__ uint32_t block_tot[2];
-  if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
-  __syncthreads();
-  uint32_t wave_local = 0, wave_host = 0;
   const int lane = (int)lane_id();
   const int sub = lane % LPR, rg = lane / LPR;
   const size_t wave_global = (size_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
@@ -208,7 +207,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
           for (int c = 0; c < CH; ++c) {
             const uint32_t col = min((uint32_t)c * LPR + sub, vpr - 1);
 #pragma unroll
-            for (int u = 0; u < U; ++u) v[c][u] = p[u][col];
+            for (int u = 0; u < U; ++u) v[c][u] = KEEP ? p[u][col] : __builtin_nontemporal_load(p[u] + col);
           }
 #pragma unroll
           for (int c = 0; c < CH; ++c) {
@@ -243,6 +242,30 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
       }
     }
   }
+}
+
+template <typename K, int KIND, int LPR, int CH, int U, typename E, bool CLIP, bool MIXED>
+__global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, const K *__restrict__ ids,
+                                                              const long long *__restrict__ seg_off,
+                                                              const float *__restrict__ weights, size_t n_rows,
+                                                              long long nnz, const u32x4 *__restrict__ cache,
+                                                              uint64_t cache_rows,
+                                                              const u32x4 *__restrict__ host, uint64_t host_rows,
+                                                              u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
+                                                              float max_norm, uint32_t *status, uint32_t *host_mirror,
+                                                              unsigned long long *counts, uint32_t keep_waves) {
+  __shared__ uint32_t block_tot[2];
+  if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
+  __syncthreads();
+  uint32_t wave_local = 0, wave_host = 0;
+  if (!MIXED || wave_in_block() < keep_waves)
+    pool_samples<K, KIND, LPR, CH, U, E, CLIP, true>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host,
+                                                     host_rows, out, vpr, combiner, bf16, max_norm, status, host_mirror,
+                                                     counts, wave_local, wave_host);
+  else if constexpr (MIXED)
+    pool_samples<K, KIND, LPR, CH, U, E, CLIP, false>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host,
+                                                      host_rows, out, vpr, combiner, bf16, max_norm, status, host_mirror,
+                                                      counts, wave_local, wave_host);
   if (counts) mix_leave_counts(block_tot, wave_local, wave_host, counts);
 }
 
@@ -259,26 +282,22 @@ constexpr int kPoolMaxRows = 8;  // output rows a lane group may own per pass
 // us for 390,625 of them against 124 with one row per group; 60 % of the table uncached behind a flat table, 262,144 of
 // them, 123 against 98 us; behind a hash table, whose lookup works on all lanes of a wavefront at once and wants them
 // to hold ids, 195,312 of them 107 against 128 us.
-template <typename K, int KIND, int LPR, typename E>
-__global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t, const K *__restrict__ ids,
-                                                              const long long *__restrict__ seg_off,
-                                                              const float *__restrict__ weights, size_t n_rows,
-                                                              long long nnz, int rows_per_group,
-                                                              const u32x4 *__restrict__ cache, uint64_t cache_rows,
-                                                              const u32x4 *__restrict__ host, uint64_t host_rows,
-                                                              u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
-                                                              uint32_t *status, uint32_t *host_mirror,
-                                                              unsigned long long *counts) {
+template <typename K, int KIND, int LPR, typename E, bool KEEP>
+__device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K *__restrict__ ids,
+                                                   const long long *__restrict__ seg_off,
+                                                   const float *__restrict__ weights, size_t n_rows, long long nnz,
+                                                   int rows_per_group, const u32x4 *__restrict__ cache,
+                                                   uint64_t cache_rows, const u32x4 *__restrict__ host,
+                                                   uint64_t host_rows, u32x4 *__restrict__ out, uint32_t vpr,
+                                                   int combiner, bool bf16, uint32_t *status, uint32_t *host_mirror,
+                                                   const unsigned long long *counts, uint32_t &wave_local,
+                                                   uint32_t &wave_host,
+                                                   long long (&seg_beg)[kWavesPerBlock][kWave / LPR][kPoolMaxRows],
+                                                   uint32_t (&seg_start)[kWavesPerBlock][kWave / LPR][kPoolMaxRows]) {
   constexpr int RPW = kWave / LPR;  // lane groups per wavefront
   constexpr int EPC = PoolElem<E>::kPerChunk;
   constexpr int U = 4;  // rows in flight per lane group
   static_assert(LPR % U == 0 && LPR >= kPoolMaxRows, "ids are taken in rounds of U; a lane per owned row");
-  __shared__ uint32_t block_tot[2];
-  __shared__ long long seg_beg[kWavesPerBlock][RPW][kPoolMaxRows];    // first id of the group's row k
-  __shared__ uint32_t seg_start[kWavesPerBlock][RPW][kPoolMaxRows];   // its first position in the group's list
-  if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
-  __syncthreads();
-  uint32_t wave_local = 0, wave_host = 0;
   const int lane = (int)lane_id();
   const int sub = lane % LPR, rg = lane / LPR, wv_in_block = (int)(threadIdx.x / kWave);
   const size_t wave_global = (size_t)blockIdx.x * kWavesPerBlock + wv_in_block;
@@ -369,7 +388,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
           if (col < vpr) {
             u32x4 v[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) v[u] = p[u][col];
+            for (int u = 0; u < U; ++u) v[u] = KEEP ? p[u][col] : __builtin_nontemporal_load(p[u] + col);
             int cc = cur;  // every chunk walks the same ids from the same state
             float ws = wsum;
 #pragma unroll
@@ -408,6 +427,32 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
     }
     __builtin_amdgcn_wave_barrier();  // the next pass rewrites the group's list
   }
+}
+
+template <typename K, int KIND, int LPR, typename E, bool MIXED>
+__global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t, const K *__restrict__ ids,
+                                                              const long long *__restrict__ seg_off,
+                                                              const float *__restrict__ weights, size_t n_rows,
+                                                              long long nnz, int rows_per_group,
+                                                              const u32x4 *__restrict__ cache, uint64_t cache_rows,
+                                                              const u32x4 *__restrict__ host, uint64_t host_rows,
+                                                              u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
+                                                              uint32_t *status, uint32_t *host_mirror,
+                                                              unsigned long long *counts, uint32_t keep_waves) {
+  __shared__ uint32_t block_tot[2];
+  __shared__ long long seg_beg[kWavesPerBlock][kWave / LPR][kPoolMaxRows];    // first id of the group's row k
+  __shared__ uint32_t seg_start[kWavesPerBlock][kWave / LPR][kPoolMaxRows];   // its first position in the group's list
+  if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
+  __syncthreads();
+  uint32_t wave_local = 0, wave_host = 0;
+  if (!MIXED || wave_in_block() < keep_waves)
+    pool_short_samples<K, KIND, LPR, E, true>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
+                                              host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
+                                              wave_local, wave_host, seg_beg, seg_start);
+  else if constexpr (MIXED)
+    pool_short_samples<K, KIND, LPR, E, false>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
+                                               host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
+                                               wave_local, wave_host, seg_beg, seg_start);
   if (counts) mix_leave_counts(block_tot, wave_local, wave_host, counts);
 }
 
@@ -443,26 +488,48 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   const bool upto2 = nnz <= rows64 * 5 / 2, upto6 = nnz <= rows64 * 6, upto12 = nnz <= rows64 * 12;
   const bool clip = max_norm > 0.f;
   int shape;
+  uint32_t keep_waves = kWavesPerBlock;
   if (clip) shape = vpr <= 32 ? 844 : vpr <= 128 ? 3244 : 6444;
-  else if (vpr <= 4) shape = upto6 ? 412 : 414;
+  else if (vpr <= 4) shape = upto6 ? 412 : nnz <= rows64 * 24 ? 414 : 814;
   else if (vpr <= 8) shape = 814;
   else if (vpr <= 16) shape = upto12 ? 822 : KIND == 0 && sizeof(E) == 2 ? 1612 : 1614;
   else if (vpr <= 32) shape = upto2 && sizeof(E) == 4 ? 842 : upto12 ? 1622 : 1624;
   else if (vpr <= 64) shape = upto12 ? 1642 : 3224;
   else if (vpr <= 128) shape = 3242;
   else shape = 6442;
+  // Rows all in HBM whose ordinary loads cost uniform ids something: some wavefronts load them non-temporally (see
+  // pool_samples), in a shape that makes up for what that costs skewed ones.  800,000 ids, fp32, without the hint / this,
+  // uniform and Zipf 1.05 (all loads non-temporal and one chunk at a time, before either): 384 bytes 4 ids 76.9 / 68.5 and
+  // 56.2 / 52.1 (71.4 and 62.4), 8 ids 68.6 / 62.7 and 39.2 / 38.9 (66.1 and 51.0), 40 ids 60.3 / 53.4 and 35.1 / 29.3
+  // (55.8 and 44.7); 512 bytes 2 ids 119.7 / 111.2 and 88.7 / 87.0 (116.1 and 121.6), 4 ids 100.6 / 93.4 and 61.6 / 59.4
+  // (92.7 and 78.7), 40 ids 78.6 / 70.9 and 40.2 / 36.9 (73.0 and 55.4).  Left alone, for it takes from skewed ids what it
+  // gives uniform ones: 512 bytes 8 ids (89.6 and 45.1; 85.5 and 66.1 before), 400,000 ids of 1 KB 4 ids (98.8 / 91.5 and
+  // 55.6 / 58.3; 92.1 and 85.6 before) and 8 ids (89.3 and 43.4; 85.1 and 66.8), of 2 KB 4 ids (192 and 116; 176 and 151).
+  // Rows of other lengths, which begin and end inside a line, are faster for uniform ids as well with ordinary loads (400
+  // bytes 4 ids 95 against 128).
+  if (KIND == 0 && !clip && vpr > 16 && vpr <= 32 && vpr % 8 == 0) {
+    if (upto2) keep_waves = vpr == 32 && sizeof(E) == 4 ? 1 : keep_waves;
+    else if (upto6) shape = 842, keep_waves = 2;
+    else if (upto12 && vpr < 32) shape = 842, keep_waves = 3;
+    else if (nnz > rows64 * 24 && sizeof(E) == 4) shape = 1622, keep_waves = 3;
+  }
   if (const char *forced = getenv("UGK_POOL_LPR")) {  // for sweeps; never a byte of the result depends on it
     const int v = atoi(forced);
-    if (!clip && (v == 8 || v == 32 || v == 64) && vpr <= (uint32_t)v * kPoolChunks) shape = v * 100 + 42;
+    if (!clip && (v == 8 || v == 32 || v == 64) && vpr <= (uint32_t)v * kPoolChunks)
+      shape = v * 100 + 42, keep_waves = kWavesPerBlock;
   }
   // Output rows per lane group and pass: one, but four as one list (extract_pool_rows_kernel) for samples of mostly one
-  // id without a flat table (see there), as long as the launch still has wavefronts for every CU.  Rows of up to 64 bytes
-  // without any table are faster with one all the same (43 / 60 us for 400,000 samples).
+  // id without a flat table (see there), as long as the launch still has wavefronts for every CU.  Without any table that
+  // is for two-byte elements of more than 64 bytes (two of 256 bytes: 127 us one by one, 107 as a list), and for fp32 rows
+  // of whole lines up to 384 bytes.  The other fp32 rows are faster one by one, 800,000 samples (400,000 from 640 bytes
+  // on) uniform and Zipf 1.05, list / one by one: 64 bytes 54 / 37 and 48 / 31, 160 bytes 95 / 81 and 81 / 72, 400 bytes
+  // 239 / 165 and 186 / 167, 512 bytes 179 / 169 and 169 / 162, 1 KB 184 / 165 and 183 / 164, 2 KB 329 / 322 and 318 / 318.
   int rows = 1;
   if constexpr (KIND != 1) {
     const int lanes = vpr <= 32 ? 8 : vpr <= 128 ? 32 : 64;
     const int groups = kWave / lanes;
-    if (n_rows && nnz <= rows64 + rows64 / 2 && (KIND != 0 || vpr > 4)) rows = 4;
+    const bool lists = KIND != 0 || (vpr > 4 && (sizeof(E) == 2 || vpr <= 8 || (vpr < 32 && vpr % 8 == 0)));
+    if (n_rows && nnz <= rows64 + rows64 / 2 && lists) rows = 4;
     const size_t enough_waves = (size_t)cu_count() * 8;
     while (rows > 1 && n_rows / ((size_t)rows * groups) < enough_waves) rows /= 2;
     if (const char *forced = getenv("UGK_POOL_ROWS")) {  // for sweeps, like the one above
@@ -474,11 +541,15 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
       const size_t rows_per_block = (size_t)rows * groups * kWavesPerBlock;
       const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
       if (num_groups) *num_groups = grid;
+      // (256 bytes uniform and Zipf 1.05, before / without the hint / one wavefront of four without: 90 / 101 / 91 and
+      // 102 / 91 / 91)
+      constexpr bool kMixed = KIND == 0 && sizeof(E) == 4;
+      const uint32_t keep = kMixed && vpr % 8 == 0 ? 1 : kWavesPerBlock;
 #define UGK_POOL_ROWS_GO(L)                                                                                            \
-  hipLaunchKernelGGL((extract_pool_rows_kernel<K, KIND, L, E>), dim3(grid), dim3(kBlock), 0, st, t, ids, seg_off,      \
-                     weights, n_rows, (long long)nnz, rows, (const u32x4 *)cache, cache_rows, (const u32x4 *)host,     \
-                     host_rows, (u32x4 *)out, vpr, combiner, bf16, status, host_mirror,                                \
-                     reinterpret_cast<unsigned long long *>(counts))
+  hipLaunchKernelGGL((extract_pool_rows_kernel<K, KIND, L, E, kMixed>), dim3(grid), dim3(kBlock), 0, st, t, ids,       \
+                     seg_off, weights, n_rows, (long long)nnz, rows, (const u32x4 *)cache, cache_rows,                 \
+                     (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, status, host_mirror,           \
+                     reinterpret_cast<unsigned long long *>(counts), keep)
       if (lanes == 8) UGK_POOL_ROWS_GO(8);
       else if (lanes == 32) UGK_POOL_ROWS_GO(32);
       else UGK_POOL_ROWS_GO(64);
@@ -490,34 +561,41 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   const size_t rows_per_block = (size_t)(kWave / (shape / 100)) * kWavesPerBlock;
   const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
   if (num_groups) *num_groups = grid;
+  const bool mixed = keep_waves < kWavesPerBlock;
   bool launched = false;
-#define UGK_POOL(L, CH, U, CLIP)                                                                                       \
-  if (shape == L * 100 + CH * 10 + U && clip == CLIP) {                                                                \
+#define UGK_POOL(L, CH, U, CLIP, MIXED)                                                                                \
+  if (shape == L * 100 + CH * 10 + U && clip == CLIP && mixed == MIXED) {                                              \
     launched = true;                                                                                                   \
-    hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, CH, U, E, CLIP>), dim3(grid), dim3(kBlock), 0, st, t, ids,       \
-                     seg_off, weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows, (const u32x4 *)host,  \
-                     host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status, host_mirror,                      \
-                     reinterpret_cast<unsigned long long *>(counts));                                                \
+    hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, CH, U, E, CLIP, MIXED>), dim3(grid), dim3(kBlock), 0, st, t,   \
+                     ids, seg_off, weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows,                  \
+                     (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status, host_mirror, \
+                     reinterpret_cast<unsigned long long *>(counts), keep_waves);                                      \
   }
-  UGK_POOL(4, 1, 2, false)
-  UGK_POOL(4, 1, 4, false)
-  UGK_POOL(8, 1, 4, false)
-  UGK_POOL(8, 2, 2, false)
+  UGK_POOL(4, 1, 2, false, false)
+  UGK_POOL(4, 1, 4, false, false)
+  UGK_POOL(8, 1, 4, false, false)
+  UGK_POOL(8, 2, 2, false, false)
   if constexpr (KIND == 0 && sizeof(E) == 2) {
-    UGK_POOL(16, 1, 2, false)
+    UGK_POOL(16, 1, 2, false, false)
   } else {
-    UGK_POOL(16, 1, 4, false)
+    UGK_POOL(16, 1, 4, false, false)
   }
-  UGK_POOL(16, 2, 4, false)
-  UGK_POOL(8, 4, 4, true)
-  UGK_POOL(32, 4, 4, true)
-  UGK_POOL(64, 4, 4, true)
-  UGK_POOL(8, 4, 2, false)
-  UGK_POOL(16, 2, 2, false)
-  UGK_POOL(16, 4, 2, false)
-  UGK_POOL(32, 2, 4, false)
-  UGK_POOL(32, 4, 2, false)
-  UGK_POOL(64, 4, 2, false)
+  UGK_POOL(16, 2, 4, false, false)
+  UGK_POOL(8, 4, 4, true, false)
+  UGK_POOL(32, 4, 4, true, false)
+  UGK_POOL(64, 4, 4, true, false)
+  UGK_POOL(8, 4, 2, false, false)
+  UGK_POOL(16, 2, 2, false, false)
+  UGK_POOL(16, 4, 2, false, false)
+  UGK_POOL(32, 2, 4, false, false)
+  UGK_POOL(32, 4, 2, false, false)
+  UGK_POOL(64, 4, 2, false, false)
+  if constexpr (KIND == 0) {
+    UGK_POOL(8, 4, 2, false, true)
+    if constexpr (sizeof(E) == 4) {
+      UGK_POOL(16, 2, 2, false, true)
+    }
+  }
 #undef UGK_POOL
   UGK_REQUIRE(launched, "ugk_extract_pool: no kernel of shape %d", shape);
   UGK_HIP(hipGetLastError());
