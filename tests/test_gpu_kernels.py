@@ -91,6 +91,36 @@ def test_gather_of_rows_that_are_no_whole_vectors(row_bytes, shift):
         assert got[dst].tobytes() == want.tobytes(), n
 
 
+# outputs on both sides of the line beyond which rows of whole vectors below 2 KB are copied by the kernel that deals the
+# output out, and beyond the 16,384 workgroups of a launch and the memory-side cache (256 MiB: the grid strides, the stores
+# are non-temporal)
+@pytest.mark.parametrize("row_bytes,mib", [(272, 8), (272, 13), (400, 17), (800, 17), (1040, 9), (1040, 11), (2064, 1), (1028, 1),
+                                           (1204, 17), (4100, 17), (272, 270), (1204, 270)])
+@pytest.mark.parametrize("hint", [0, 1])
+def test_gather_that_deals_the_output_out(row_bytes, mib, hint):
+    """whole vectors and rows at 4-byte boundaries, ordinary (0: by size) and non-temporal (1) stores, a few keys without a
+    row among them: their rows, and the bytes around the output, stay as they were"""
+    gen = torch.Generator(device="cuda").manual_seed(row_bytes + mib)
+    rows, n, words = 5_003, (mib << 20) // row_bytes, row_bytes // 4
+    table = torch.randint(-(1 << 31), 1 << 31, (rows, words), dtype=torch.int32, device="cuda", generator=gen)
+    keys = torch.randint(0, rows, (n,), device="cuda", generator=gen)
+    bad = torch.rand(n, device="cuda", generator=gen) < 0.01
+    bad[0] = bad[n - 1] = False
+    q = torch.where(bad, rows, keys)
+    out = torch.full((n * words + 8,), 0x7E7E7E7E, dtype=torch.int32, device="cuda")
+    st = dev_zeros_u32(1)
+    hip.call("ugk_set_output_hint", hint)
+    try:
+        hip.call("ugk_gather_direct_i64", ptr(table), rows, ptr(q), n, ptr(out) + 16, row_bytes, 0, ptr(st), None, None)
+    finally:
+        hip.call("ugk_set_output_hint", 0)
+    assert status_value(st) == hip.ST_KEY_OUT_OF_RANGE
+    want = table[keys]
+    want[bad] = 0x7E7E7E7E
+    assert torch.equal(out[4 : 4 + n * words].view(n, words), want)
+    assert (out[:4] == 0x7E7E7E7E).all() and (out[4 + n * words :] == 0x7E7E7E7E).all()
+
+
 def test_gather_direct_empty_and_capped_grid():
     rng = np.random.default_rng(1)
     table = _rand_table(rng, 100, 512)

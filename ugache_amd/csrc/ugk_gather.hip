@@ -477,17 +477,28 @@ uint32_t flat_tile(size_t row_bytes) {
   return best;
 }
 
-// Which dense gathers deal the output out instead of the rows.  Measured, us per launch, rows out of 4 GiB of HBM:
-//   rows of whole vectors, against gather_kernel's 2^k lanes per row, which idle unless the row is 2^k vectors:
-//     160 bytes: 65,536 keys 7.4 -> 8.2, 262,144 keys 23.4 -> 22.1, 1 M keys 73.0 -> 70.8; 400 bytes: 13.9 -> 13.7, 42.6 ->
-//     40.8, 165.1 -> 165.4; 640 bytes: 18.4 -> 18.0, 58.6 -> 53.4; 800 bytes: 23.1 -> 22.0, 78.6 -> 79.3; 1600 bytes: 38.0 ->
-//     36.4, 153.6 -> 148.3; rows of 2^k vectors from 256 to 2048 bytes are level or up to 3 % slower
+// Which dense gathers deal the output out instead of the rows.  Measured, us per launch, rows out of HBM:
+//   rows of whole vectors, against gather_kernel's 2^k lanes per row, which idle unless the row is 2^k vectors; by
+//   wavefronts of that kernel (four rows of up to 64 vectors each, eight of up to 32), lanes -> this: 272 bytes 3,855 6.3 ->
+//   6.8, 5,782 9.2 -> 8.4, 30,840 32.6 -> 30.4; 400 bytes 3,932 7.6 -> 8.1, 5,243 10.5 -> 9.6, 20,971 30.4 -> 28.9; 528 bytes
+//   3,972 6.0 -> 6.6, 5,958 8.8 -> 8.0, 31,775 30.1 -> 28.2; 912 bytes 3,449 7.3 -> 7.9, 4,599 9.7 -> 9.3, 18,396 28.3 ->
+//   27.0.  Up to four wavefronts per SIMD the lanes are the faster ones, beyond that this.  Rows of more than 64 vectors,
+//   by bytes of output, 1 / 8 / 12 / 64 MiB: 1200 bytes 3.9 / 6.4 / 8.1 / 30.0 -> 3.7 / 6.4 / 7.8 / 26.8; 1616 bytes 3.9 / 6.0 /
+//   7.7 / 27.2 -> 3.7 / 6.4 / 7.8 / 26.4; 2064 bytes 4.3 / 6.5 / 8.3 / 29.1 -> 3.7 / 6.4 / 7.7 / 26.2; 9008 bytes 8.3 / 10.4 /
+//   11.2 / 26.9 -> 3.7 / 6.2 / 7.7 / 25.7.  Rows of 160 bytes and rows of 2^k vectors are level or slower at any size
 //   other rows, against gather_flat_kernel: 404 bytes: 65,536 keys 13.4 -> 14.4, 262,144 keys 42.5 -> 44.6; 804 bytes: 21.9
 //     -> 22.3, 71.6 -> 74.3; 1204 bytes: 32.3 -> 30.5, 137.6 -> 124.4; 2404 bytes: 55.1 -> 52.3; 3000 bytes: 66.1 -> 62.6
 //     (the vectors that two rows share cost two loads and a store per row, which short rows have too many of)
-bool stream_pays(uintptr_t align, const void *out, size_t row_bytes) {
-  if (align % 16 == 0) return row_bytes >= kStreamMinBytes && (row_bytes & (row_bytes - 1)) != 0;
-  return align % 4 == 0 && (uintptr_t)out % 16 == 0 && row_bytes >= 1024;
+// Over the host link a row is better asked for by one instruction: 24 MiB of 272 bytes with 32 / 128 workgroups 654 / 654 ->
+// 675 / 697, 800 bytes 508 / 508 -> 524 / 519, 1600 bytes 475 / 476 -> 491 / 479, 2404 bytes (flat) 493 / 482 -> 503 / 481.  A
+// launch whose grid the caller caps is one of those.
+bool stream_pays(uintptr_t align, const void *out, size_t row_bytes, size_t n, unsigned max_blocks) {
+  if (max_blocks) return false;
+  if (align % 16 != 0) return align % 4 == 0 && (uintptr_t)out % 16 == 0 && row_bytes >= 1024;
+  if (row_bytes < kStreamMinBytes || (row_bytes & (row_bytes - 1)) == 0) return false;
+  if (row_bytes > 1024) return row_bytes >= 2048 || n * row_bytes >= (size_t)10 << 20;
+  const size_t rows_per_wave = row_bytes > 512 ? 4 : 8;
+  return n / rows_per_wave > (size_t)cu_count() * 16;
 }
 
 template <typename Idx>
@@ -540,7 +551,7 @@ int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_
   return launch_vec<V, Idx>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks, status,      \
                             host_mirror, st)
   if constexpr (Idx::kDense) {
-    if (stream_pays(align, out, row_bytes))
+    if (stream_pays(align, out, row_bytes, n, max_blocks))
       return launch_stream<Idx>(ix, src, src_rows, out, row_bytes, n, max_blocks, status, host_mirror, st);
   }
   if (align % 16 == 0) UGK_VEC(u32x4);
