@@ -98,14 +98,26 @@ def test_gather_of_rows_that_are_no_whole_vectors(row_bytes, shift):
                                            (1204, 17), (4100, 17), (272, 270), (1204, 270)])
 @pytest.mark.parametrize("hint", [0, 1])
 def test_gather_that_deals_the_output_out(row_bytes, mib, hint):
-    """whole vectors and rows at 4-byte boundaries, ordinary (0: by size) and non-temporal (1) stores, a few keys without a
-    row among them: their rows, and the bytes around the output, stay as they were"""
-    gen = torch.Generator(device="cuda").manual_seed(row_bytes + mib)
-    rows, n, words = 5_003, (mib << 20) // row_bytes, row_bytes // 4
+    """whole vectors and rows at 4-byte boundaries, ordinary (0: by size) and non-temporal (1) stores"""
+    _gather_with_keys_that_miss(row_bytes, (mib << 20) // row_bytes, hint)
+
+
+# both sides of the lines between 16 lanes of 4 bytes, small tiles of the flat copy and full ones
+@pytest.mark.parametrize("row_bytes,n", [(20, 65_536), (36, 65_537), (60, 65_536), (68, 65_536), (100, 83_886), (300, 27_962),
+                                         (804, 10_433), (804, 10_434), (1020, 9_001)])
+def test_flat_gather_at_the_edges_of_its_tiles(row_bytes, n):
+    _gather_with_keys_that_miss(row_bytes, n, 0)
+
+
+def _gather_with_keys_that_miss(row_bytes, n, hint):
+    """a few keys without a row: their rows, and the bytes around the output, stay as they were"""
+    gen = torch.Generator(device="cuda").manual_seed(row_bytes + n)
+    rows, words = 5_003, row_bytes // 4
     table = torch.randint(-(1 << 31), 1 << 31, (rows, words), dtype=torch.int32, device="cuda", generator=gen)
     keys = torch.randint(0, rows, (n,), device="cuda", generator=gen)
     bad = torch.rand(n, device="cuda", generator=gen) < 0.01
     bad[0] = bad[n - 1] = False
+    bad[n // 2] = True
     q = torch.where(bad, rows, keys)
     out = torch.full((n * words + 8,), 0x7E7E7E7E, dtype=torch.int32, device="cuda")
     st = dev_zeros_u32(1)

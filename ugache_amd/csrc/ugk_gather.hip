@@ -16,6 +16,7 @@
 //     gather_stream_kernel (long ones that come out in the order of the keys);
 //   * keys / index records are range-checked against the source's row count: a bad key sets a status bit
 //     and its row is skipped instead of faulting.
+#include <algorithm>
 #include <cstdlib>
 
 #include "ugk_internal.h"
@@ -451,9 +452,10 @@ int launch_vec(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t o
     if (vpr <= 16) UGK_GO(16);
     if (vpr <= 32) UGK_GO(32);
     UGK_GO(64);
-  } else if constexpr (sizeof(V) == 4) {  // rows of up to 16 bytes: the longer ones are copied flat
+  } else if constexpr (sizeof(V) == 4) {  // rows of up to 16 bytes, longer ones in small launches (see launch_gather)
     if (vpr <= 1) UGK_GO(1);
-    UGK_GO(4);
+    if (vpr <= 4) UGK_GO(4);
+    UGK_GO(16);
   } else {
     if (vpr <= 1) UGK_GO(1);
     if (vpr <= 16) UGK_GO(16);
@@ -464,9 +466,13 @@ int launch_vec(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t o
 
 // Rows per wavefront of a flat copy: the fewest that fill nine tenths of the last round of 4 vectors per lane, or the
 // number that fills it best.  Few, because wavefronts that start in order keep the rows being written in one window
-// (see gather_grid).
-uint32_t flat_tile(size_t row_bytes) {
+// (see gather_grid).  A small launch is a wavefront's own time, not bandwidth: up to 65,536 rows and 8 MiB are spread over
+// more wavefronts of half a round, at most 16 rows (100 bytes x 2,048 3.8 -> 3.4 us, 252 bytes x 2,048 3.6 -> 3.4, 600 bytes x
+// 2,048 4.8 -> 3.7, x 16,384 7.6 -> 6.6; 4-byte or 8-byte lanes, which the flat copy replaces, 3.3, 3.3, 4.1 and 7.6).
+uint32_t flat_tile(size_t row_bytes, size_t n) {
   const size_t chunks = (row_bytes + 15) / 16, round = 4 * kWave;
+  if (n <= 65536 && n * row_bytes <= (size_t)8 << 20)
+    return (uint32_t)std::min<size_t>(std::max<size_t>(round / 2 / chunks, 1), 16);
   uint32_t best = 1;
   double best_fill = 0;
   for (uint32_t t = 1; t <= (uint32_t)kWave && t * chunks <= 4 * round; ++t) {
@@ -505,7 +511,7 @@ template <typename Idx>
 int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, size_t row_bytes,
                 const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
                 uint32_t *host_mirror, hipStream_t stream) {
-  const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes));
+  const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes, n));
   const size_t per_block = (size_t)f.tile * kWavesPerBlock;
   const unsigned grid = gather_grid((n + per_block - 1) / per_block, max_blocks);
   hipLaunchKernelGGL((gather_flat_kernel<Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src, src_rows,
@@ -555,6 +561,9 @@ int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_
       return launch_stream<Idx>(ix, src, src_rows, out, row_bytes, n, max_blocks, status, host_mirror, st);
   }
   if (align % 16 == 0) UGK_VEC(u32x4);
+  // short rows in small launches: 16 lanes of 4 bytes have less to do before their first load than the flat copy (36 bytes x
+  // 2,048 3.2 / 3.8 us, x 65,536 5.0 / 5.3, x 262,144 14.6 / 10.6; 52 bytes x 8,192 3.3 / 4.0, x 65,536 5.4 / 6.1)
+  if (align % 4 == 0 && row_bytes <= 64 && n <= 65536) UGK_VEC(uint32_t);
   if (flat_row_ok(align, row_bytes))
     return launch_flat<Idx>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks, status,
                             host_mirror, st);
