@@ -102,9 +102,10 @@ def test_gather_that_deals_the_output_out(row_bytes, mib, hint):
     _gather_with_keys_that_miss(row_bytes, (mib << 20) // row_bytes, hint)
 
 
-# both sides of the lines between 16 lanes of 4 bytes, small tiles of the flat copy and full ones
+# both sides of the lines between 16 lanes of 4 bytes, small tiles of the flat copy and full ones, and between four lanes
+# of 4 bytes and one of 8 bytes
 @pytest.mark.parametrize("row_bytes,n", [(20, 65_536), (36, 65_537), (60, 65_536), (68, 65_536), (100, 83_886), (300, 27_962),
-                                         (804, 10_433), (804, 10_434), (1020, 9_001)])
+                                         (804, 10_433), (804, 10_434), (1020, 9_001), (8, 262_144), (8, 262_145)])
 def test_flat_gather_at_the_edges_of_its_tiles(row_bytes, n):
     _gather_with_keys_that_miss(row_bytes, n, 0)
 
