@@ -110,6 +110,31 @@ def test_flat_gather_at_the_edges_of_its_tiles(row_bytes, n):
     _gather_with_keys_that_miss(row_bytes, n, 0)
 
 
+@pytest.mark.parametrize("row_bytes", [36, 68, 200, 320, 324])
+@pytest.mark.parametrize("capped", [0, 32])
+def test_host_group_of_rows_that_are_no_whole_vectors(row_bytes, capped):
+    """the host group of a batch, which comes last in its list, over the host link, with and without a cap on the grid"""
+    rng = np.random.default_rng(row_bytes)
+    rows, n, n_host = 3_000, 9_001, 7_777
+    table = _rand_table(rng, rows, row_bytes)
+    pin = pinned_from(table)
+    try:
+        idx = np.zeros(n, IDX_DTYPE)
+        idx["src"] = rng.integers(0, rows, size=n)
+        idx["dst_off"] = rng.permutation(n)
+        d_idx, counts, st = to_dev(idx), to_dev(np.array([n - n_host, n_host], np.uint32)), dev_zeros_u32(1)
+        out = dev_bytes(n * row_bytes, fill=0xCD)
+        hip.call("ugk_gather_group", pin.ptr, rows, ptr(d_idx), ptr(counts), hip.LOC_HOST, n, ptr(out), n, row_bytes, capped,
+                 ptr(st), None, None)
+        assert status_value(st) == 0
+        want = np.full((n, row_bytes), 0xCD, np.uint8)
+        want[idx["dst_off"][n - n_host :]] = table[idx["src"][n - n_host :]]
+        assert to_np(out)[: n * row_bytes].tobytes() == want.tobytes()
+    finally:
+        sync()
+        pin.free()
+
+
 def _gather_with_keys_that_miss(row_bytes, n, hint):
     """a few keys without a row: their rows, and the bytes around the output, stay as they were"""
     gen = torch.Generator(device="cuda").manual_seed(row_bytes + n)

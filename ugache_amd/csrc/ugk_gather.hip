@@ -457,7 +457,8 @@ int launch_vec(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t o
   } else if constexpr (sizeof(V) == 4) {  // rows of up to 16 bytes, longer ones in small launches (see launch_gather)
     if (vpr <= 1) UGK_GO(1);
     if (vpr <= 4) UGK_GO(4);
-    UGK_GO(16);
+    if (vpr <= 16) UGK_GO(16);
+    UGK_GO(64);
   } else {
     if (vpr <= 1) UGK_GO(1);
     if (vpr <= 16) UGK_GO(16);
@@ -566,6 +567,11 @@ int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_
   // short rows in small launches: 16 lanes of 4 bytes have less to do before their first load than the flat copy (36 bytes x
   // 2,048 3.2 / 3.8 us, x 65,536 5.0 / 5.3, x 262,144 14.6 / 10.6; 52 bytes x 8,192 3.3 / 4.0, x 65,536 5.4 / 6.1)
   if (align % 4 == 0 && row_bytes <= 64 && n <= 65536) UGK_VEC(uint32_t);
+  // the host group of a batch, with no cap on the grid: so many requests at once the link answers better where each is one
+  // instruction of 4-byte lanes (16 MiB of 100 / 148 / 200 / 252 / 300 bytes 753 / 587 / 497 / 455 / 459 us, flat 815 / 661 /
+  // 571 / 519 / 485; 404 bytes 436 and 433); behind a cap the flat copy is the faster one (32 workgroups, 200 bytes 663 and
+  // 522 us)
+  if (align % 4 == 0 && counts && group == UGK_LOC_HOST && max_blocks == 0 && row_bytes <= 320) UGK_VEC(uint32_t);
   if (flat_row_ok(align, row_bytes))
     return launch_flat<Idx>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks, status,
                             host_mirror, st);
