@@ -1097,6 +1097,46 @@ def test_pooled_extraction_at_the_edges_of_its_shapes(kind, vpr):
             pin.free()
 
 
+@pytest.mark.parametrize("kind", ["none", "flat"])
+@pytest.mark.parametrize("vpr", [4, 16, 24, 32, 64])
+def test_pooled_sample_does_not_depend_on_the_others_of_its_batch(kind, vpr):
+    """weighted mean and sqrtn of 200 samples of 3 to 60 ids, the same bytes whether the batch's other samples have two ids
+    or ninety, which the shape of the launch follows"""
+    rng = np.random.default_rng(vpr)
+    nkeys, rb, probes = 2_000, vpr * 16, 200
+    host = rng.standard_normal((nkeys, rb // 4)).astype(np.float32)
+    pin = pinned_from(host.view(np.uint8).reshape(nkeys, rb))
+    cached = rng.choice(nkeys, nkeys // 2, replace=False).astype(np.int64)
+    cache = host[cached].view(np.uint8).reshape(len(cached), rb).copy()
+    mem, tb = (None, hip.table(0, None, 0)) if kind == "none" else _make_flat(nkeys)
+    if kind == "flat":
+        assert _insert(tb, cached) == 0
+    lens = rng.integers(3, 61, size=probes)
+    ids = [rng.integers(0, nkeys, size=n) for n in lens]
+    wts = [(rng.random(n) + 0.5).astype(np.float32) for n in lens]
+    try:
+        d_cache, st = to_dev(cache), dev_zeros_u32(1)
+        for combiner in (1, 2):
+            seen = []
+            for others in (2, 9, 20, 90):
+                more = 20_000 // others
+                all_ids = np.concatenate(ids + [rng.integers(0, nkeys, size=more * others)]).astype(np.int64)
+                all_w = np.concatenate(wts + [np.ones(more * others, np.float32)])
+                off = np.concatenate([[0], np.cumsum(np.concatenate([lens, np.full(more, others)]))]).astype(np.int64)
+                n_rows = probes + more
+                out = dev_bytes(n_rows * rb)
+                d_ids, d_off, d_w = to_dev(all_ids), to_dev(off), to_dev(all_w)
+                hip.call("ugk_extract_pool_i64", tb, ptr(d_ids), ptr(d_off), ptr(d_w), n_rows, len(all_ids), combiner, 4,
+                         ptr(d_cache), 0 if kind == "none" else len(cached), pin.ptr, nkeys, ptr(out), rb, ptr(st), None,
+                         None, None, None)
+                assert status_value(st) == 0
+                seen.append(to_np(out)[: probes * rb].tobytes())
+            assert all(b == seen[0] for b in seen), (combiner, [b == seen[0] for b in seen])
+    finally:
+        sync()
+        pin.free()
+
+
 @pytest.mark.parametrize("rows_per_group", ["", "2", "8"])
 def test_pooled_extraction_hand_worked(rows_per_group, monkeypatch):
     if rows_per_group:

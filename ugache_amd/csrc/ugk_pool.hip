@@ -103,6 +103,8 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
   constexpr int RPW = kWave / LPR;  // output rows per wavefront and pass
   constexpr int EPC = PoolElem<E>::kPerChunk;
   static_assert(LPR % U == 0, "ids are taken in rounds of U");
+  constexpr int kParts = LPR * CH <= 32 ? 8 : LPR * CH <= 128 ? 32 : 64;  // sums of weights per sample (see below)
+  static_assert(LPR * 2 >= kParts && LPR <= kParts * 2, "a lane has one sum of weights, two, or half of one");
   const int lane = (int)lane_id();
   const int sub = lane % LPR, rg = lane / LPR;
   const size_t wave_global = (size_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
@@ -128,8 +130,10 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
     for (int c = 0; c < CH; ++c)
 #pragma unroll
       for (int e = 0; e < EPC; ++e) acc[c][e] = 0.f;
-    // this lane's share of the row's sum of weights (or of their squares); with four lanes the rounds alternate between
-    // two sums, so that the weights are added in the order in which eight lanes add them
+    // This lane's share of the row's sum of weights (or of their squares), added in an order that the row's length fixes and
+    // the shape does not: kParts sums, sum k over the ids k, k + kParts, ... of the sample.  Fewer lanes than sums take two
+    // in turn; twice as many lanes keep each sum twice and add two ids a round to it.  (The shape depends on the whole
+    // batch: without this a sample's last bits would depend on the samples beside it.)
     float wsum = 0.f, wsum_odd = 0.f;
     bool odd = false;
     for (long long j0 = beg; __ballot(j0 < end) != 0ull; j0 += LPR) {  // until every group of the wavefront is through
@@ -144,10 +148,6 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
       }
       const bool use = active && row.has_row;  // a key without a row adds nothing (the launch is flagged)
       const float w = use ? (weights ? weights[j] : 1.f) : 0.f;
-      const float wterm = combiner == 2 ? w * w : w;
-      if (LPR == 4 && odd) wsum_odd += wterm;
-      else wsum += wterm;
-      odd = !odd;
       for (int s0 = 0; s0 < LPR; s0 += U) {
         if (__ballot(active && sub >= s0) == 0ull) break;  // no group has an id left in this round
         grow_t p[U];
@@ -223,11 +223,27 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
           }
         }
       }
+      // (behind the rows: in front of them their loads would wait for the weights)
+      const float wterm = combiner == 2 ? w * w : w;
+      if constexpr (LPR < kParts) {
+        if (odd) wsum_odd += wterm;
+        else wsum += wterm;
+        odd = !odd;
+      } else if constexpr (LPR > kParts) {
+        static_assert(LPR == 16 && kParts == 8, "lane l and lane l xor 8 of 16");
+        constexpr int kRowRor8 = 0x128;  // DPP control: the 16 lanes of a row rotated by 8, no trip through LDS
+        const float other = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(wterm), kRowRor8, 0xf, 0xf, true));
+        const bool second = (sub & kParts) != 0;
+        wsum += second ? other : wterm;
+        wsum += second ? wterm : other;
+      } else {
+        wsum += wterm;
+      }
     }
     // the row's denominator: every lane of the group holds a share
-    if (LPR == 4) wsum += wsum_odd;
+    if constexpr (LPR < kParts) wsum += wsum_odd;
 #pragma unroll
-    for (int d = LPR / 2; d > 0; d >>= 1) wsum += __shfl_xor(wsum, d);
+    for (int d = (LPR < kParts ? LPR : kParts) / 2; d > 0; d >>= 1) wsum += __shfl_xor(wsum, d);
     const float denom = combiner == 1 ? wsum : combiner == 2 ? sqrtf(wsum) : 1.f;
     if (row_ok) {
 #pragma unroll
@@ -513,7 +529,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
     else if (upto12 && vpr < 32) shape = 842, keep_waves = 3;
     else if (nnz > rows64 * 24 && sizeof(E) == 4) shape = 1622, keep_waves = 3;
   }
-  if (const char *forced = getenv("UGK_POOL_LPR")) {  // for sweeps; never a byte of the result depends on it
+  if (const char *forced = getenv("UGK_POOL_LPR")) {  // for sweeps; a weighted mean's last bits may vary with it
     const int v = atoi(forced);
     if (!clip && (v == 8 || v == 32 || v == 64) && vpr <= (uint32_t)v * kPoolChunks)
       shape = v * 100 + 42, keep_waves = kWavesPerBlock;
