@@ -177,7 +177,9 @@ int ugk_copy_rows(void *dst_dev, const void *src_dev, size_t nbytes, void *strea
  * non-temporal stores whatever the size (a caller that rotates its outputs over more buffers than the cache holds: the
  * rows of one launch are evicted by the next anyway, and evicting them costs more than streaming them, 51.4 us against
  * 47.5 us for 262,144 rows of 512 bytes).  UGK_OUTPUT_STAYS: ordinary stores whatever the size.  Never a byte of the
- * result depends on it.  The environment variable UGK_GATHER_NT_STORE=0/1 overrides both. */
+ * result depends on it.  The environment variable UGK_GATHER_NT_STORE=0/1 overrides both.  Rows whose length or buffers
+ * are multiples of 4 bytes only are written with ordinary stores whatever the hint says, but for dense gathers of 1024
+ * bytes a row and more: their lines leave in pieces, and at no size did non-temporal stores gain more than 2 %. */
 #define UGK_OUTPUT_AUTO 0
 #define UGK_OUTPUT_STREAMS 1
 #define UGK_OUTPUT_STAYS 2

@@ -23,8 +23,11 @@ typedef __attribute__((address_space(1))) u32x4 *gout_t;
 // bytes: a row of R bytes at a random multiple of 4 touches (R + 124) / 128 of them.  What it replaced were lanes of 4 or
 // 8 bytes, 16 or 64 to a row; gathers of 262,144 rows out of 4 GiB of HBM, before -> after: 36 bytes 14.6 -> 10.6 us,
 // 100 bytes 38.0 -> 17.0 us (5.0 TB/s of lines read and rows written), 200 bytes 44.3 -> 25.7, 404 bytes 64.3 -> 42.7,
-// 804 bytes 137.8 -> 71.6.  The stores are ordinary ones whatever the size of the output: rows that end inside a line
-// leave it in two pieces, which non-temporal stores write out apart (804 bytes: 71.6 us, non-temporal 89.3).
+// 804 bytes 137.8 -> 71.6.  The stores are ordinary ones whatever the size of the output and whatever ugk_set_output_hint says:
+// rows that end inside a line leave it in two pieces, which non-temporal stores write out apart.  us per launch, ordinary /
+// non-temporal: 804 bytes, one buffer of 224 / 288 / 600 MiB 80 / 100, 123 / 130, 266 / 270, four of 224 MiB in turn 99.5 /
+// 100; 200 bytes 99 / 119, 151 / 155, 319 / 323 and 116 / 119; 1020 bytes 78 / 100, 121 / 132, 265 / 278 and 96 / 101; only
+// rows of 36 bytes are 2 % the other way beyond the memory-side cache, 317 / 312 for 288 MiB.
 typedef u32x4 u32x4_by4 __attribute__((aligned(4)));
 typedef const __attribute__((address_space(1))) u32x4_by4 *grow_by4_t;
 typedef __attribute__((address_space(1))) u32x4_by4 *gout_by4_t;

@@ -594,16 +594,11 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
     }                                               \
     UGK_GO2(L, kWave);                              \
   } while (0)
-#define UGK_FLAT(W)                 \
-  do {                              \
-    if (nt) UGK_GO4(0, W, true, false); \
-    else UGK_GO4(0, W, false, false);   \
-  } while (0)
-  if (flat) {
-    if (kpw == 8) UGK_FLAT(8);
-    else if (kpw == 16) UGK_FLAT(16);
-    else if (kpw == 32) UGK_FLAT(32);
-    else UGK_FLAT(kWave);
+  if (flat) {  // ordinary stores whatever the size (see flat_copy)
+    if (kpw == 8) UGK_GO4(0, 8, false, false);
+    else if (kpw == 16) UGK_GO4(0, 16, false, false);
+    else if (kpw == 32) UGK_GO4(0, 32, false, false);
+    else UGK_GO4(0, kWave, false, false);
   } else if (vpr <= 1) UGK_GO2(1, kWave);
   else if (vpr <= 2) UGK_GO(2);
   else if (vpr <= 4) UGK_GO(4);
@@ -611,7 +606,6 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   else if (vpr <= 16) UGK_GO(16);
   else if (vpr <= 32) UGK_GO(32);
   else UGK_GO(64);
-#undef UGK_FLAT
 #undef UGK_GO
 #undef UGK_GO2
 #undef UGK_GO3
