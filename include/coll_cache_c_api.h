@@ -129,7 +129,8 @@ void coll_cache_forward_pooled_i64(int replica_id, const int64_t *key, const int
  * (COLL_GPU_RECORD=1) the counting is one more kernel of the recorded lookup, so every replay counts the keys it
  * reads.  Batches the
  * one-kernel paths cannot take (COLL_DEDUP_KEYS, a factored
- * SAMGRAPH_COLL_CACHE_CONCURRENT_LINK_IMPL, rows not multiples of 16 bytes with a partial cache) block as usual. */
+ * SAMGRAPH_COLL_CACHE_CONCURRENT_LINK_IMPL, and with a partial cache rows or an output that are neither multiples of 16
+ * bytes nor multiples of 4 with rows of at least 20) block as usual. */
 void coll_cache_lookup_async(int replica_id, const uint32_t *key, size_t num_keys, void *output, StreamHandle stream);
 void coll_cache_lookup_async_i64(int replica_id, const int64_t *key, size_t num_keys, void *output,
                                  StreamHandle stream);

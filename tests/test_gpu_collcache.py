@@ -450,7 +450,7 @@ def test_bfloat16_table_is_looked_up_as_its_bytes(pct):
 @pytest.mark.parametrize("dim,dtype", [(3, torch.float32), (5, torch.float16), (1, torch.float32), (7, torch.float32)])
 @pytest.mark.parametrize("pct", [0.2, 1.0, 0.0])
 def test_rows_that_are_not_multiples_of_16_bytes(dim, dtype, pct):
-    """12-, 10-, 4- and 28-byte rows: the 16-byte-lane kernels do not apply, narrower lanes take over"""
+    """12-, 10- and 4-byte rows, which narrower lanes take, and 28-byte rows, 16-byte vectors at 4-byte boundaries"""
     rng = np.random.default_rng(dim)
     n_item = 9_000
     if dtype == torch.float16 and dim % 2:

@@ -296,8 +296,9 @@ class ExtractSession {
   // Stream-ordered variants (an extension; the reference's lookup always blocks): the kernels of the batch are
   // enqueued on `stream` and the call returns without waiting; `output` is complete for whatever is enqueued on the
   // same stream afterwards.  All stream-ordered lookups of a session must use one stream.  Error flags, group sizes
-  // and profiler values are collected by Wait().  Batches the fused / direct kernels cannot take (deduplication on,
-  // rows not multiples of 16 bytes, a factored mode selected) run through the blocking path instead.
+  // and profiler values are collected by Wait().  Batches the fused / direct kernels cannot take (deduplication on, a
+  // factored mode selected, with a partial cache rows or buffers that are neither multiples of 16 bytes nor multiples of 4
+  // with rows of at least 20) run through the blocking path instead.
   void ExtractFeatAsync(const IdType *nodes, const size_t num_nodes, void *output, StreamHandle stream);
   void ExtractFeatAsync64(const Id64Type *nodes, const size_t num_nodes, void *output, StreamHandle stream);
   // blocks until every stream-ordered lookup enqueued so far has finished, aborts if one of them met a key outside
