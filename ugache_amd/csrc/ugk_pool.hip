@@ -294,10 +294,10 @@ constexpr int kPoolMaxRows = 8;  // output rows a lane group may own per pass
 // moves on to a later one.  What keeps memory busy is then the number of ids, not the shape of the segments: with one
 // row per group a sample of one id leaves most of the group's lookups and loads unused.  The bookkeeping costs
 // registers (three wavefronts per SIMD instead of four) and a lane's chunks are read one after the other, so it is not
-// for flat tables, behind which rows come over the host link: samples of one id over rows of 512 bytes, all in HBM, 115
-// us for 390,625 of them against 124 with one row per group; 60 % of the table uncached behind a flat table, 262,144 of
-// them, 123 against 98 us; behind a hash table, whose lookup works on all lanes of a wavefront at once and wants them
-// to hold ids, 195,312 of them 107 against 128 us.
+// for flat tables, behind which rows come over the host link: 60 % of the table uncached behind a flat table, 262,144 samples
+// of one id over rows of 512 bytes, 123 against 98 us with one row per group; behind a hash table, whose lookup works on all
+// lanes of a wavefront at once and wants them to hold ids, 195,312 of them 107 against 128 us.  (Without any table the rule
+// in extract_pool_lpr says which rows it is for.)
 template <typename K, int KIND, int LPR, typename E, bool KEEP>
 __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K *__restrict__ ids,
                                                    const long long *__restrict__ seg_off,
@@ -514,18 +514,19 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   else if (vpr <= 128) shape = 3242;
   else shape = 6442;
   // Rows all in HBM whose ordinary loads cost uniform ids something: some wavefronts load them non-temporally (see
-  // pool_samples), in a shape that makes up for what that costs skewed ones.  800,000 ids, fp32, without the hint / this,
-  // uniform and Zipf 1.05 (all loads non-temporal and one chunk at a time, before either): 384 bytes 4 ids 76.9 / 68.5 and
-  // 56.2 / 52.1 (71.4 and 62.4), 8 ids 68.6 / 62.7 and 39.2 / 38.9 (66.1 and 51.0), 40 ids 60.3 / 53.4 and 35.1 / 29.3
-  // (55.8 and 44.7); 512 bytes 2 ids 119.7 / 111.2 and 88.7 / 87.0 (116.1 and 121.6), 4 ids 100.6 / 93.4 and 61.6 / 59.4
-  // (92.7 and 78.7), 40 ids 78.6 / 70.9 and 40.2 / 36.9 (73.0 and 55.4).  Left alone, for it takes from skewed ids what it
-  // gives uniform ones: 512 bytes 8 ids (89.6 and 45.1; 85.5 and 66.1 before), 400,000 ids of 1 KB 4 ids (98.8 / 91.5 and
-  // 55.6 / 58.3; 92.1 and 85.6 before) and 8 ids (89.3 and 43.4; 85.1 and 66.8), of 2 KB 4 ids (192 and 116; 176 and 151).
-  // Rows of other lengths, which begin and end inside a line, are faster for uniform ids as well with ordinary loads (400
-  // bytes 4 ids 95 against 128).
+  // pool_samples), in a shape that makes up for what that costs skewed ones.  800,000 ids out of 2 GiB, fp32, without the
+  // hint / this, uniform and Zipf 1.05 (all loads non-temporal and one chunk at a time, before either): 384 bytes 4 ids
+  // 76.9 / 68.5 and 56.2 / 52.1 (71.4 and 62.4), 8 ids 68.6 / 62.7 and 39.2 / 38.9 (66.1 and 51.0), 40 ids 60.3 / 53.4 and
+  // 35.1 / 29.3 (55.8 and 44.7); 512 bytes 2 ids 119.7 / 111.2 and 88.7 / 87.0 (116.1 and 121.6), 4 ids 99.6 / 86.8 and 61.3 /
+  // 60.7 (92.0 and 81.5), 6 ids 92.9 / 83.8 and 50.5 / 50.6 (91.3 and 75.6), 40 ids 78.6 / 70.9 and 40.2 / 36.9 (73.0 and
+  // 55.4); out of 6 GiB 4 ids 105 / 89 and 64 / 62 (92 and 80).  Left alone, for it takes from skewed ids what it gives uniform
+  // ones: 512 bytes 8 ids (89.6 and 45.1; 85.5 and 66.1 before; 94 and 47, 86 and 68 out of 6 GiB) and 16 ids (81 and 38; 80
+  // and 62; 88 and 40, 80 and 63 out of 6 GiB), 400,000 ids of 1 KB 4 ids (98.8 / 91.5 and 55.6 / 58.3; 92.1 and 85.6 before)
+  // and 8 ids (89.3 and 43.4; 85.1 and 66.8), of 2 KB 4 ids (192 and 116; 176 and 151).  Rows of other lengths, which begin
+  // and end inside a line, are faster for uniform ids as well with ordinary loads (400 bytes 4 ids 95 against 128).
   if (KIND == 0 && !clip && vpr > 16 && vpr <= 32 && vpr % 8 == 0) {
     if (upto2) keep_waves = vpr == 32 && sizeof(E) == 4 ? 1 : keep_waves;
-    else if (upto6) shape = 842, keep_waves = 2;
+    else if (upto6) shape = 842, keep_waves = vpr == 32 && nnz <= rows64 * 9 / 2 ? 1 : 2;
     else if (upto12 && vpr < 32) shape = 842, keep_waves = 3;
     else if (nnz > rows64 * 24 && sizeof(E) == 4) shape = 1622, keep_waves = 3;
   }
