@@ -282,7 +282,7 @@ int ugk_select_keys_i64(const int64_t *keys_dev, const uint32_t *sel_dev, size_t
 
 /* ---- single-kernel mixed-source extraction: kDirectNoGroup with DataIterMixLoc
  *      (cache_context.cu:137-159, 1295-1329): lookup and gather fused, source picked per row ----------
- * Rows and buffers are multiples of 16 bytes, or of 4 bytes with rows of at least 20 (ugk_extract_mix_staged_*: of 16).
+ * Rows and buffers are multiples of 16 bytes, or of 4 bytes with rows of 20 to 2^30 (ugk_extract_mix_staged_*: of 16).
  * group_counts_host (may be NULL): pinned, GPU-mapped host memory (ugk_host_malloc) of ugk_extract_mix_max_groups()
  * 8-byte words.  Workgroup b leaves in word b, for the keys it handled, (rows not taken from the cache << 32) | rows
  * taken from the cache — a posted write nobody waits for.  *num_groups_host (ordinary host memory, written by the call
