@@ -159,6 +159,15 @@ def _gather_with_keys_that_miss(row_bytes, n, hint):
     assert (out[:4] == 0x7E7E7E7E).all() and (out[4 + n * words :] == 0x7E7E7E7E).all()
 
 
+# launches of one round of workgroups (2,048 on 256 CUs) and of one more, with rows of one vector per lane and of several;
+# wavefronts with a bad key and the batch's last one copy behind a branch, all others without
+@pytest.mark.parametrize("row_bytes,n", [(128, 131_072), (128, 131_073), (512, 32_769), (512, 40_003), (1024, 16_385),
+                                         (4096, 9), (4096, 4097), (4096 + 2048, 1030), (64, 262_145)])
+@pytest.mark.parametrize("hint", [0, 1])
+def test_gather_of_more_than_one_round_of_workgroups(row_bytes, n, hint):
+    _gather_with_keys_that_miss(row_bytes, n, hint)
+
+
 def test_gather_direct_empty_and_capped_grid():
     rng = np.random.default_rng(1)
     table = _rand_table(rng, 100, 512)

@@ -5,8 +5,7 @@
 //   * a row of V 16-byte vectors is copied by LPR = min(64, pow2ceil(V)) adjacent lanes, so one wavefront
 //     instruction moves 64/LPR whole rows as fully coalesced segments (512-B rows: 2 rows, 128-B rows: 8);
 //   * every lane keeps UNROLL = 2 independent rows in flight (both loads issued before the first store) and the
-//     launch uses many small workgroups of one pass each:
-//     measured on MI355X this beats deeper unrolling with fewer, longer-lived workgroups by ~15 %;
+//     launch uses many small workgroups of one pass each (gather_kernel has the figures of one, four and eight rows);
 //   * loads carry the non-temporal hint (table rows are touched once); stores are ordinary write-back stores
 //     while the output fits the 256 MiB memory-side cache, so the consumer finds it there, and non-temporal
 //     beyond that or when the caller says its outputs do not stay there (ugk_set_output_hint);
@@ -84,11 +83,20 @@ __device__ __forceinline__ void st_stream(V *p, V v) {
 
 // NT_STORE is a template parameter, not a launch argument: with a run-time flag the optimiser merges the two stores
 // of `if (nt) stream(p, v); else *p = v;` into one and the non-temporal hint is lost (seen with UNROLL = 1).
+// Bound by HBM.  Where the launch is more than one round of workgroups (many_groups), or a lane has several vectors of a
+// row, a wavefront whose rows are all there and all good, which is every one but the batch's last, copies them without a
+// branch: behind one each load waits for the one before.  Rows out of 5 GiB, us per launch with the branch / without:
+// 512 bytes x 65,536 15.5 / 14.7, x 262,144 45.5 / 44.8 (6.0 TB/s); 1 KB x 32,768 15.5 / 14.7, x 262,144 83.1 / 81.5; 4 KB x 2,048
+// 6.8 / 6.4, x 8,192 15.5 / 14.1, x 131,072 193 / 188; 128 bytes x 196,608 13.4 / 12.2.  A launch that is all on the chip at
+// once is no faster for it and up to 5 % slower near that size: 512 bytes x 16,384 5.8 / 5.7, x 32,768 8.5 / 9.0, x 36,000
+// 10.5 / 10.3, 64 bytes x 262,144 11.3 / 11.7, 128 bytes x 131,072 8.7 / 9.1.  Rows in flight per lane, one / two / four /
+// eight, all without: 512 bytes x 65,536 15.9 / 14.7 / 15.1 / 15.5, x 524,288 91.1 / 82.4 / 82.5 / 83.5; 4 KB x 32,768 43.4 /
+// 43.4 / 51.9 / 48.4; 16 bytes x 32,768 3.8 / 4.5 / 5.8 / 9.0.
 template <typename V, int LPR, int UNROLL, bool NT_STORE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restrict__ src, uint64_t src_rows,
                                                         V *__restrict__ out, uint64_t out_rows, uint32_t vpr,
                                                         const uint32_t *__restrict__ counts, uint32_t group, size_t n,
-                                                        uint32_t *status, uint32_t *host_mirror) {
+                                                        bool many_groups, uint32_t *status, uint32_t *host_mirror) {
   size_t begin = 0, count = n;
   if (counts) {
     const uint32_t c = counts[group];
@@ -122,19 +130,34 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
         }
       }
     }
+    bool whole = true;
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) whole = whole && ok[u];
+    // (rows of up to 64 bytes gain nothing and stay as they were)
+    const bool no_branch = LPR >= 8 && (many_groups || vpr > LPR) && __ballot(!whole) == 0ull;
     for (uint32_t c0 = 0; c0 < vpr; c0 += LPR) {
       const uint32_t col = c0 + lane;
       if (col < vpr) {
         V v[UNROLL];
+        if (no_branch) {
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u)
-          if (ok[u]) v[u] = ld_stream(src + s[u] * vpr + col);
+          for (int u = 0; u < UNROLL; ++u) v[u] = ld_stream(src + s[u] * vpr + col);
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u)
-          if (ok[u]) {
+          for (int u = 0; u < UNROLL; ++u) {
             if constexpr (NT_STORE) st_stream(out + d[u] * vpr + col, v[u]);
             else out[d[u] * vpr + col] = v[u];
           }
+        } else {
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+            if (ok[u]) v[u] = ld_stream(src + s[u] * vpr + col);
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+            if (ok[u]) {
+              if constexpr (NT_STORE) st_stream(out + d[u] * vpr + col, v[u]);
+              else out[d[u] * vpr + col] = v[u];
+            }
+        }
       }
     }
   }
@@ -414,14 +437,15 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
                     uint32_t *host_mirror, bool nt, hipStream_t stream) {
   constexpr size_t kPerIter = (size_t)(kBlock / LPR) * UNROLL;
   const unsigned grid = gather_grid((n + kPerIter - 1) / kPerIter, max_blocks);
+  const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
   if (nt)
     hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, true, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,
                        reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,
-                       group, n, status, host_mirror);
+                       group, n, many_groups, status, host_mirror);
   else
     hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, false, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,
                        reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,
-                       group, n, status, host_mirror);
+                       group, n, many_groups, status, host_mirror);
   UGK_HIP(hipGetLastError());
   return 0;
 }
