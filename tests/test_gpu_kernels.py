@@ -542,6 +542,22 @@ def test_hash_table_dense_collisions_and_host_entries():
     assert loc[0] == 1
 
 
+# tables of one line, of less than one pass of the census, of whole passes and of a remainder
+@pytest.mark.parametrize("kind,words", [(2, 2), (3, 1)])
+@pytest.mark.parametrize("entries", [64, 80, 262_144, 1 << 21, (1 << 21) + 16, 3_000_016])
+def test_census_counts_every_entry_once(kind, words, entries):
+    gen = torch.Generator(device="cuda").manual_seed(entries)
+    state = torch.randint(0, 3, (entries,), device="cuda", generator=gen)
+    key = torch.randint(0, 1 << 30, (entries, words), dtype=torch.int64, device="cuda", generator=gen)
+    never, tomb = (-1, -2) if kind == 2 else (-1, 0xFFFFFFFE)
+    key[:, 0] = torch.where(state == 0, key[:, 0], torch.where(state == 1, tomb, never))
+    tb, census = hip.table(kind, ptr(key), entries), torch.full((6,), 77, dtype=torch.int32, device="cuda")
+    assert ptr(key) % 128 == 0
+    hip.call("ugk_table_census", tb, ptr(census), None)
+    sync()
+    assert to_np(census, np.uint64).tolist() == [int((state == k).sum()) for k in range(3)]
+
+
 # ---- the compact hash table (kind 3): keyed by the row a key stands for --------------------------------------------
 def _census(tb):
     cen = torch.zeros(3, dtype=torch.int64, device="cuda")

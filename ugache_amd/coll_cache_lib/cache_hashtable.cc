@@ -28,6 +28,7 @@ void CacheEntryManager::CreateFlat(const std::function<MemHandle(size_t)> &alloc
 }
 
 namespace {
+constexpr unsigned kCensusWord = 16;  // status words 16 .. 21: the counts of ugk_table_census
 size_t HashEntryBytes(int kind) { return kind == 3 ? sizeof(uint64_t) : sizeof(ugk_bucket_t); }
 size_t HashEntriesFor(int kind, size_t num_entries) {
   return kind == 3 ? ugk_hash32_entries_for(num_entries, RunConfig::hash_load_factor)
@@ -123,7 +124,7 @@ void CacheEntryManager::Evict(TensorPtr keys_to_evict, StreamHandle stream) {
   else
     UGK_CALL(ugk_table_evict_u32(RowView(), keys_to_evict->CPtr<uint32_t>(), keys_to_evict->NumItem(),
                                  StatusPtr(this, stream), stream));
-  if (_table.kind >= 2) _num_tombstones += keys_to_evict->NumItem();
+  NoteEvicted(keys_to_evict->NumItem());
 }
 
 void CacheEntryManager::EvictRelease(TensorPtr keys_to_evict, StreamHandle stream) {
@@ -133,22 +134,32 @@ void CacheEntryManager::EvictRelease(TensorPtr keys_to_evict, StreamHandle strea
   else
     UGK_CALL(ugk_table_evict_release_u32(RowView(), keys_to_evict->CPtr<uint32_t>(), keys_to_evict->NumItem(),
                                          SlotUsedBits(), _cache_space_capacity, StatusPtr(this, stream), stream));
-  if (_table.kind >= 2) _num_tombstones += keys_to_evict->NumItem();
+  NoteEvicted(keys_to_evict->NumItem());
+}
+
+void CacheEntryManager::NoteEvicted(size_t n) {
+  if (_table.kind >= 2) _num_tombstones += n;
+  _census_fresh = false;
+}
+
+bool CacheEntryManager::CensusDue() const {
+  return _table.kind >= 2 && (double)_num_tombstones > RunConfig::hash_rebuild_tombstone_frac * (double)_table.size;
 }
 
 bool CacheEntryManager::MaybeRebuild(const std::function<MemHandle(size_t)> &allocator, Context ctx, int loc,
                                      StreamHandle stream, const std::function<void()> &wait_for_lookups) {
-  if (_table.kind < 2) return false;
-  const double limit = RunConfig::hash_rebuild_tombstone_frac * (double)_table.size;
-  if ((double)_num_tombstones <= limit) return false;
-  // _num_tombstones counts evictions; inserts reuse tombstones they pass, so look before rebuilding
-  uint64_t *census_dev = reinterpret_cast<uint64_t *>(StatusPtr(this, stream) + 16);
-  uint64_t census[3] = {0, 0, 0};
-  UGK_CALL(ugk_table_census(_table, census_dev, stream));
-  UGK_CALL(ugk_memcpy_async(census, census_dev, sizeof(census), stream));
-  UGK_CALL(ugk_stream_sync(stream));
-  _num_tombstones = census[1];
-  if ((double)_num_tombstones <= limit) return false;
+  if (!CensusDue()) return false;
+  // _num_tombstones counts evictions; inserts reuse tombstones they pass, so look before rebuilding (unless
+  // StatusAndWords has looked since the last of them)
+  if (!_census_fresh) {
+    uint64_t *census_dev = reinterpret_cast<uint64_t *>(StatusPtr(this, stream) + kCensusWord);
+    uint64_t census[3] = {0, 0, 0};
+    UGK_CALL(ugk_table_census(_table, census_dev, stream));
+    UGK_CALL(ugk_memcpy_async(census, census_dev, sizeof(census), stream));
+    UGK_CALL(ugk_stream_sync(stream));
+    _num_tombstones = census[1];
+    if (!CensusDue()) return false;
+  }
   TensorPtr keys, offs, key_buffer;
   size_t n = 0;
   if (_dev_lists_valid) {  // the cached rows are known on the device: the key list never leaves it
@@ -193,6 +204,7 @@ bool CacheEntryManager::MaybeRebuild(const std::function<MemHandle(size_t)> &all
   if (wait_for_lookups) wait_for_lookups();
   fresh_handle = nullptr;  // the old buckets
   _num_tombstones = 0;
+  _census_fresh = false;
   _num_rebuilds++;
   return true;
 }
@@ -274,13 +286,22 @@ void CacheEntryManager::WaitByTicket(StreamHandle stream) {
 
 uint32_t CacheEntryManager::StatusAndWords(const uint32_t *extra_dev, unsigned n_extra, uint32_t *extra_out,
                                            StreamHandle stream) {
-  CHECK_LE(n_extra, 30u);
   CHECK(_dev_words) << "the table's pinned words come with its device lists";
+  // a census of the table that MaybeRebuild would ask for next comes along, for it costs a wait of its own there
+  const bool census = CensusDue() && !_census_fresh;
+  uint32_t *status = StatusPtr(this, stream);
+  if (census) UGK_CALL(ugk_table_census(_table, reinterpret_cast<uint64_t *>(status + kCensusWord), stream));
+  const unsigned n_own = census ? kCensusWord + 6 : 1;
+  CHECK_LE(n_own + n_extra, 31u);
   if (++_ticket == 0) _ticket = 1;
   uint32_t *dst = DevWords() + 32;
-  UGK_CALL(ugk_words_to_host_ticket(StatusPtr(this, stream), 1, extra_dev, n_extra, dst, _ticket,
-                                    RunConfig::spin_wait_us, stream));
-  for (unsigned i = 0; i < n_extra; ++i) extra_out[i] = dst[2 + i];
+  UGK_CALL(ugk_words_to_host_ticket(status, n_own, extra_dev, n_extra, dst, _ticket, RunConfig::spin_wait_us, stream));
+  for (unsigned i = 0; i < n_extra; ++i) extra_out[i] = dst[1 + n_own + i];
+  if (census) {
+    const uint32_t *tombstones = dst + 1 + kCensusWord + 2;  // the second of three 64-bit counts
+    _num_tombstones = ((size_t)tombstones[1] << 32) | tombstones[0];
+    _census_fresh = true;
+  }
   return dst[1];
 }
 

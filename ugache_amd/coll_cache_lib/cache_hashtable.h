@@ -95,7 +95,10 @@ class CacheEntryManager {
   // only when no lookup that took the old handle is still running, after which the old buckets are released.
   bool MaybeRebuild(const std::function<MemHandle(size_t)> &allocator, Context ctx, int loc, StreamHandle stream,
                     const std::function<void()> &wait_for_lookups);
-  size_t _num_tombstones = 0;
+  bool CensusDue() const;       // more evictions since the last census than the rebuild limit
+  void NoteEvicted(size_t n);
+  size_t _num_tombstones = 0;   // at the last census, and the keys evicted since
+  bool _census_fresh = false;   // _num_tombstones is a census, nothing has been evicted since
   size_t _num_rebuilds = 0;
 
   // ---- the same bookkeeping on the device, for refreshes that never leave it -----------------------------------
@@ -169,8 +172,9 @@ class CacheEntryManager {
                 const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream);
   // waits for `stream` by a ticket in the table's pinned words (spin_us == 0: by the runtime)
   void WaitByTicket(StreamHandle stream);
-  // status words of the table's kernels and n_extra more device words (<= 30), brought to the host by one launch and
-  // one wait by ticket; returns the table's status word, the extra words land in extra_out
+  // status words of the table's kernels and n_extra more device words (<= 9), brought to the host by one launch and
+  // one wait by ticket, with a census of the table where one is due; returns the table's status word, the extra words land
+  // in extra_out
   uint32_t StatusAndWords(const uint32_t *extra_dev, unsigned n_extra, uint32_t *extra_out, StreamHandle stream);
   // device list of host rows -> device list of table keys (the rows themselves, or their ids in sparse-id mode)
   TensorPtr RowsToTableKeys(TensorPtr rows_dev, TensorPtr &buffer, const std::function<MemHandle(size_t)> &allocator,
