@@ -103,7 +103,7 @@ typedef struct {
 const char *ugk_last_error(void);
 /* version of this ABI; bumped on any signature change.  ugk_abi_version() is what the loaded library was built with:
  * a caller compiled against another UGK_ABI_VERSION must not go on. */
-#define UGK_ABI_VERSION 22
+#define UGK_ABI_VERSION 23
 int ugk_abi_version(void);
 
 /* ---- runtime plumbing: Device::{AllocDataSpace,FreeDataSpace,CopyDataFromTo,StreamSync,CreateStream}
@@ -138,6 +138,30 @@ int ugk_stream_is_capturing(void *stream, int *capturing);
  * wait).  `value` must differ from what the word holds (a counter).  What kernels enqueued before the ticket wrote into
  * pinned host memory is visible once the ticket is. */
 int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, unsigned spin_us);
+/* The end of one launch polled for without a kernel behind it.  ugk_leave_done_words: the next ugk_gather_*,
+ * ugk_extract_mix_* or ugk_extract_pool_* call of this thread (that one only; after a call that failed, and where none
+ * comes, NULL takes the request back) makes its workgroups leave words in words_host as they end, and stores the number of
+ * words in done->num_words before it returns: 0 where the launch cannot (outputs written with non-temporal stores, nothing
+ * to do, counts of 2^24 and more), and the caller then waits for the stream in another way.  With words a launch leaves no
+ * group_counts_host and *num_groups_host is 0.  ugk_done_wait polls them for up to
+ * spin_us microseconds before it falls back to waiting for the stream, and returns with the two group sizes of the launch
+ * (0 where it keeps none; either may be NULL).  What the launch wrote is complete then, for kernels and copies on any
+ * stream and for the host: a launch with words writes its rows through to memory, and a workgroup leaves its word when its
+ * stores have been acknowledged; so is everything enqueued in front of it.
+ * words_host: UGK_DONE_WORDS words of pinned, GPU-mapped memory (ugk_host_malloc); tag: differs from call to call until
+ * the words are cleared (no launch may be using them then); counters_dev: UGK_DONE_COUNTERS * 16 8-byte device words that
+ * are zero before the first launch (and are left so by every launch).  Neither is shared by launches in flight together. */
+#define UGK_DONE_WORDS 256
+#define UGK_DONE_COUNTERS 64
+#define UGK_DONE_MAX_TAG 0xffffu
+typedef struct {
+  uint64_t *words_host;
+  uint64_t *counters_dev;
+  uint32_t tag;
+  uint32_t num_words; /* set by the launch */
+} ugk_done_t;
+int ugk_leave_done_words(ugk_done_t *done);
+int ugk_done_wait(const ugk_done_t *done, unsigned spin_us, void *stream, uint64_t *local, uint64_t *others);
 /* The same wait with a few device words brought along: one launch behind everything enqueued on `stream` copies
  * a_dev[0 .. n_a) and b_dev[0 .. n_b) (either may be NULL with a count of 0; n_a + n_b <= 63) to dst_host[1 ...] and
  * then writes `value` to dst_host[0]; the host polls dst_host[0] as above.  dst_host: pinned host words from

@@ -158,6 +158,17 @@ int check_table(const ugk_table_t &t, const char *who) {
 
 void copy_row(void *dst, const void *src, size_t bytes) { memcpy(dst, src, bytes); }
 
+// ugk_leave_done_words: work has been done when a call of the model returns, so its one word is written there
+thread_local ugk_done_t *g_done = nullptr;
+bool leave_done(uint64_t local, uint64_t others) {
+  ugk_done_t *d = g_done;
+  g_done = nullptr;
+  if (!d || local + others >= (1u << 24)) return false;
+  d->num_words = 1;
+  d->words_host[0] = ((uint64_t)d->tag << 48) | (others << 24) | local;
+  return true;
+}
+
 template <typename K>
 int gather_direct(const void *src, uint64_t src_rows, const K *keys, const uint32_t *dst, size_t n, void *out,
                   uint64_t out_rows, size_t rb, uint32_t *status, uint32_t *mirror) {
@@ -171,6 +182,7 @@ int gather_direct(const void *src, uint64_t src_rows, const K *keys, const uint3
     }
     copy_row((char *)out + d * rb, (const char *)src + s * rb, rb);
   }
+  if (dst == nullptr) leave_done(0, 0);
   return 0;
 }
 
@@ -425,8 +437,9 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
     if (from_cache) ++local;
     else ++others;
   }
-  if (counts) counts[0] = (others << 32) | local;
-  if (num_groups) *num_groups = 1;
+  const bool polled = leave_done(local, others);
+  if (counts && !polled) counts[0] = (others << 32) | local;
+  if (num_groups) *num_groups = polled ? 0 : 1;
   return 0;
 }
 
@@ -553,8 +566,9 @@ int extract_pool(ugk_table_t t, const K *ids, const int64_t *seg_off, const floa
       }
     }
   }
-  if (counts) counts[0] = (others << 32) | local;
-  if (num_groups) *num_groups = 1;
+  const bool polled = leave_done(local, others);
+  if (counts && !polled) counts[0] = (others << 32) | local;
+  if (num_groups) *num_groups = polled ? 0 : 1;
   return 0;
 }
 
@@ -832,6 +846,26 @@ int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, 
     note_stream_idle(as_stream(stream));
   }
   *ticket_host = value;
+  return 0;
+}
+int ugk_leave_done_words(ugk_done_t *done) {
+  if (done) {
+    REQUIRE(done->words_host && done->counters_dev && done->tag > 0 && done->tag <= UGK_DONE_MAX_TAG,
+            "ugk_leave_done_words: bad argument");
+    done->num_words = 0;
+  }
+  g_done = done;
+  return 0;
+}
+int ugk_done_wait(const ugk_done_t *done, unsigned, void *stream, uint64_t *local, uint64_t *others) {
+  REQUIRE(done && done->num_words == 1 && (done->words_host[0] >> 48) == done->tag, "ugk_done_wait: no words");
+  {
+    std::lock_guard<std::mutex> g(g_rt_mu);
+    if (as_stream(stream)->capture) violation("the host waited for the words of a launch that was recorded into a graph");
+    note_stream_idle(as_stream(stream));
+  }
+  if (local) *local = done->words_host[0] & 0xffffffu;
+  if (others) *others = (done->words_host[0] >> 24) & 0xffffffu;
   return 0;
 }
 int ugk_words_to_host_ticket(const uint32_t *a, unsigned n_a, const uint32_t *b, unsigned n_b, uint32_t *dst,

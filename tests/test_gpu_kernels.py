@@ -823,6 +823,136 @@ def _extract_mix(fn, tb, keys_dev, n, cache_dev, cache_rows, pin, host_rows, out
         words.free()
 
 
+class _DoneWords:
+    """the words and counters of ugk_leave_done_words, and the check that a launch leaves the counters at zero"""
+
+    def __init__(self):
+        self.words = PinnedArray((256,), np.uint64)
+        self.words.array[:] = 0
+        self.counters = torch.zeros(64 * 16, dtype=torch.int64, device="cuda")
+        self.done = hip.Done(self.words.ptr, ptr(self.counters), 0, 0)
+
+    def run(self, launch, spin_us, groups):
+        self.done.tag = self.done.tag + 1
+        hip.call("ugk_leave_done_words", C.byref(self.done))
+        launch()
+        if groups is None:
+            assert self.done.num_words == 0
+            sync()
+            return None
+        assert self.done.num_words == (groups if groups <= 256 else 64)
+        local, others = C.c_uint64(), C.c_uint64()
+        hip.call("ugk_done_wait", C.byref(self.done), spin_us, None, C.byref(local), C.byref(others))
+        sync()
+        assert not self.counters.any().item()
+        return local.value, others.value
+
+
+# gathers of one workgroup, of the most that leave a word each, of one more, of as many as make some counters one longer than
+# the others, and of several rounds; every kernel and every kind of lane
+@pytest.mark.parametrize("row_bytes,rows_per_group", [(512, 16), (16, 512), (64, 128), (8192, 8), (1, 512), (2, 512), (4, 512),
+                                                      (12, 128), (100, 0), (404, 0), (1204, 0), (800, 0)])
+@pytest.mark.parametrize("spin_us", [0, 1_000_000])
+def test_gather_that_tells_its_end_by_words(row_bytes, rows_per_group, spin_us):
+    gen = torch.Generator(device="cuda").manual_seed(row_bytes)
+    rows, done = 5_003, _DoneWords()
+    table = torch.randint(0, 256, (rows, row_bytes), dtype=torch.uint8, device="cuda", generator=gen)
+    for groups in (1, 255, 256, 257, 321, 4_099 if row_bytes < 1024 else 400):
+        n = groups * (rows_per_group or 16) - (1 if groups > 1 else 0)
+        keys = torch.randint(0, rows, (n,), device="cuda", generator=gen)
+        bad = torch.zeros(n, dtype=torch.bool, device="cuda")
+        bad[n // 2] = n > 4
+        q, want = torch.where(bad, rows, keys), table[keys]
+        want[bad] = 0x7E
+        out = torch.full((n, row_bytes), 0x7E, dtype=torch.uint8, device="cuda")
+        st = dev_zeros_u32(1)
+        sync()
+
+        def launch():
+            hip.call("ugk_gather_direct_i64", ptr(table), rows, ptr(q), n, ptr(out), row_bytes, 0, ptr(st), None, None)
+
+        if rows_per_group:
+            assert done.run(launch, spin_us, groups) == (0, 0)
+        else:  # the number of workgroups is the kernel's own affair
+            done.done.tag += 1
+            hip.call("ugk_leave_done_words", C.byref(done.done))
+            launch()
+            assert done.done.num_words > 0
+            hip.call("ugk_done_wait", C.byref(done.done), spin_us, None, None, None)
+            assert not done.counters.any().item()
+        assert torch.equal(out, want)
+        assert status_value(st) == (hip.ST_KEY_OUT_OF_RANGE if n > 4 else 0)
+    # the request met one call: the next one leaves nothing; and streaming outputs are waited for in another way
+    before = done.words.array.copy()
+    launch()
+    sync()
+    assert (done.words.array == before).all()
+    if row_bytes % 16 == 0:
+        hip.call("ugk_set_output_hint", 1)
+        try:
+            done.run(launch, spin_us, None)
+        finally:
+            hip.call("ugk_set_output_hint", 0)
+
+
+@pytest.mark.parametrize("kind", ["flat", "hash", "hash32"])
+@pytest.mark.parametrize("rb", [36, 128, 512])
+@pytest.mark.parametrize("stage", [False, True])
+def test_fused_and_pooled_lookups_that_tell_their_end_by_words(kind, rb, stage):
+    if stage and rb % 16:
+        pytest.skip("a stage takes rows of whole vectors")
+    rng = np.random.default_rng(rb)
+    nkeys, done = 6_000, _DoneWords()
+    table = _rand_table(rng, nkeys, rb)
+    if rb % 16 == 0:
+        table = rng.integers(-8, 8, size=(nkeys, rb // 4)).astype(np.float32).view(np.uint8)  # sums are exact
+    cached = rng.permutation(nkeys)[:4_000].astype(np.int64)
+    mem, tb = (_make_flat(nkeys) if kind == "flat" else (_make_hash if kind == "hash" else _make_hash32)(len(cached))[:2])
+    assert _insert(tb, cached.astype(np.uint32)) == 0
+    pin, d_cache = pinned_from(table), to_dev(table[cached])
+    d_table = to_dev(table)
+    if stage:
+        s_rows, s_owner = dev_bytes(1024 * rb), torch.zeros(1024, dtype=torch.int64, device="cuda")
+    st, groups = dev_zeros_u32(1), C.c_uint32(7)
+    in_cache = np.zeros(nkeys, bool)
+    in_cache[cached] = True
+    for epoch, n in enumerate((1, 31, 4_096, 8_192, 8_193, 20_000, 300_000), 1):
+        keys = rng.integers(0, nkeys, size=n).astype(np.int64)
+        d_keys, out = to_dev(keys), dev_bytes(n * rb, fill=0xEE)
+        sync()
+        args = [tb, ptr(d_keys), n, ptr(d_cache), len(cached), pin.ptr, nkeys, ptr(out), rb, ptr(st), None, None,
+                C.byref(groups), hip.HINT_UNKNOWN]
+        done.done.tag += 1
+        hip.call("ugk_leave_done_words", C.byref(done.done))
+        if stage:
+            hip.call("ugk_extract_mix_staged_i64", *args, hip.Stage(ptr(s_rows), ptr(s_owner), 1023, epoch, 0), None)
+        else:
+            hip.call("ugk_extract_mix_i64", *args, None)
+        local, others = C.c_uint64(), C.c_uint64()
+        assert done.done.num_words > 0 and groups.value == 0
+        hip.call("ugk_done_wait", C.byref(done.done), 1_000_000, None, C.byref(local), C.byref(others))
+        assert (local.value, others.value) == (in_cache[keys].sum(), (~in_cache[keys]).sum())
+        assert torch.equal(out[: n * rb].view(n, rb), d_table[torch.from_numpy(keys).cuda()])
+        assert not done.counters.any().item()
+        if rb % 16 == 0 and not stage:
+            per = 3 if n > 3 else 1
+            n_rows = n // per
+            off = torch.arange(0, n_rows * per + 1, per, device="cuda")
+            pooled = torch.empty((n_rows, rb // 4), dtype=torch.float32, device="cuda")
+            sync()
+            done.done.tag += 1
+            hip.call("ugk_leave_done_words", C.byref(done.done))
+            hip.call("ugk_extract_pool_i64", tb, ptr(d_keys), ptr(off), None, n_rows, n_rows * per, 0, 4, ptr(d_cache),
+                     len(cached), pin.ptr, nkeys, ptr(pooled), rb, ptr(st), None, None, C.byref(groups), None)
+            assert done.done.num_words > 0 and groups.value == 0
+            hip.call("ugk_done_wait", C.byref(done.done), 0, None, C.byref(local), C.byref(others))
+            used = keys[: n_rows * per]
+            assert (local.value, others.value) == (in_cache[used].sum(), (~in_cache[used]).sum())
+            want = d_table.view(torch.float32)[torch.from_numpy(used).cuda()].view(n_rows, per, -1).sum(1)
+            assert torch.equal(pooled, want)
+    assert status_value(st) == 0
+
+
 def test_outputs_beyond_4_GiB():
     """9M keys of 512-byte rows: the output (4.6 GB) passes 2^32 bytes, so every byte offset the kernels form must be a
     64-bit one.  table[r, c] is a closed form of (r, c); all three extraction paths are checked against it on the

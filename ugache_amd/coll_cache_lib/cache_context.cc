@@ -328,6 +328,13 @@ ExtractSession::ExtractSession(std::shared_ptr<CacheContext> cache_ctx) : _cache
   _counts[1] = state + kStCounts1;
   _status = state + kStStatus;
   _mix_counts = PinnedHostAlloc((size_t)ugk_extract_mix_max_groups() * sizeof(uint64_t));
+  _done_words = PinnedHostAlloc(UGK_DONE_WORDS * sizeof(uint64_t));
+  memset(_done_words->ptr(), 0, UGK_DONE_WORDS * sizeof(uint64_t));
+  _done_counters = EagerGPUAlloc(dev, UGK_DONE_COUNTERS * 16 * sizeof(uint64_t));
+  UGK_CALL(ugk_fill_u32(_done_counters->ptr<uint32_t>(), 0, UGK_DONE_COUNTERS * 16 * 2, nullptr));
+  UGK_CALL(ugk_stream_sync(nullptr));
+  _done.words_host = _done_words->ptr<uint64_t>();
+  _done.counters_dev = _done_counters->ptr<uint64_t>();
   _host_mirror_handle = PinnedHostAlloc(256);
   _host_mirror = _host_mirror_handle->ptr<uint32_t>();
   memset(_host_mirror, 0, 256);
@@ -808,8 +815,10 @@ void ExtractSession::NoteOutput(const void *output, size_t nbytes) {
   _out_hint = hint;
 }
 
-// group sizes of the last fused launch: the sum of the words its workgroups left in pinned host memory
+// group sizes of the last fused launch: the sum of the words its workgroups left in pinned host memory (no words: the
+// wait has brought the sizes along, see WaitForBatch)
 void ExtractSession::SumMixCounts() {
+  if (_mix_groups == 0) return;
   const uint64_t *w = _mix_counts->ptr<uint64_t>();
   uint64_t local = 0, others = 0;
   for (uint32_t g = 0; g < _mix_groups; g++) {
@@ -820,10 +829,31 @@ void ExtractSession::SumMixCounts() {
   _host_mirror[kMirGroupSizes + UGK_LOC_HOST] = (uint32_t)others;
 }
 
-// The wait of a blocking lookup.  By default a ticket written by a one-lane kernel behind the batch's kernels is polled
-// in the pinned mirror: it turns up a few microseconds before a wait for the stream returns (COLL_SPIN_WAIT=0: wait for
-// the stream, as the reference does).
+// In front of the one launch of a blocking lookup that is waited for by WaitForBatch next: asks that its workgroups leave
+// words for the wait to poll.
+void ExtractSession::AskForDoneWords() {
+  _done.num_words = 0;
+  if (RunConfig::spin_wait_us == 0) return;
+  if (++_done.tag > UGK_DONE_MAX_TAG) {  // nothing is in flight that uses the words: blocking lookups follow each other
+    memset(_done.words_host, 0, UGK_DONE_WORDS * sizeof(uint64_t));
+    _done.tag = 1;
+  }
+  UGK_CALL(ugk_leave_done_words(&_done));
+}
+
+// The wait of a blocking lookup.  A launch that leaves words is polled for by them, which also bring its group sizes.
+// For others a ticket written by a one-lane kernel behind the batch's kernels is polled in the pinned mirror: it turns up a
+// few microseconds before a wait for the stream returns (COLL_SPIN_WAIT=0: wait for the stream, as the reference does).
 void ExtractSession::WaitForBatch(StreamHandle stream) {
+  if (_done.num_words) {
+    uint64_t local = 0, others = 0;
+    UGK_CALL(ugk_done_wait(&_done, RunConfig::spin_wait_us, stream, &local, &others));
+    _done.num_words = 0;
+    _mix_groups = 0;
+    _host_mirror[kMirGroupSizes + UGK_LOC_LOCAL] = (uint32_t)local;
+    _host_mirror[kMirGroupSizes + UGK_LOC_HOST] = (uint32_t)others;
+    return;
+  }
   if (RunConfig::spin_wait_us == 0) {
     UGK_CALL(ugk_stream_sync(stream));
     return;
@@ -891,6 +921,7 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
     Timer t_host;
     if (events) UGK_CALL(ugk_event_record(_ev_t[0], stream));
     if (dst_map == nullptr) {
+      AskForDoneWords();
       UGK_CALL(GatherDirect(ctx->_device_cache_data[0], ctx->_num_total_nodes, nodes, num_nodes, output, rb,
                             from_host ? _cpu_blocks : 0, _status, _host_mirror, stream));
     } else {
@@ -958,9 +989,10 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
     // slow for one that mostly hits: it is given where the share is known (the keys COLL_SKIP_LOCAL selected all come
     // from outside the cache), not guessed from the previous batch.
     const uint32_t hint = skip_local ? (uint32_t)num_nodes : UGK_HINT_UNKNOWN;
+    const ugk_stage_t *stage = StageTakes(output) ? NextStage(stream, false) : nullptr;
+    AskForDoneWords();
     UGK_CALL(ExtractMix(table, nodes, num_nodes, cache, cache_rows, host, host_rows, output, rb, _status,
-                        _host_mirror, _mix_counts->ptr<uint64_t>(), &_mix_groups, hint,
-                        StageTakes(output) ? NextStage(stream, false) : nullptr, stream));
+                        _host_mirror, _mix_counts->ptr<uint64_t>(), &_mix_groups, hint, stage, stream));
     if (events) UGK_CALL(ugk_event_record(_ev_t[1], stream));
     RecordLaunch(input_nodes, num_input, keys_ready);
     WaitForBatch(stream);
@@ -1226,7 +1258,8 @@ void ExtractSession::Wait(StreamHandle stream) {
 // direct mapping is the HBM copy (the kernel then counts its ids as "from the host table")
 template <typename KeyT>
 bool ExtractSession::LaunchPooled(const KeyT *nodes, const int64_t *seg_off, const float *weights, size_t num_rows,
-                                  size_t num_nodes, int combiner, int elem_bytes, void *output, StreamHandle stream) {
+                                  size_t num_nodes, int combiner, int elem_bytes, void *output, bool blocking,
+                                  StreamHandle stream) {
   CacheContext *ctx = _cache_ctx.get();
   const size_t rb = ctx->_row_bytes;
   CHECK_NOTNULL(seg_off);
@@ -1255,6 +1288,7 @@ bool ExtractSession::LaunchPooled(const KeyT *nodes, const int64_t *seg_off, con
   }
   CHECK((((uintptr_t)cache | (uintptr_t)host | (uintptr_t)output) & 15u) == 0) << "pooled lookup: misaligned buffer";
   const RecordPlan keys_ready = RecordBegin(stream);
+  if (blocking) AskForDoneWords();
   UGK_CALL(ExtractPool(table, nodes, seg_off, weights, num_rows, num_nodes, combiner, elem_bytes, _pool_max_norm, cache,
                        cache_rows, host, ctx->_num_total_nodes, output, rb, _status, _host_mirror,
                        _mix_counts->ptr<uint64_t>(), &_mix_groups, stream));
@@ -1279,7 +1313,7 @@ void ExtractSession::ExtractPooledImpl(const KeyT *nodes, const int64_t *seg_off
   }
   Timer t_host;
   const bool all_from_hbm =
-      LaunchPooled(nodes, seg_off, weights, num_rows, num_nodes, combiner, elem_bytes, output, stream);
+      LaunchPooled(nodes, seg_off, weights, num_rows, num_nodes, combiner, elem_bytes, output, true, stream);
   WaitForBatch(stream);
   const double host_time = t_host.Passed();
   JoinRecordOnHost();
@@ -1316,7 +1350,7 @@ void ExtractSession::ExtractPooledAsyncImpl(const KeyT *nodes, const int64_t *se
   NoteAsyncStream(stream);
   InFlight enqueueing(this);  // see ExtractFeatAsyncImpl
   _async_swap_counts =
-      LaunchPooled(nodes, seg_off, weights, num_rows, num_nodes, combiner, elem_bytes, output, stream);
+      LaunchPooled(nodes, seg_off, weights, num_rows, num_nodes, combiner, elem_bytes, output, false, stream);
   JoinRecord(stream);
   _async_last_fused = true;
   _async_pending++;

@@ -174,6 +174,10 @@ class ExtractSession {
   void SumMixCounts();
   uint32_t _ticket = 0;  // last ticket a blocking lookup waited for (kMirTicket)
   void WaitForBatch(StreamHandle stream);
+  // what a blocking lookup's launch tells its end with (ugk_leave_done_words); num_words > 0: the launch in flight does
+  MemHandle _done_words, _done_counters;
+  ugk_done_t _done{};
+  void AskForDoneWords();
   // Rows that crossed the host link, kept for the next refresh (COLL_MISS_STAGE_ROWS): written by the fused extraction,
   // read by the refresh's row copy.  A foreground refresh runs while no lookup does and reads the stage the lookups
   // write.  A background refresh runs beside lookups, so there are two stages then: it switches the lookups over to
@@ -230,7 +234,7 @@ class ExtractSession {
                          uint64_t task_key);
   template <typename KeyT>
   bool LaunchPooled(const KeyT *nodes, const int64_t *seg_off, const float *weights, size_t num_rows, size_t num_nodes,
-                    int combiner, int elem_bytes, void *output, StreamHandle stream);
+                    int combiner, int elem_bytes, void *output, bool blocking, StreamHandle stream);
   template <typename KeyT>
   void ExtractPooledAsyncImpl(const KeyT *nodes, const int64_t *seg_off, const float *weights, size_t num_rows,
                               size_t num_nodes, int combiner, int elem_bytes, void *output, StreamHandle stream);

@@ -96,7 +96,8 @@ template <typename V, int LPR, int UNROLL, bool NT_STORE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restrict__ src, uint64_t src_rows,
                                                         V *__restrict__ out, uint64_t out_rows, uint32_t vpr,
                                                         const uint32_t *__restrict__ counts, uint32_t group, size_t n,
-                                                        bool many_groups, uint32_t *status, uint32_t *host_mirror) {
+                                                        bool many_groups, uint32_t *status, uint32_t *host_mirror,
+                                                        DoneWords done) {
   size_t begin = 0, count = n;
   if (counts) {
     const uint32_t c = counts[group];
@@ -104,6 +105,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
     begin = (group == UGK_LOC_LOCAL) ? 0 : n - c;
     if (host_mirror && blockIdx.x == 0 && threadIdx.x == 0) host_mirror[1 + group] = c;
   }
+  const bool through = !NT_STORE && done.tag != 0;
   constexpr int RPB = kBlock / LPR;  // rows copied by one block instruction
   const uint32_t lane = threadIdx.x % LPR;
   const uint32_t rib = threadIdx.x / LPR;
@@ -142,15 +144,22 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
         if (no_branch) {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) v[u] = ld_stream(src + s[u] * vpr + col);
+        } else {
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+            if (ok[u]) v[u] = ld_stream(src + s[u] * vpr + col);
+        }
+        if (through) {
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+            if (ok[u]) store_through(reinterpret_cast<uint64_t>(out + d[u] * vpr + col), v[u]);
+        } else if (no_branch) {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) {
             if constexpr (NT_STORE) st_stream(out + d[u] * vpr + col, v[u]);
             else out[d[u] * vpr + col] = v[u];
           }
         } else {
-#pragma unroll
-          for (int u = 0; u < UNROLL; ++u)
-            if (ok[u]) v[u] = ld_stream(src + s[u] * vpr + col);
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
             if (ok[u]) {
@@ -161,6 +170,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
       }
     }
   }
+  if (done.tag) leave_done(done, nullptr);
 }
 
 // The same for rows the lanes of gather_kernel do not fit (see flat_copy): a wavefront takes f.tile rows, one index
@@ -169,7 +179,8 @@ template <typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                              char *__restrict__ out, uint64_t out_rows, FlatRow f,
                                                              const uint32_t *__restrict__ counts, uint32_t group,
-                                                             size_t n, uint32_t *status, uint32_t *host_mirror) {
+                                                             size_t n, uint32_t *status, uint32_t *host_mirror,
+                                                             DoneWords done) {
   size_t begin = 0, count = n;
   if (counts) {
     const uint32_t c = counts[group];
@@ -194,8 +205,9 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
     // a row that is skipped is read where the tile's first good row is
     const uint64_t at = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
     const uint64_t dummy = shfl64(at, __ffsll(good) - 1);
-    flat_copy<Idx::kDense>(ok ? at : dummy | kNoRowBit, (uint32_t)d, out, base, 0, rows, f);
+    flat_copy<Idx::kDense>(ok ? at : dummy | kNoRowBit, (uint32_t)d, out, base, 0, rows, f, done.tag != 0);
   }
+  if (done.tag) leave_done(done, nullptr);
 }
 
 // ... and with the output dealt out instead of the rows, for batches whose row i becomes output row i: a wavefront owns
@@ -220,10 +232,15 @@ StreamRow stream_row(size_t row_bytes, size_t n) {
 template <bool NT_STORE, bool SHARE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                                char *__restrict__ out, StreamRow f, uint32_t *status,
-                                                               uint32_t *host_mirror) {
+                                                               uint32_t *host_mirror, DoneWords done) {
   static_assert(Idx::kDense, "row i goes to output row i");
   typedef __attribute__((address_space(1))) uint32_t *gword_t;
   constexpr int U = (int)(kStreamPart / (kWave * 16));
+  const bool through = !NT_STORE && done.tag != 0;
+  auto put = [through](auto *q, auto w) {
+    if (through) store_through(reinterpret_cast<uint64_t>(q), w);
+    else *q = w;
+  };
   const uint32_t lane = lane_id();
   const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock * kStreamPart;
   for (uint64_t begin = ((uint64_t)blockIdx.x * kWavesPerBlock + wave_in_block()) * kStreamPart; begin < f.total;
@@ -289,13 +306,13 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
         w.w = head == 12 ? sb.x : head == 8 ? sb.y : sb.z;
         if (row_a && row_b) {
           if constexpr (NT_STORE) __builtin_nontemporal_store(w, q);
-          else *q = w;
+          else put(q, w);
         } else {  // a skipped row leaves its words of the output alone
           const gword_t q1 = reinterpret_cast<gword_t>(q);
-          if (row_a) q1[0] = w.x;
-          if (head > 4 ? row_a : row_b) q1[1] = w.y;
-          if (head > 8 ? row_a : row_b) q1[2] = w.z;
-          if (row_b) q1[3] = w.w;
+          if (row_a) put(q1, (uint32_t)w.x);
+          if (head > 4 ? row_a : row_b) put(q1 + 1, (uint32_t)w.y);
+          if (head > 8 ? row_a : row_b) put(q1 + 2, (uint32_t)w.z);
+          if (row_b) put(q1 + 3, (uint32_t)w.w);
         }
       }
     }
@@ -304,7 +321,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
       if (copy[u]) {
         const gout_t q = reinterpret_cast<gout_t>(to + (u * kWave + lane) * 16);
         if constexpr (NT_STORE) __builtin_nontemporal_store(v[u], q);
-        else *q = v[u];
+        else put(q, v[u]);
       }
     if constexpr (SHARE) {
       const uint32_t rest = bytes % 16;  // the words behind the last whole vector of the output: the end of its last row
@@ -313,11 +330,12 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
         const uint32_t rlo = __shfl(lo, (int)r), rhi = __shfl(hi, (int)r);
         if (lane < rest / 4 && (rlo & kNoRowBit) == 0) {
           const uint64_t from = (((uint64_t)rhi << 32) | rlo) + f.row_bytes - rest;
-          reinterpret_cast<gword_t>(to + bytes - rest)[lane] = reinterpret_cast<gword_t>(from)[lane];
+          put(reinterpret_cast<gword_t>(to + bytes - rest) + lane, (uint32_t)reinterpret_cast<gword_t>(from)[lane]);
         }
       }
     }
   }
+  if (done.tag) leave_done(done, nullptr);
 }
 
 // Re-expansion of duplicates inside one buffer: row i takes the bytes of its representative row.  Source and
@@ -434,18 +452,19 @@ unsigned gather_grid(size_t passes, unsigned max_blocks) {
 template <typename V, int LPR, int UNROLL, typename Idx>
 int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, uint32_t vpr,
                     const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
-                    uint32_t *host_mirror, bool nt, hipStream_t stream) {
+                    uint32_t *host_mirror, bool nt, DoneRequest &request, hipStream_t stream) {
   constexpr size_t kPerIter = (size_t)(kBlock / LPR) * UNROLL;
   const unsigned grid = gather_grid((n + kPerIter - 1) / kPerIter, max_blocks);
   const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
+  const DoneWords done = nt ? DoneWords{nullptr, nullptr, 0} : request.take(grid);
   if (nt)
     hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, true, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,
                        reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,
-                       group, n, many_groups, status, host_mirror);
+                       group, n, many_groups, status, host_mirror, done);
   else
     hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, false, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,
                        reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,
-                       group, n, many_groups, status, host_mirror);
+                       group, n, many_groups, status, host_mirror, done);
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -453,21 +472,21 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
 template <typename V, int LPR, typename Idx>
 int launch_one(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, uint32_t vpr,
                const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
-               uint32_t *host_mirror, hipStream_t stream) {
+               uint32_t *host_mirror, DoneRequest &request, hipStream_t stream) {
   // two rows in flight per lane; one was measured with streaming stores and is no better (262,144 keys of 512 bytes
   // into rotating outputs 49.3 us against 47.9 us, 1 M keys 184 against 180 us)
   return launch_unrolled<V, LPR, 2, Idx>(ix, src, src_rows, out, out_rows, vpr, counts, group, n, max_blocks, status,
-                                         host_mirror, nt_store_for(n * (size_t)vpr * sizeof(V)), stream);
+                                         host_mirror, nt_store_for(n * (size_t)vpr * sizeof(V)), request, stream);
 }
 
 template <typename V, typename Idx>
 int launch_vec(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, size_t row_bytes,
                const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
-               uint32_t *host_mirror, hipStream_t stream) {
+               uint32_t *host_mirror, DoneRequest &request, hipStream_t stream) {
   const uint32_t vpr = (uint32_t)(row_bytes / sizeof(V));
 #define UGK_GO(L) \
   return launch_one<V, L, Idx>(ix, src, src_rows, out, out_rows, vpr, counts, group, n, max_blocks, status, host_mirror, \
-                               stream)
+                               request, stream)
   if constexpr (sizeof(V) == 16) {
     if (vpr <= 1) UGK_GO(1);
     if (vpr <= 2) UGK_GO(2);
@@ -537,26 +556,27 @@ bool stream_pays(uintptr_t align, const void *out, size_t row_bytes, size_t n, u
 template <typename Idx>
 int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, size_t row_bytes,
                 const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
-                uint32_t *host_mirror, hipStream_t stream) {
+                uint32_t *host_mirror, DoneRequest &request, hipStream_t stream) {
   const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes, n));
   const size_t per_block = (size_t)f.tile * kWavesPerBlock;
   const unsigned grid = gather_grid((n + per_block - 1) / per_block, max_blocks);
   hipLaunchKernelGGL((gather_flat_kernel<Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src, src_rows,
-                     (char *)out, out_rows, f, counts, group, n, status, host_mirror);
+                     (char *)out, out_rows, f, counts, group, n, status, host_mirror, request.take(grid));
   UGK_HIP(hipGetLastError());
   return 0;
 }
 
 template <typename Idx>
 int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t row_bytes, size_t n,
-                  unsigned max_blocks, uint32_t *status, uint32_t *host_mirror, hipStream_t stream) {
+                  unsigned max_blocks, uint32_t *status, uint32_t *host_mirror, DoneRequest &request, hipStream_t stream) {
   const StreamRow f = stream_row(row_bytes, n);
   const uint64_t per_block = (uint64_t)kStreamPart * kWavesPerBlock;
   const unsigned grid = gather_grid((f.total + per_block - 1) / per_block, max_blocks);
   const bool nt = nt_store_for(n * row_bytes);
+  const DoneWords done = nt ? DoneWords{nullptr, nullptr, 0} : request.take(grid);
 #define UGK_GO(NT, SHARE)                                                                                             \
   hipLaunchKernelGGL((gather_stream_kernel<NT, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,                \
-                     (const char *)src, src_rows, (char *)out, f, status, host_mirror)
+                     (const char *)src, src_rows, (char *)out, f, status, host_mirror, done)
   if (row_bytes % 16 == 0) {
     if (nt) UGK_GO(true, false);
     else UGK_GO(false, false);
@@ -573,6 +593,7 @@ template <typename Idx>
 int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, size_t row_bytes,
                   const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
                   uint32_t *host_mirror, void *stream) {
+  DoneRequest request;
   if (n == 0) return 0;
   UGK_REQUIRE(src && out, "gather: null source or output");
   UGK_REQUIRE(status, "gather: null status word");
@@ -582,10 +603,11 @@ int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_
   hipStream_t st = as_stream(stream);
 #define UGK_VEC(V)                                                                                                  \
   return launch_vec<V, Idx>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks, status,      \
-                            host_mirror, st)
+                            host_mirror, request, st)
   if constexpr (Idx::kDense) {
     if (stream_pays(align, out, row_bytes, n, max_blocks))
-      return launch_stream<Idx>(ix, src, src_rows, out, row_bytes, n, max_blocks, status, host_mirror, st);
+      return launch_stream<Idx>(ix, src, src_rows, out, row_bytes, n, max_blocks, status, host_mirror, request,
+                                st);
   }
   if (align % 16 == 0) UGK_VEC(u32x4);
   // short rows in small launches: 16 lanes of 4 bytes have less to do before their first load than the flat copy (36 bytes x
@@ -598,7 +620,7 @@ int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_
   if (align % 4 == 0 && counts && group == UGK_LOC_HOST && max_blocks == 0 && row_bytes <= 320) UGK_VEC(uint32_t);
   if (flat_row_ok(align, row_bytes))
     return launch_flat<Idx>(ix, src, src_rows, out, out_rows, row_bytes, counts, group, n, max_blocks, status,
-                            host_mirror, st);
+                            host_mirror, request, st);
   // rows of 8 bytes: one lane of 8 bytes each in large launches, where four of 4 bytes, two of them idle, are too many (us:
   // 2 M rows 49.4 / 51.6, 262,144 rows 8.5 / 8.6, 8,192 rows 4.0 / 3.2)
   if (row_bytes == 8 && align % 8 == 0 && n > 262144) UGK_VEC(unsigned long long);

@@ -55,6 +55,32 @@ static inline unsigned clamp_grid(size_t want, unsigned max_blocks) {
 constexpr size_t kMemorySideCacheBytes = (size_t)256 << 20;
 bool nt_store_for(size_t out_bytes);
 
+// What a launch leaves for a host that polls for its end (ugk_leave_done_words; leave_done in ugk_mix.cuh); tag 0: nobody
+// polls, and words, if there are any, are the per-workgroup counts of ugk_extract_mix_*.
+struct DoneWords {
+  unsigned long long *words, *counters;
+  uint32_t tag;
+};
+// Up to kDoneDirect workgroups leave a word each.  More of them meet in kDoneFan counters, workgroup b in counter b %
+// kDoneFan, and the last one of a counter leaves its word: writes into host memory cost 2 us per thousand, and a host that
+// polls thousands of words falls behind.  262,144 rows of 512 bytes gathered, launch to end of poll, with 32 / 64 / 128 /
+// 256 / 512 / 1024 counters 48.6 / 48.7 / 49.0 / 49.3 / 49.7 / 50.8 us, a word per workgroup (16,384) 53.0, one-lane ticket
+// kernel behind the gather 52.0; 8,192 rows (512 workgroups) 8.9 / 8.8 / 9.0 / 9.3 / 9.2 / 9.2, 9.1 and 9.8; 1,664 rows 8.4 /
+// 8.6 / 8.2 / 8.2 / 8.1 / 8.1, 8.0 and 9.4; 8 rows 6.3 against 8.5.
+constexpr uint32_t kDoneDirect = UGK_DONE_WORDS, kDoneFan = UGK_DONE_COUNTERS;
+
+// The request of ugk_leave_done_words, if this thread has made one: the entry points that can fulfil it take it as they
+// begin, so that it never meets a later launch.
+class DoneRequest {
+ public:
+  DoneRequest();
+  // grid: workgroups of the launch; count_limit: no counter of it reaches this, 0 where none are kept
+  DoneWords take(unsigned grid, uint64_t count_limit = 0);
+
+ private:
+  ugk_done_t *_done;
+};
+
 __device__ __forceinline__ unsigned lane_id() { return __lane_id(); }
 // number of the wavefront in its workgroup, in a scalar register: what is computed from it stays scalar
 __device__ __forceinline__ unsigned wave_in_block() { return __builtin_amdgcn_readfirstlane(threadIdx.x / kWave); }

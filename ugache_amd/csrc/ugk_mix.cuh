@@ -15,6 +15,49 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 typedef const __attribute__((address_space(1))) u32x4 *grow_t;  // a row in global memory (HBM, or mapped host memory)
 typedef __attribute__((address_space(1))) u32x4 *gout_t;
 
+// ---- the end of a launch a host polls for --------------------------------------------------------------------------
+// Stores that are written through the caches (system scope): once such a store has been acknowledged its bytes are in
+// memory, and not in the L2 of an XCD that is written back when the kernel has ended.  In assembler, for the language has
+// no such stores of 16 bytes; the s_nop is for the vector instruction that may overwrite the stored registers next.
+template <typename V>
+__device__ __forceinline__ void store_through(uint64_t to, V v) {
+  typedef __attribute__((address_space(1))) char *gbyte_t;
+  const gbyte_t p = reinterpret_cast<gbyte_t>(to);
+  if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+  else if constexpr (sizeof(V) == 8) asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+  else if constexpr (sizeof(V) == 4) asm volatile("global_store_dword %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+  else if constexpr (sizeof(V) == 2) asm volatile("global_store_short %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"((uint32_t)v) : "memory");
+  else asm volatile("global_store_byte %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"((uint32_t)v) : "memory");
+}
+
+// The last thing a workgroup does: its counts, and with a tag the news that it has ended.  All threads call it; tot (in LDS,
+// may be NULL) holds the rows taken from the cache and all others.
+__device__ __forceinline__ void leave_done(const DoneWords &done, const uint32_t *tot) {
+  if (done.tag) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have been acknowledged
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const uint32_t local = tot ? tot[0] : 0u, others = tot ? tot[1] : 0u;
+  if (done.tag == 0) {
+    done.words[blockIdx.x] = ((unsigned long long)others << 32) | local;
+    return;
+  }
+  const unsigned long long tag = (unsigned long long)done.tag << 48, mine = ((unsigned long long)others << 24) | local;
+  if (gridDim.x <= kDoneDirect) {
+    done.words[blockIdx.x] = tag | mine;
+    return;
+  }
+  const uint32_t g = blockIdx.x % kDoneFan, members = gridDim.x / kDoneFan + (g < gridDim.x % kDoneFan ? 1u : 0u);
+  const unsigned long long add = (1ull << 48) | mine;
+  unsigned long long *counter = done.counters + g * 16;  // a line each
+  const unsigned long long sum =
+      __hip_atomic_fetch_add(counter, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
+  if ((uint32_t)(sum >> 48) == members) {
+    // zero again for the next launch, which does not start before this one has ended
+    __hip_atomic_store(counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    done.words[g] = tag | (sum & 0xffffffffffffull);
+  }
+}
+
 // ---- flat row copy -------------------------------------------------------------------------------------------------
 // Rows of any multiple of 4 bytes above 16, as 16-byte vectors all the same: a vector load or store of global memory
 // needs 4-byte alignment only, and the last vector of a row is moved back so that it ends with the row (it overlaps
@@ -61,7 +104,7 @@ static inline FlatRow flat_row(size_t row_bytes, uint32_t tile) {
 // lanes call it with the same r0 and count.
 template <bool DENSE>
 __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, char *out, size_t d0, uint32_t r0,
-                                          uint32_t count, const FlatRow &f) {
+                                          uint32_t count, const FlatRow &f, bool through) {
   constexpr int U = 4;  // vectors in flight per lane
   const uint32_t total = count * f.chunks;
   const uint32_t tail = f.row_bytes - 16;
@@ -85,9 +128,15 @@ __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, c
     u32x4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
+    if (through) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (ok[u]) *q[u] = v[u];
+      for (int u = 0; u < U; ++u)
+        if (ok[u]) store_through(reinterpret_cast<uint64_t>(q[u]), v[u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (ok[u]) *q[u] = v[u];
+    }
   }
 }
 
@@ -132,14 +181,14 @@ __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key
 // launch at 99 % hits (same-address atomics are performed one after the other at the memory side), one add whose
 // result tells the last workgroup still 5 us (every workgroup ends by waiting for the round trip), and a device-scope
 // fence per workgroup 13-49 % of a whole step (each writes back and invalidates the L2 of its XCD).
+// (A launch that a host polls for waits for its stores anyway, and adds its workgroups up in a few counters: leave_done.)
 __device__ __forceinline__ void mix_leave_counts(uint32_t *block_tot, uint32_t wave_local, uint32_t wave_host,
-                                                 unsigned long long *counts) {
+                                                 const DoneWords &done) {
   if (lane_id() == 0) {
     if (wave_local) atomicAdd(&block_tot[0], wave_local);
     if (wave_host) atomicAdd(&block_tot[1], wave_host);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) counts[blockIdx.x] = ((unsigned long long)block_tot[1] << 32) | block_tot[0];
+  leave_done(done, block_tot);
 }
 
 }  // namespace

@@ -164,7 +164,8 @@ __global__ __launch_bounds__(kBlock) void select_keys_kernel(const K *__restrict
 // the rows of one wavefront's KPW keys, lane l holding the address of key b0 + l's row
 // stage_bits (STAGE only): where the lane's row is filed as well, 0 for a row that is not
 template <int LPR, int KPW, bool NT_STORE, bool STAGE>
-__device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits, u32x4 *out, size_t b0, uint32_t vpr) {
+__device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits, u32x4 *out, size_t b0, uint32_t vpr,
+                                         bool through) {
   constexpr int RPW = kWave / LPR;  // rows per wavefront instruction
   constexpr int UNROLL = (RPW * 4 <= KPW) ? 4 : (KPW / RPW);
   static_assert(KPW <= kWave && KPW % (RPW * UNROLL) == 0, "keys per wavefront must be whole rounds of rows");
@@ -188,18 +189,29 @@ __device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits,
         u32x4 v[UNROLL];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) v[u] = __builtin_nontemporal_load(p[u] + col);
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u)
-          if (ok[u]) {
-            gout_t dst = (gout_t)out + (b0 + r0 + u * RPW + rg) * vpr + col;
-            // a template parameter: the two stores of a run-time choice get merged and lose the hint
-            if constexpr (NT_STORE) __builtin_nontemporal_store(v[u], dst);
-            else *dst = v[u];
-          }
-        if constexpr (STAGE) {
+        const gout_t dst = (gout_t)out + (b0 + r0 + rg) * vpr + col;
+        if (!NT_STORE && through) {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
-            if (ps[u]) ps[u][col] = v[u];
+            if (ok[u]) store_through(reinterpret_cast<uint64_t>(dst + (size_t)u * RPW * vpr), v[u]);
+          if constexpr (STAGE) {
+#pragma unroll
+            for (int u = 0; u < UNROLL; ++u)
+              if (ps[u]) store_through(reinterpret_cast<uint64_t>(ps[u] + col), v[u]);
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+            if (ok[u]) {
+              // a template parameter: the two stores of a run-time choice get merged and lose the hint
+              if constexpr (NT_STORE) __builtin_nontemporal_store(v[u], dst + (size_t)u * RPW * vpr);
+              else dst[(size_t)u * RPW * vpr] = v[u];
+            }
+          if constexpr (STAGE) {
+#pragma unroll
+            for (int u = 0; u < UNROLL; ++u)
+              if (ps[u]) ps[u][col] = v[u];
+          }
         }
       }
     }
@@ -230,7 +242,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
                                                              const void *__restrict__ host, uint64_t host_rows,
                                                              void *__restrict__ out, FlatRow f_row,
                                                              uint32_t *status, uint32_t *host_mirror,
-                                                             unsigned long long *counts, ugk_stage_t stage) {
+                                                             DoneWords done, ugk_stage_t stage) {
   __shared__ uint32_t block_tot[2];
   if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
   __syncthreads();
@@ -250,7 +262,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
     const MixRow row = mix_resolve(t, key, active, f, static_cast<const unit_t *>(cache), cache_rows,
                                    static_cast<const unit_t *>(host), host_rows, out,
                                    LPR == 0 ? f_row.row_bytes : f_row.chunks, status, host_mirror);
-    if (counts) {
+    if (done.words) {
       // rows from the cache, and all others (host rows, and rows skipped for a key without a row: the launch is
       // flagged then and its group sizes mean nothing, but the two sums still add up to n)
       wave_local += __popcll(__ballot(row.from_cache));
@@ -260,15 +272,17 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       const uint64_t bits = row.has_row ? row.bits : row.bits | kNoRowBit;
       const uint32_t here = (uint32_t)min((size_t)KPW, n - b0);
       for (uint32_t r0 = 0; r0 < here; r0 += f_row.tile)
-        flat_copy<true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
+        flat_copy<true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row,
+                        done.tag != 0);
     } else {
       const uint32_t vpr = f_row.chunks;
       uint64_t stage_bits = 0;
       if constexpr (STAGE) stage_bits = stage_claim(stage, row, vpr);
-      mix_copy<LPR, KPW, NT_STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
+      mix_copy<LPR, KPW, NT_STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr,
+                                          done.tag != 0);
     }
   }
-  if (counts) mix_leave_counts(block_tot, wave_local, wave_host, counts);
+  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
 }
 
 // ---- dedup -----------------------------------------------------------------------------------------------
@@ -505,7 +519,7 @@ template <typename K, int KIND>
 int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, uint64_t cache_rows, const void *host,
                     uint64_t host_rows, void *out, size_t row_bytes, bool flat, uint32_t *status,
                     uint32_t *host_mirror, uint64_t *counts, uint32_t *num_groups, uint32_t others_hint, const ugk_stage_t *stage,
-                    hipStream_t st) {
+                    DoneRequest &request, hipStream_t st) {
   // ordinary write-back stores while the output fits the memory-side cache (the consumer finds it there),
   // non-temporal beyond, or as the caller's hint says
   const bool nt = nt_store_for(n * row_bytes);
@@ -556,12 +570,14 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const FlatRow f_row = flat_row(row_bytes, (uint32_t)kpw);
   const size_t keys_per_group = (size_t)kpw * kWavesPerBlock;
   const unsigned grid = clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u);
-  if (num_groups) *num_groups = grid;
+  DoneWords done = nt && !flat ? DoneWords{nullptr, nullptr, 0} : request.take(grid, n);
+  if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
+  if (num_groups) *num_groups = done.tag ? 0 : grid;
   const ugk_stage_t no_stage{};
 #define UGK_GO4(L, W, NT, ST)                                                                                       \
   hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, NT, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
-                     cache, cache_rows, host, host_rows, out, f_row, status, host_mirror,                          \
-                     reinterpret_cast<unsigned long long *>(counts), ST ? *stage : no_stage)
+                     cache, cache_rows, host, host_rows, out, f_row, status, host_mirror, done,                    \
+                     ST ? *stage : no_stage)
 #define UGK_GO3(L, W, NT)               \
   do {                                  \
     if (stage) UGK_GO4(L, W, NT, true); \
@@ -618,6 +634,7 @@ template <typename K>
 int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint64_t cache_rows, const void *host,
                 uint64_t host_rows, void *out, size_t row_bytes, uint32_t *status, uint32_t *host_mirror,
                 uint64_t *counts, uint32_t *num_groups, uint32_t others_hint, const ugk_stage_t *stage, void *stream) {
+  DoneRequest request;
   if (num_groups) *num_groups = 0;
   if (n == 0) return 0;
   UGK_REQUIRE(keys && out && status, "ugk_extract_mix: null keys, output or status");
@@ -648,12 +665,12 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
   }
   if (t.kind == 1)
     return extract_mix_lpr<K, 1>(t, keys, n, cache, cache_rows, host, host_rows, out, row_bytes, flat, status,
-                                 host_mirror, counts, num_groups, others_hint, stage, as_stream(stream));
+                                 host_mirror, counts, num_groups, others_hint, stage, request, as_stream(stream));
   if (t.kind == 2)
     return extract_mix_lpr<K, 2>(t, keys, n, cache, cache_rows, host, host_rows, out, row_bytes, flat, status,
-                                 host_mirror, counts, num_groups, others_hint, stage, as_stream(stream));
+                                 host_mirror, counts, num_groups, others_hint, stage, request, as_stream(stream));
   return extract_mix_lpr<K, 3>(t, keys, n, cache, cache_rows, host, host_rows, out, row_bytes, flat, status,
-                               host_mirror, counts, num_groups, others_hint, stage, as_stream(stream));
+                               host_mirror, counts, num_groups, others_hint, stage, request, as_stream(stream));
 }
 
 // The workspace is laid out by its own size, not by the batch's: `cap` slot words, then cap / 2 words of unique ids by

@@ -98,7 +98,7 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
                                              uint64_t cache_rows, const u32x4 *__restrict__ host, uint64_t host_rows,
                                              u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
                                              float max_norm, uint32_t *status, uint32_t *host_mirror,
-                                             const unsigned long long *counts, uint32_t &wave_local,
+                                             const DoneWords &done, uint32_t &wave_local,
                                              uint32_t &wave_host) {
   constexpr int RPW = kWave / LPR;  // output rows per wavefront and pass
   constexpr int EPC = PoolElem<E>::kPerChunk;
@@ -142,7 +142,7 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
       const Found f = table_lookup<KIND>(t, key, active);
       const MixRow row = mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
-      if (counts) {
+      if (done.words) {
         wave_local += __popcll(__ballot(row.from_cache));
         wave_host += __popcll(__ballot(active && !row.from_cache));
       }
@@ -253,7 +253,9 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
           float y[EPC];
 #pragma unroll
           for (int e = 0; e < EPC; ++e) y[e] = denom != 0.f ? acc[c][e] / denom : 0.f;  // div_no_nan
-          out[r * vpr + col] = PoolElem<E>::pack(y, bf16);
+          const u32x4 packed = PoolElem<E>::pack(y, bf16);
+          if (done.tag) store_through(reinterpret_cast<uint64_t>(out + r * vpr + col), packed);
+          else out[r * vpr + col] = packed;
         }
       }
     }
@@ -269,7 +271,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
                                                               const u32x4 *__restrict__ host, uint64_t host_rows,
                                                               u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
                                                               float max_norm, uint32_t *status, uint32_t *host_mirror,
-                                                              unsigned long long *counts, uint32_t keep_waves) {
+                                                              DoneWords done, uint32_t keep_waves) {
   __shared__ uint32_t block_tot[2];
   if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
   __syncthreads();
@@ -277,12 +279,12 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
   if (!MIXED || wave_in_block() < keep_waves)
     pool_samples<K, KIND, LPR, CH, U, E, CLIP, true>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host,
                                                      host_rows, out, vpr, combiner, bf16, max_norm, status, host_mirror,
-                                                     counts, wave_local, wave_host);
+                                                     done, wave_local, wave_host);
   else if constexpr (MIXED)
     pool_samples<K, KIND, LPR, CH, U, E, CLIP, false>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host,
                                                       host_rows, out, vpr, combiner, bf16, max_norm, status, host_mirror,
-                                                      counts, wave_local, wave_host);
-  if (counts) mix_leave_counts(block_tot, wave_local, wave_host, counts);
+                                                      done, wave_local, wave_host);
+  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
 }
 
 constexpr int kPoolMaxRows = 8;  // output rows a lane group may own per pass
@@ -306,7 +308,7 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
                                                    uint64_t cache_rows, const u32x4 *__restrict__ host,
                                                    uint64_t host_rows, u32x4 *__restrict__ out, uint32_t vpr,
                                                    int combiner, bool bf16, uint32_t *status, uint32_t *host_mirror,
-                                                   const unsigned long long *counts, uint32_t &wave_local,
+                                                   const DoneWords &done, uint32_t &wave_local,
                                                    uint32_t &wave_host,
                                                    long long (&seg_beg)[kWavesPerBlock][kWave / LPR][kPoolMaxRows],
                                                    uint32_t (&seg_start)[kWavesPerBlock][kWave / LPR][kPoolMaxRows]) {
@@ -365,7 +367,9 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
       float y[EPC];
 #pragma unroll
       for (int e = 0; e < EPC; ++e) y[e] = denom != 0.f ? acc[c][e] / denom : 0.f, acc[c][e] = 0.f;
-      out[(g0 + k) * vpr + col] = PoolElem<E>::pack(y, bf16);
+      const u32x4 packed = PoolElem<E>::pack(y, bf16);
+      if (done.tag) store_through(reinterpret_cast<uint64_t>(out + (g0 + k) * vpr + col), packed);
+      else out[(g0 + k) * vpr + col] = packed;
     };
     for (uint32_t f0 = 0; __ballot(f0 < total) != 0ull; f0 += LPR) {  // until every group of the wavefront is through
       const uint32_t f = f0 + sub;
@@ -379,7 +383,7 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
       const Found fd = table_lookup<KIND>(t, key, active);
       const MixRow row = mix_resolve(t, key, active, fd, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
-      if (counts) {
+      if (done.words) {
         wave_local += __popcll(__ballot(row.from_cache));
         wave_host += __popcll(__ballot(active && !row.from_cache));
       }
@@ -454,7 +458,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
                                                               const u32x4 *__restrict__ host, uint64_t host_rows,
                                                               u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
                                                               uint32_t *status, uint32_t *host_mirror,
-                                                              unsigned long long *counts, uint32_t keep_waves) {
+                                                              DoneWords done, uint32_t keep_waves) {
   __shared__ uint32_t block_tot[2];
   __shared__ long long seg_beg[kWavesPerBlock][kWave / LPR][kPoolMaxRows];    // first id of the group's row k
   __shared__ uint32_t seg_start[kWavesPerBlock][kWave / LPR][kPoolMaxRows];   // its first position in the group's list
@@ -463,20 +467,20 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
   uint32_t wave_local = 0, wave_host = 0;
   if (!MIXED || wave_in_block() < keep_waves)
     pool_short_samples<K, KIND, LPR, E, true>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
-                                              host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
+                                              host, host_rows, out, vpr, combiner, bf16, status, host_mirror, done,
                                               wave_local, wave_host, seg_beg, seg_start);
   else if constexpr (MIXED)
     pool_short_samples<K, KIND, LPR, E, false>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
-                                               host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
+                                               host, host_rows, out, vpr, combiner, bf16, status, host_mirror, done,
                                                wave_local, wave_host, seg_beg, seg_start);
-  if (counts) mix_leave_counts(block_tot, wave_local, wave_host, counts);
+  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
 }
 
 template <typename K, int KIND, typename E>
 int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, const float *weights, size_t n_rows,
                      const void *cache, uint64_t cache_rows, const void *host, uint64_t host_rows, void *out,
                      uint32_t vpr, uint64_t nnz, int combiner, bool bf16, float max_norm, uint32_t *status,
-                     uint32_t *host_mirror, uint64_t *counts, uint32_t *num_groups, hipStream_t st) {
+                     uint32_t *host_mirror, uint64_t *counts, uint32_t *num_groups, DoneRequest &request, hipStream_t st) {
   // Lanes per output row, chunks per lane and ids in flight (LPR, CH, U).  The fewest lanes that hold a row with the
   // fewest registers are best for few ids per sample (a lane group resolves LPR ids at a time and keeps U rows on
   // their way, and both are wasted on a sample that has fewer), more lanes and more rows in flight for many.  us per
@@ -541,6 +545,8 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   // of whole lines up to 384 bytes.  The other fp32 rows are faster one by one, 800,000 samples (400,000 from 640 bytes
   // on) uniform and Zipf 1.05, list / one by one: 64 bytes 54 / 37 and 48 / 31, 160 bytes 95 / 81 and 81 / 72, 400 bytes
   // 239 / 165 and 186 / 167, 512 bytes 179 / 169 and 169 / 162, 1 KB 184 / 165 and 183 / 164, 2 KB 329 / 322 and 318 / 318.
+  // (an output that does not fit the memory-side cache is not written through: 131,072 samples of one id of 2 KB 120 -> 122 us)
+  const uint64_t polled_nnz = n_rows * (size_t)vpr * 16 <= kMemorySideCacheBytes ? nnz : ~0ull;
   int rows = 1;
   if constexpr (KIND != 1) {
     const int lanes = vpr <= 32 ? 8 : vpr <= 128 ? 32 : 64;
@@ -557,7 +563,9 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
     if (rows > 1) {
       const size_t rows_per_block = (size_t)rows * groups * kWavesPerBlock;
       const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
-      if (num_groups) *num_groups = grid;
+      DoneWords done = request.take(grid, polled_nnz);
+      if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
+      if (num_groups) *num_groups = done.tag ? 0 : grid;
       // (256 bytes uniform and Zipf 1.05, before / without the hint / one wavefront of four without: 90 / 101 / 91 and
       // 102 / 91 / 91)
       constexpr bool kMixed = KIND == 0 && sizeof(E) == 4;
@@ -566,7 +574,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   hipLaunchKernelGGL((extract_pool_rows_kernel<K, KIND, L, E, kMixed>), dim3(grid), dim3(kBlock), 0, st, t, ids,       \
                      seg_off, weights, n_rows, (long long)nnz, rows, (const u32x4 *)cache, cache_rows,                 \
                      (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, status, host_mirror,           \
-                     reinterpret_cast<unsigned long long *>(counts), keep)
+                     done, keep)
       if (lanes == 8) UGK_POOL_ROWS_GO(8);
       else if (lanes == 32) UGK_POOL_ROWS_GO(32);
       else UGK_POOL_ROWS_GO(64);
@@ -577,7 +585,9 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   }
   const size_t rows_per_block = (size_t)(kWave / (shape / 100)) * kWavesPerBlock;
   const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
-  if (num_groups) *num_groups = grid;
+  DoneWords done = request.take(grid, polled_nnz);
+  if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
+  if (num_groups) *num_groups = done.tag ? 0 : grid;
   const bool mixed = keep_waves < kWavesPerBlock;
   bool launched = false;
 #define UGK_POOL(L, CH, U, CLIP, MIXED)                                                                                \
@@ -586,7 +596,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
     hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, CH, U, E, CLIP, MIXED>), dim3(grid), dim3(kBlock), 0, st, t,   \
                      ids, seg_off, weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows,                  \
                      (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status, host_mirror, \
-                     reinterpret_cast<unsigned long long *>(counts), keep_waves);                                      \
+                     done, keep_waves);                                                                                \
   }
   UGK_POOL(4, 1, 2, false, false)
   UGK_POOL(4, 1, 4, false, false)
@@ -657,6 +667,7 @@ int extract_pool(ugk_table_t t, const K *ids, const int64_t *seg_off, const floa
                  int combiner, int elem_bytes, const void *cache, uint64_t cache_rows, const void *host,
                  uint64_t host_rows, void *out, size_t row_bytes, float max_norm, uint32_t *status,
                  uint32_t *host_mirror, uint64_t *counts, uint32_t *num_groups, void *stream) {
+  DoneRequest request;
   if (num_groups) *num_groups = 0;
   if (n_rows == 0) return 0;
   UGK_REQUIRE(seg_off && out && status, "ugk_extract_pool: null offsets, output or status");
@@ -686,10 +697,10 @@ int extract_pool(ugk_table_t t, const K *ids, const int64_t *seg_off, const floa
 #define UGK_POOL_KIND(KIND)                                                                                          \
   (elem_bytes == 4 ? extract_pool_lpr<K, KIND, float>(t, ids, so, weights, n_rows, cache, cache_rows, host, host_rows, \
                                                       out, vpr, nnz, combiner, false, max_norm, status, host_mirror,  \
-                                                      counts, num_groups, st)                                         \
+                                                      counts, num_groups, request, st)                                      \
                    : extract_pool_lpr<K, KIND, __half>(t, ids, so, weights, n_rows, cache, cache_rows, host,          \
                                                        host_rows, out, vpr, nnz, combiner, bf16, max_norm, status,    \
-                                                       host_mirror, counts, num_groups, st))
+                                                       host_mirror, counts, num_groups, request, st))
   if (t.kind == 0) return UGK_POOL_KIND(0);
   if (t.kind == 1) return UGK_POOL_KIND(1);
   if (t.kind == 2) return UGK_POOL_KIND(2);

@@ -31,6 +31,20 @@ int cu_count() {
   return cached[dev];
 }
 
+static thread_local ugk_done_t *g_done = nullptr;
+
+DoneRequest::DoneRequest() : _done(g_done) { g_done = nullptr; }
+
+// a counter holds 16 bits of workgroups and two counts of 24 bits
+DoneWords DoneRequest::take(unsigned grid, uint64_t count_limit) {
+  if (!_done || grid / kDoneFan >= 0xffffu || count_limit >= (1u << 24)) return DoneWords{nullptr, nullptr, 0};
+  ugk_done_t *d = _done;
+  _done = nullptr;
+  d->num_words = grid <= kDoneDirect ? grid : kDoneFan;
+  return DoneWords{reinterpret_cast<unsigned long long *>(d->words_host),
+                   reinterpret_cast<unsigned long long *>(d->counters_dev), d->tag};
+}
+
 int blocks_per_cu() {
   static int v = 0;
   if (v == 0) {
@@ -244,6 +258,43 @@ int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, 
   // microseconds the poll saved
   if (*word == value) return 0;
   UGK_HIP(hipStreamSynchronize(as_stream(stream)));
+  return 0;
+}
+
+int ugk_leave_done_words(ugk_done_t *done) {
+  if (done) {
+    UGK_REQUIRE(done->words_host && done->counters_dev, "ugk_leave_done_words: null words or counters");
+    UGK_REQUIRE(done->tag > 0 && done->tag <= UGK_DONE_MAX_TAG, "ugk_leave_done_words: tag %u is not in [1, %u]", done->tag,
+                UGK_DONE_MAX_TAG);
+    done->num_words = 0;
+  }
+  ugk::g_done = done;
+  return 0;
+}
+
+int ugk_done_wait(const ugk_done_t *done, unsigned spin_us, void *stream, uint64_t *local, uint64_t *others) {
+  UGK_REQUIRE(done && done->num_words > 0 && done->num_words <= UGK_DONE_WORDS, "ugk_done_wait: no words to wait for");
+  const volatile uint64_t *words = done->words_host;
+  const auto t0 = std::chrono::steady_clock::now();
+  uint64_t sum_local = 0, sum_others = 0;
+  bool spin = true;
+  for (uint32_t i = 0; i < done->num_words; ++i) {
+    uint64_t w = words[i];
+    for (unsigned polls = 1; (w >> 48) != done->tag && spin; w = words[i], ++polls)
+      if ((polls & 63u) == 0)
+        spin = std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0).count() <
+               (long long)spin_us;
+    if ((w >> 48) != done->tag) {
+      UGK_HIP(hipStreamSynchronize(as_stream(stream)));
+      w = words[i];
+      UGK_REQUIRE((w >> 48) == done->tag, "ugk_done_wait: the launch has ended without word %u", i);
+    }
+    sum_local += w & 0xffffffu;
+    sum_others += (w >> 24) & 0xffffffu;
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  if (local) *local = sum_local;
+  if (others) *others = sum_others;
   return 0;
 }
 

@@ -44,6 +44,11 @@ class Stage(C.Structure):
                 ("reserved", C.c_uint32)]
 
 
+class Done(C.Structure):
+    """ugk_done_t"""
+    _fields_ = [("words_host", C.c_void_p), ("counters_dev", C.c_void_p), ("tag", C.c_uint32), ("num_words", C.c_uint32)]
+
+
 class DeviceInfo(C.Structure):
     """ugk_device_info_t"""
     _fields_ = [("name", C.c_char * 256), ("arch", C.c_char * 64), ("compute_units", C.c_int32),
@@ -70,6 +75,8 @@ SIGNATURES = {
     "ugk_stream_sync": [_vp],
     "ugk_stream_is_capturing": [_vp, _vp],
     "ugk_stream_sync_ticket": [_vp, _vp, _u32, C.c_uint],
+    "ugk_leave_done_words": [C.POINTER(Done)],
+    "ugk_done_wait": [C.POINTER(Done), C.c_uint, _vp, C.POINTER(_u64), C.POINTER(_u64)],
     "ugk_words_to_host_ticket": [_vp, C.c_uint, _vp, C.c_uint, _vp, _u32, C.c_uint, _vp],
     "ugk_preload_kernels": [],
     "ugk_device_sync": [],
