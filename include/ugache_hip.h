@@ -159,6 +159,8 @@ typedef struct {
   uint64_t *counters_dev;
   uint32_t tag;
   uint32_t num_words; /* set by the launch */
+  void *keys_host;    /* pinned: a launch with words leaves its first num_keys keys there, complete as its rows are */
+  uint64_t num_keys;  /* 0: none */
 } ugk_done_t;
 int ugk_leave_done_words(ugk_done_t *done);
 int ugk_done_wait(const ugk_done_t *done, unsigned spin_us, void *stream, uint64_t *local, uint64_t *others);

@@ -160,12 +160,14 @@ void copy_row(void *dst, const void *src, size_t bytes) { memcpy(dst, src, bytes
 
 // ugk_leave_done_words: work has been done when a call of the model returns, so its one word is written there
 thread_local ugk_done_t *g_done = nullptr;
-bool leave_done(uint64_t local, uint64_t others) {
+template <typename K>
+bool leave_done(uint64_t local, uint64_t others, const K *keys, size_t n) {
   ugk_done_t *d = g_done;
   g_done = nullptr;
   if (!d || local + others >= (1u << 24)) return false;
   d->num_words = 1;
   d->words_host[0] = ((uint64_t)d->tag << 48) | (others << 24) | local;
+  for (size_t i = 0; i < std::min<size_t>(n, d->num_keys); ++i) static_cast<K *>(d->keys_host)[i] = keys[i];
   return true;
 }
 
@@ -182,7 +184,7 @@ int gather_direct(const void *src, uint64_t src_rows, const K *keys, const uint3
     }
     copy_row((char *)out + d * rb, (const char *)src + s * rb, rb);
   }
-  if (dst == nullptr) leave_done(0, 0);
+  if (dst == nullptr) leave_done(0, 0, keys, n);
   return 0;
 }
 
@@ -437,7 +439,7 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
     if (from_cache) ++local;
     else ++others;
   }
-  const bool polled = leave_done(local, others);
+  const bool polled = leave_done(local, others, keys, n);
   if (counts && !polled) counts[0] = (others << 32) | local;
   if (num_groups) *num_groups = polled ? 0 : 1;
   return 0;
@@ -566,7 +568,7 @@ int extract_pool(ugk_table_t t, const K *ids, const int64_t *seg_off, const floa
       }
     }
   }
-  const bool polled = leave_done(local, others);
+  const bool polled = leave_done(local, others, ids, nnz);
   if (counts && !polled) counts[0] = (others << 32) | local;
   if (num_groups) *num_groups = polled ? 0 : 1;
   return 0;

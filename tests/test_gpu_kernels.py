@@ -830,11 +830,22 @@ class _DoneWords:
         self.words = PinnedArray((256,), np.uint64)
         self.words.array[:] = 0
         self.counters = torch.zeros(64 * 16, dtype=torch.int64, device="cuda")
-        self.done = hip.Done(self.words.ptr, ptr(self.counters), 0, 0)
+        self.keys = PinnedArray((4_096,), np.int64)
+        self.done = hip.Done(self.words.ptr, ptr(self.counters), 0, 0, self.keys.ptr, 0)
 
-    def run(self, launch, spin_us, groups):
-        self.done.tag = self.done.tag + 1
+    def ask(self, num_keys):
+        """the first num_keys keys of the launch are wanted too"""
+        self.keys.array[:] = -7
+        self.done.num_keys, self.done.tag = min(num_keys, 4_096), self.done.tag + 1
         hip.call("ugk_leave_done_words", C.byref(self.done))
+
+    def check_keys(self, keys):
+        """they came, all of them and nothing behind them"""
+        n = self.done.num_keys
+        assert (self.keys.array[:n] == keys[:n]).all() and (self.keys.array[n:] == -7).all()
+
+    def run(self, launch, spin_us, groups, num_keys=0):
+        self.ask(num_keys)
         launch()
         if groups is None:
             assert self.done.num_words == 0
@@ -871,16 +882,17 @@ def test_gather_that_tells_its_end_by_words(row_bytes, rows_per_group, spin_us):
         def launch():
             hip.call("ugk_gather_direct_i64", ptr(table), rows, ptr(q), n, ptr(out), row_bytes, 0, ptr(st), None, None)
 
+        wanted = (0, 1, n // 2 + 1, n, n // 20)[groups % 5]
         if rows_per_group:
-            assert done.run(launch, spin_us, groups) == (0, 0)
+            assert done.run(launch, spin_us, groups, wanted) == (0, 0)
         else:  # the number of workgroups is the kernel's own affair
-            done.done.tag += 1
-            hip.call("ugk_leave_done_words", C.byref(done.done))
+            done.ask(wanted)
             launch()
             assert done.done.num_words > 0
             hip.call("ugk_done_wait", C.byref(done.done), spin_us, None, None, None)
             assert not done.counters.any().item()
         assert torch.equal(out, want)
+        done.check_keys(to_np(q))
         assert status_value(st) == (hip.ST_KEY_OUT_OF_RANGE if n > 4 else 0)
     # the request met one call: the next one leaves nothing; and streaming outputs are waited for in another way
     before = done.words.array.copy()
@@ -922,8 +934,7 @@ def test_fused_and_pooled_lookups_that_tell_their_end_by_words(kind, rb, stage):
         sync()
         args = [tb, ptr(d_keys), n, ptr(d_cache), len(cached), pin.ptr, nkeys, ptr(out), rb, ptr(st), None, None,
                 C.byref(groups), hip.HINT_UNKNOWN]
-        done.done.tag += 1
-        hip.call("ugk_leave_done_words", C.byref(done.done))
+        done.ask((0, 1, n // 20, n)[epoch % 4])
         if stage:
             hip.call("ugk_extract_mix_staged_i64", *args, hip.Stage(ptr(s_rows), ptr(s_owner), 1023, epoch, 0), None)
         else:
@@ -932,6 +943,7 @@ def test_fused_and_pooled_lookups_that_tell_their_end_by_words(kind, rb, stage):
         assert done.done.num_words > 0 and groups.value == 0
         hip.call("ugk_done_wait", C.byref(done.done), 1_000_000, None, C.byref(local), C.byref(others))
         assert (local.value, others.value) == (in_cache[keys].sum(), (~in_cache[keys]).sum())
+        done.check_keys(keys)
         assert torch.equal(out[: n * rb].view(n, rb), d_table[torch.from_numpy(keys).cuda()])
         assert not done.counters.any().item()
         if rb % 16 == 0 and not stage:
@@ -940,13 +952,13 @@ def test_fused_and_pooled_lookups_that_tell_their_end_by_words(kind, rb, stage):
             off = torch.arange(0, n_rows * per + 1, per, device="cuda")
             pooled = torch.empty((n_rows, rb // 4), dtype=torch.float32, device="cuda")
             sync()
-            done.done.tag += 1
-            hip.call("ugk_leave_done_words", C.byref(done.done))
+            done.ask((1, n // 20, n_rows * per, 0)[epoch % 4])
             hip.call("ugk_extract_pool_i64", tb, ptr(d_keys), ptr(off), None, n_rows, n_rows * per, 0, 4, ptr(d_cache),
                      len(cached), pin.ptr, nkeys, ptr(pooled), rb, ptr(st), None, None, C.byref(groups), None)
             assert done.done.num_words > 0 and groups.value == 0
             hip.call("ugk_done_wait", C.byref(done.done), 0, None, C.byref(local), C.byref(others))
             used = keys[: n_rows * per]
+            done.check_keys(used)
             assert (local.value, others.value) == (in_cache[used].sum(), (~in_cache[used]).sum())
             want = d_table.view(torch.float32)[torch.from_numpy(used).cuda()].view(n_rows, per, -1).sum(1)
             assert torch.equal(pooled, want)

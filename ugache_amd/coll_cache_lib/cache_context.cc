@@ -831,14 +831,31 @@ void ExtractSession::SumMixCounts() {
 
 // In front of the one launch of a blocking lookup that is waited for by WaitForBatch next: asks that its workgroups leave
 // words for the wait to poll.
-void ExtractSession::AskForDoneWords() {
+void ExtractSession::AskForDoneWords(StreamHandle stream) {
   _done.num_words = 0;
-  if (RunConfig::spin_wait_us == 0) return;
+  if (RunConfig::spin_wait_us == 0) {
+    CopyKeysNow(stream);
+    return;
+  }
   if (++_done.tag > UGK_DONE_MAX_TAG) {  // nothing is in flight that uses the words: blocking lookups follow each other
     memset(_done.words_host, 0, UGK_DONE_WORDS * sizeof(uint64_t));
     _done.tag = 1;
   }
+  _done.keys_host = _along_dst;
+  _done.num_keys = _along_num;
   UGK_CALL(ugk_leave_done_words(&_done));
+}
+
+void ExtractSession::CopyKeysNow(StreamHandle stream) {
+  if (_along_num == 0) return;
+  UGK_CALL(ugk_copy_rows(_along_dst, _along_src, _along_bytes, stream));
+  _along_num = 0;
+}
+
+void ExtractSession::FinishKeysAlong(StreamHandle stream) {
+  if (_along_num == 0) return;
+  CopyKeysNow(stream);
+  UGK_CALL(ugk_stream_sync(stream));
 }
 
 // The wait of a blocking lookup.  A launch that leaves words is polled for by them, which also bring its group sizes.
@@ -849,11 +866,13 @@ void ExtractSession::WaitForBatch(StreamHandle stream) {
     uint64_t local = 0, others = 0;
     UGK_CALL(ugk_done_wait(&_done, RunConfig::spin_wait_us, stream, &local, &others));
     _done.num_words = 0;
+    _along_num = 0;
     _mix_groups = 0;
     _host_mirror[kMirGroupSizes + UGK_LOC_LOCAL] = (uint32_t)local;
     _host_mirror[kMirGroupSizes + UGK_LOC_HOST] = (uint32_t)others;
     return;
   }
+  CopyKeysNow(stream);
   if (RunConfig::spin_wait_us == 0) {
     UGK_CALL(ugk_stream_sync(stream));
     return;
@@ -898,7 +917,9 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
   const uint32_t *dst_map = nullptr, *inverse = nullptr;
   float ms_dedup = 0;
   const bool skip_local = !ctx->IsDirectMapping() && GetEnv("COLL_SKIP_LOCAL") == "1";
-  if (RunConfig::dedup_keys && num_nodes >= RunConfig::dedup_min_keys && !_skip_dedup && !skip_local) {
+  const bool dedup = RunConfig::dedup_keys && num_nodes >= RunConfig::dedup_min_keys && !_skip_dedup && !skip_local;
+  if (dedup || skip_local) CopyKeysNow(stream);  // the launches work on other keys than the caller's
+  if (dedup) {
     UGK_CALL(ugk_event_record(_ev_t[2], stream));
     const size_t nu = DedupKeys(nodes, num_nodes, stream);
     UGK_CALL(ugk_event_record(_ev_t[3], stream));
@@ -921,7 +942,7 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
     Timer t_host;
     if (events) UGK_CALL(ugk_event_record(_ev_t[0], stream));
     if (dst_map == nullptr) {
-      AskForDoneWords();
+      AskForDoneWords(stream);
       UGK_CALL(GatherDirect(ctx->_device_cache_data[0], ctx->_num_total_nodes, nodes, num_nodes, output, rb,
                             from_host ? _cpu_blocks : 0, _status, _host_mirror, stream));
     } else {
@@ -990,7 +1011,7 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
     // from outside the cache), not guessed from the previous batch.
     const uint32_t hint = skip_local ? (uint32_t)num_nodes : UGK_HINT_UNKNOWN;
     const ugk_stage_t *stage = StageTakes(output) ? NextStage(stream, false) : nullptr;
-    AskForDoneWords();
+    AskForDoneWords(stream);
     UGK_CALL(ExtractMix(table, nodes, num_nodes, cache, cache_rows, host, host_rows, output, rb, _status,
                         _host_mirror, _mix_counts->ptr<uint64_t>(), &_mix_groups, hint, stage, stream));
     if (events) UGK_CALL(ugk_event_record(_ev_t[1], stream));
@@ -1022,6 +1043,7 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
   }
 
   // classify + partition on the caller's stream, then one gather per source
+  CopyKeysNow(stream);
   EnsureIdx(num_nodes);
   ugk_idx_t *idx = _idx_handle->ptr<ugk_idx_t>();
   uint32_t *cur = _counts[_cur], *next = _counts[_cur ^ 1];
@@ -1288,7 +1310,7 @@ bool ExtractSession::LaunchPooled(const KeyT *nodes, const int64_t *seg_off, con
   }
   CHECK((((uintptr_t)cache | (uintptr_t)host | (uintptr_t)output) & 15u) == 0) << "pooled lookup: misaligned buffer";
   const RecordPlan keys_ready = RecordBegin(stream);
-  if (blocking) AskForDoneWords();
+  if (blocking) AskForDoneWords(stream);
   UGK_CALL(ExtractPool(table, nodes, seg_off, weights, num_rows, num_nodes, combiner, elem_bytes, _pool_max_norm, cache,
                        cache_rows, host, ctx->_num_total_nodes, output, rb, _status, _host_mirror,
                        _mix_counts->ptr<uint64_t>(), &_mix_groups, stream));

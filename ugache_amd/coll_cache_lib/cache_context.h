@@ -177,7 +177,11 @@ class ExtractSession {
   // what a blocking lookup's launch tells its end with (ugk_leave_done_words); num_words > 0: the launch in flight does
   MemHandle _done_words, _done_counters;
   ugk_done_t _done{};
-  void AskForDoneWords();
+  void AskForDoneWords(StreamHandle stream);
+  const void *_along_src = nullptr;  // CopyKeysAlong: the batch's keys, where a copy of the first of them goes
+  void *_along_dst = nullptr;
+  size_t _along_num = 0, _along_bytes = 0;
+  void CopyKeysNow(StreamHandle stream);
   // Rows that crossed the host link, kept for the next refresh (COLL_MISS_STAGE_ROWS): written by the fused extraction,
   // read by the refresh's row copy.  A foreground refresh runs while no lookup does and reads the stage the lookups
   // write.  A background refresh runs beside lookups, so there are two stages then: it switches the lookups over to
@@ -350,6 +354,13 @@ class ExtractSession {
   // the device-side counting of the following lookups covers only the first `num_keys` keys of a batch
   // (the recorded prefix of LookupManager's record thread); SIZE_MAX, the default: the whole batch
   void SetRecordLimit(size_t num_keys) { _record_limit = num_keys; }
+  // The next blocking lookup of `keys` leaves a copy of the first num_keys of them in pinned host memory: its own launch
+  // where that leaves words for the wait, a copy kernel on its stream otherwise.  FinishKeysAlong, behind the lookup: the
+  // copy is complete (a lookup that launched nothing has not made it).
+  void CopyKeysAlong(const void *keys, void *pinned, size_t num_keys, size_t key_bytes) {
+    _along_src = keys, _along_dst = pinned, _along_num = num_keys, _along_bytes = num_keys * key_bytes;
+  }
+  void FinishKeysAlong(StreamHandle stream);
   // the pooled lookups that follow clip every looked-up row to this l2 norm before it is weighted (the max_norm of
   // the sparse layer, sparse_lookup_layer.py:95-140); 0, the default: no clipping
   void SetPooledMaxNorm(float max_norm) { _pool_max_norm = max_norm; }

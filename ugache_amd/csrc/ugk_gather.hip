@@ -30,6 +30,7 @@ constexpr uint64_t kNoLimit = ~0ull;
 // ---- index functors (what the reference calls IdxStore*) -------------------------------------------
 struct DirectU32 {
   static constexpr bool kDense = true;  // row i goes to output row i
+  typedef uint32_t key_t;
   const uint32_t *keys;
   __device__ __forceinline__ void get(size_t i, uint64_t &s, uint64_t &d) const {
     s = keys[i];
@@ -38,6 +39,7 @@ struct DirectU32 {
 };
 struct DirectI64 {
   static constexpr bool kDense = true;
+  typedef int64_t key_t;
   const int64_t *keys;
   __device__ __forceinline__ void get(size_t i, uint64_t &s, uint64_t &d) const {
     s = (uint64_t)keys[i];  // negative keys become huge and fail the range check
@@ -112,6 +114,11 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
   constexpr size_t kPerIter = (size_t)RPB * UNROLL;
 
   for (size_t base = (size_t)blockIdx.x * kPerIter; base < count; base += (size_t)gridDim.x * kPerIter) {
+    if constexpr (Idx::kDense) {
+      if (base < done.num_keys)
+        for (size_t i = base + threadIdx.x; i < min(base + kPerIter, count); i += kBlock)
+          copy_key_along(done, i, ix.keys[i]);
+    }
     // the index words of all rows of the pass first, in flight together (a row past the end takes the last one's),
     // then the checks: a check between two of them would make the second wait for the first
     uint64_t s[UNROLL], d[UNROLL];
@@ -195,6 +202,9 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
     uint64_t s = 0, d = 0;
     bool ok = lane_id() < rows;
     if (ok) ix.get(begin + base + lane_id(), s, d);
+    if constexpr (Idx::kDense) {
+      if (ok) copy_key_along(done, base + lane_id(), (typename Idx::key_t)s);
+    }
     if (ok && (s >= src_rows || d >= out_rows)) {
       ok = false;
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
@@ -254,6 +264,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     const bool active = (uint64_t)lane * f.row_bytes < (uint64_t)off0 + bytes;
     bool ok = active;
     if (ok) ix.get(row0 + lane, s, d);
+    if (ok) copy_key_along(done, row0 + lane, (typename Idx::key_t)s);  // a row in two parts: twice the same key
     if (ok && s >= src_rows) {
       ok = false;
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
@@ -456,7 +467,7 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
   constexpr size_t kPerIter = (size_t)(kBlock / LPR) * UNROLL;
   const unsigned grid = gather_grid((n + kPerIter - 1) / kPerIter, max_blocks);
   const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
-  const DoneWords done = nt ? DoneWords{nullptr, nullptr, 0} : request.take(grid);
+  const DoneWords done = nt ? DoneWords{} : request.take(grid);
   if (nt)
     hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, true, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,
                        reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,
@@ -573,7 +584,7 @@ int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t 
   const uint64_t per_block = (uint64_t)kStreamPart * kWavesPerBlock;
   const unsigned grid = gather_grid((f.total + per_block - 1) / per_block, max_blocks);
   const bool nt = nt_store_for(n * row_bytes);
-  const DoneWords done = nt ? DoneWords{nullptr, nullptr, 0} : request.take(grid);
+  const DoneWords done = nt ? DoneWords{} : request.take(grid);
 #define UGK_GO(NT, SHARE)                                                                                             \
   hipLaunchKernelGGL((gather_stream_kernel<NT, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,                \
                      (const char *)src, src_rows, (char *)out, f, status, host_mirror, done)

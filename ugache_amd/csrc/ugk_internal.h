@@ -59,6 +59,8 @@ bool nt_store_for(size_t out_bytes);
 // polls, and words, if there are any, are the per-workgroup counts of ugk_extract_mix_*.
 struct DoneWords {
   unsigned long long *words, *counters;
+  void *keys;         // the launch leaves its first num_keys keys here (pinned host memory)
+  uint64_t num_keys;
   uint32_t tag;
 };
 // Up to kDoneDirect workgroups leave a word each.  More of them meet in kDoneFan counters, workgroup b in counter b %

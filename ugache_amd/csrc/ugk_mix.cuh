@@ -30,6 +30,12 @@ __device__ __forceinline__ void store_through(uint64_t to, V v) {
   else asm volatile("global_store_byte %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"((uint32_t)v) : "memory");
 }
 
+// key i of the launch, where the host wants a copy (a lane per key: neighbouring lanes' keys leave as one write)
+template <typename K>
+__device__ __forceinline__ void copy_key_along(const DoneWords &done, uint64_t i, K key) {
+  if (i < done.num_keys) static_cast<K *>(done.keys)[i] = key;
+}
+
 // The last thing a workgroup does: its counts, and with a tag the news that it has ended.  All threads call it; tot (in LDS,
 // may be NULL) holds the rows taken from the cache and all others.
 __device__ __forceinline__ void leave_done(const DoneWords &done, const uint32_t *tot) {

@@ -254,6 +254,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
     const size_t i = b0 + lane;
     const bool active = lane < KPW && i < n;
     const uint64_t key = active ? key_to_u64<K>(keys[i]) : 0;
+    if (active) copy_key_along<K>(done, i, (K)key);
     // a full wavefront of keys probes its eight home lines in one go (see hash_probe_home)
     // (fewer keys: their home lines in one go as well, and only the rounds of the probe that have keys to serve)
     constexpr int ROUNDS = KPW >= 8 ? KPW / 8 : 1;
@@ -570,7 +571,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const FlatRow f_row = flat_row(row_bytes, (uint32_t)kpw);
   const size_t keys_per_group = (size_t)kpw * kWavesPerBlock;
   const unsigned grid = clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u);
-  DoneWords done = nt && !flat ? DoneWords{nullptr, nullptr, 0} : request.take(grid, n);
+  DoneWords done = nt && !flat ? DoneWords{} : request.take(grid, n);
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;
   const ugk_stage_t no_stage{};

@@ -140,6 +140,7 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
       const long long j = j0 + sub;
       const bool active = j < end;
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
+      if (active) copy_key_along<K>(done, (uint64_t)j, (K)key);
       const Found f = table_lookup<KIND>(t, key, active);
       const MixRow row = mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
       if (done.words) {
@@ -381,6 +382,7 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
       }
       const long long j = active ? my_beg[k] + (long long)(f - my_start[k]) : 0;
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
+      if (active) copy_key_along<K>(done, (uint64_t)j, (K)key);
       const Found fd = table_lookup<KIND>(t, key, active);
       const MixRow row = mix_resolve(t, key, active, fd, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
       if (done.words) {

@@ -37,12 +37,12 @@ DoneRequest::DoneRequest() : _done(g_done) { g_done = nullptr; }
 
 // a counter holds 16 bits of workgroups and two counts of 24 bits
 DoneWords DoneRequest::take(unsigned grid, uint64_t count_limit) {
-  if (!_done || grid / kDoneFan >= 0xffffu || count_limit >= (1u << 24)) return DoneWords{nullptr, nullptr, 0};
+  if (!_done || grid / kDoneFan >= 0xffffu || count_limit >= (1u << 24)) return DoneWords{};
   ugk_done_t *d = _done;
   _done = nullptr;
   d->num_words = grid <= kDoneDirect ? grid : kDoneFan;
   return DoneWords{reinterpret_cast<unsigned long long *>(d->words_host),
-                   reinterpret_cast<unsigned long long *>(d->counters_dev), d->tag};
+                   reinterpret_cast<unsigned long long *>(d->counters_dev), d->keys_host, d->num_keys, d->tag};
 }
 
 int blocks_per_cu() {
@@ -266,6 +266,7 @@ int ugk_leave_done_words(ugk_done_t *done) {
     UGK_REQUIRE(done->words_host && done->counters_dev, "ugk_leave_done_words: null words or counters");
     UGK_REQUIRE(done->tag > 0 && done->tag <= UGK_DONE_MAX_TAG, "ugk_leave_done_words: tag %u is not in [1, %u]", done->tag,
                 UGK_DONE_MAX_TAG);
+    UGK_REQUIRE(done->keys_host || done->num_keys == 0, "ugk_leave_done_words: null buffer for the keys");
     done->num_words = 0;
   }
   ugk::g_done = done;
