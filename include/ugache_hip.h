@@ -138,6 +138,8 @@ int ugk_stream_is_capturing(void *stream, int *capturing);
  * wait).  `value` must differ from what the word holds (a counter).  What kernels enqueued before the ticket wrote into
  * pinned host memory is visible once the ticket is. */
 int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, unsigned spin_us);
+/* the poll of ugk_stream_sync_ticket alone, for a ticket that some launch on `stream` writes itself */
+int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned spin_us, void *stream);
 /* The end of one launch polled for without a kernel behind it.  ugk_leave_done_words: the next ugk_gather_*,
  * ugk_extract_mix_* or ugk_extract_pool_* call of this thread (that one only; after a call that failed, and where none
  * comes, NULL takes the request back) makes its workgroups leave words in words_host as they end, and stores the number of
@@ -539,6 +541,12 @@ int ugk_rank_place_keep(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, voi
 int ugk_rank_place_observed(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, void *ws_dev, uint64_t *in_new_dev,
                             uint64_t *observed_dev, int reset_counts, const uint64_t *cached_dev, void *evict_ws_dev,
                             void *insert_ws_dev, uint32_t *totals_host, uint32_t *status_dev, void *stream);
+/* the same with a ticket (non-zero; 0: none) in totals_host[3], a fourth pinned word: once it is there the sums are, and the
+ * bitmap and the two workspaces may be read by launches on any stream (ugk_ticket_wait); cached_dev must not be NULL */
+int ugk_rank_place_observed_ticket(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, void *ws_dev,
+                                   uint64_t *in_new_dev, uint64_t *observed_dev, int reset_counts,
+                                   const uint64_t *cached_dev, void *evict_ws_dev, void *insert_ws_dev,
+                                   uint32_t *totals_host, uint32_t *status_dev, uint32_t ticket, void *stream);
 int ugk_rank_threshold(const void *ws_dev, uint64_t *threshold_host, void *stream);
 /* Ordered compaction over bitmaps.  The set S = { p < nbits : bit p of m is set }, m = (invert_a ? ~a : a) & ~b
  * (b_dev may be NULL).  ugk_bitmap_count writes |S| to *total_host (pinned host word, may be NULL) and leaves the
@@ -551,6 +559,10 @@ int ugk_bitmap_count(const uint64_t *a_dev, const uint64_t *b_dev, int invert_a,
                      uint32_t *total_host, void *stream);
 int ugk_bitmap_emit(const uint64_t *a_dev, const uint64_t *b_dev, int invert_a, uint64_t nbits, const void *ws_dev,
                     uint32_t *out_dev, uint64_t max_out, void *stream);
+/* the same, and |S| to *total_host (pinned, may be NULL): for callers that do not wait between the two, whose count then
+ * needs no launch of its own for the total (ugk_bitmap_count with total_host NULL) */
+int ugk_bitmap_emit_counted(const uint64_t *a_dev, const uint64_t *b_dev, int invert_a, uint64_t nbits, const void *ws_dev,
+                            uint32_t *out_dev, uint64_t max_out, uint32_t *total_host, void *stream);
 /* ugk_bitmap_count(a, b, 0, ..., ws_ab) and ugk_bitmap_count(b, a, 0, ..., ws_ba) in one pass over the two bitmaps:
  * totals_host (two pinned words, may be NULL) receives [0] |a & ~b| and [1] |b & ~a| */
 int ugk_bitmap_count_diff(const uint64_t *a_dev, const uint64_t *b_dev, uint64_t nbits, void *ws_ab_dev,

@@ -850,6 +850,13 @@ int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, 
   *ticket_host = value;
   return 0;
 }
+int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned, void *stream) {
+  REQUIRE(ticket_host && *ticket_host == value, "ugk_ticket_wait: nobody has written the ticket");
+  std::lock_guard<std::mutex> g(g_rt_mu);
+  if (as_stream(stream)->capture) violation("the host waited for a ticket on a stream that records into a graph");
+  note_stream_idle(as_stream(stream));
+  return 0;
+}
 int ugk_leave_done_words(ugk_done_t *done) {
   if (done) {
     REQUIRE(done->words_host && done->counters_dev && done->tag > 0 && done->tag <= UGK_DONE_MAX_TAG,
@@ -1418,6 +1425,16 @@ int ugk_rank_place_observed(uint32_t *counts, uint64_t num_rows, uint64_t k, voi
   *static_cast<uint64_t *>(ws) = 0xffffffffull - last_row;
   return 0;
 }
+int ugk_rank_place_observed_ticket(uint32_t *counts, uint64_t num_rows, uint64_t k, void *ws, uint64_t *in_new,
+                                   uint64_t *observed, int reset_counts, const uint64_t *cached, void *evict_ws,
+                                   void *insert_ws, uint32_t *totals_host, uint32_t *status, uint32_t ticket, void *stream) {
+  REQUIRE(ticket == 0 || cached, "ugk_rank_place_observed: a ticket comes with the counts of what changes");
+  if (int rc = ugk_rank_place_observed(counts, num_rows, k, ws, in_new, observed, reset_counts, cached, evict_ws, insert_ws,
+                                       totals_host, status, stream))
+    return rc;
+  if (ticket) totals_host[3] = ticket;
+  return 0;
+}
 int ugk_rank_threshold(const void *ws, uint64_t *threshold_host, void *) {
   *threshold_host = *static_cast<const uint64_t *>(ws);
   return 0;
@@ -1446,6 +1463,11 @@ int ugk_bitmap_emit(const uint64_t *a, const uint64_t *b, int invert_a, uint64_t
     }
   }
   return 0;
+}
+int ugk_bitmap_emit_counted(const uint64_t *a, const uint64_t *b, int invert_a, uint64_t nbits, const void *ws, uint32_t *out,
+                            uint64_t max_out, uint32_t *total_host, void *stream) {
+  if (total_host) *total_host = *static_cast<const uint32_t *>(ws);
+  return ugk_bitmap_emit(a, b, invert_a, nbits, ws, out, max_out, stream);
 }
 int ugk_bitmap_count_diff(const uint64_t *a, const uint64_t *b, uint64_t nbits, void *ws_ab, void *ws_ba,
                           uint32_t *totals_host, void *stream) {

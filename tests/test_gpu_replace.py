@@ -4,6 +4,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from gpu_util import PinnedArray, dev_bytes, dev_zeros_u32, ptr, status_value, sync, to_dev, to_np
 from ugache_amd import hip
@@ -403,6 +404,86 @@ def test_bitmap_emit_diff_writes_both_lists_as_two_emits_would(nbits, shape):
     finally:
         sync()
         total.free()
+
+
+# chunks of one block, of two and (beyond 2^26 bits) of more; the pass that adds the chunk counts up itself and the one
+# behind a scan
+@pytest.mark.parametrize("nbits", [1, 4096, 8192, (1 << 25) - 1, 1 << 25, (1 << 25) + 1, 1 << 26, (1 << 26) + 1])
+@pytest.mark.parametrize("scanned", [False, True])
+def test_bitmap_lists_at_the_edges_of_the_emit_passes(nbits, scanned):
+    gen = torch.Generator(device="cuda").manual_seed(nbits)
+    words = (nbits + 63) // 64
+    a = torch.randint(-(1 << 62), 1 << 62, (words,), dtype=torch.int64, device="cuda", generator=gen)
+    for _ in range(4):  # a bit in 64 or so
+        a &= torch.randint(-(1 << 62), 1 << 62, (words,), dtype=torch.int64, device="cuda", generator=gen)
+    a[words // 2 : words // 2 + 200] = -1  # and a run of them
+    bits = ((a.unsqueeze(1) >> torch.arange(64, device="cuda")) & 1).view(-1)[:nbits]
+    want = torch.nonzero(bits).view(-1).to(torch.int32)
+    del bits
+    ws, total = dev_bytes(hip.lib().ugk_bitmap_workspace_bytes(), fill=0xA5), PinnedArray((4,), np.uint32)
+    sync()
+    try:
+        total.array[...] = 0xFFFFFFFF
+        hip.call("ugk_bitmap_count", ptr(a), None, 0, nbits, ptr(ws), total.ptr if scanned else None, None)
+        for max_out in sorted({0, 1, len(want) // 2, len(want)}):
+            out = torch.full((len(want) + 8,), -1, dtype=torch.int32, device="cuda")
+            hip.call("ugk_bitmap_emit_counted", ptr(a), None, 0, nbits, ptr(ws), ptr(out), max_out, total.ptr + 4, None)
+            sync()
+            assert total.array[1] == len(want) and total.array[0] == (len(want) if scanned else 0xFFFFFFFF)
+            assert torch.equal(out[:max_out], want[:max_out]) and (out[max_out:] == -1).all()
+            total.array[1] = 0xFFFFFFFF
+    finally:
+        sync()
+        total.free()
+
+
+@pytest.mark.parametrize("n", [1000, 2_000_001, 40_000_000, (1 << 26) + 77])
+def test_placement_polled_for_by_its_ticket(n):
+    """once the ticket is there the sums are, and launches on another stream, which nothing orders behind the placement on
+    the device, list what leaves and comes in as they do behind a wait"""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    words, k = (n + 63) // 64, n // 3
+    obs = torch.zeros(words * 64, dtype=torch.bool, device="cuda")
+    obs[torch.randint(0, n, (n // 50 + 1,), device="cuda", generator=gen)] = True
+    cached = torch.zeros(words * 64, dtype=torch.bool, device="cuda")
+    cached[n // 5 : n // 5 + k - 1] = True
+    fill = torch.cumsum(~obs[:n], 0, dtype=torch.int32) <= k - int(obs.sum())
+    new = obs[:n] | fill
+    leaving = torch.nonzero(cached[:n] & ~new).view(-1).to(torch.int32)
+    coming = torch.nonzero(new & ~cached[:n]).view(-1).to(torch.int32)
+    shift = torch.arange(64, device="cuda")
+    pack = lambda b: torch.cat([(c.view(-1, 64).long() << shift).sum(1) for c in b.split(64 << 16)])  # noqa: E731
+    d_obs, d_cached, d_new = pack(obs), pack(cached), torch.empty(words, dtype=torch.int64, device="cuda")
+    del obs, cached, fill, new
+    ws, st = dev_bytes(hip.lib().ugk_rank_workspace_bytes()), dev_zeros_u32(1)
+    ws_out, ws_in = (dev_bytes(hip.lib().ugk_bitmap_workspace_bytes()) for _ in range(2))
+    one, other = torch.cuda.Stream(), torch.cuda.Stream()
+    totals = PinnedArray((4,), np.uint32)
+    totals.array[...] = 0
+    sync()
+    try:
+        for ticket in (5, 6, 7):
+            hip.call("ugk_rank_place_observed_ticket", None, n, k, ptr(ws), ptr(d_new), ptr(d_obs), 0, ptr(d_cached),
+                     ptr(ws_out), ptr(ws_in), totals.ptr, ptr(st), ticket, one.cuda_stream)
+            hip.call("ugk_ticket_wait", totals.ptr + 12, ticket, 1_000_000, one.cuda_stream)
+            assert totals.array.tolist()[:2] == [len(leaving), len(coming)] and totals.array[3] == ticket
+            out_l, in_l = torch.empty_like(leaving), torch.empty_like(coming)
+            hip.call("ugk_bitmap_emit_diff", ptr(d_cached), ptr(d_new), n, ptr(ws_out), ptr(ws_in), ptr(out_l), len(leaving),
+                     ptr(in_l), len(coming), other.cuda_stream)
+            sync()
+            assert torch.equal(out_l, leaving) and torch.equal(in_l, coming)
+            d_new.fill_(-1)
+            sync()
+        assert status_value(st) == 0
+        # a promise that does not hold: told at once, with nothing placed
+        hip.call("ugk_rank_place_observed_ticket", None, n, 1, ptr(ws), ptr(d_new), ptr(d_obs), 0, ptr(d_cached),
+                 ptr(ws_out), ptr(ws_in), totals.ptr, ptr(st), 8, one.cuda_stream)
+        hip.call("ugk_ticket_wait", totals.ptr + 12, 8, 1_000_000, one.cuda_stream)
+        assert totals.array.tolist()[:2] == [0, 0] and status_value(st) == hip.ST_PLACE_PROMISE
+        assert (d_new == -1).all()
+    finally:
+        sync()
+        totals.free()
 
 
 def test_bitmap_compaction_of_an_empty_and_a_full_set():

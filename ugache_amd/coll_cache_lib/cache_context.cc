@@ -583,9 +583,10 @@ bool ExtractSession::PlaceOnDevice(size_t num_cached, uint64_t *in_new_bits, uin
   const bool few_observed = diff != nullptr && keep_bits == nullptr && !replays_count && ObservedBits() != nullptr &&
                             num_cached > 0 && num_cached < rows && bound < num_cached;
   if (few_observed) {
-    UGK_CALL(ugk_rank_place_observed(_hot_counts->ptr<uint32_t>(), rows, num_cached, rank_ws, in_new_bits,
-                                     ObservedBits(), reset_counts ? 1 : 0, diff->cached_bits, diff->evict_ws,
-                                     diff->insert_ws, diff->totals_host, diff->status_dev, _record_stream));
+    UGK_CALL(ugk_rank_place_observed_ticket(_hot_counts->ptr<uint32_t>(), rows, num_cached, rank_ws, in_new_bits,
+                                            ObservedBits(), reset_counts ? 1 : 0, diff->cached_bits, diff->evict_ws,
+                                            diff->insert_ws, diff->totals_host, diff->status_dev, diff->ticket,
+                                            _record_stream));
   } else {
     UGK_CALL(ugk_rank_place_keep(_hot_counts->ptr<uint32_t>(), rows, num_cached, rank_ws, in_new_bits, scratch_bits,
                                  ObservedBits(), keep_bits, reset_counts ? 1 : 0, _record_stream));
@@ -596,6 +597,7 @@ bool ExtractSession::PlaceOnDevice(size_t num_cached, uint64_t *in_new_bits, uin
   }
   _observed_word = diff && ObservedBits() ? diff->totals_host + 2 : nullptr;
   _placement_reset = reset_counts;
+  if (few_observed && diff->ticket) return true;
   UGK_CALL(ugk_event_record(_ev_placed, _record_stream));
   UGK_CALL(ugk_stream_wait_event(stream, _ev_placed));
   return few_observed;
@@ -1684,13 +1686,19 @@ void RefreshSession::refresh_on_device(ExtractSession *session, size_t num_cache
   // sets are counted before the one wait that tells the host their sizes.
   // COLL_GPU_REFRESH_STABLE: rows that tie at the last count that gets in stay where they are (cached or not)
   // (a placement that knows that fewer rows were observed than the cache holds counts both sets on its way)
+  // (and leaves a ticket behind the counts: the host, which needs them next, polls for it, and the refresh's stream, which
+  // gets its next launch after that, does not wait for the stream of the placement on the device)
   const ExtractSession::DiffCount diff = {table->InCacheBits(), table->_dev_bm_ws->ptr(), table->_dev_bm_ws2->ptr(),
-                                          table->DevWords() + 8, _status_handle->ptr<uint32_t>()};
+                                          table->DevWords() + 8, _status_handle->ptr<uint32_t>(), table->NextTicket()};
   const bool counted = session->PlaceOnDevice(
       num_cached, table->InNewBits(), table->_dev_scratch_bits->ptr<uint64_t>(),
       RunConfig::gpu_refresh_stable ? table->InCacheBits() : nullptr, table->_dev_rank_ws->ptr(),
       !RunConfig::gpu_refresh_keep, &diff, stream);
   if (!counted) table->CountDiff(table->InCacheBits(), table->InNewBits(), num_rows, stream);  // the same pinned words
+  if (counted && diff.ticket)
+    UGK_CALL(ugk_ticket_wait(diff.totals_host + 3, diff.ticket, RunConfig::spin_wait_us, session->RecordStream()));
+  else
+    table->WaitByTicket(stream);
   ApplyPlacedBits(session, num_cached, foreground, stage, true,
                   counted ? "placement (from the observed rows alone)" : "placement", sync_s, t_phase);
 }
@@ -1742,11 +1750,12 @@ void RefreshSession::refresh_from_ranked_rows(ExtractSession *session, TensorPtr
   } else {
     table->CountDiff(table->InCacheBits(), table->InNewBits(), num_rows, stream);
   }
+  table->WaitByTicket(stream);
   ApplyPlacedBits(session, num_cached, foreground, stage, false, "placement ranked on the host", sync_s, t_phase);
 }
 
 // The second half of a refresh whose new placement stands in the table's bitmap of rows cached after it, with the two
-// counts (rows that leave, rows that come in) on their way into the pinned words 8 and 9: waits for the counts, lists
+// counts (rows that leave, rows that come in) in the pinned words 8 and 9 (the caller has waited for them): lists
 // evict = cached & ~new and insert = new & ~cached, then steps 4 - 6 of refresh_after_solve_new on device lists.
 void RefreshSession::ApplyPlacedBits(ExtractSession *session, size_t num_cached, bool foreground,
                                      const ugk_stage_t *stage, bool placed_from_counters, const char *how,
@@ -1757,7 +1766,6 @@ void RefreshSession::ApplyPlacedBits(ExtractSession *session, size_t num_cached,
   const auto &alloc = ctx->_eager_gpu_mem_allocator;
   const size_t num_rows = ctx->_num_total_nodes, capacity = ctx->_cache_space_capacity;
   volatile uint32_t *n_evict_word = table->DevWords() + 8, *n_insert_word = table->DevWords() + 9;
-  table->WaitByTicket(stream);
   if (placed_from_counters) session->PlacementWaitedFor();
   const size_t num_evicted = *n_evict_word, num_insert = *n_insert_word;
   TensorPtr evict_rows, insert_rows;  // both lists in one pass over the two bitmaps
@@ -1798,9 +1806,7 @@ void RefreshSession::ApplyPlacedBits(ExtractSession *session, size_t num_cached,
     CHECK_LE(num_insert, num_free_expected) << "free cache slots exhausted";
     // how many slots are free is known without looking (what was free plus what was evicted); the count the compaction
     // makes on its way is compared with that once the refresh has been waited for
-    n_free_word = table->CountBits(table->SlotUsedBits(), nullptr, true, capacity, 0, stream);
-    TensorPtr slots =
-        table->EmitBits(table->SlotUsedBits(), nullptr, true, capacity, 0, num_insert, __free_slots, alloc, gpu_ctx, stream);
+    TensorPtr slots = table->FreeSlots(num_insert, &n_free_word, __free_slots, alloc, gpu_ctx, stream);
     if (foreground) {
       // nothing runs beside a foreground refresh: the copy goes on the refresh's own stream, behind the lists it reads
       CopyRowsIntoSlots(insert_rows->CPtr<uint32_t>(), slots->CPtr<uint32_t>(), num_insert, true, stream, stage);

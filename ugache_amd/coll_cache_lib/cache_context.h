@@ -344,9 +344,11 @@ class ExtractSession {
   struct DiffCount {
     const uint64_t *cached_bits;
     void *evict_ws, *insert_ws;
-    uint32_t *totals_host;  // three pinned words; [2] receives the rows observed
+    uint32_t *totals_host;  // four pinned words; [2] receives the rows observed
     uint32_t *status_dev;
+    uint32_t ticket;        // non-zero: a placement that counts leaves it in totals_host[3], `stream` does not wait for it
   };
+  StreamHandle RecordStream() const { return _record_stream; }
   bool PlaceOnDevice(size_t num_cached, uint64_t *in_new_bits, uint64_t *scratch_bits, const uint64_t *keep_bits,
                      void *rank_ws, bool reset_counts, const DiffCount *diff, StreamHandle stream);
   // after `stream` has been waited for: the host learns how many rows the placement saw observed

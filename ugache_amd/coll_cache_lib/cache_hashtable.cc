@@ -240,22 +240,22 @@ TensorPtr CacheEntryManager::CompactBits(const uint64_t *a, const uint64_t *b, b
   return list;
 }
 
-volatile uint32_t *CacheEntryManager::CountBits(const uint64_t *a, const uint64_t *b, bool invert_a, uint64_t nbits,
-                                                int which, StreamHandle stream) {
-  CHECK(which == 0 || which == 1);
-  uint32_t *total = DevWords() + 8 + which;
-  void *ws = which == 0 ? _dev_bm_ws->ptr() : _dev_bm_ws2->ptr();
-  UGK_CALL(ugk_bitmap_count(a, b, invert_a ? 1 : 0, nbits, ws, total, stream));
-  return total;
+TensorPtr CacheEntryManager::FreeSlots(size_t n, volatile uint32_t **num_free, TensorPtr &buffer,
+                                       const std::function<MemHandle(size_t)> &allocator, Context ctx,
+                                       StreamHandle stream) {
+  TensorPtr list = ReuseList(buffer, kI32, n, allocator, ctx);
+  uint32_t *total = DevWords() + 8;
+  UGK_CALL(ugk_bitmap_count(SlotUsedBits(), nullptr, 1, _cache_space_capacity, _dev_bm_ws->ptr(), nullptr, stream));
+  UGK_CALL(ugk_bitmap_emit_counted(SlotUsedBits(), nullptr, 1, _cache_space_capacity, _dev_bm_ws->ptr(),
+                                   list->Ptr<uint32_t>(), n, total, stream));
+  *num_free = total;
+  return list;
 }
 
-TensorPtr CacheEntryManager::EmitBits(const uint64_t *a, const uint64_t *b, bool invert_a, uint64_t nbits, int which,
-                                      size_t n, TensorPtr &buffer, const std::function<MemHandle(size_t)> &allocator,
-                                      Context ctx, StreamHandle stream) {
-  TensorPtr list = ReuseList(buffer, kI32, n, allocator, ctx);
-  const void *ws = which == 0 ? _dev_bm_ws->ptr() : _dev_bm_ws2->ptr();
-  if (n) UGK_CALL(ugk_bitmap_emit(a, b, invert_a ? 1 : 0, nbits, ws, list->Ptr<uint32_t>(), n, stream));
-  return list;
+uint32_t CacheEntryManager::NextTicket() {
+  if (RunConfig::spin_wait_us == 0) return 0;
+  if (++_ticket == 0) _ticket = 1;
+  return _ticket;
 }
 
 void CacheEntryManager::CountDiff(const uint64_t *a, const uint64_t *b, uint64_t nbits, StreamHandle stream) {
@@ -272,7 +272,7 @@ void CacheEntryManager::EmitDiff(const uint64_t *a, const uint64_t *b, uint64_t 
                                 n_ba ? (*list_ba)->Ptr<uint32_t>() : nullptr, n_ba, stream));
 }
 
-// pinned words of the table (64): [0] CompactBits' total, [8..10] the counts of a refresh, [16] the ticket of
+// pinned words of the table (64): [0] CompactBits' total, [8..10] the counts of a refresh and [11] their ticket, [16] the ticket of
 // WaitByTicket, [32] the ticket of StatusAndWords and [33 ...] its words
 void CacheEntryManager::WaitByTicket(StreamHandle stream) {
   CHECK(_dev_words) << "the table's pinned words come with its device lists";

@@ -143,15 +143,10 @@ class CacheEntryManager {
   TensorPtr CompactBits(const uint64_t *a, const uint64_t *b, bool invert_a, uint64_t nbits, size_t limit,
                         TensorPtr &buffer, const std::function<MemHandle(size_t)> &allocator, Context ctx,
                         StreamHandle stream, size_t *total_out);
-  // The two halves of CompactBits for callers that count several sets before they wait once: CountBits enqueues the
-  // count of set `which` (0 or 1, each with a workspace of its own) and returns the pinned word it will land in;
-  // EmitBits, after the bitmaps' count is known (waited for, or known by other means), enqueues the list of the first n
-  // elements.
-  volatile uint32_t *CountBits(const uint64_t *a, const uint64_t *b, bool invert_a, uint64_t nbits, int which,
-                               StreamHandle stream);
-  TensorPtr EmitBits(const uint64_t *a, const uint64_t *b, bool invert_a, uint64_t nbits, int which, size_t n,
-                     TensorPtr &buffer, const std::function<MemHandle(size_t)> &allocator, Context ctx,
-                     StreamHandle stream);
+  // Enqueues the list of the first n free cache slots, ascending; how many are free is in the pinned word *num_free once the
+  // stream has been waited for.
+  TensorPtr FreeSlots(size_t n, volatile uint32_t **num_free, TensorPtr &buffer,
+                      const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream);
   // A build that made its key list from a bitmap on the device hands the bitmap over: until a refresh changes the
   // cache it is the bitmap of cached rows, and the slots taken are 0 .. cached - 1 (the build fills them in list
   // order), so the first refresh finds both bitmaps without a pass over the key list and a lookup of every key.
@@ -163,7 +158,7 @@ class CacheEntryManager {
   }
   void DropBuildBits() { _build_bits_fresh = false; }
   // the counts of both differences of two bitmaps (sets 0 = a & ~b and 1 = b & ~a) from one pass, into the pinned
-  // words CountBits would write
+  // words 8 and 9
   void CountDiff(const uint64_t *a, const uint64_t *b, uint64_t nbits, StreamHandle stream);
   // both differences of two bitmaps in one launch, counted as sets 0 (a & ~b) and 1 (b & ~a): the first n_ab and n_ba
   // elements into lists taken from the two buffers
@@ -172,6 +167,8 @@ class CacheEntryManager {
                 const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream);
   // waits for `stream` by a ticket in the table's pinned words (spin_us == 0: by the runtime)
   void WaitByTicket(StreamHandle stream);
+  // a value for a ticket that a launch leaves itself; 0 where waits go through the runtime
+  uint32_t NextTicket();
   // status words of the table's kernels and n_extra more device words (<= 9), brought to the host by one launch and
   // one wait by ticket, with a census of the table where one is due; returns the table's status word, the extra words land
   // in extra_out

@@ -20,9 +20,26 @@
 //          setting / clearing listed bits.  Membership of the cache and occupancy of its slots live in such bitmaps,
 //          so evict = cached & ~new, insert = new & ~cached, free slots = ~used are all the same three launches.
 #include "ugk_internal.h"
+#include "ugk_mix.cuh"
 
 namespace ugk {
 namespace {
+
+// sums over the wavefront by DPP (adds within rows of 16 lanes, then across them): no trip through LDS, where the six dependent
+// permutes of a shuffled scan wait for each other and for those of the CU's other wavefronts
+__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t x) {  // of lanes 0 .. mine
+  constexpr int kRowShr = 0x110, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kRowShr + 1, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kRowShr + 2, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kRowShr + 4, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kRowShr + 8, 0xf, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kRowBcast15, 0xa, 0xf, false);
+  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kRowBcast31, 0xc, 0xf, false);
+  return x;
+}
+__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {  // of all lanes, the same in each
+  return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_sum(x), kWave - 1);
+}
 
 constexpr int kHistBins = 2048;        // 11-bit digits at most
 constexpr uint32_t kSatCount = kHistBins - 1;
@@ -38,10 +55,37 @@ constexpr uint64_t kBmMaxBits = 1ull << 32;
 constexpr uint32_t kBmMaxBlocks = (uint32_t)(kBmMaxBits / 64 / kWave);  // 2^20
 struct BmWs {
   uint32_t total;
-  uint32_t pad[3];
+  uint32_t scanned;              // base holds the prefix; 0: still the counts (the emit pass adds them up itself)
+  uint32_t pad[2];
   uint32_t base[kBmChunks];      // per chunk: first the count, after the scan the exclusive prefix
   uint32_t block[kBmMaxBlocks];  // per 64-word block: its count
 };
+
+// The workgroups of a launch that add up two counts: each comes to one of kArriveLines lines, the last of a line to the
+// top one (adds on one word are performed one after the other).  A line's first word counts arrivals above the first
+// count, the second count is complete before its arrival is seen.
+constexpr uint32_t kArriveLines = 32;
+struct Arrivals {
+  unsigned long long line[kArriveLines + 1][16];
+};
+// one thread of the workgroup, all of whose stores have been acknowledged; true for the last workgroup of the launch,
+// which then has both sums
+__device__ __forceinline__ bool arrive(Arrivals *at, uint32_t &a, uint32_t &b) {
+  const uint32_t lines = min(gridDim.x, kArriveLines), mine = blockIdx.x % lines;
+  uint32_t members = gridDim.x / lines + (mine < gridDim.x % lines ? 1u : 0u);
+  for (int level = 0; level < 2; ++level) {
+    unsigned long long *w = at->line[level ? kArriveLines : mine];
+    __hip_atomic_fetch_add(w + 1, (unsigned long long)b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned long long add = (1ull << 32) | a;
+    const unsigned long long sum = __hip_atomic_fetch_add(w, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
+    if ((uint32_t)(sum >> 32) != members) return false;
+    a = (uint32_t)sum;
+    b = (uint32_t)__hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    members = lines;
+  }
+  return true;
+}
 
 // workspace of a placement
 struct RankWs {
@@ -58,6 +102,7 @@ struct RankWs {
   uint32_t split_done;           // the guess was T: gt and eq are written, the second pass is not needed
 
   uint32_t hist[kHistBins];
+  Arrivals arrivals;             // of rank_combine_observed_kernel
   BmWs bm;                       // chunk offsets of `eq`
 };
 
@@ -357,12 +402,7 @@ __global__ __launch_bounds__(kBlock) void rank_locate_kernel(RankWs *ws, const u
     const uint64_t w = w0 + tid;
     unsigned long long m = w < end ? tie_word(ws, eq, keep, w) : 0ull;
     const uint32_t mine = __popcll(m);
-    uint32_t incl = mine;
-#pragma unroll
-    for (int s = 1; s < kWave; s <<= 1) {
-      const uint32_t up = __shfl_up(incl, s);
-      if (tid >= s) incl += up;
-    }
+    const uint32_t incl = wave_incl_sum(mine);
     const uint32_t all = __shfl(incl, kWave - 1);
     if (skip < all) {  // in this group of words; wavefront-uniform
       if (incl - mine <= skip && skip < incl) {
@@ -398,18 +438,46 @@ __global__ __launch_bounds__(kBlock) void rank_combine_kernel(const RankWs *ws, 
   }
 }
 
-__device__ __forceinline__ void scan_chunks(BmWs *ws, uint32_t *total_host);  // with the bitmap kernels below
+// The counts of all chunks scanned by one workgroup of kScanBlock threads, eight neighbouring chunks a thread, in registers:
+// pre[j] = counts in front of chunk 8 * tid + j, total = all of them.  (With 256 threads, a scan in LDS and the counts read
+// from memory twice rank_locate_unobserved_kernel took 13.5 us; 5.7 this way.)
+constexpr int kScanBlock = kBmChunks / 8;
+__device__ __forceinline__ void scan_chunks(const uint32_t *counts, uint32_t (&pre)[8], uint32_t &total) {
+  constexpr int kWaves = kScanBlock / kWave;
+  __shared__ uint32_t wave_sum[kWaves];
+  const int tid = threadIdx.x, lane = tid % kWave;
+  // (a workspace is 8-byte aligned)
+  const u32x4_by4 *c4 = reinterpret_cast<const u32x4_by4 *>(counts) + 2 * tid;
+  const u32x4 lo = c4[0], hi = c4[1];
+  const uint32_t c[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  uint32_t sum = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) pre[j] = sum, sum += c[j];
+  const uint32_t incl = wave_incl_sum(sum);
+  if (lane == kWave - 1) wave_sum[tid / kWave] = incl;
+  __syncthreads();
+  uint32_t before = incl - sum;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < tid / kWave) before += wave_sum[w];
+    total += wave_sum[w];
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) pre[j] += before;
+}
 
 // ---- the placement when the caller knows that fewer rows were observed than are wanted ----------------------------
 // One workgroup, after `observed` was counted into ws->bm: scans the chunk counts, checks the caller's promise and
 // finds the last needed never-observed row, the (want - observed rows - 1)-th clear bit of `observed`, ascending (clear
-// bits in front of chunk c = its first bit number - set bits in front of it).  Three dependent reads after the scan:
-// the chunk offsets, the block counts of the one chunk, the 64 words of the one block.
-__global__ __launch_bounds__(kBlock) void rank_locate_unobserved_kernel(RankWs *ws, const unsigned long long *observed,
-                                                                        uint64_t nbits, uint64_t per_chunk,
-                                                                        unsigned long long want, uint32_t *status,
-                                                                        uint32_t *observed_host) {
+// bits in front of chunk c = its first bit number - set bits in front of it).  Three dependent reads: the chunk counts,
+// the block counts of the one chunk, the 64 words of the one block.
+__global__ __launch_bounds__(kScanBlock) void rank_locate_unobserved_kernel(RankWs *ws, const unsigned long long *observed,
+                                                                            uint64_t nbits, uint64_t per_chunk,
+                                                                            unsigned long long want, uint32_t *status,
+                                                                            uint32_t *observed_host) {
   __shared__ uint32_t chunk_of;
+  __shared__ uint64_t skip_of;
   const int tid = threadIdx.x;
   if (tid == 0) {  // what rank_init_kernel sets, for the readers of a placement (the histogram is not used here)
     ws->threshold = 0;
@@ -420,9 +488,10 @@ __global__ __launch_bounds__(kBlock) void rank_locate_unobserved_kernel(RankWs *
     ws->from_bitmap = 0;
     ws->keep_mode = 0;
   }
-  scan_chunks(&ws->bm, nullptr);
-  __syncthreads();
-  const uint32_t total = ws->bm.total;
+  for (uint32_t i = tid; i < (kArriveLines + 1) * 16; i += kScanBlock) (&ws->arrivals.line[0][0])[i] = 0ull;
+  uint32_t pre[8], total;
+  scan_chunks(ws->bm.base, pre, total);
+  if (tid == 0) ws->bm.total = total;
   if (tid == 0 && observed_host) *observed_host = total;
   if (total >= want) {  // uniform: the promise does not hold, nothing is placed
     if (tid == 0) atomicOr(status, UGK_ST_PLACE_PROMISE);
@@ -430,18 +499,16 @@ __global__ __launch_bounds__(kBlock) void rank_locate_unobserved_kernel(RankWs *
   }
   const uint64_t index = want - total - 1;  // among the clear bits, from 0
   const uint64_t chunk_bits = per_chunk * 64;
-  auto clear_before = [&](int c) -> uint64_t {  // c in [0, kBmChunks]
-    if (c >= kBmChunks) return nbits - total;
-    const uint64_t first = (uint64_t)c * chunk_bits;
-    return (first < nbits ? first : nbits) - ws->bm.base[c];
-  };
-  constexpr int kPer = kBmChunks / kBlock;
-  uint64_t lo = clear_before(tid * kPer);
-  for (int j = 0; j < kPer; ++j) {
-    const int c = tid * kPer + j;
-    const uint64_t hi = clear_before(c + 1);
-    if (lo <= index && index < hi) chunk_of = (uint32_t)c;  // exactly one chunk holds it
-    lo = hi;
+  // the last chunk with no more than `index` clear bits in front of it holds the bit, and it is the one whose clear bits
+  // reach beyond: exactly one chunk
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint64_t c = (uint64_t)tid * 8 + j;
+    const uint64_t first = min(c * chunk_bits, nbits), behind = min((c + 1) * chunk_bits, nbits);
+    const uint64_t lo = first - pre[j];
+    // set bits up to the chunk's end: the next one's prefix, which the last of a thread's eight finds from its count
+    const uint32_t upto = j < 7 ? pre[j < 7 ? j + 1 : 7] : pre[7] + ws->bm.base[c];
+    if (lo <= index && index < behind - upto) chunk_of = (uint32_t)c, skip_of = index - lo;
   }
   __syncthreads();
   if (tid >= kWave) return;
@@ -450,7 +517,7 @@ __global__ __launch_bounds__(kBlock) void rank_locate_unobserved_kernel(RankWs *
   const uint64_t n_blocks = (n_words + kWave - 1) / kWave;
   const uint64_t blocks_per_chunk = per_chunk / kWave, first_blk = (uint64_t)c * blocks_per_chunk;
   constexpr uint64_t kBlockBits = (uint64_t)kWave * 64;
-  uint64_t skip = index - clear_before((int)c);  // clear bits of the chunk below the wanted one
+  uint64_t skip = skip_of;  // clear bits of the chunk below the wanted one
   // the block: a lane per block of the chunk
   uint64_t blk = 0;
   bool found = false;
@@ -461,12 +528,7 @@ __global__ __launch_bounds__(kBlock) void rank_locate_unobserved_kernel(RankWs *
       const uint64_t bits = min(nbits - b * kBlockBits, kBlockBits);
       mine = (uint32_t)bits - ws->bm.block[b];
     }
-    uint32_t incl = mine;
-#pragma unroll
-    for (int s = 1; s < kWave; s <<= 1) {
-      const uint32_t up = __shfl_up(incl, s);
-      if (tid >= s) incl += up;
-    }
+    const uint32_t incl = wave_incl_sum(mine);
     const uint32_t all = __shfl(incl, kWave - 1);
     if (skip < all) {  // wavefront-uniform
       const unsigned long long holds = __ballot(incl - mine <= skip && skip < incl);
@@ -487,12 +549,7 @@ __global__ __launch_bounds__(kBlock) void rank_locate_unobserved_kernel(RankWs *
     if (nbits - w * 64 < 64) m &= (1ull << (nbits - w * 64)) - 1ull;
   }
   const uint32_t mine = __popcll(m);
-  uint32_t incl = mine;
-#pragma unroll
-  for (int s = 1; s < kWave; s <<= 1) {
-    const uint32_t up = __shfl_up(incl, s);
-    if (tid >= s) incl += up;
-  }
+  const uint32_t incl = wave_incl_sum(mine);
   if (incl - mine <= skip && skip < incl) {
     uint32_t drop = (uint32_t)skip - (incl - mine);
     while (drop--) m &= m - 1;
@@ -506,22 +563,39 @@ __global__ __launch_bounds__(kBlock) void rank_locate_unobserved_kernel(RankWs *
 }
 
 // in_new = observed | (never observed, up to last_row); with `cached`, the rows that leave (cached & ~in_new) and come
-// in (in_new & ~cached) are counted per 64-word block and per chunk on the way, as bitmap_count_kernel would.  One
-// wavefront per chunk.
+// in (in_new & ~cached) are counted per 64-word block and per chunk on the way, as bitmap_count_kernel would, and all in
+// all: the last workgroup to end writes both sums to totals_host.  One wavefront per chunk.  With a ticket, which that
+// workgroup writes behind the sums, a host that polls for it may go on at once, on any stream: what the refresh reads next is
+// written through to memory then (leave_done has the why).
 __global__ __launch_bounds__(kBlock) void rank_combine_observed_kernel(uint32_t *counts, uint64_t nbits,
-                                                                       uint64_t per_chunk, const RankWs *ws,
+                                                                       uint64_t per_chunk, RankWs *ws,
                                                                        unsigned long long *observed,
                                                                        unsigned long long *in_new,
                                                                        const unsigned long long *cached,
                                                                        BmWs *evict_ws, BmWs *insert_ws,
-                                                                       int reset_counts) {
-  if (!ws->from_bitmap) return;
+                                                                       int reset_counts, uint32_t *totals_host,
+                                                                       uint32_t ticket) {
+  __shared__ uint32_t leaving_of[kBlock / kWave], coming_of[kBlock / kWave];
+  if (!ws->from_bitmap) {  // nothing was placed
+    if (cached && blockIdx.x == 0 && threadIdx.x == 0) {
+      totals_host[0] = totals_host[1] = 0;
+      __threadfence_system();
+      if (ticket) *(volatile uint32_t *)(totals_host + 3) = ticket;
+    }
+    return;
+  }
   const uint64_t wl = ws->last_row >> 6;
   const unsigned bl = ws->last_row & 63u;
   const int lane = (int)lane_id();
   const uint64_t n_words = (nbits + 63) / 64;
   const uint64_t wave = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
   const uint64_t n_waves = (uint64_t)gridDim.x * (kBlock / kWave);
+  auto put = [ticket](auto *to, auto v) {
+    if (ticket) store_through(reinterpret_cast<uint64_t>(to), v);
+    else *to = v;
+  };
+  if (cached && blockIdx.x == 0 && threadIdx.x == 0) put(&evict_ws->scanned, 0u), put(&insert_ws->scanned, 0u);
+  uint32_t out_all = 0, in_all = 0;
   for (uint64_t chunk = wave; chunk < (uint64_t)kBmChunks; chunk += n_waves) {
     const uint64_t begin = chunk * per_chunk, end = min(n_words, begin + per_chunk);
     uint32_t out_sum = 0, in_sum = 0;
@@ -533,7 +607,7 @@ __global__ __launch_bounds__(kBlock) void rank_combine_observed_kernel(uint32_t 
         unsigned long long upto = w < wl ? ~0ull : (w == wl ? (bl == 63 ? ~0ull : (1ull << (bl + 1)) - 1ull) : 0ull);
         if (nbits - w * 64 < 64) upto &= (1ull << (nbits - w * 64)) - 1ull;
         const unsigned long long nw = obs | (~obs & upto);
-        in_new[w] = nw;
+        put(in_new + w, nw);
         if (cached) {
           const unsigned long long c = cached[w];
           leaving = __popcll(c & ~nw);
@@ -548,23 +622,37 @@ __global__ __launch_bounds__(kBlock) void rank_combine_observed_kernel(uint32_t 
         }
       }
       if (cached) {  // uniform
-#pragma unroll
-        for (int d = kWave / 2; d > 0; d >>= 1) {
-          leaving += __shfl_xor(leaving, d);
-          coming += __shfl_xor(coming, d);
-        }
+        leaving = wave_sum(leaving);
+        coming = wave_sum(coming);
         if (lane == 0) {
-          evict_ws->block[w0 / kWave] = leaving;  // chunks begin on block boundaries
-          insert_ws->block[w0 / kWave] = coming;
+          put(&evict_ws->block[w0 / kWave], leaving);  // chunks begin on block boundaries
+          put(&insert_ws->block[w0 / kWave], coming);
         }
         out_sum += leaving;
         in_sum += coming;
       }
     }
     if (cached && lane == 0) {
-      evict_ws->base[chunk] = out_sum;
-      insert_ws->base[chunk] = in_sum;
+      put(&evict_ws->base[chunk], out_sum);
+      put(&insert_ws->base[chunk], in_sum);
     }
+    out_all += out_sum;
+    in_all += in_sum;
+  }
+  if (!cached) return;  // uniform
+  if (ticket) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have been acknowledged
+  if (lane == 0) leaving_of[threadIdx.x / kWave] = out_all, coming_of[threadIdx.x / kWave] = in_all;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  uint32_t out_wg = 0, in_wg = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / kWave; ++w) out_wg += leaving_of[w], in_wg += coming_of[w];
+  if (!arrive(&ws->arrivals, out_wg, in_wg)) return;
+  totals_host[0] = out_wg;
+  totals_host[1] = in_wg;
+  if (ticket) {
+    __threadfence_system();
+    *(volatile uint32_t *)(totals_host + 3) = ticket;
   }
 }
 
@@ -606,6 +694,7 @@ __global__ __launch_bounds__(kBlock) void bitmap_count_kernel(const unsigned lon
                                                               int flags, uint64_t nbits, uint64_t per_chunk,
                                                               BmWs *ws, const RankWs *gate) {
   if (gate && gate->keep_mode != 2) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) ws->scanned = 0;
   const int lane = (int)lane_id();
   const uint64_t n_words = (nbits + 63) / 64;
   const uint64_t wave = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
@@ -616,8 +705,7 @@ __global__ __launch_bounds__(kBlock) void bitmap_count_kernel(const unsigned lon
     for (uint64_t w0 = begin; w0 < end; w0 += kWave) {
       const uint64_t w = w0 + lane;
       uint32_t mine = w < end ? __popcll(bm_word(a, b, flags, nbits, w)) : 0u;
-#pragma unroll
-      for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_xor(mine, d);
+      mine = wave_sum(mine);
       if (lane == 0) ws->block[w0 / kWave] = mine;  // chunks begin on block boundaries
       found += mine;
     }
@@ -650,11 +738,8 @@ __global__ __launch_bounds__(kBlock) void bitmap_count_diff_kernel(const unsigne
         n_ab = __popcll(wa & ~wb);
         n_ba = __popcll(wb & ~wa);
       }
-#pragma unroll
-      for (int d = kWave / 2; d > 0; d >>= 1) {
-        n_ab += __shfl_xor(n_ab, d);
-        n_ba += __shfl_xor(n_ba, d);
-      }
+      n_ab = wave_sum(n_ab);
+      n_ba = wave_sum(n_ba);
       if (lane == 0) {
         ws_ab->block[w0 / kWave] = n_ab;  // chunks begin on block boundaries
         ws_ba->block[w0 / kWave] = n_ba;
@@ -669,46 +754,28 @@ __global__ __launch_bounds__(kBlock) void bitmap_count_diff_kernel(const unsigne
   }
 }
 
-__device__ __forceinline__ void scan_chunks(BmWs *ws, uint32_t *total_host) {
-  constexpr int kPer = kBmChunks / kBlock;  // 32 chunks per thread
-  __shared__ uint32_t part[kBlock];
-  const int tid = threadIdx.x;
-  uint32_t sum = 0;
-  for (int j = 0; j < kPer; ++j) sum += ws->base[tid * kPer + j];
-  part[tid] = sum;
-  __syncthreads();
-  for (int s = 1; s < kBlock; s <<= 1) {  // inclusive prefix sums
-    const uint32_t add = tid >= s ? part[tid - s] : 0;
-    __syncthreads();
-    part[tid] += add;
-    __syncthreads();
-  }
-  uint32_t run = part[tid] - sum;
-  for (int j = 0; j < kPer; ++j) {
-    const uint32_t c = ws->base[tid * kPer + j];
-    ws->base[tid * kPer + j] = run;
-    run += c;
-  }
-  if (tid == kBlock - 1) {
-    ws->total = part[tid];
-    if (total_host) *total_host = part[tid];
+// one workgroup of kScanBlock threads: the counts of the chunks become their prefix
+__device__ __forceinline__ void scan_ws(BmWs *ws, uint32_t *total_host) {
+  uint32_t pre[8], total;
+  scan_chunks(ws->base, pre, total);
+  u32x4_by4 *to = reinterpret_cast<u32x4_by4 *>(ws->base) + 2 * threadIdx.x;
+  to[0] = u32x4{pre[0], pre[1], pre[2], pre[3]};
+  to[1] = u32x4{pre[4], pre[5], pre[6], pre[7]};
+  if (threadIdx.x == 0) {
+    ws->total = total;
+    ws->scanned = 1;
+    if (total_host) *total_host = total;
   }
 }
 
-__global__ __launch_bounds__(kBlock) void bitmap_scan_kernel(BmWs *ws, uint32_t *total_host, const RankWs *gate) {
+__global__ __launch_bounds__(kScanBlock) void bitmap_scan_kernel(BmWs *ws, uint32_t *total_host, const RankWs *gate) {
   if (gate && gate->keep_mode != 2) return;
-  scan_chunks(ws, total_host);
+  scan_ws(ws, total_host);
 }
 
-// two workspaces in one launch (one workgroup each), totals to totals_host[0] and [1]; gate: a placement that must have
-// taken the observed-rows path
-__global__ __launch_bounds__(kBlock) void bitmap_scan2_kernel(BmWs *a, BmWs *b, uint32_t *totals_host,
-                                                              const RankWs *gate) {
-  if (gate && !gate->from_bitmap) {
-    if (threadIdx.x == 0) totals_host[blockIdx.x] = 0;
-    return;
-  }
-  scan_chunks(blockIdx.x == 0 ? a : b, totals_host ? totals_host + blockIdx.x : (uint32_t *)nullptr);
+// two workspaces in one launch (one workgroup each), totals to totals_host[0] and [1]
+__global__ __launch_bounds__(kScanBlock) void bitmap_scan2_kernel(BmWs *a, BmWs *b, uint32_t *totals_host) {
+  scan_ws(blockIdx.x == 0 ? a : b, totals_host ? totals_host + blockIdx.x : (uint32_t *)nullptr);
 }
 
 // The set bits of one 64-word block, a lane per word on entry (m), to out[pos0 ...] in ascending order; n_set: how
@@ -719,16 +786,12 @@ __global__ __launch_bounds__(kBlock) void bitmap_scan2_kernel(BmWs *a, BmWs *b, 
 // long after the rest had finished; for blocks with a few bits the word-at-a-time form is the slower one, 51 against
 // 37 us over 122 k blocks with four bits each).
 constexpr uint32_t kEmitDense = 2 * kWave;
-__device__ __forceinline__ void emit_word(unsigned long long m, uint32_t n_set, uint64_t pos0, uint64_t w, int lane,
-                                          uint32_t *out, uint64_t max_out) {
-  const uint32_t mine = __popcll(m);
-  uint32_t incl = mine;
-#pragma unroll
-  for (int s = 1; s < kWave; s <<= 1) {
-    const uint32_t up = __shfl_up(incl, s);
-    if (lane >= s) incl += up;
-  }
-  const uint32_t excl = incl - mine;
+__device__ __forceinline__ uint32_t set_bits_upto(unsigned long long m) {  // in the words of this lane and the ones below
+  return wave_incl_sum(__popcll(m));
+}
+__device__ __forceinline__ void emit_word(unsigned long long m, uint32_t incl, uint32_t n_set, uint64_t pos0, uint64_t w,
+                                          int lane, uint32_t *out, uint64_t max_out) {
+  const uint32_t excl = incl - __popcll(m);
   if (n_set <= kEmitDense) {
     uint64_t pos = pos0 + excl;
     while (m) {
@@ -755,7 +818,9 @@ __device__ __forceinline__ void emit_word(unsigned long long m, uint32_t n_set, 
 
 __global__ __launch_bounds__(kBlock) void bitmap_emit_kernel(const unsigned long long *a, const unsigned long long *b,
                                                              int flags, uint64_t nbits, uint64_t per_chunk,
-                                                             const BmWs *ws, uint32_t *out, uint64_t max_out) {
+                                                             const BmWs *ws, uint32_t *out, uint64_t max_out,
+                                                             uint32_t *total_host) {
+  if (total_host && blockIdx.x == 0 && threadIdx.x == 0) *total_host = ws->total;
   const int lane = (int)lane_id();
   const uint64_t n_words = (nbits + 63) / 64;
   const uint64_t n_blocks = (n_words + kWave - 1) / kWave;
@@ -769,13 +834,12 @@ __global__ __launch_bounds__(kBlock) void bitmap_emit_kernel(const unsigned long
     const uint64_t chunk = blk / blocks_per_chunk, first = chunk * blocks_per_chunk;
     uint32_t before = 0;
     for (uint64_t q = first + lane; q < blk; q += kWave) before += ws->block[q];
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) before += __shfl_xor(before, d);
+    before = wave_sum(before);
     const uint64_t pos0 = (uint64_t)ws->base[chunk] + before;
     if (pos0 >= max_out) continue;
     const uint64_t w = blk * kWave + lane;
     unsigned long long m = w < n_words ? bm_word(a, b, flags, nbits, w) : 0ull;
-    emit_word(m, n_here, pos0, w, lane, out, max_out);
+    emit_word(m, set_bits_upto(m), n_here, pos0, w, lane, out, max_out);
   }
 }
 
@@ -819,11 +883,8 @@ __global__ __launch_bounds__(kBlock) void bitmap_emit_diff_kernel(const unsigned
 #pragma unroll
     for (int j = 0; j < kDiffBlocks; ++j) any |= n_ab[j] | n_ba[j];
     if (any == 0) continue;  // wavefront-uniform
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) {
-      before_ab += __shfl_xor(before_ab, d);
-      before_ba += __shfl_xor(before_ba, d);
-    }
+    before_ab = wave_sum(before_ab);
+    before_ba = wave_sum(before_ba);
     // where each block's elements go: its chunk's offset plus the counts of the chunk's earlier blocks
     uint64_t pos_ab[kDiffBlocks], pos_ba[kDiffBlocks];
 #pragma unroll
@@ -858,8 +919,93 @@ __global__ __launch_bounds__(kBlock) void bitmap_emit_diff_kernel(const unsigned
 #pragma unroll
     for (int j = 0; j < kDiffBlocks; ++j) {
       const uint64_t w = (blk0 + j) * kWave + lane;
-      if (do_ab[j]) emit_word(wa[j] & ~wb[j], n_ab[j], pos_ab[j], w, lane, out_ab, max_ab);
-      if (do_ba[j]) emit_word(wb[j] & ~wa[j], n_ba[j], pos_ba[j], w, lane, out_ba, max_ba);
+      const unsigned long long ab = wa[j] & ~wb[j], ba = wb[j] & ~wa[j];
+      if (do_ab[j]) emit_word(ab, set_bits_upto(ab), n_ab[j], pos_ab[j], w, lane, out_ab, max_ab);
+      if (do_ba[j]) emit_word(ba, set_bits_upto(ba), n_ba[j], pos_ba[j], w, lane, out_ba, max_ba);
+    }
+  }
+}
+
+// The emit pass over a bitmap of up to kSmallBits bits, whose chunks are at most kSmallBlocks blocks long: a workgroup of a
+// wavefront per chunk.  The words are asked for together with the counts of the chunks in front of the workgroup, which it adds up
+// itself where no scan has run: one round of reads, and no one-workgroup launch between the count and this one (40 M
+// bits, 72,000 rows that leave and as many that come: 7.9 us, against 5.0 for the scan and 8.0; 72,000 free slots among 4 M:
+// 11.3 against 5.7 and 9.0, and a hand-over less).  Longer chunks would make a wavefront of a dense one work long after
+// the others.
+constexpr uint64_t kSmallBlocks = 2, kSmallBits = (uint64_t)kBmChunks * kSmallBlocks * kWave * 64;
+constexpr int kSmallBlock = 1024, kSmallWaves = kSmallBlock / kWave;
+static inline unsigned small_grid(uint64_t nbits, uint64_t per_chunk) {
+  return (unsigned)(((nbits + 63) / 64 + per_chunk * kSmallWaves - 1) / (per_chunk * kSmallWaves));
+}
+struct BmList {
+  const BmWs *ws;
+  uint32_t *out;
+  uint64_t max_out;
+};
+// sets S of one (LISTS == 1: bm_word's of a and b) or two lists (a & ~b, b & ~a); total_host (LISTS == 1): |S|
+template <int LISTS>
+__global__ __launch_bounds__(kSmallBlock) void bitmap_emit_small_kernel(const unsigned long long *a,
+                                                                        const unsigned long long *b, int flags,
+                                                                        uint64_t nbits, uint64_t per_chunk, BmList first,
+                                                                        BmList second, uint32_t *total_host) {
+  __shared__ uint32_t part[LISTS][kSmallWaves];
+  const BmList list[2] = {first, second};
+  const int tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
+  const uint64_t n_words = (nbits + 63) / 64;
+  const uint32_t chunk0 = blockIdx.x * kSmallWaves;
+  const uint64_t w_first = (uint64_t)(chunk0 + wv) * per_chunk + lane;
+  unsigned long long m[LISTS][kSmallBlocks];
+#pragma unroll
+  for (uint64_t j = 0; j < kSmallBlocks; ++j) {
+    const uint64_t w = w_first + j * kWave;
+    const bool in = j * kWave < per_chunk && w < n_words;
+    const uint64_t at = in ? w : 0;  // no branch around the loads
+    if constexpr (LISTS == 1) {
+      m[0][j] = in ? bm_word(a, b, flags, nbits, at) : 0ull;
+    } else {
+      const unsigned long long valid = !in ? 0ull : nbits - at * 64 < 64 ? (1ull << (nbits - at * 64)) - 1ull : ~0ull;
+      const unsigned long long wa = a[at], wb = b[at];
+      m[0][j] = wa & ~wb & valid;
+      m[1][j] = wb & ~wa & valid;
+    }
+  }
+  // the counts in front of the workgroup, and of its own chunks (a chunk behind the last word has a count of zero)
+  uint32_t before[LISTS], own[LISTS], scanned[LISTS];
+#pragma unroll
+  for (int l = 0; l < LISTS; ++l) {
+    const uint32_t *counts = list[l].ws->base;
+    scanned[l] = list[l].ws->scanned;
+    own[l] = counts[chunk0 + lane % kSmallWaves];
+    before[l] = 0;
+#pragma unroll
+    for (int q = 0; q < kBmChunks / kSmallBlock; ++q) {
+      const uint32_t c = q * kSmallBlock + tid;
+      const uint32_t n = counts[c];
+      if (c < chunk0) before[l] += n;
+    }
+  }
+#pragma unroll
+  for (int l = 0; l < LISTS; ++l) {
+    before[l] = wave_sum(before[l]);
+    if (lane == 0) part[l][wv] = before[l];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int l = 0; l < LISTS; ++l) {
+    // (lane q of the first sixteen: what wavefront q added up, and the count of its chunk)
+    const uint32_t front = wave_sum(lane < kSmallWaves ? part[l][lane] : 0u);
+    uint32_t pos = front + wave_sum(lane < wv ? own[l] : 0u);
+    uint32_t all = front + wave_sum(lane < kSmallWaves ? own[l] : 0u);
+    if (scanned[l]) pos = __shfl(own[l], wv), all = list[l].ws->total;
+    if (LISTS == 1 && total_host && blockIdx.x == gridDim.x - 1 && tid == 0) *total_host = all;
+#pragma unroll
+    for (uint64_t j = 0; j < kSmallBlocks; ++j) {
+      if (__ballot(m[l][j] != 0ull) == 0ull) continue;
+      const uint32_t incl = set_bits_upto(m[l][j]);
+      const uint32_t n_set = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+      if (pos < list[l].max_out)
+        emit_word(m[l][j], incl, n_set, pos, w_first + j * kWave, lane, list[l].out, list[l].max_out);
+      pos += n_set;
     }
   }
 }
@@ -953,7 +1099,7 @@ int ugk_rank_place_keep(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, voi
   if (observed) {
     hipLaunchKernelGGL(bitmap_count_kernel, dim3(bm_grid), dim3(kBlock), 0, st, observed, none, 0, num_rows, per_chunk,
                        &ws->bm, no_gate);
-    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kBlock), 0, st, &ws->bm, (uint32_t *)nullptr, no_gate);
+    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, &ws->bm, (uint32_t *)nullptr, no_gate);
     hipLaunchKernelGGL(rank_decide_kernel, dim3(1), dim3(1), 0, st, ws);
     hipLaunchKernelGGL(rank_split_bitmap_kernel, dim3(word_grid), dim3(kBlock), 0, st, counts_dev, num_rows, ws,
                        observed, in_new, eq, reset_counts);
@@ -984,16 +1130,16 @@ int ugk_rank_place_keep(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, voi
     // rows that tie at the K-th count: the kept ones first.  The second count runs only when they do not suffice.
     hipLaunchKernelGGL(bitmap_count_kernel, dim3(bm_grid), dim3(kBlock), 0, st, eq, keep, kBmAndB, num_rows, per_chunk,
                        &ws->bm, no_gate);
-    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kBlock), 0, st, &ws->bm, (uint32_t *)nullptr, no_gate);
+    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, &ws->bm, (uint32_t *)nullptr, no_gate);
     hipLaunchKernelGGL(rank_keep_decide_kernel, dim3(1), dim3(1), 0, st, ws);
     hipLaunchKernelGGL(bitmap_count_kernel, dim3(bm_grid), dim3(kBlock), 0, st, eq, keep, 0, num_rows, per_chunk,
                        &ws->bm, (const RankWs *)ws);
-    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kBlock), 0, st, &ws->bm, (uint32_t *)nullptr,
+    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, &ws->bm, (uint32_t *)nullptr,
                        (const RankWs *)ws);
   } else {
     hipLaunchKernelGGL(bitmap_count_kernel, dim3(bm_grid), dim3(kBlock), 0, st, eq, none, 0, num_rows, per_chunk,
                        &ws->bm, no_gate);
-    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kBlock), 0, st, &ws->bm, (uint32_t *)nullptr, no_gate);
+    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, &ws->bm, (uint32_t *)nullptr, no_gate);
   }
   hipLaunchKernelGGL(rank_locate_kernel, dim3(1), dim3(kBlock), 0, st, ws, eq, keep, num_rows, per_chunk);
   hipLaunchKernelGGL(rank_combine_kernel, dim3(word_grid), dim3(kBlock), 0, st, ws, in_new, eq, keep, n_words,
@@ -1005,6 +1151,15 @@ int ugk_rank_place_keep(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, voi
 int ugk_rank_place_observed(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, void *ws_dev, uint64_t *in_new_dev,
                             uint64_t *observed_dev, int reset_counts, const uint64_t *cached_dev, void *evict_ws_dev,
                             void *insert_ws_dev, uint32_t *totals_host, uint32_t *status_dev, void *stream) {
+  return ugk_rank_place_observed_ticket(counts_dev, num_rows, k, ws_dev, in_new_dev, observed_dev, reset_counts, cached_dev,
+                                        evict_ws_dev, insert_ws_dev, totals_host, status_dev, 0, stream);
+}
+
+int ugk_rank_place_observed_ticket(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, void *ws_dev,
+                                   uint64_t *in_new_dev, uint64_t *observed_dev, int reset_counts,
+                                   const uint64_t *cached_dev, void *evict_ws_dev, void *insert_ws_dev,
+                                   uint32_t *totals_host, uint32_t *status_dev, uint32_t ticket, void *stream) {
+  UGK_REQUIRE(ticket == 0 || cached_dev, "ugk_rank_place_observed: a ticket comes with the counts of what changes");
   UGK_REQUIRE(ws_dev && in_new_dev && observed_dev && status_dev, "ugk_rank_place_observed: null pointer");
   UGK_REQUIRE(counts_dev || !reset_counts, "ugk_rank_place_observed: counters to reset, but no counters");
   UGK_REQUIRE(num_rows > 0 && num_rows < 0xffffffffull, "ugk_rank_place_observed: %llu rows do not fit 32 bits",
@@ -1025,15 +1180,15 @@ int ugk_rank_place_observed(uint32_t *counts_dev, uint64_t num_rows, uint64_t k,
   const unsigned bm_grid = clamp_grid((kBmChunks + (kBlock / kWave) - 1) / (kBlock / kWave), (unsigned)cu_count() * 8u);
   hipLaunchKernelGGL(bitmap_count_kernel, dim3(bm_grid), dim3(kBlock), 0, st, observed, none, 0, num_rows, per_chunk,
                      &ws->bm, no_gate);
-  hipLaunchKernelGGL(rank_locate_unobserved_kernel, dim3(1), dim3(kBlock), 0, st, ws, observed, num_rows, per_chunk,
+  hipLaunchKernelGGL(rank_locate_unobserved_kernel, dim3(1), dim3(kScanBlock), 0, st, ws, observed, num_rows, per_chunk,
                      (unsigned long long)k, status_dev, totals_host ? totals_host + 2 : (uint32_t *)nullptr);
   hipLaunchKernelGGL(rank_combine_observed_kernel, dim3(bm_grid), dim3(kBlock), 0, st, counts_dev, num_rows, per_chunk,
-                     (const RankWs *)ws, observed, reinterpret_cast<unsigned long long *>(in_new_dev),
+                     ws, observed, reinterpret_cast<unsigned long long *>(in_new_dev),
                      reinterpret_cast<const unsigned long long *>(cached_dev), static_cast<BmWs *>(evict_ws_dev),
-                     static_cast<BmWs *>(insert_ws_dev), reset_counts);
-  if (cached_dev)
-    hipLaunchKernelGGL(bitmap_scan2_kernel, dim3(2), dim3(kBlock), 0, st, static_cast<BmWs *>(evict_ws_dev),
-                       static_cast<BmWs *>(insert_ws_dev), totals_host, (const RankWs *)ws);
+                     static_cast<BmWs *>(insert_ws_dev), reset_counts, totals_host, ticket);
+  if (cached_dev && num_rows > kSmallBits)  // the emit pass of longer bitmaps wants the chunk counts scanned
+    hipLaunchKernelGGL(bitmap_scan2_kernel, dim3(2), dim3(kScanBlock), 0, st, static_cast<BmWs *>(evict_ws_dev),
+                       static_cast<BmWs *>(insert_ws_dev), (uint32_t *)nullptr);
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -1060,8 +1215,9 @@ int ugk_bitmap_count(const uint64_t *a_dev, const uint64_t *b_dev, int invert_a,
                      reinterpret_cast<const unsigned long long *>(a_dev),
                      reinterpret_cast<const unsigned long long *>(b_dev), invert_a ? kBmInvertA : 0, nbits,
                      per_chunk, static_cast<BmWs *>(ws_dev), (const RankWs *)nullptr);
-  hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kBlock), 0, as_stream(stream), static_cast<BmWs *>(ws_dev),
-                     total_host, (const RankWs *)nullptr);
+  if (total_host || nbits > kSmallBits)
+    hipLaunchKernelGGL(bitmap_scan_kernel, dim3(1), dim3(kScanBlock), 0, as_stream(stream), static_cast<BmWs *>(ws_dev),
+                       total_host, (const RankWs *)nullptr);
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -1078,27 +1234,40 @@ int ugk_bitmap_count_diff(const uint64_t *a_dev, const uint64_t *b_dev, uint64_t
                      reinterpret_cast<const unsigned long long *>(a_dev),
                      reinterpret_cast<const unsigned long long *>(b_dev), nbits, per_chunk,
                      static_cast<BmWs *>(ws_ab_dev), static_cast<BmWs *>(ws_ba_dev));
-  hipLaunchKernelGGL(bitmap_scan2_kernel, dim3(2), dim3(kBlock), 0, as_stream(stream), static_cast<BmWs *>(ws_ab_dev),
-                     static_cast<BmWs *>(ws_ba_dev), totals_host, (const RankWs *)nullptr);
+  hipLaunchKernelGGL(bitmap_scan2_kernel, dim3(2), dim3(kScanBlock), 0, as_stream(stream), static_cast<BmWs *>(ws_ab_dev),
+                     static_cast<BmWs *>(ws_ba_dev), totals_host);
   UGK_HIP(hipGetLastError());
   return 0;
 }
 
 int ugk_bitmap_emit(const uint64_t *a_dev, const uint64_t *b_dev, int invert_a, uint64_t nbits, const void *ws_dev,
                     uint32_t *out_dev, uint64_t max_out, void *stream) {
+  return ugk_bitmap_emit_counted(a_dev, b_dev, invert_a, nbits, ws_dev, out_dev, max_out, nullptr, stream);
+}
+
+int ugk_bitmap_emit_counted(const uint64_t *a_dev, const uint64_t *b_dev, int invert_a, uint64_t nbits, const void *ws_dev,
+                            uint32_t *out_dev, uint64_t max_out, uint32_t *total_host, void *stream) {
   UGK_REQUIRE(a_dev && ws_dev, "ugk_bitmap_emit: null pointer");
   UGK_REQUIRE(nbits > 0 && nbits <= 0xffffffffull, "ugk_bitmap_emit: %llu bits do not fit 32-bit positions",
               (unsigned long long)nbits);
-  if (max_out == 0) return 0;
-  UGK_REQUIRE(out_dev, "ugk_bitmap_emit: null output list");
+  if (max_out == 0 && !total_host) return 0;
+  UGK_REQUIRE(out_dev || max_out == 0, "ugk_bitmap_emit: null output list");
   const uint64_t n_words = (nbits + 63) / 64;
   const uint64_t per_chunk = bm_words_per_chunk(n_words);
+  if (nbits <= kSmallBits) {
+    hipLaunchKernelGGL((bitmap_emit_small_kernel<1>), dim3(small_grid(nbits, per_chunk)), dim3(kSmallBlock), 0, as_stream(stream),
+                       reinterpret_cast<const unsigned long long *>(a_dev),
+                       reinterpret_cast<const unsigned long long *>(b_dev), invert_a ? kBmInvertA : 0, nbits, per_chunk,
+                       BmList{static_cast<const BmWs *>(ws_dev), out_dev, max_out}, BmList{nullptr, nullptr, 0}, total_host);
+    UGK_HIP(hipGetLastError());
+    return 0;
+  }
   const uint64_t n_blocks = (n_words + kWave - 1) / kWave;
   const unsigned grid = clamp_grid((n_blocks + (kBlock / kWave) - 1) / (kBlock / kWave), 0);
   hipLaunchKernelGGL(bitmap_emit_kernel, dim3(grid), dim3(kBlock), 0, as_stream(stream),
                      reinterpret_cast<const unsigned long long *>(a_dev),
                      reinterpret_cast<const unsigned long long *>(b_dev), invert_a ? kBmInvertA : 0, nbits,
-                     per_chunk, static_cast<const BmWs *>(ws_dev), out_dev, max_out);
+                     per_chunk, static_cast<const BmWs *>(ws_dev), out_dev, max_out, total_host);
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -1113,6 +1282,15 @@ int ugk_bitmap_emit_diff(const uint64_t *a_dev, const uint64_t *b_dev, uint64_t 
   UGK_REQUIRE((out_ab_dev || max_ab == 0) && (out_ba_dev || max_ba == 0), "ugk_bitmap_emit_diff: null output list");
   const uint64_t n_words = (nbits + 63) / 64;
   const uint64_t per_chunk = bm_words_per_chunk(n_words);
+  if (nbits <= kSmallBits) {
+    hipLaunchKernelGGL((bitmap_emit_small_kernel<2>), dim3(small_grid(nbits, per_chunk)), dim3(kSmallBlock), 0, as_stream(stream),
+                       reinterpret_cast<const unsigned long long *>(a_dev),
+                       reinterpret_cast<const unsigned long long *>(b_dev), 0, nbits, per_chunk,
+                       BmList{static_cast<const BmWs *>(ws_ab_dev), out_ab_dev, max_ab},
+                       BmList{static_cast<const BmWs *>(ws_ba_dev), out_ba_dev, max_ba}, (uint32_t *)nullptr);
+    UGK_HIP(hipGetLastError());
+    return 0;
+  }
   const uint64_t n_groups = ((n_words + kWave - 1) / kWave + kDiffBlocks - 1) / kDiffBlocks;
   const unsigned grid = clamp_grid((n_groups + (kBlock / kWave) - 1) / (kBlock / kWave), 0);
   hipLaunchKernelGGL(bitmap_emit_diff_kernel, dim3(grid), dim3(kBlock), 0, as_stream(stream),

@@ -240,11 +240,9 @@ __global__ void words_ticket_kernel(const uint32_t *a, unsigned n_a, const uint3
 }
 }  // namespace
 
-int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, unsigned spin_us) {
-  UGK_REQUIRE(ticket_host, "ugk_stream_sync_ticket: null ticket word");
-  hipLaunchKernelGGL(ticket_kernel, dim3(1), dim3(1), 0, as_stream(stream), ticket_host, value);
-  UGK_HIP(hipGetLastError());
-  volatile uint32_t *word = ticket_host;
+int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned spin_us, void *stream) {
+  UGK_REQUIRE(ticket_host, "ugk_ticket_wait: null ticket word");
+  const volatile uint32_t *word = ticket_host;
   const auto t0 = std::chrono::steady_clock::now();
   unsigned polls = 0;
   while (*word != value) {
@@ -256,9 +254,16 @@ int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, 
   }
   // the ticket says that everything enqueued in front of it has run: asking the runtime as well would give back the
   // microseconds the poll saved
-  if (*word == value) return 0;
-  UGK_HIP(hipStreamSynchronize(as_stream(stream)));
+  if (*word != value) UGK_HIP(hipStreamSynchronize(as_stream(stream)));
+  std::atomic_thread_fence(std::memory_order_acquire);
   return 0;
+}
+
+int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, unsigned spin_us) {
+  UGK_REQUIRE(ticket_host, "ugk_stream_sync_ticket: null ticket word");
+  hipLaunchKernelGGL(ticket_kernel, dim3(1), dim3(1), 0, as_stream(stream), ticket_host, value);
+  UGK_HIP(hipGetLastError());
+  return ugk_ticket_wait(ticket_host, value, spin_us, stream);
 }
 
 int ugk_leave_done_words(ugk_done_t *done) {
@@ -307,18 +312,7 @@ int ugk_words_to_host_ticket(const uint32_t *a_dev, unsigned n_a, const uint32_t
   hipLaunchKernelGGL(words_ticket_kernel, dim3(1), dim3(64), 0, as_stream(stream), a_dev, n_a, b_dev, n_b, dst_host,
                      value);
   UGK_HIP(hipGetLastError());
-  volatile uint32_t *word = dst_host;
-  const auto t0 = std::chrono::steady_clock::now();
-  unsigned polls = 0;
-  while (*word != value) {
-    if ((++polls & 63u) == 0 &&
-        std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0).count() >=
-            (long long)spin_us)
-      break;
-  }
-  if (*word != value) UGK_HIP(hipStreamSynchronize(as_stream(stream)));
-  std::atomic_thread_fence(std::memory_order_acquire);
-  return 0;
+  return ugk_ticket_wait(dst_host, value, spin_us, stream);
 }
 
 int ugk_preload_kernels(void) {

@@ -76,6 +76,7 @@ SIGNATURES = {
     "ugk_stream_sync": [_vp],
     "ugk_stream_is_capturing": [_vp, _vp],
     "ugk_stream_sync_ticket": [_vp, _vp, _u32, C.c_uint],
+    "ugk_ticket_wait": [_vp, _u32, C.c_uint, _vp],
     "ugk_leave_done_words": [C.POINTER(Done)],
     "ugk_done_wait": [C.POINTER(Done), C.c_uint, _vp, C.POINTER(_u64), C.POINTER(_u64)],
     "ugk_words_to_host_ticket": [_vp, C.c_uint, _vp, C.c_uint, _vp, _u32, C.c_uint, _vp],
@@ -148,10 +149,12 @@ SIGNATURES = {
     "ugk_rank_place": [_vp, _u64, _u64, _vp, _vp, _vp, _vp, C.c_int, _vp],
     "ugk_rank_place_keep": [_vp, _u64, _u64, _vp, _vp, _vp, _vp, _vp, C.c_int, _vp],
     "ugk_rank_place_observed": [_vp, _u64, _u64, _vp, _vp, _vp, C.c_int, _vp, _vp, _vp, _vp, _vp, _vp],
+    "ugk_rank_place_observed_ticket": [_vp, _u64, _u64, _vp, _vp, _vp, C.c_int, _vp, _vp, _vp, _vp, _vp, _u32, _vp],
     "ugk_rank_threshold": [_vp, _vp, _vp],
     "ugk_bitmap_workspace_bytes": [],
     "ugk_bitmap_count": [_vp, _vp, C.c_int, _u64, _vp, _vp, _vp],
     "ugk_bitmap_emit": [_vp, _vp, C.c_int, _u64, _vp, _vp, _u64, _vp],
+    "ugk_bitmap_emit_counted": [_vp, _vp, C.c_int, _u64, _vp, _vp, _u64, _vp, _vp],
     "ugk_bitmap_count_diff": [_vp, _vp, _u64, _vp, _vp, _vp, _vp],
     "ugk_bitmap_emit_diff": [_vp, _vp, _u64, _vp, _vp, _vp, _u64, _vp, _u64, _vp],
     "ugk_bitmap_update": [_vp, _u64, _vp, _sz, C.c_int, _vp, _vp],
