@@ -140,6 +140,8 @@ int ugk_stream_is_capturing(void *stream, int *capturing);
 int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, unsigned spin_us);
 /* the poll of ugk_stream_sync_ticket alone, for a ticket that some launch on `stream` writes itself */
 int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned spin_us, void *stream);
+/* the same until the word is no longer `value` */
+int ugk_word_wait(const uint32_t *word_host, uint32_t value, unsigned spin_us, void *stream);
 /* The end of one launch polled for without a kernel behind it.  ugk_leave_done_words: the next ugk_gather_*,
  * ugk_extract_mix_* or ugk_extract_pool_* call of this thread (that one only; after a call that failed, and where none
  * comes, NULL takes the request back) makes its workgroups leave words in words_host as they end, and stores the number of
@@ -447,6 +449,14 @@ int ugk_dedup_u32(const uint32_t *keys_dev, size_t n, void *workspace_dev, size_
 int ugk_dedup_i64(const int64_t *keys_dev, size_t n, void *workspace_dev, size_t workspace_bytes, uint32_t epoch,
                   int64_t *unique_out_dev, uint32_t *inverse_out_dev, uint32_t *rep_out_dev, uint32_t *n_unique_dev,
                   uint32_t *n_unique_host, void *stream);
+
+/* The same for keys of key_bytes 4 or 8, with two count words that calls take in turn: n_unique_dev is zero on entry as above,
+ * and the call leaves next_n_unique_dev at zero for the next one.  *n_unique_host, which the caller sets to 0 (a batch of one
+ * key and more has one distinct key at least), can be polled (ugk_word_wait): once it changes, launches behind this call on
+ * `stream` may be sized by it. */
+int ugk_dedup_rotating(const void *keys_dev, uint32_t key_bytes, size_t n, void *workspace_dev, size_t workspace_bytes,
+                       uint32_t epoch, void *unique_out_dev, uint32_t *inverse_out_dev, uint32_t *rep_out_dev,
+                       uint32_t *n_unique_dev, uint32_t *next_n_unique_dev, uint32_t *n_unique_host, void *stream);
 
 /* The same deduplication for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.  The slot set and the per-occurrence ids,

@@ -857,6 +857,12 @@ int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned, void 
   note_stream_idle(as_stream(stream));
   return 0;
 }
+int ugk_word_wait(const uint32_t *word_host, uint32_t value, unsigned, void *stream) {
+  REQUIRE(word_host && *word_host != value, "ugk_word_wait: nobody has written the word");
+  std::lock_guard<std::mutex> g(g_rt_mu);
+  if (as_stream(stream)->capture) violation("the host waited for a word on a stream that records into a graph");
+  return 0;
+}
 int ugk_leave_done_words(ugk_done_t *done) {
   if (done) {
     REQUIRE(done->words_host && done->counters_dev && done->tag > 0 && done->tag <= UGK_DONE_MAX_TAG,
@@ -1266,6 +1272,18 @@ int ugk_gather_scatter_staged_u32(const void *host, uint64_t host_rows, const ui
   return 0;
 }
 
+int ugk_dedup_rotating(const void *keys, uint32_t key_bytes, size_t n, void *, size_t, uint32_t, void *unique_out,
+                       uint32_t *inverse, uint32_t *rep, uint32_t *n_unique, uint32_t *next_n_unique,
+                       uint32_t *n_unique_host, void *) {
+  REQUIRE((key_bytes == 4 || key_bytes == 8) && next_n_unique && next_n_unique != n_unique, "ugk_dedup_rotating: bad argument");
+  REQUIRE(n == 0 || *n_unique == 0, "ugk_dedup_rotating: the count word is not zero");
+  if (n) *next_n_unique = 0;
+  if (key_bytes == 4)
+    return dedup(static_cast<const uint32_t *>(keys), n, static_cast<uint32_t *>(unique_out), inverse, rep, n_unique,
+                 n_unique_host);
+  return dedup(static_cast<const int64_t *>(keys), n, static_cast<int64_t *>(unique_out), inverse, rep, n_unique,
+               n_unique_host);
+}
 size_t ugk_dedup_workspace_bytes(size_t) { return 64; }
 int ugk_dedup_u32(const uint32_t *keys, size_t n, void *, size_t, uint32_t epoch, uint32_t *unique_out,
                   uint32_t *inverse, uint32_t *rep, uint32_t *n_unique, uint32_t *n_unique_host, void *) {

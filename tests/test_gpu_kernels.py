@@ -1875,6 +1875,40 @@ def test_dedup_of_small_and_large_batches_sharing_one_workspace(kdtype):
                  ptr(dev_zeros_u32(n)), None, ptr(dev_zeros_u32(1)), None, None)
 
 
+@pytest.mark.parametrize("kdtype", [np.uint32, np.int64])
+def test_dedup_with_two_count_words_in_turn(kdtype):
+    """each call finds its word at zero and leaves the other so; the number of distinct keys can be polled for, and what is
+    launched behind the poll reads complete lists"""
+    rng = np.random.default_rng(5)
+    cap = 300_000
+    ws_bytes = hip.lib().ugk_dedup_workspace_bytes(cap)
+    ws = torch.zeros(ws_bytes, dtype=torch.uint8, device="cuda")
+    counts, found = dev_zeros_u32(2), PinnedArray((1,), np.uint32)
+    uniq, inv, rep = dev_bytes(cap * 8), dev_zeros_u32(cap), dev_zeros_u32(cap)
+    sync()
+    try:
+        for epoch, (n, space) in enumerate([(1, 5), (255, 40), (65_536, 1 << 20), (65_537, 3_000), (65_537, 1 << 40),
+                                              (131_072, 50_000), (131_073, 1 << 40), (cap, 1 << 40), (cap, 7)], 1):
+            keys = rng.integers(0, min(space, np.iinfo(kdtype).max), size=n).astype(kdtype)
+            d_keys = to_dev(keys)
+            found.array[0] = 0
+            sync()
+            hip.call("ugk_dedup_rotating", ptr(d_keys), keys.itemsize, n, ptr(ws), ws_bytes, epoch, ptr(uniq), ptr(inv),
+                     ptr(rep), ptr(counts) + 4 * (epoch & 1), ptr(counts) + 4 * (1 - (epoch & 1)), found.ptr, None)
+            hip.call("ugk_word_wait", found.ptr, 0, (0, 1_000_000)[epoch & 1], None)
+            want = np.unique(keys)
+            assert found.array[0] == len(want)
+            got = to_np(uniq, kdtype)[: len(want)]  # a copy on the same stream
+            assert np.array_equal(np.sort(got), want)
+            assert np.array_equal(got[to_np(inv, np.uint32)[:n]], keys)
+            r = to_np(rep, np.uint32)[: len(want)]
+            assert np.array_equal(keys[r], got)
+            assert to_np(counts, np.uint32)[1 - (epoch & 1)] == 0
+    finally:
+        sync()
+        found.free()
+
+
 @pytest.mark.parametrize("mode", ["flat", "hash", "hash32"])
 @pytest.mark.parametrize("kdtype", [np.uint32, np.int64])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 4097, 200_000])

@@ -461,15 +461,6 @@ static int Classify(ugk_table_t t, const Id64Type *keys, size_t n, uint64_t host
                     ugk_idx_t *idx, uint32_t *c, uint32_t *next, uint32_t *st, uint32_t *mirror, StreamHandle s) {
   return ugk_classify_i64(t, keys, n, host_rows, dst_map, idx, c, next, st, mirror, s);
 }
-static int Dedup(const IdType *keys, size_t n, void *ws, size_t ws_bytes, uint32_t epoch, IdType *uniq, uint32_t *inv,
-                 uint32_t *rep, uint32_t *nu, uint32_t *nu_host, StreamHandle s) {
-  return ugk_dedup_u32(keys, n, ws, ws_bytes, epoch, uniq, inv, rep, nu, nu_host, s);
-}
-static int Dedup(const Id64Type *keys, size_t n, void *ws, size_t ws_bytes, uint32_t epoch, Id64Type *uniq,
-                 uint32_t *inv, uint32_t *rep, uint32_t *nu, uint32_t *nu_host, StreamHandle s) {
-  return ugk_dedup_i64(keys, n, ws, ws_bytes, epoch, uniq, inv, rep, nu, nu_host, s);
-}
-
 static int Record(const IdType *keys, size_t n, uint64_t mul, uint64_t mask, uint32_t *counts, uint64_t rows,
                   uint64_t *observed, uint32_t *st, uint32_t *mirror, StreamHandle s) {
   return ugk_record_u32(keys, n, mul, mask, counts, rows, observed, st, mirror, s);
@@ -674,7 +665,7 @@ size_t ExtractSession::DrainHotness(FreqRecorder *recorder) {
 // each (where its row is gathered to) and, per input position, which distinct key it is.  One blocking wait: the
 // host needs the number of distinct keys to size the launches that follow.
 template <typename KeyT>
-size_t ExtractSession::DedupKeys(const KeyT *nodes, size_t num_nodes, StreamHandle stream) {
+size_t ExtractSession::DedupKeys(const KeyT *nodes, size_t num_nodes, uint32_t *inverse, StreamHandle stream) {
   const size_t ws_bytes = ugk_dedup_workspace_bytes(num_nodes);
   auto alloc = _cache_ctx->_gpu_mem_allocator;
   if (_dedup_ws == nullptr || _dedup_ws_bytes < ws_bytes) {
@@ -696,12 +687,19 @@ size_t ExtractSession::DedupKeys(const KeyT *nodes, size_t num_nodes, StreamHand
     UGK_CALL(ugk_fill_u32(_dedup_ws->ptr<uint32_t>(), 0, _dedup_ws_bytes / 4, stream));
     _dedup_epoch = 1;
   }
-  uint32_t *n_unique = _state + kStNumUnique;
-  UGK_CALL(ugk_fill_u32(n_unique, 0, 1, stream));
-  UGK_CALL(Dedup(nodes, num_nodes, _dedup_ws->ptr<void>(), _dedup_ws_bytes, _dedup_epoch, DedupUnique<KeyT>(),
-                 DedupInverse(), DedupRep(), n_unique, _host_mirror + kMirNumUnique, stream));
-  UGK_CALL(ugk_stream_sync(stream));
-  const size_t nu = _host_mirror[kMirNumUnique];
+  // two count words in turn: each call finds its own at zero, left so by the call before (or by the session's start)
+  uint32_t *n_unique = _state + (_dedup_odd ? kStNumUnique2 : kStNumUnique);
+  uint32_t *next = _state + (_dedup_odd ? kStNumUnique : kStNumUnique2);
+  _dedup_odd = !_dedup_odd;
+  volatile uint32_t *found = _host_mirror + kMirNumUnique;
+  *found = 0;
+  UGK_CALL(ugk_dedup_rotating(nodes, sizeof(KeyT), num_nodes, _dedup_ws->ptr<void>(), _dedup_ws_bytes, _dedup_epoch,
+                              DedupUnique<KeyT>(), inverse ? inverse : DedupInverse(), DedupRep(), n_unique, next,
+                              _host_mirror + kMirNumUnique, stream));
+  // the number is there as the second of the two kernels starts, which what is launched next stands behind
+  if (RunConfig::spin_wait_us == 0) UGK_CALL(ugk_stream_sync(stream));
+  else UGK_CALL(ugk_word_wait(_host_mirror + kMirNumUnique, 0, RunConfig::spin_wait_us, stream));
+  const size_t nu = *found;
   CHECK(nu >= 1 && nu <= num_nodes) << "deduplication produced " << nu << " keys from " << num_nodes;
   return nu;
 }
@@ -923,7 +921,7 @@ void ExtractSession::ExtractFeatImpl(const KeyT *nodes, size_t num_nodes, void *
   if (dedup || skip_local) CopyKeysNow(stream);  // the launches work on other keys than the caller's
   if (dedup) {
     UGK_CALL(ugk_event_record(_ev_t[2], stream));
-    const size_t nu = DedupKeys(nodes, num_nodes, stream);
+    const size_t nu = DedupKeys(nodes, num_nodes, nullptr, stream);
     UGK_CALL(ugk_event_record(_ev_t[3], stream));
     nodes = DedupUnique<KeyT>();
     dst_map = DedupRep();
@@ -1196,10 +1194,9 @@ size_t ExtractSession::ExtractUniqueImpl(const KeyT *nodes, size_t num_nodes, vo
   CHECK_NOTNULL(nodes);
   CHECK_NOTNULL(output);
   CHECK_NOTNULL(inverse_out);
-  const size_t nu = DedupKeys(nodes, num_nodes, stream);
-  UGK_CALL(ugk_memcpy_async(inverse_out, DedupInverse(), num_nodes * sizeof(uint32_t), stream));
+  const size_t nu = DedupKeys(nodes, num_nodes, inverse_out, stream);
   _skip_dedup = true;
-  ExtractFeatImpl<KeyT>(DedupUnique<KeyT>(), nu, output, stream, task_key);  // blocks: the copy above is done too
+  ExtractFeatImpl<KeyT>(DedupUnique<KeyT>(), nu, output, stream, task_key);  // blocks: the kernels above are done too
   _skip_dedup = false;
   return nu;
 }

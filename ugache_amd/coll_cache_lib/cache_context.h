@@ -93,7 +93,8 @@ class CacheContext {
 
 class ExtractSession {
   // words of the device-side state block (64 zero-filled uint32)
-  enum StateWord { kStCounts0 = 0, kStCounts1 = 2, kStStatus = 4, kStNumUnique = 5, kStDrainEntries = 6 };
+  enum StateWord { kStCounts0 = 0, kStCounts1 = 2, kStStatus = 4, kStNumUnique = 5, kStDrainEntries = 6,
+                   kStNumUnique2 = 7 };
   // words of the pinned host mirror the kernels write; [1] and [2] are indexed 1 + location
   enum MirrorWord { kMirError = 0, kMirGroupSizes = 1, kMirNumUnique = 3, kMirDrainCount = 4, kMirDrainMore = 5,
                     kMirSkipCount = 6, kMirTicket = 7 };
@@ -124,7 +125,8 @@ class ExtractSession {
   uint32_t *DedupInverse() const { return reinterpret_cast<uint32_t *>(_dedup_out->ptr<char>() + _dedup_cap * 8); }
   uint32_t *DedupRep() const { return DedupInverse() + _dedup_cap; }
   template <typename KeyT>
-  size_t DedupKeys(const KeyT *nodes, size_t num_nodes, StreamHandle stream);
+  size_t DedupKeys(const KeyT *nodes, size_t num_nodes, uint32_t *inverse, StreamHandle stream);
+  bool _dedup_odd = false;  // which of the two count words the next deduplication uses
 
   // hotness counters on the device (RunConfig::gpu_record)
   MemHandle _hot_counts;         // uint32 per row of the host table

@@ -424,8 +424,11 @@ __global__ __launch_bounds__(kBlock) void dedup_claim_kernel(const K *__restrict
 
 __global__ __launch_bounds__(kBlock) void dedup_resolve_kernel(size_t n, const uint32_t *__restrict__ uid_of,
                                                                uint32_t *inverse, const uint32_t *n_unique,
-                                                               uint32_t *n_unique_host) {
-  if (n_unique_host && blockIdx.x == 0 && threadIdx.x == 0) *n_unique_host = *n_unique;
+                                                               uint32_t *n_unique_host, uint32_t *next_n_unique) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (next_n_unique) *next_n_unique = 0;
+    if (n_unique_host) *n_unique_host = *n_unique;
+  }
   for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
     inverse[i] = uid_of[inverse[i]];
 }
@@ -686,7 +689,7 @@ size_t dedup_capacity_of_workspace(size_t bytes) {
 template <typename K>
 int dedup(const K *keys, size_t n, void *workspace, size_t workspace_bytes, uint32_t epoch, const uint32_t *epoch_dev,
           K *unique_out, uint32_t *inverse, uint32_t *rep_of, uint32_t *n_unique, uint32_t *n_unique_host,
-          void *stream) {
+          uint32_t *next_n_unique, void *stream) {
   if (n == 0) return 0;
   UGK_REQUIRE(keys && workspace && unique_out && inverse && n_unique, "ugk_dedup: null pointer");
   UGK_REQUIRE(epoch != 0 || epoch_dev, "ugk_dedup: epoch must be non-zero");
@@ -697,13 +700,19 @@ int dedup(const K *keys, size_t n, void *workspace, size_t workspace_bytes, uint
               workspace_bytes, cap / 2, n);
   unsigned long long *slots = reinterpret_cast<unsigned long long *>(workspace);
   uint32_t *uid_of = reinterpret_cast<uint32_t *>(slots + cap);
-  // 256-key tiles while 1024-key ones would leave compute units idle; beyond that the larger tile wins, because more
-  // of a skewed batch's duplicates meet in LDS (212,992 keys, Zipf 1.1: 24.7 us against 43.8 us)
-  const int items = n <= (size_t)cu_count() * kBlock ? 1 : kItems;
+  // 256-key tiles while larger ones would leave compute units idle, 512-key ones up to twice as many keys; beyond that the
+  // larger tile wins, because more of a skewed batch's duplicates meet in LDS.  us with the set cleared in front of it (about
+  // 5 of them), 256 / 512 / 1024-key tiles: 65,536 keys uniform 29 / 38 / 57, Zipf 0.9 27 / 30 / 41, Zipf 1.3 18 / 18 / 20;
+  // 100,000 keys 27 / 32 / 46, 29 / 28 / 36, 24 / 21 / 21; 200,000 keys 36 / 38 / 51, 43 / 35 / 39, 39 / 29 / 23.
+  const size_t per_cu = (size_t)cu_count() * kBlock;
+  const int items = n <= per_cu ? 1 : n <= 2 * per_cu ? 2 : kItems;
   const size_t tile = (size_t)kBlock * items;
   const unsigned claim_grid = clamp_grid((n + tile - 1) / tile, 0);
   if (items == 1)
     hipLaunchKernelGGL((dedup_claim_kernel<K, 1>), dim3(claim_grid), dim3(kBlock), 0, as_stream(stream), keys, n,
+                       slots, cap - 1, epoch, epoch_dev, uid_of, unique_out, inverse, rep_of, n_unique);
+  else if (items == 2)
+    hipLaunchKernelGGL((dedup_claim_kernel<K, 2>), dim3(claim_grid), dim3(kBlock), 0, as_stream(stream), keys, n,
                        slots, cap - 1, epoch, epoch_dev, uid_of, unique_out, inverse, rep_of, n_unique);
   else
     hipLaunchKernelGGL((dedup_claim_kernel<K, kItems>), dim3(claim_grid), dim3(kBlock), 0, as_stream(stream), keys, n,
@@ -711,7 +720,7 @@ int dedup(const K *keys, size_t n, void *workspace, size_t workspace_bytes, uint
   UGK_HIP(hipGetLastError());
   const unsigned grid = clamp_grid((n + kBlock - 1) / kBlock, 0);
   hipLaunchKernelGGL(dedup_resolve_kernel, dim3(grid), dim3(kBlock), 0, as_stream(stream), n, uid_of, inverse,
-                     n_unique, n_unique_host);
+                     n_unique, n_unique_host, next_n_unique);
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -832,23 +841,37 @@ int ugk_dedup_static(const void *keys_dev, uint32_t key_bytes, size_t n, void *u
   if (key_bytes == 4)
     return dedup<uint32_t>(static_cast<const uint32_t *>(keys_dev), n, ws, UGK_DEDUP_STATIC_WS_BYTES, 0, epoch_dev,
                            static_cast<uint32_t *>(unique_out_dev), inverse_out_dev, rep_out_dev, n_unique_dev,
-                           n_unique_host, stream);
+                           n_unique_host, nullptr, stream);
   return dedup<int64_t>(static_cast<const int64_t *>(keys_dev), n, ws, UGK_DEDUP_STATIC_WS_BYTES, 0, epoch_dev,
                         static_cast<int64_t *>(unique_out_dev), inverse_out_dev, rep_out_dev, n_unique_dev,
-                        n_unique_host, stream);
+                        n_unique_host, nullptr, stream);
+}
+
+int ugk_dedup_rotating(const void *keys_dev, uint32_t key_bytes, size_t n, void *workspace_dev, size_t workspace_bytes,
+                       uint32_t epoch, void *unique_out_dev, uint32_t *inverse_out_dev, uint32_t *rep_out_dev,
+                       uint32_t *n_unique_dev, uint32_t *next_n_unique_dev, uint32_t *n_unique_host, void *stream) {
+  UGK_REQUIRE(key_bytes == 4 || key_bytes == 8, "ugk_dedup_rotating: keys of %u bytes (4 or 8 are supported)", key_bytes);
+  UGK_REQUIRE(next_n_unique_dev && next_n_unique_dev != n_unique_dev, "ugk_dedup_rotating: one count word for two calls");
+  if (key_bytes == 4)
+    return dedup<uint32_t>(static_cast<const uint32_t *>(keys_dev), n, workspace_dev, workspace_bytes, epoch, nullptr,
+                           static_cast<uint32_t *>(unique_out_dev), inverse_out_dev, rep_out_dev, n_unique_dev,
+                           n_unique_host, next_n_unique_dev, stream);
+  return dedup<int64_t>(static_cast<const int64_t *>(keys_dev), n, workspace_dev, workspace_bytes, epoch, nullptr,
+                        static_cast<int64_t *>(unique_out_dev), inverse_out_dev, rep_out_dev, n_unique_dev, n_unique_host,
+                        next_n_unique_dev, stream);
 }
 
 int ugk_dedup_u32(const uint32_t *keys_dev, size_t n, void *workspace_dev, size_t workspace_bytes, uint32_t epoch,
                   uint32_t *unique_out_dev, uint32_t *inverse_out_dev, uint32_t *rep_out_dev, uint32_t *n_unique_dev,
                   uint32_t *n_unique_host, void *stream) {
   return dedup<uint32_t>(keys_dev, n, workspace_dev, workspace_bytes, epoch, nullptr, unique_out_dev, inverse_out_dev,
-                         rep_out_dev, n_unique_dev, n_unique_host, stream);
+                         rep_out_dev, n_unique_dev, n_unique_host, nullptr, stream);
 }
 int ugk_dedup_i64(const int64_t *keys_dev, size_t n, void *workspace_dev, size_t workspace_bytes, uint32_t epoch,
                   int64_t *unique_out_dev, uint32_t *inverse_out_dev, uint32_t *rep_out_dev, uint32_t *n_unique_dev,
                   uint32_t *n_unique_host, void *stream) {
   return dedup<int64_t>(keys_dev, n, workspace_dev, workspace_bytes, epoch, nullptr, unique_out_dev, inverse_out_dev,
-                        rep_out_dev, n_unique_dev, n_unique_host, stream);
+                        rep_out_dev, n_unique_dev, n_unique_host, nullptr, stream);
 }
 
 }  // extern "C"

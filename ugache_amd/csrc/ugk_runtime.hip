@@ -240,23 +240,33 @@ __global__ void words_ticket_kernel(const uint32_t *a, unsigned n_a, const uint3
 }
 }  // namespace
 
-int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned spin_us, void *stream) {
-  UGK_REQUIRE(ticket_host, "ugk_ticket_wait: null ticket word");
-  const volatile uint32_t *word = ticket_host;
+// polls a pinned word for up to spin_us until it is `value` (or, with until_other, something else), then waits for the stream
+static int poll_word(const uint32_t *word_host, uint32_t value, bool until_other, unsigned spin_us, void *stream) {
+  const volatile uint32_t *word = word_host;
   const auto t0 = std::chrono::steady_clock::now();
   unsigned polls = 0;
-  while (*word != value) {
+  while ((*word != value) != until_other) {
     // the clock is read every 64 polls: a poll is a load of a line the device writes into, the clock a system call away
     if ((++polls & 63u) == 0 &&
         std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now() - t0).count() >=
             (long long)spin_us)
       break;
   }
-  // the ticket says that everything enqueued in front of it has run: asking the runtime as well would give back the
-  // microseconds the poll saved
-  if (*word != value) UGK_HIP(hipStreamSynchronize(as_stream(stream)));
+  // the word says that what it stands for has run: asking the runtime as well would give back the microseconds the poll
+  // saved
+  if ((*word != value) != until_other) UGK_HIP(hipStreamSynchronize(as_stream(stream)));
   std::atomic_thread_fence(std::memory_order_acquire);
   return 0;
+}
+
+int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned spin_us, void *stream) {
+  UGK_REQUIRE(ticket_host, "ugk_ticket_wait: null ticket word");
+  return poll_word(ticket_host, value, false, spin_us, stream);
+}
+
+int ugk_word_wait(const uint32_t *word_host, uint32_t value, unsigned spin_us, void *stream) {
+  UGK_REQUIRE(word_host, "ugk_word_wait: null word");
+  return poll_word(word_host, value, true, spin_us, stream);
 }
 
 int ugk_stream_sync_ticket(void *stream, uint32_t *ticket_host, uint32_t value, unsigned spin_us) {

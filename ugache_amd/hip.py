@@ -77,6 +77,7 @@ SIGNATURES = {
     "ugk_stream_is_capturing": [_vp, _vp],
     "ugk_stream_sync_ticket": [_vp, _vp, _u32, C.c_uint],
     "ugk_ticket_wait": [_vp, _u32, C.c_uint, _vp],
+    "ugk_word_wait": [_vp, _u32, C.c_uint, _vp],
     "ugk_leave_done_words": [C.POINTER(Done)],
     "ugk_done_wait": [C.POINTER(Done), C.c_uint, _vp, C.POINTER(_u64), C.POINTER(_u64)],
     "ugk_words_to_host_ticket": [_vp, C.c_uint, _vp, C.c_uint, _vp, _u32, C.c_uint, _vp],
@@ -140,6 +141,7 @@ SIGNATURES = {
     "ugk_dedup_workspace_bytes": [_sz],
     "ugk_dedup_u32": [_vp, _sz, _vp, _sz, _u32, _vp, _vp, _vp, _vp, _vp, _vp],
     "ugk_dedup_i64": [_vp, _sz, _vp, _sz, _u32, _vp, _vp, _vp, _vp, _vp, _vp],
+    "ugk_dedup_rotating": [_vp, _u32, _sz, _vp, _sz, _u32, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "ugk_dedup_static": [_vp, _u32, _sz, _vp, _vp, _vp, _vp, _vp, _vp],
     "ugk_record_u32": [_vp, _sz, _u64, _u64, _vp, _u64, _vp, _vp, _vp, _vp],
     "ugk_record_i64": [_vp, _sz, _u64, _u64, _vp, _u64, _vp, _vp, _vp, _vp],
