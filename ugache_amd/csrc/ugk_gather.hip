@@ -83,8 +83,6 @@ __device__ __forceinline__ void st_stream(V *p, V v) {
   __builtin_nontemporal_store(v, p);
 }
 
-// NT_STORE is a template parameter, not a launch argument: with a run-time flag the optimiser merges the two stores
-// of `if (nt) stream(p, v); else *p = v;` into one and the non-temporal hint is lost (seen with UNROLL = 1).
 // Bound by HBM.  Where the launch is more than one round of workgroups (many_groups), or a lane has several vectors of a
 // row, a wavefront whose rows are all there and all good, which is every one but the batch's last, copies them without a
 // branch: behind one each load waits for the one before.  Rows out of 5 GiB, us per launch with the branch / without:
@@ -94,7 +92,7 @@ __device__ __forceinline__ void st_stream(V *p, V v) {
 // 10.5 / 10.3, 64 bytes x 262,144 11.3 / 11.7, 128 bytes x 131,072 8.7 / 9.1.  Rows in flight per lane, one / two / four /
 // eight, all without: 512 bytes x 65,536 15.9 / 14.7 / 15.1 / 15.5, x 524,288 91.1 / 82.4 / 82.5 / 83.5; 4 KB x 32,768 43.4 /
 // 43.4 / 51.9 / 48.4; 16 bytes x 32,768 3.8 / 4.5 / 5.8 / 9.0.
-template <typename V, int LPR, int UNROLL, bool NT_STORE, typename Idx>
+template <typename V, int LPR, int UNROLL, Store STORE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restrict__ src, uint64_t src_rows,
                                                         V *__restrict__ out, uint64_t out_rows, uint32_t vpr,
                                                         const uint32_t *__restrict__ counts, uint32_t group, size_t n,
@@ -107,18 +105,12 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
     begin = (group == UGK_LOC_LOCAL) ? 0 : n - c;
     if (host_mirror && blockIdx.x == 0 && threadIdx.x == 0) host_mirror[1 + group] = c;
   }
-  const bool through = !NT_STORE && done.tag != 0;
   constexpr int RPB = kBlock / LPR;  // rows copied by one block instruction
   const uint32_t lane = threadIdx.x % LPR;
   const uint32_t rib = threadIdx.x / LPR;
   constexpr size_t kPerIter = (size_t)RPB * UNROLL;
 
   for (size_t base = (size_t)blockIdx.x * kPerIter; base < count; base += (size_t)gridDim.x * kPerIter) {
-    if constexpr (Idx::kDense) {
-      if (base < done.num_keys)
-        for (size_t i = base + threadIdx.x; i < min(base + kPerIter, count); i += kBlock)
-          copy_key_along(done, i, ix.keys[i]);
-    }
     // the index words of all rows of the pass first, in flight together (a row past the end takes the last one's),
     // then the checks: a check between two of them would make the second wait for the first
     uint64_t s[UNROLL], d[UNROLL];
@@ -148,41 +140,39 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
       const uint32_t col = c0 + lane;
       if (col < vpr) {
         V v[UNROLL];
+        auto put = [&](int u) {
+          V *to = out + d[u] * vpr + col;
+          if constexpr (STORE == kThrough) store_through(reinterpret_cast<uint64_t>(to), v[u]);
+          else if constexpr (STORE == kStreaming) st_stream(to, v[u]);
+          else *to = v[u];
+        };
         if (no_branch) {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) v[u] = ld_stream(src + s[u] * vpr + col);
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) put(u);
         } else {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
             if (ok[u]) v[u] = ld_stream(src + s[u] * vpr + col);
-        }
-        if (through) {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
-            if (ok[u]) store_through(reinterpret_cast<uint64_t>(out + d[u] * vpr + col), v[u]);
-        } else if (no_branch) {
-#pragma unroll
-          for (int u = 0; u < UNROLL; ++u) {
-            if constexpr (NT_STORE) st_stream(out + d[u] * vpr + col, v[u]);
-            else out[d[u] * vpr + col] = v[u];
-          }
-        } else {
-#pragma unroll
-          for (int u = 0; u < UNROLL; ++u)
-            if (ok[u]) {
-              if constexpr (NT_STORE) st_stream(out + d[u] * vpr + col, v[u]);
-              else out[d[u] * vpr + col] = v[u];
-            }
+            if (ok[u]) put(u);
         }
       }
     }
+    if constexpr (Idx::kDense && STORE == kThrough) {
+      if (base < done.num_keys)
+        for (size_t i = base + threadIdx.x; i < min(base + kPerIter, count); i += kBlock)
+          copy_key_along(done, i, ix.keys[i]);
+    }
   }
-  if (done.tag) leave_done(done, nullptr);
+  if constexpr (STORE == kThrough) leave_done<true>(done, nullptr);
 }
 
 // The same for rows the lanes of gather_kernel do not fit (see flat_copy): a wavefront takes f.tile rows, one index
 // word per lane, and copies their vectors numbered through.
-template <typename Idx>
+template <Store STORE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                              char *__restrict__ out, uint64_t out_rows, FlatRow f,
                                                              const uint32_t *__restrict__ counts, uint32_t group,
@@ -202,22 +192,23 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
     uint64_t s = 0, d = 0;
     bool ok = lane_id() < rows;
     if (ok) ix.get(begin + base + lane_id(), s, d);
-    if constexpr (Idx::kDense) {
-      if (ok) copy_key_along(done, base + lane_id(), (typename Idx::key_t)s);
-    }
     if (ok && (s >= src_rows || d >= out_rows)) {
       ok = false;
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
       if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
     }
     const unsigned long long good = __ballot(ok);
-    if (good == 0ull) continue;
-    // a row that is skipped is read where the tile's first good row is
-    const uint64_t at = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
-    const uint64_t dummy = shfl64(at, __ffsll(good) - 1);
-    flat_copy<Idx::kDense>(ok ? at : dummy | kNoRowBit, (uint32_t)d, out, base, 0, rows, f, done.tag != 0);
+    if (good != 0ull) {
+      // a row that is skipped is read where the tile's first good row is
+      const uint64_t at = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
+      const uint64_t dummy = shfl64(at, __ffsll(good) - 1);
+      flat_copy<Idx::kDense, STORE == kThrough>(ok ? at : dummy | kNoRowBit, (uint32_t)d, out, base, 0, rows, f);
+    }
+    if constexpr (Idx::kDense && STORE == kThrough) {
+      if (lane_id() < rows) copy_key_along(done, base + lane_id(), (typename Idx::key_t)s);
+    }
   }
-  if (done.tag) leave_done(done, nullptr);
+  if constexpr (STORE == kThrough) leave_done<true>(done, nullptr);
 }
 
 // ... and with the output dealt out instead of the rows, for batches whose row i becomes output row i: a wavefront owns
@@ -239,16 +230,15 @@ StreamRow stream_row(size_t row_bytes, size_t n) {
                    (uint64_t)n * row_bytes};
 }
 
-template <bool NT_STORE, bool SHARE, typename Idx>
+template <Store STORE, bool SHARE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                                char *__restrict__ out, StreamRow f, uint32_t *status,
                                                                uint32_t *host_mirror, DoneWords done) {
   static_assert(Idx::kDense, "row i goes to output row i");
   typedef __attribute__((address_space(1))) uint32_t *gword_t;
   constexpr int U = (int)(kStreamPart / (kWave * 16));
-  const bool through = !NT_STORE && done.tag != 0;
-  auto put = [through](auto *q, auto w) {
-    if (through) store_through(reinterpret_cast<uint64_t>(q), w);
+  auto put = [](auto *q, auto w) {
+    if constexpr (STORE == kThrough) store_through(reinterpret_cast<uint64_t>(q), w);
     else *q = w;
   };
   const uint32_t lane = lane_id();
@@ -264,14 +254,16 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     const bool active = (uint64_t)lane * f.row_bytes < (uint64_t)off0 + bytes;
     bool ok = active;
     if (ok) ix.get(row0 + lane, s, d);
-    if (ok) copy_key_along(done, row0 + lane, (typename Idx::key_t)s);  // a row in two parts: twice the same key
     if (ok && s >= src_rows) {
       ok = false;
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
       if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
     }
     const unsigned long long good = __ballot(ok);
-    if (good == 0ull) continue;
+    if (good == 0ull) {
+      if (STORE == kThrough && active) copy_key_along(done, row0 + lane, (typename Idx::key_t)s);
+      continue;
+    }
     // a row that is skipped is read where the first good one is (all lanes take part in the shuffle)
     const uint64_t mine = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
     const uint64_t dummy = shfl64(mine, __ffsll(good) - 1);
@@ -316,7 +308,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
         w.z = head == 12 ? sa.w : head == 8 ? sb.x : sb.y;
         w.w = head == 12 ? sb.x : head == 8 ? sb.y : sb.z;
         if (row_a && row_b) {
-          if constexpr (NT_STORE) __builtin_nontemporal_store(w, q);
+          if constexpr (STORE == kStreaming) __builtin_nontemporal_store(w, q);
           else put(q, w);
         } else {  // a skipped row leaves its words of the output alone
           const gword_t q1 = reinterpret_cast<gword_t>(q);
@@ -331,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     for (int u = 0; u < U; ++u)
       if (copy[u]) {
         const gout_t q = reinterpret_cast<gout_t>(to + (u * kWave + lane) * 16);
-        if constexpr (NT_STORE) __builtin_nontemporal_store(v[u], q);
+        if constexpr (STORE == kStreaming) __builtin_nontemporal_store(v[u], q);
         else put(q, v[u]);
       }
     if constexpr (SHARE) {
@@ -345,8 +337,10 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
         }
       }
     }
+    if (STORE == kThrough && active)
+      copy_key_along(done, row0 + lane, (typename Idx::key_t)s);  // a row in two parts: twice the same key
   }
-  if (done.tag) leave_done(done, nullptr);
+  if constexpr (STORE == kThrough) leave_done<true>(done, nullptr);
 }
 
 // Re-expansion of duplicates inside one buffer: row i takes the bytes of its representative row.  Source and
@@ -479,14 +473,14 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
   const unsigned grid = gather_grid((n + kPerIter - 1) / kPerIter, max_blocks);
   const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
   const DoneWords done = nt ? DoneWords{} : request.take(grid);
-  if (nt)
-    hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, true, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,
-                       reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,
-                       group, n, many_groups, status, host_mirror, done);
-  else
-    hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, false, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,
-                       reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,
-                       group, n, many_groups, status, host_mirror, done);
+#define UGK_GO(STORE)                                                                                                  \
+  hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,            \
+                     reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,   \
+                     group, n, many_groups, status, host_mirror, done)
+  if (done.tag) UGK_GO(kThrough);
+  else if (nt) UGK_GO(kStreaming);
+  else UGK_GO(kOrdinary);
+#undef UGK_GO
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -582,8 +576,13 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
   const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes, n));
   const size_t per_block = (size_t)f.tile * kWavesPerBlock;
   const unsigned grid = gather_grid((n + per_block - 1) / per_block, max_blocks);
-  hipLaunchKernelGGL((gather_flat_kernel<Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src, src_rows,
-                     (char *)out, out_rows, f, counts, group, n, status, host_mirror, request.take(grid));
+  const DoneWords done = request.take(grid);
+  if (done.tag)
+    hipLaunchKernelGGL((gather_flat_kernel<kThrough, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,
+                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, done);
+  else
+    hipLaunchKernelGGL((gather_flat_kernel<kOrdinary, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,
+                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, done);
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -596,16 +595,16 @@ int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t 
   const unsigned grid = gather_grid((f.total + per_block - 1) / per_block, max_blocks);
   const bool nt = nt_store_for(n * row_bytes);
   const DoneWords done = nt ? DoneWords{} : request.take(grid);
-#define UGK_GO(NT, SHARE)                                                                                             \
-  hipLaunchKernelGGL((gather_stream_kernel<NT, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,                \
+#define UGK_GO(STORE, SHARE)                                                                                          \
+  hipLaunchKernelGGL((gather_stream_kernel<STORE, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,             \
                      (const char *)src, src_rows, (char *)out, f, status, host_mirror, done)
-  if (row_bytes % 16 == 0) {
-    if (nt) UGK_GO(true, false);
-    else UGK_GO(false, false);
-  } else {
-    if (nt) UGK_GO(true, true);
-    else UGK_GO(false, true);
-  }
+  const bool share = row_bytes % 16 != 0;
+  if (done.tag && share) UGK_GO(kThrough, true);
+  else if (done.tag) UGK_GO(kThrough, false);
+  else if (nt && share) UGK_GO(kStreaming, true);
+  else if (nt) UGK_GO(kStreaming, false);
+  else if (share) UGK_GO(kOrdinary, true);
+  else UGK_GO(kOrdinary, false);
 #undef UGK_GO
   UGK_HIP(hipGetLastError());
   return 0;

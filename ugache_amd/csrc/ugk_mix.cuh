@@ -30,20 +30,26 @@ __device__ __forceinline__ void store_through(uint64_t to, V v) {
   else asm volatile("global_store_byte %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"((uint32_t)v) : "memory");
 }
 
+// how a kernel stores its rows: a template parameter, not a launch argument, for with a run-time choice the optimiser merges
+// an ordinary and a non-temporal store into one and the hint is lost, and the code of all of them costs a small launch
+// 0.2 to 0.4 us (26,624 rows of 64 bytes 3.6 -> 4.0)
+enum Store { kOrdinary, kStreaming, kThrough };
+
 // key i of the launch, where the host wants a copy (a lane per key: neighbouring lanes' keys leave as one write)
 template <typename K>
 __device__ __forceinline__ void copy_key_along(const DoneWords &done, uint64_t i, K key) {
   if (i < done.num_keys) static_cast<K *>(done.keys)[i] = key;
 }
 
-// The last thing a workgroup does: its counts, and with a tag the news that it has ended.  All threads call it; tot (in LDS,
+// The last thing a workgroup does: its counts, and where a host polls the news that it has ended.  All threads call it; tot (in LDS,
 // may be NULL) holds the rows taken from the cache and all others.
+template <bool POLLED>
 __device__ __forceinline__ void leave_done(const DoneWords &done, const uint32_t *tot) {
-  if (done.tag) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have been acknowledged
+  if constexpr (POLLED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have been acknowledged
   __syncthreads();
   if (threadIdx.x != 0) return;
   const uint32_t local = tot ? tot[0] : 0u, others = tot ? tot[1] : 0u;
-  if (done.tag == 0) {
+  if constexpr (!POLLED) {
     done.words[blockIdx.x] = ((unsigned long long)others << 32) | local;
     return;
   }
@@ -108,9 +114,9 @@ static inline FlatRow flat_row(size_t row_bytes, uint32_t tile) {
 // Copies the rows r0 .. r0 + count - 1 of the wavefront, count <= f.tile: lane r holds where row r is read (kNoRowBit:
 // not at all) and, with DENSE false, which output row it becomes; with DENSE row r becomes output row d0 + r.  All
 // lanes call it with the same r0 and count.
-template <bool DENSE>
+template <bool DENSE, bool THROUGH>
 __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, char *out, size_t d0, uint32_t r0,
-                                          uint32_t count, const FlatRow &f, bool through) {
+                                          uint32_t count, const FlatRow &f) {
   constexpr int U = 4;  // vectors in flight per lane
   const uint32_t total = count * f.chunks;
   const uint32_t tail = f.row_bytes - 16;
@@ -134,15 +140,12 @@ __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, c
     u32x4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
-    if (through) {
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (ok[u]) store_through(reinterpret_cast<uint64_t>(q[u]), v[u]);
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (ok[u]) *q[u] = v[u];
-    }
+    for (int u = 0; u < U; ++u)
+      if (ok[u]) {
+        if constexpr (THROUGH) store_through(reinterpret_cast<uint64_t>(q[u]), v[u]);
+        else *q[u] = v[u];
+      }
   }
 }
 
@@ -188,13 +191,14 @@ __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key
 // result tells the last workgroup still 5 us (every workgroup ends by waiting for the round trip), and a device-scope
 // fence per workgroup 13-49 % of a whole step (each writes back and invalidates the L2 of its XCD).
 // (A launch that a host polls for waits for its stores anyway, and adds its workgroups up in a few counters: leave_done.)
+template <bool POLLED>
 __device__ __forceinline__ void mix_leave_counts(uint32_t *block_tot, uint32_t wave_local, uint32_t wave_host,
                                                  const DoneWords &done) {
   if (lane_id() == 0) {
     if (wave_local) atomicAdd(&block_tot[0], wave_local);
     if (wave_host) atomicAdd(&block_tot[1], wave_host);
   }
-  leave_done(done, block_tot);
+  leave_done<POLLED>(done, block_tot);
 }
 
 }  // namespace

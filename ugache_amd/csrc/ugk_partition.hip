@@ -163,9 +163,8 @@ __global__ __launch_bounds__(kBlock) void select_keys_kernel(const K *__restrict
 // that workgroups started in order write.
 // the rows of one wavefront's KPW keys, lane l holding the address of key b0 + l's row
 // stage_bits (STAGE only): where the lane's row is filed as well, 0 for a row that is not
-template <int LPR, int KPW, bool NT_STORE, bool STAGE>
-__device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits, u32x4 *out, size_t b0, uint32_t vpr,
-                                         bool through) {
+template <int LPR, int KPW, Store STORE, bool STAGE>
+__device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits, u32x4 *out, size_t b0, uint32_t vpr) {
   constexpr int RPW = kWave / LPR;  // rows per wavefront instruction
   constexpr int UNROLL = (RPW * 4 <= KPW) ? 4 : (KPW / RPW);
   static_assert(KPW <= kWave && KPW % (RPW * UNROLL) == 0, "keys per wavefront must be whole rounds of rows");
@@ -190,28 +189,21 @@ __device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits,
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) v[u] = __builtin_nontemporal_load(p[u] + col);
         const gout_t dst = (gout_t)out + (b0 + r0 + rg) * vpr + col;
-        if (!NT_STORE && through) {
 #pragma unroll
-          for (int u = 0; u < UNROLL; ++u)
-            if (ok[u]) store_through(reinterpret_cast<uint64_t>(dst + (size_t)u * RPW * vpr), v[u]);
-          if constexpr (STAGE) {
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
-              if (ps[u]) store_through(reinterpret_cast<uint64_t>(ps[u] + col), v[u]);
+        for (int u = 0; u < UNROLL; ++u)
+          if (ok[u]) {
+            const gout_t to = dst + (size_t)u * RPW * vpr;
+            if constexpr (STORE == kThrough) store_through(reinterpret_cast<uint64_t>(to), v[u]);
+            else if constexpr (STORE == kStreaming) __builtin_nontemporal_store(v[u], to);
+            else *to = v[u];
           }
-        } else {
+        if constexpr (STAGE) {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
-            if (ok[u]) {
-              // a template parameter: the two stores of a run-time choice get merged and lose the hint
-              if constexpr (NT_STORE) __builtin_nontemporal_store(v[u], dst + (size_t)u * RPW * vpr);
-              else dst[(size_t)u * RPW * vpr] = v[u];
+            if (ps[u]) {
+              if constexpr (STORE == kThrough) store_through(reinterpret_cast<uint64_t>(ps[u] + col), v[u]);
+              else ps[u][col] = v[u];
             }
-          if constexpr (STAGE) {
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
-              if (ps[u]) ps[u][col] = v[u];
-          }
         }
       }
     }
@@ -236,7 +228,7 @@ __device__ __forceinline__ uint64_t stage_claim(const ugk_stage_t &stage, const 
 }
 
 // LPR: lanes per row, or 0 for rows that are copied flat (flat_copy; f.tile rows at a time)
-template <typename K, int KIND, int LPR, int KPW, bool NT_STORE, bool STAGE>
+template <typename K, int KIND, int LPR, int KPW, Store STORE, bool STAGE>
 __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, const K *__restrict__ keys, size_t n,
                                                              const void *__restrict__ cache, uint64_t cache_rows,
                                                              const void *__restrict__ host, uint64_t host_rows,
@@ -254,7 +246,6 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
     const size_t i = b0 + lane;
     const bool active = lane < KPW && i < n;
     const uint64_t key = active ? key_to_u64<K>(keys[i]) : 0;
-    if (active) copy_key_along<K>(done, i, (K)key);
     // a full wavefront of keys probes its eight home lines in one go (see hash_probe_home)
     // (fewer keys: their home lines in one go as well, and only the rounds of the probe that have keys to serve)
     constexpr int ROUNDS = KPW >= 8 ? KPW / 8 : 1;
@@ -273,17 +264,19 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       const uint64_t bits = row.has_row ? row.bits : row.bits | kNoRowBit;
       const uint32_t here = (uint32_t)min((size_t)KPW, n - b0);
       for (uint32_t r0 = 0; r0 < here; r0 += f_row.tile)
-        flat_copy<true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row,
-                        done.tag != 0);
+        flat_copy<true, STORE == kThrough>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
     } else {
       const uint32_t vpr = f_row.chunks;
       uint64_t stage_bits = 0;
       if constexpr (STAGE) stage_bits = stage_claim(stage, row, vpr);
-      mix_copy<LPR, KPW, NT_STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr,
-                                          done.tag != 0);
+      mix_copy<LPR, KPW, STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
+    }
+    // behind the rows: in front of them it would be in the way of the lookup
+    if constexpr (STORE == kThrough) {
+      if (active) copy_key_along<K>(done, i, (K)key);
     }
   }
-  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
+  if (done.words) mix_leave_counts<STORE == kThrough>(block_tot, wave_local, wave_host, done);
 }
 
 // ---- dedup -----------------------------------------------------------------------------------------------
@@ -587,10 +580,16 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
     if (stage) UGK_GO4(L, W, NT, true); \
     else UGK_GO4(L, W, NT, false);      \
   } while (0)
-#define UGK_GO2(L, W)         \
-  do {                        \
-    if (nt) UGK_GO3(L, W, true); \
-    else UGK_GO3(L, W, false);   \
+#define UGK_GO2(L, W)                          \
+  do {                                         \
+    if (done.tag) UGK_GO3(L, W, kThrough);     \
+    else if (nt) UGK_GO3(L, W, kStreaming);    \
+    else UGK_GO3(L, W, kOrdinary);             \
+  } while (0)
+#define UGK_FLAT(W)                                   \
+  do {                                                \
+    if (done.tag) UGK_GO4(0, W, kThrough, false);     \
+    else UGK_GO4(0, W, kOrdinary, false);             \
   } while (0)
 #define UGK_GO(L)                                   \
   do {                                              \
@@ -615,10 +614,10 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
     UGK_GO2(L, kWave);                              \
   } while (0)
   if (flat) {  // ordinary stores whatever the size (see flat_copy)
-    if (kpw == 8) UGK_GO4(0, 8, false, false);
-    else if (kpw == 16) UGK_GO4(0, 16, false, false);
-    else if (kpw == 32) UGK_GO4(0, 32, false, false);
-    else UGK_GO4(0, kWave, false, false);
+    if (kpw == 8) UGK_FLAT(8);
+    else if (kpw == 16) UGK_FLAT(16);
+    else if (kpw == 32) UGK_FLAT(32);
+    else UGK_FLAT(kWave);
   } else if (vpr <= 1) UGK_GO2(1, kWave);
   else if (vpr <= 2) UGK_GO(2);
   else if (vpr <= 4) UGK_GO(4);
@@ -630,6 +629,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
 #undef UGK_GO2
 #undef UGK_GO3
 #undef UGK_GO4
+#undef UGK_FLAT
   UGK_HIP(hipGetLastError());
   return 0;
 }

@@ -140,7 +140,6 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
       const long long j = j0 + sub;
       const bool active = j < end;
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
-      if (active) copy_key_along<K>(done, (uint64_t)j, (K)key);
       const Found f = table_lookup<KIND>(t, key, active);
       const MixRow row = mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
       if (done.words) {
@@ -224,6 +223,7 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
           }
         }
       }
+      if (active) copy_key_along<K>(done, (uint64_t)j, (K)key);
       // (behind the rows: in front of them their loads would wait for the weights)
       const float wterm = combiner == 2 ? w * w : w;
       if constexpr (LPR < kParts) {
@@ -285,7 +285,8 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
     pool_samples<K, KIND, LPR, CH, U, E, CLIP, false>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host,
                                                       host_rows, out, vpr, combiner, bf16, max_norm, status, host_mirror,
                                                       done, wave_local, wave_host);
-  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
+  if (done.tag) mix_leave_counts<true>(block_tot, wave_local, wave_host, done);
+  else if (done.words) mix_leave_counts<false>(block_tot, wave_local, wave_host, done);
 }
 
 constexpr int kPoolMaxRows = 8;  // output rows a lane group may own per pass
@@ -309,7 +310,7 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
                                                    uint64_t cache_rows, const u32x4 *__restrict__ host,
                                                    uint64_t host_rows, u32x4 *__restrict__ out, uint32_t vpr,
                                                    int combiner, bool bf16, uint32_t *status, uint32_t *host_mirror,
-                                                   const DoneWords &done, uint32_t &wave_local,
+                                                   const unsigned long long *counts, uint32_t &wave_local,
                                                    uint32_t &wave_host,
                                                    long long (&seg_beg)[kWavesPerBlock][kWave / LPR][kPoolMaxRows],
                                                    uint32_t (&seg_start)[kWavesPerBlock][kWave / LPR][kPoolMaxRows]) {
@@ -368,9 +369,7 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
       float y[EPC];
 #pragma unroll
       for (int e = 0; e < EPC; ++e) y[e] = denom != 0.f ? acc[c][e] / denom : 0.f, acc[c][e] = 0.f;
-      const u32x4 packed = PoolElem<E>::pack(y, bf16);
-      if (done.tag) store_through(reinterpret_cast<uint64_t>(out + (g0 + k) * vpr + col), packed);
-      else out[(g0 + k) * vpr + col] = packed;
+      out[(g0 + k) * vpr + col] = PoolElem<E>::pack(y, bf16);
     };
     for (uint32_t f0 = 0; __ballot(f0 < total) != 0ull; f0 += LPR) {  // until every group of the wavefront is through
       const uint32_t f = f0 + sub;
@@ -382,10 +381,9 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
       }
       const long long j = active ? my_beg[k] + (long long)(f - my_start[k]) : 0;
       const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
-      if (active) copy_key_along<K>(done, (uint64_t)j, (K)key);
       const Found fd = table_lookup<KIND>(t, key, active);
       const MixRow row = mix_resolve(t, key, active, fd, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
-      if (done.words) {
+      if (counts) {
         wave_local += __popcll(__ballot(row.from_cache));
         wave_host += __popcll(__ballot(active && !row.from_cache));
       }
@@ -460,7 +458,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
                                                               const u32x4 *__restrict__ host, uint64_t host_rows,
                                                               u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
                                                               uint32_t *status, uint32_t *host_mirror,
-                                                              DoneWords done, uint32_t keep_waves) {
+                                                              unsigned long long *counts, uint32_t keep_waves) {
   __shared__ uint32_t block_tot[2];
   __shared__ long long seg_beg[kWavesPerBlock][kWave / LPR][kPoolMaxRows];    // first id of the group's row k
   __shared__ uint32_t seg_start[kWavesPerBlock][kWave / LPR][kPoolMaxRows];   // its first position in the group's list
@@ -469,13 +467,13 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
   uint32_t wave_local = 0, wave_host = 0;
   if (!MIXED || wave_in_block() < keep_waves)
     pool_short_samples<K, KIND, LPR, E, true>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
-                                              host, host_rows, out, vpr, combiner, bf16, status, host_mirror, done,
+                                              host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
                                               wave_local, wave_host, seg_beg, seg_start);
   else if constexpr (MIXED)
     pool_short_samples<K, KIND, LPR, E, false>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
-                                               host, host_rows, out, vpr, combiner, bf16, status, host_mirror, done,
+                                               host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
                                                wave_local, wave_host, seg_beg, seg_start);
-  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
+  if (counts) mix_leave_counts<false>(block_tot, wave_local, wave_host, DoneWords{counts, nullptr, nullptr, 0, 0});
 }
 
 template <typename K, int KIND, typename E>
@@ -547,7 +545,8 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   // of whole lines up to 384 bytes.  The other fp32 rows are faster one by one, 800,000 samples (400,000 from 640 bytes
   // on) uniform and Zipf 1.05, list / one by one: 64 bytes 54 / 37 and 48 / 31, 160 bytes 95 / 81 and 81 / 72, 400 bytes
   // 239 / 165 and 186 / 167, 512 bytes 179 / 169 and 169 / 162, 1 KB 184 / 165 and 183 / 164, 2 KB 329 / 322 and 318 / 318.
-  // (an output that does not fit the memory-side cache is not written through: 131,072 samples of one id of 2 KB 120 -> 122 us)
+  // (an output that does not fit the memory-side cache is not written through: 131,072 samples of one id of 2 KB 120 -> 122 us;
+  // nor does the list kernel below leave words: the choice of stores where it writes a row cost it a quarter of its speed)
   const uint64_t polled_nnz = n_rows * (size_t)vpr * 16 <= kMemorySideCacheBytes ? nnz : ~0ull;
   int rows = 1;
   if constexpr (KIND != 1) {
@@ -565,9 +564,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
     if (rows > 1) {
       const size_t rows_per_block = (size_t)rows * groups * kWavesPerBlock;
       const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
-      DoneWords done = request.take(grid, polled_nnz);
-      if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
-      if (num_groups) *num_groups = done.tag ? 0 : grid;
+      if (num_groups) *num_groups = grid;
       // (256 bytes uniform and Zipf 1.05, before / without the hint / one wavefront of four without: 90 / 101 / 91 and
       // 102 / 91 / 91)
       constexpr bool kMixed = KIND == 0 && sizeof(E) == 4;
@@ -576,7 +573,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   hipLaunchKernelGGL((extract_pool_rows_kernel<K, KIND, L, E, kMixed>), dim3(grid), dim3(kBlock), 0, st, t, ids,       \
                      seg_off, weights, n_rows, (long long)nnz, rows, (const u32x4 *)cache, cache_rows,                 \
                      (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, status, host_mirror,           \
-                     done, keep)
+                     reinterpret_cast<unsigned long long *>(counts), keep)
       if (lanes == 8) UGK_POOL_ROWS_GO(8);
       else if (lanes == 32) UGK_POOL_ROWS_GO(32);
       else UGK_POOL_ROWS_GO(64);
