@@ -831,20 +831,26 @@ class _DoneWords:
         self.words.array[:] = 0
         self.counters = torch.zeros(64 * 16, dtype=torch.int64, device="cuda")
         self.keys = PinnedArray((4_096,), np.int64)
+        self.mirror = PinnedArray((16,), np.uint32)
         self.done = hip.Done(self.words.ptr, ptr(self.counters), 0, 0, self.keys.ptr, 0)
 
     def ask(self, num_keys):
         """the first num_keys keys of the launch are wanted too"""
         self.keys.array[:] = -7
         self.done.num_keys, self.done.tag = min(num_keys, 4_096), self.done.tag + 1
+        self.mirror.array[:] = 0
         hip.call("ugk_leave_done_words", C.byref(self.done))
+
+    def check_flag(self, flag):
+        """as soon as the words are there: the error flag is too"""
+        assert self.mirror.array[0] == flag
 
     def check_keys(self, keys):
         """they came, all of them and nothing behind them"""
         n = self.done.num_keys
         assert (self.keys.array[:n] == keys[:n]).all() and (self.keys.array[n:] == -7).all()
 
-    def run(self, launch, spin_us, groups, num_keys=0):
+    def run(self, launch, spin_us, groups, num_keys=0, flag=0):
         self.ask(num_keys)
         launch()
         if groups is None:
@@ -854,6 +860,7 @@ class _DoneWords:
         assert self.done.num_words == (groups if groups <= 256 else 64)
         local, others = C.c_uint64(), C.c_uint64()
         hip.call("ugk_done_wait", C.byref(self.done), spin_us, None, C.byref(local), C.byref(others))
+        self.check_flag(flag)
         sync()
         assert not self.counters.any().item()
         return local.value, others.value
@@ -880,20 +887,22 @@ def test_gather_that_tells_its_end_by_words(row_bytes, rows_per_group, spin_us):
         sync()
 
         def launch():
-            hip.call("ugk_gather_direct_i64", ptr(table), rows, ptr(q), n, ptr(out), row_bytes, 0, ptr(st), None, None)
+            hip.call("ugk_gather_direct_i64", ptr(table), rows, ptr(q), n, ptr(out), row_bytes, 0, ptr(st), done.mirror.ptr, None)
 
         wanted = (0, 1, n // 2 + 1, n, n // 20)[groups % 5]
+        flag = hip.ST_KEY_OUT_OF_RANGE if n > 4 else 0
         if rows_per_group:
-            assert done.run(launch, spin_us, groups, wanted) == (0, 0)
+            assert done.run(launch, spin_us, groups, wanted, flag) == (0, 0)
         else:  # the number of workgroups is the kernel's own affair
             done.ask(wanted)
             launch()
             assert done.done.num_words > 0
             hip.call("ugk_done_wait", C.byref(done.done), spin_us, None, None, None)
+            done.check_flag(flag)
             assert not done.counters.any().item()
-        assert torch.equal(out, want)
         done.check_keys(to_np(q))
-        assert status_value(st) == (hip.ST_KEY_OUT_OF_RANGE if n > 4 else 0)
+        assert torch.equal(out, want)
+        assert status_value(st) == flag
     # the request met one call: the next one leaves nothing; and streaming outputs are waited for in another way
     before = done.words.array.copy()
     launch()

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
     const uint32_t c = counts[group];
     count = c;
     begin = (group == UGK_LOC_LOCAL) ? 0 : n - c;
-    if (host_mirror && blockIdx.x == 0 && threadIdx.x == 0) host_mirror[1 + group] = c;
+    if (host_mirror && blockIdx.x == 0 && threadIdx.x == 0) tell_host(host_mirror + 1 + group, c);
   }
   constexpr int RPB = kBlock / LPR;  // rows copied by one block instruction
   const uint32_t lane = threadIdx.x % LPR;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
         ok[u] = false;
         if (lane == 0) {
           atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
-          if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
+          if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_KEY_OUT_OF_RANGE);
         }
       }
     }
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
     const uint32_t c = counts[group];
     count = c;
     begin = (group == UGK_LOC_LOCAL) ? 0 : n - c;
-    if (host_mirror && blockIdx.x == 0 && threadIdx.x == 0) host_mirror[1 + group] = c;
+    if (host_mirror && blockIdx.x == 0 && threadIdx.x == 0) tell_host(host_mirror + 1 + group, c);
   }
   const size_t wave = (size_t)blockIdx.x * kWavesPerBlock + wave_in_block();
   const size_t stride = (size_t)gridDim.x * kWavesPerBlock * f.tile;
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
     if (ok && (s >= src_rows || d >= out_rows)) {
       ok = false;
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
-      if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
+      if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_KEY_OUT_OF_RANGE);
     }
     const unsigned long long good = __ballot(ok);
     if (good != 0ull) {
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     if (ok && s >= src_rows) {
       ok = false;
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
-      if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
+      if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_KEY_OUT_OF_RANGE);
     }
     const unsigned long long good = __ballot(ok);
     if (good == 0ull) {

@@ -35,10 +35,18 @@ __device__ __forceinline__ void store_through(uint64_t to, V v) {
 // 0.2 to 0.4 us (26,624 rows of 64 bytes 3.6 -> 4.0)
 enum Store { kOrdinary, kStreaming, kThrough };
 
+// A word for the host beside the rows (an error flag, a key).  The same kind of store: an ordinary one into host memory is
+// acknowledged before it is there, and the words of leave_done, which say that all of this is complete, may overtake it
+// (a lookup of four keys, one of them out of range, returned without its error that way).
+template <typename T>
+__device__ __forceinline__ void tell_host(T *word, T v) {
+  __hip_atomic_store(word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // key i of the launch, where the host wants a copy (a lane per key: neighbouring lanes' keys leave as one write)
 template <typename K>
 __device__ __forceinline__ void copy_key_along(const DoneWords &done, uint64_t i, K key) {
-  if (i < done.num_keys) static_cast<K *>(done.keys)[i] = key;
+  if (i < done.num_keys) tell_host(static_cast<K *>(done.keys) + i, key);
 }
 
 // The last thing a workgroup does: its counts, and where a host polls the news that it has ended.  All threads call it; tot (in LDS,
@@ -170,7 +178,7 @@ __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key
     else if (!f.hit && fallback_row(t, key) < host_rows) host_row = fallback_row(t, key);
     else {
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
-      if (host_mirror) host_mirror[0] = UGK_ST_KEY_OUT_OF_RANGE;
+      if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_KEY_OUT_OF_RANGE);
     }
   }
   // A key without a row copies nothing; its lanes read the head of the output instead (mapped whatever the key), so

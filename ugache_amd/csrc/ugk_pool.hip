@@ -116,14 +116,14 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
     if (beg < 0 || end > nnz || end < beg) {  // a segment outside the ids: nothing is read for it, its row is zeros
       if (sub == 0) {
         atomicOr(status, UGK_ST_BAD_SEGMENT);
-        if (host_mirror) host_mirror[0] = UGK_ST_BAD_SEGMENT;
+        if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_BAD_SEGMENT);
       }
       beg = end = 0;
     } else if (row_ok && sub == 0 && ((r == 0 && beg != 0) || (r + 1 == n_rows && end != nnz))) {
       // the offsets do not cover the ids from the first to the last (neighbouring segments share their boundary word,
       // so the two ends are all that can be wrong): the per-source id counts would not add up to nnz
       atomicOr(status, UGK_ST_BAD_SEGMENT);
-      if (host_mirror) host_mirror[0] = UGK_ST_BAD_SEGMENT;
+      if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_BAD_SEGMENT);
     }
     float acc[CH][EPC];
 #pragma unroll
@@ -336,12 +336,12 @@ __device__ __forceinline__ void pool_short_samples(const ugk_table_t &t, const K
       // bits; the launcher keeps batches of 2^28 ids and more away from this kernel, so the last test never fires.)
       if (b < 0 || e > nnz || e < b || e - b >= (1ll << 28)) {
         atomicOr(status, UGK_ST_BAD_SEGMENT);
-        if (host_mirror) host_mirror[0] = UGK_ST_BAD_SEGMENT;
+        if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_BAD_SEGMENT);
       } else {
         beg = b, len = (uint32_t)(e - b);
         if ((g0 + sub == 0 && b != 0) || (g0 + sub + 1 == n_rows && e != nnz)) {  // the ids are not covered end to end
           atomicOr(status, UGK_ST_BAD_SEGMENT);
-          if (host_mirror) host_mirror[0] = UGK_ST_BAD_SEGMENT;
+          if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_BAD_SEGMENT);
         }
       }
     }
@@ -646,7 +646,7 @@ __global__ __launch_bounds__(kBlock) void segment_offsets_kernel(const long long
       if (cur < prev || cur < 0 || (i > 0 && prev < 0) || (i < nnz && cur >= (long long)n_rows) ||
           prev >= (long long)n_rows) {
         if (status) atomicOr(status, UGK_ST_BAD_SEGMENT);
-        if (host_mirror) host_mirror[0] = UGK_ST_BAD_SEGMENT;
+        if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_BAD_SEGMENT);
         prev = 0, cur = -1;
       }
     }
