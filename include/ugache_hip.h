@@ -103,7 +103,7 @@ typedef struct {
 const char *ugk_last_error(void);
 /* version of this ABI; bumped on any signature change.  ugk_abi_version() is what the loaded library was built with:
  * a caller compiled against another UGK_ABI_VERSION must not go on. */
-#define UGK_ABI_VERSION 23
+#define UGK_ABI_VERSION 24
 int ugk_abi_version(void);
 
 /* ---- runtime plumbing: Device::{AllocDataSpace,FreeDataSpace,CopyDataFromTo,StreamSync,CreateStream}
@@ -154,9 +154,10 @@ int ugk_word_wait(const uint32_t *word_host, uint32_t value, unsigned spin_us, v
  * stores have been acknowledged; so is everything enqueued in front of it.
  * words_host: UGK_DONE_WORDS words of pinned, GPU-mapped memory (ugk_host_malloc); tag: differs from call to call until
  * the words are cleared (no launch may be using them then); counters_dev: UGK_DONE_COUNTERS * 16 8-byte device words that
- * are zero before the first launch (and are left so by every launch).  Neither is shared by launches in flight together. */
+ * are zero before the first launch: two sets of counters that launches take in turn (counter_set), each of which clears the
+ * other's for the next.  Neither is shared by launches in flight together. */
 #define UGK_DONE_WORDS 256
-#define UGK_DONE_COUNTERS 64
+#define UGK_DONE_COUNTERS 128
 #define UGK_DONE_MAX_TAG 0xffffu
 typedef struct {
   uint64_t *words_host;
@@ -165,6 +166,8 @@ typedef struct {
   uint32_t num_words; /* set by the launch */
   void *keys_host;    /* pinned: a launch with words leaves its first num_keys keys there, complete as its rows are */
   uint64_t num_keys;  /* 0: none */
+  uint32_t counter_set; /* 0 before the first launch, kept by the launches from then on */
+  uint32_t reserved;
 } ugk_done_t;
 int ugk_leave_done_words(ugk_done_t *done);
 int ugk_done_wait(const ugk_done_t *done, unsigned spin_us, void *stream, uint64_t *local, uint64_t *others);

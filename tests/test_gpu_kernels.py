@@ -824,15 +824,15 @@ def _extract_mix(fn, tb, keys_dev, n, cache_dev, cache_rows, pin, host_rows, out
 
 
 class _DoneWords:
-    """the words and counters of ugk_leave_done_words, and the check that a launch leaves the counters at zero"""
+    """the words and counters of ugk_leave_done_words, and the check that a launch leaves the next one's counters at zero"""
 
     def __init__(self):
         self.words = PinnedArray((256,), np.uint64)
         self.words.array[:] = 0
-        self.counters = torch.zeros(64 * 16, dtype=torch.int64, device="cuda")
+        self.counters = torch.zeros((2, 64 * 16), dtype=torch.int64, device="cuda")
         self.keys = PinnedArray((4_096,), np.int64)
         self.mirror = PinnedArray((16,), np.uint32)
-        self.done = hip.Done(self.words.ptr, ptr(self.counters), 0, 0, self.keys.ptr, 0)
+        self.done = hip.Done(self.words.ptr, ptr(self.counters), 0, 0, self.keys.ptr, 0, 0, 0)
 
     def ask(self, num_keys):
         """the first num_keys keys of the launch are wanted too"""
@@ -861,9 +861,14 @@ class _DoneWords:
         local, others = C.c_uint64(), C.c_uint64()
         hip.call("ugk_done_wait", C.byref(self.done), spin_us, None, C.byref(local), C.byref(others))
         self.check_flag(flag)
-        sync()
-        assert not self.counters.any().item()
+        self.check_counters()
         return local.value, others.value
+
+    def check_counters(self):
+        """no wait for the launch in front of it: the words say that what it cleared is zero"""
+        other = torch.cuda.Stream()
+        with torch.cuda.stream(other):
+            assert not self.counters[self.done.counter_set ^ 1].any().item()
 
 
 # gathers of one workgroup, of the most that leave a word each, of one more, of as many as make some counters one longer than
@@ -899,7 +904,7 @@ def test_gather_that_tells_its_end_by_words(row_bytes, rows_per_group, spin_us):
             assert done.done.num_words > 0
             hip.call("ugk_done_wait", C.byref(done.done), spin_us, None, None, None)
             done.check_flag(flag)
-            assert not done.counters.any().item()
+            done.check_counters()
         done.check_keys(to_np(q))
         assert torch.equal(out, want)
         assert status_value(st) == flag
@@ -954,7 +959,7 @@ def test_fused_and_pooled_lookups_that_tell_their_end_by_words(kind, rb, stage):
         assert (local.value, others.value) == (in_cache[keys].sum(), (~in_cache[keys]).sum())
         done.check_keys(keys)
         assert torch.equal(out[: n * rb].view(n, rb), d_table[torch.from_numpy(keys).cuda()])
-        assert not done.counters.any().item()
+        done.check_counters()
         if rb % 16 == 0 and not stage:
             per = 3 if n > 3 else 1
             n_rows = n // per

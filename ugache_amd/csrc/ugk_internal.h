@@ -62,6 +62,7 @@ struct DoneWords {
   void *keys;         // the launch leaves its first num_keys keys here (pinned host memory)
   uint64_t num_keys;
   uint32_t tag;
+  uint32_t set;       // which of the two sets of counters
 };
 // Up to kDoneDirect workgroups leave a word each.  More of them meet in kDoneFan counters, workgroup b in counter b %
 // kDoneFan, and the last one of a counter leaves its word: writes into host memory cost 2 us per thousand, and a host that
@@ -69,7 +70,7 @@ struct DoneWords {
 // 256 / 512 / 1024 counters 48.6 / 48.7 / 49.0 / 49.3 / 49.7 / 50.8 us, a word per workgroup (16,384) 53.0, one-lane ticket
 // kernel behind the gather 52.0; 8,192 rows (512 workgroups) 8.9 / 8.8 / 9.0 / 9.3 / 9.2 / 9.2, 9.1 and 9.8; 1,664 rows 8.4 /
 // 8.6 / 8.2 / 8.2 / 8.1 / 8.1, 8.0 and 9.4; 8 rows 6.3 against 8.5.
-constexpr uint32_t kDoneDirect = UGK_DONE_WORDS, kDoneFan = UGK_DONE_COUNTERS;
+constexpr uint32_t kDoneDirect = UGK_DONE_WORDS, kDoneFan = UGK_DONE_COUNTERS / 2;
 
 // The request of ugk_leave_done_words, if this thread has made one: the entry points that can fulfil it take it as they
 // begin, so that it never meets a later launch.

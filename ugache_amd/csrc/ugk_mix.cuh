@@ -53,7 +53,15 @@ __device__ __forceinline__ void copy_key_along(const DoneWords &done, uint64_t i
 // may be NULL) holds the rows taken from the cache and all others.
 template <bool POLLED>
 __device__ __forceinline__ void leave_done(const DoneWords &done, const uint32_t *tot) {
-  if constexpr (POLLED) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have been acknowledged
+  if constexpr (POLLED) {
+    // The set of counters this launch does not use is made zero for the next one, in front of the wait: once all words are
+    // there that is complete, also for a launch on another stream, which does not wait for this one to end.  (A counter
+    // cleared by the workgroup that finds it complete would need a wait between that and its word.)
+    if (gridDim.x > kDoneDirect && blockIdx.x < kDoneFan && threadIdx.x == 0)
+      __hip_atomic_store(done.counters + ((done.set ^ 1u) * kDoneFan + blockIdx.x) * 16, 0ull, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have been acknowledged
+  }
   __syncthreads();
   if (threadIdx.x != 0) return;
   const uint32_t local = tot ? tot[0] : 0u, others = tot ? tot[1] : 0u;
@@ -68,14 +76,10 @@ __device__ __forceinline__ void leave_done(const DoneWords &done, const uint32_t
   }
   const uint32_t g = blockIdx.x % kDoneFan, members = gridDim.x / kDoneFan + (g < gridDim.x % kDoneFan ? 1u : 0u);
   const unsigned long long add = (1ull << 48) | mine;
-  unsigned long long *counter = done.counters + g * 16;  // a line each
+  unsigned long long *counter = done.counters + (done.set * kDoneFan + g) * 16;  // a line each
   const unsigned long long sum =
       __hip_atomic_fetch_add(counter, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
-  if ((uint32_t)(sum >> 48) == members) {
-    // zero again for the next launch, which does not start before this one has ended
-    __hip_atomic_store(counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    done.words[g] = tag | (sum & 0xffffffffffffull);
-  }
+  if ((uint32_t)(sum >> 48) == members) done.words[g] = tag | (sum & 0xffffffffffffull);
 }
 
 // ---- flat row copy -------------------------------------------------------------------------------------------------

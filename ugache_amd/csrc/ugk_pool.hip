@@ -473,7 +473,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
     pool_short_samples<K, KIND, LPR, E, false>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
                                                host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
                                                wave_local, wave_host, seg_beg, seg_start);
-  if (counts) mix_leave_counts<false>(block_tot, wave_local, wave_host, DoneWords{counts, nullptr, nullptr, 0, 0});
+  if (counts) mix_leave_counts<false>(block_tot, wave_local, wave_host, DoneWords{counts, nullptr, nullptr, 0, 0, 0});
 }
 
 template <typename K, int KIND, typename E>

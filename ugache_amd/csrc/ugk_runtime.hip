@@ -41,8 +41,10 @@ DoneWords DoneRequest::take(unsigned grid, uint64_t count_limit) {
   ugk_done_t *d = _done;
   _done = nullptr;
   d->num_words = grid <= kDoneDirect ? grid : kDoneFan;
+  if (grid > kDoneDirect) d->counter_set ^= 1u;
   return DoneWords{reinterpret_cast<unsigned long long *>(d->words_host),
-                   reinterpret_cast<unsigned long long *>(d->counters_dev), d->keys_host, d->num_keys, d->tag};
+                   reinterpret_cast<unsigned long long *>(d->counters_dev), d->keys_host, d->num_keys, d->tag,
+                   d->counter_set & 1u};
 }
 
 int blocks_per_cu() {
