@@ -554,8 +554,9 @@ int ugk_rank_place_keep(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, voi
 int ugk_rank_place_observed(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, void *ws_dev, uint64_t *in_new_dev,
                             uint64_t *observed_dev, int reset_counts, const uint64_t *cached_dev, void *evict_ws_dev,
                             void *insert_ws_dev, uint32_t *totals_host, uint32_t *status_dev, void *stream);
-/* the same with a ticket (non-zero; 0: none) in totals_host[3], a fourth pinned word: once it is there the sums are, and the
- * bitmap and the two workspaces may be read by launches on any stream (ugk_ticket_wait); cached_dev must not be NULL */
+/* the same with a ticket (non-zero; 0: none) in totals_host[3], a fourth pinned word, left by the last launch of the placement:
+ * once it is there the sums are, and the bitmap and the two workspaces may be read and written by launches on any stream
+ * (ugk_ticket_wait); cached_dev must not be NULL */
 int ugk_rank_place_observed_ticket(uint32_t *counts_dev, uint64_t num_rows, uint64_t k, void *ws_dev,
                                    uint64_t *in_new_dev, uint64_t *observed_dev, int reset_counts,
                                    const uint64_t *cached_dev, void *evict_ws_dev, void *insert_ws_dev,

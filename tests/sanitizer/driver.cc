@@ -133,6 +133,13 @@ int main(int argc, char **argv) {
       coll_cache_lookup_i64(0, k64.data(), k64.size(), out.data(), nullptr);
       bad_rows += check_rows(table, out.data(), k32.data(), k32.size());
       coll_cache_refresh(0, nullptr, /*foreground=*/1);
+      // ... and one for which fewer rows were observed than the cache holds, whose placement the host polls for; in the
+      // second round by the passes for long bitmaps (the model reports a list made in front of the scan it is made from)
+      ugk_model_small_bits(round == 0 ? (size_t)1 << 26 : 1024);
+      coll_cache_lookup(0, k32.data(), 1000, out.data(), nullptr);
+      coll_cache_refresh(0, nullptr, /*foreground=*/1);
+      coll_cache_lookup(0, k32.data(), k32.size(), out.data(), nullptr);
+      bad_rows += check_rows(table, out.data(), k32.data(), k32.size());
       const size_t nu = coll_cache_lookup_unique(0, k32.data(), k32.size(), out.data(), inverse.data(), nullptr);
       for (size_t i = 0; i < k32.size(); ++i)
         if (inverse[i] >= nu ||

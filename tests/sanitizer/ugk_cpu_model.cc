@@ -637,16 +637,24 @@ uint64_t bm_word(const uint64_t *a, const uint64_t *b, int invert_a, uint64_t nb
 //   - a stream or event that took part in a capture must not be destroyed while the recorded graph lives, and -- the
 //     rule of the library itself -- only the caller's stream takes part in the caller's capture: an event recorded or a
 //     second stream joined while capturing is reported even where the runtime would accept it.
+// Launches of a placement and of the lists made from it are numbered, and every stream, event and ticket knows per stream
+// which of them it stands behind: what one launch wrote another may read or write only where it is ordered behind it.
+typedef std::map<const void *, uint64_t> Clock;  // stream -> number of a launch on it
+void merge(Clock &into, const Clock &from) {
+  for (auto &kv : from) into[kv.first] = std::max(into[kv.first], kv.second);
+}
 struct Stream {
   int capture = 0;      // id of the capture this stream records into, 0: runs its work
   bool origin = false;  // the capture was begun on this stream
   void *join_event = nullptr;  // joined stream: the last event recorded on it
   bool joined_back = true;
+  Clock behind;                // per stream, the last launch that the next one on this stream is ordered behind
 };
 struct Event {
   std::chrono::steady_clock::time_point at;
   int captured_in = 0;  // id of the capture its last record went into, 0: recorded on a running stream
   Stream *recorded_on = nullptr;
+  Clock behind;
 };
 struct Graph {
   std::vector<Stream *> streams;
@@ -670,10 +678,36 @@ void violation(const char *fmt, ...) {
   va_end(ap);
   g_violations.emplace_back(buf);
 }
+uint64_t g_launches = 0;
+Clock g_host_behind;                              // what the host has waited for: what it launches next is behind it
+std::map<const uint32_t *, Clock> g_ticket_behind;  // a ticket's word -> what stands in front of it
+std::map<const void *, std::pair<Stream *, uint64_t>> g_written;  // buffer -> the launch that wrote it last
+uint64_t g_small_bits = (uint64_t)1 << 26;        // longer bitmaps: a placement ends with a scan of its own
+
 // caller holds g_rt_mu: the host has waited for `s` (null: for every stream)
 void note_stream_idle(Stream *s) {
   for (auto &kv : g_stage_writers)
     if (s == nullptr || kv.second.first == s) kv.second.second = false;
+  if (s) merge(g_host_behind, s->behind);
+  else for (auto &kv : g_written) g_host_behind[kv.second.first] = g_launches;
+}
+// a launch on `stream` that reads `in` and writes `out` (null pointers: nothing)
+void note_launch(void *stream, const char *what, std::initializer_list<const void *> in,
+                 std::initializer_list<const void *> out, const uint32_t *ticket = nullptr) {
+  std::lock_guard<std::mutex> g(g_rt_mu);
+  Stream *s = as_stream(stream);
+  merge(s->behind, g_host_behind);
+  for (auto *list : {&in, &out})
+    for (const void *p : *list) {
+      auto w = g_written.find(p);
+      if (w == g_written.end() || w->second.first == s) continue;
+      if (s->behind[w->second.first] < w->second.second)
+        violation("%s on a stream that is not ordered behind the launch on another stream that wrote its data", what);
+    }
+  s->behind[s] = ++g_launches;
+  for (const void *p : out)
+    if (p) g_written[p] = {s, g_launches};
+  if (ticket) g_ticket_behind[ticket] = s->behind;
 }
 void note_staged_launch(const ugk_stage_t &stage, void *stream) {
   std::lock_guard<std::mutex> g(g_rt_mu);
@@ -746,6 +780,11 @@ void ugk_model_reset(void) {
   g_violations.clear();
   g_graphs.clear();
   g_stage_writers.clear();
+  g_written.clear();
+}
+void ugk_model_small_bits(size_t nbits) {
+  std::lock_guard<std::mutex> g(g_rt_mu);
+  g_small_bits = nbits;
 }
 }
 
@@ -788,6 +827,13 @@ int ugk_malloc(void **ptr, size_t nbytes) {
 }
 int ugk_free(void *ptr) {
   if (ptr) note_allocation("device memory freed");
+  if (ptr) {
+    std::lock_guard<std::mutex> m(g_mem_mu), g(g_rt_mu);
+    auto block = g_blocks.find((uintptr_t)ptr);  // what is allocated there next has not been written
+    if (block != g_blocks.end())
+      g_written.erase(g_written.lower_bound(ptr),
+                      g_written.lower_bound(static_cast<char *>(ptr) + std::max<size_t>(block->second.first, 1)));
+  }
   return free_block(ptr, 2);
 }
 int ugk_host_malloc(void **ptr, size_t nbytes) {
@@ -825,6 +871,7 @@ int ugk_stream_destroy(void *stream) {
     for (auto &kv : g_graphs)
       for (auto &m : kv.second.streams)
         if (m == stream) m = nullptr;
+    for (auto it = g_written.begin(); it != g_written.end();) it = it->second.first == stream ? g_written.erase(it) : std::next(it);
   }
   delete static_cast<Stream *>(stream);
   return 0;
@@ -854,7 +901,7 @@ int ugk_ticket_wait(const uint32_t *ticket_host, uint32_t value, unsigned, void 
   REQUIRE(ticket_host && *ticket_host == value, "ugk_ticket_wait: nobody has written the ticket");
   std::lock_guard<std::mutex> g(g_rt_mu);
   if (as_stream(stream)->capture) violation("the host waited for a ticket on a stream that records into a graph");
-  note_stream_idle(as_stream(stream));
+  merge(g_host_behind, g_ticket_behind[ticket_host]);  // not behind what the stream holds behind the ticket
   return 0;
 }
 int ugk_word_wait(const uint32_t *word_host, uint32_t value, unsigned, void *stream) {
@@ -904,7 +951,7 @@ int ugk_device_sync(void) {
   return 0;
 }
 int ugk_event_create(void **event) {
-  *event = new Event{std::chrono::steady_clock::now()};
+  *event = new Event{std::chrono::steady_clock::now(), 0, nullptr, {}};
   return 0;
 }
 int ugk_event_destroy(void *event) {
@@ -927,6 +974,8 @@ int ugk_event_record(void *event, void *stream) {
   e->at = std::chrono::steady_clock::now();
   e->captured_in = s->capture;
   e->recorded_on = s;
+  e->behind = s->behind;
+  merge(e->behind, g_host_behind);
   if (s->capture) {
     violation("an event was recorded on a stream that records into a graph: it belongs to the caller's capture now");
     g_graphs[s->capture].events.push_back(event);
@@ -938,6 +987,7 @@ int ugk_event_sync(void *event) {
   REQUIRE(event, "null event");
   std::lock_guard<std::mutex> g(g_rt_mu);
   if (static_cast<Event *>(event)->captured_in) violation("the host waited for a captured event");
+  merge(g_host_behind, static_cast<Event *>(event)->behind);
   return 0;
 }
 int ugk_event_query(void *event, int *complete) {
@@ -953,6 +1003,7 @@ int ugk_stream_wait_event(void *stream, void *event) {
   Event *e = static_cast<Event *>(event);
   Stream *s = as_stream(stream);
   const bool live_capture = e->captured_in != 0 && e->captured_in == g_capture_active;
+  merge(s->behind, e->behind);
   if (live_capture && s->capture == 0) {
     // the waiting stream joins the capture the event belongs to
     violation("a second stream joined the caller's capture by waiting for a captured event");
@@ -1359,8 +1410,9 @@ int ugk_rank_place(uint32_t *counts, uint64_t num_rows, uint64_t k, void *ws, ui
 // rows ordered by (count, kept, tie) with tie = row for counted rows and 0xffffffff - row for the others: three
 // 32-bit fields do not fit one word, so the kept bit goes between the count and the tie of a 128-bit key
 int ugk_rank_place_keep(uint32_t *counts, uint64_t num_rows, uint64_t k, void *ws, uint64_t *in_new,
-                        uint64_t *scratch, uint64_t *observed, const uint64_t *keep, int reset_counts, void *) {
+                        uint64_t *scratch, uint64_t *observed, const uint64_t *keep, int reset_counts, void *stream) {
   REQUIRE(counts && ws && in_new && scratch, "ugk_rank_place: null pointer");
+  note_launch(stream, "a placement", {keep}, {in_new, scratch});
   REQUIRE(keep != in_new && keep != scratch, "ugk_rank_place_keep: the keep bitmap is one of the output bitmaps");
   REQUIRE(num_rows > 0 && num_rows < 0xffffffffull, "ugk_rank_place: rows do not fit 32 bits");
   const uint64_t n_words = (num_rows + 63) / 64;
@@ -1398,7 +1450,13 @@ int ugk_rank_place_keep(uint32_t *counts, uint64_t num_rows, uint64_t k, void *w
 }
 int ugk_rank_place_observed(uint32_t *counts, uint64_t num_rows, uint64_t k, void *ws, uint64_t *in_new,
                             uint64_t *observed, int reset_counts, const uint64_t *cached, void *evict_ws,
-                            void *insert_ws, uint32_t *totals_host, uint32_t *status, void *) {
+                            void *insert_ws, uint32_t *totals_host, uint32_t *status, void *stream) {
+  return ugk_rank_place_observed_ticket(counts, num_rows, k, ws, in_new, observed, reset_counts, cached, evict_ws, insert_ws,
+                                        totals_host, status, 0, stream);
+}
+static int place_observed(uint32_t *counts, uint64_t num_rows, uint64_t k, void *ws, uint64_t *in_new, uint64_t *observed,
+                          int reset_counts, const uint64_t *cached, void *evict_ws, void *insert_ws, uint32_t *totals_host,
+                          uint32_t *status) {
   REQUIRE(ws && in_new && observed && status, "ugk_rank_place_observed: null pointer");
   REQUIRE(counts || !reset_counts, "ugk_rank_place_observed: counters to reset, but no counters");
   REQUIRE(num_rows > 0 && num_rows < 0xffffffffull, "ugk_rank_place_observed: rows do not fit 32 bits");
@@ -1447,8 +1505,12 @@ int ugk_rank_place_observed_ticket(uint32_t *counts, uint64_t num_rows, uint64_t
                                    uint64_t *observed, int reset_counts, const uint64_t *cached, void *evict_ws,
                                    void *insert_ws, uint32_t *totals_host, uint32_t *status, uint32_t ticket, void *stream) {
   REQUIRE(ticket == 0 || cached, "ugk_rank_place_observed: a ticket comes with the counts of what changes");
-  if (int rc = ugk_rank_place_observed(counts, num_rows, k, ws, in_new, observed, reset_counts, cached, evict_ws, insert_ws,
-                                       totals_host, status, stream))
+  const uint32_t *word = ticket ? totals_host + 3 : nullptr;
+  const bool scan = cached && num_rows > g_small_bits;
+  note_launch(stream, "a placement", {cached}, {in_new, evict_ws, insert_ws}, scan ? nullptr : word);
+  if (scan) note_launch(stream, "the scan behind a placement", {}, {evict_ws, insert_ws}, word);
+  if (int rc = place_observed(counts, num_rows, k, ws, in_new, observed, reset_counts, cached, evict_ws, insert_ws,
+                              totals_host, status))
     return rc;
   if (ticket) totals_host[3] = ticket;
   return 0;
@@ -1459,8 +1521,9 @@ int ugk_rank_threshold(const void *ws, uint64_t *threshold_host, void *) {
 }
 size_t ugk_bitmap_workspace_bytes(void) { return 64; }
 int ugk_bitmap_count(const uint64_t *a, const uint64_t *b, int invert_a, uint64_t nbits, void *ws,
-                     uint32_t *total_host, void *) {
+                     uint32_t *total_host, void *stream) {
   REQUIRE(a && ws && nbits > 0 && nbits <= 0xffffffffull, "ugk_bitmap_count: bad argument");
+  note_launch(stream, "a count of a bitmap", {a, b}, {ws});
   uint32_t total = 0;
   for (uint64_t w = 0; w < (nbits + 63) / 64; ++w) total += __builtin_popcountll(bm_word(a, b, invert_a, nbits, w));
   *static_cast<uint32_t *>(ws) = total;
@@ -1468,9 +1531,10 @@ int ugk_bitmap_count(const uint64_t *a, const uint64_t *b, int invert_a, uint64_
   return 0;
 }
 int ugk_bitmap_emit(const uint64_t *a, const uint64_t *b, int invert_a, uint64_t nbits, const void *ws, uint32_t *out,
-                    uint64_t max_out, void *) {
+                    uint64_t max_out, void *stream) {
   REQUIRE(a && ws && nbits > 0 && nbits <= 0xffffffffull, "ugk_bitmap_emit: bad argument");
   if (max_out == 0) return 0;
+  note_launch(stream, "a list of a bitmap", {a, b, ws}, {out});
   REQUIRE(out, "ugk_bitmap_emit: null output list");
   uint64_t pos = 0;
   for (uint64_t w = 0; w < (nbits + 63) / 64 && pos < max_out; ++w) {

@@ -14,4 +14,6 @@ void ugk_model_graph_destroy(int graph_id);
 // number of rule violations seen so far; their texts, one a line, into text[capacity]
 size_t ugk_model_violations(char *text, size_t capacity);
 void ugk_model_reset(void);
+// bitmaps longer than this take the passes that the kernel layer has for those of more than 2^26 bits
+void ugk_model_small_bits(size_t nbits);
 }

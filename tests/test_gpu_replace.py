@@ -463,13 +463,17 @@ def test_placement_polled_for_by_its_ticket(n):
     sync()
     try:
         for ticket in (5, 6, 7):
+            # nothing but the two calls between the ticket and the lists
+            out_l, in_l = torch.full_like(leaving, -1), torch.full_like(coming, -1)
+            lists = (ptr(d_cached), ptr(d_new), n, ptr(ws_out), ptr(ws_in), ptr(out_l), len(leaving), ptr(in_l), len(coming),
+                     other.cuda_stream)
+            wait = (totals.ptr + 12, ticket, 1_000_000, one.cuda_stream)
+            sync()
             hip.call("ugk_rank_place_observed_ticket", None, n, k, ptr(ws), ptr(d_new), ptr(d_obs), 0, ptr(d_cached),
                      ptr(ws_out), ptr(ws_in), totals.ptr, ptr(st), ticket, one.cuda_stream)
-            hip.call("ugk_ticket_wait", totals.ptr + 12, ticket, 1_000_000, one.cuda_stream)
+            hip.call("ugk_ticket_wait", *wait)
+            hip.call("ugk_bitmap_emit_diff", *lists)
             assert totals.array.tolist()[:2] == [len(leaving), len(coming)] and totals.array[3] == ticket
-            out_l, in_l = torch.empty_like(leaving), torch.empty_like(coming)
-            hip.call("ugk_bitmap_emit_diff", ptr(d_cached), ptr(d_new), n, ptr(ws_out), ptr(ws_in), ptr(out_l), len(leaving),
-                     ptr(in_l), len(coming), other.cuda_stream)
             sync()
             assert torch.equal(out_l, leaving) and torch.equal(in_l, coming)
             d_new.fill_(-1)

@@ -100,6 +100,7 @@ struct RankWs {
   uint32_t last_t;               // T of the placement before this one (whatever the memory held, the first time)
   uint32_t guess_t;              // the T the first pass over the counters split by on the way (= last_t)
   uint32_t split_done;           // the guess was T: gt and eq are written, the second pass is not needed
+  uint32_t scans_done;           // of bitmap_scan2_kernel behind a placement with a ticket
 
   uint32_t hist[kHistBins];
   Arrivals arrivals;             // of rank_combine_observed_kernel
@@ -487,6 +488,7 @@ __global__ __launch_bounds__(kScanBlock) void rank_locate_unobserved_kernel(Rank
     ws->last_row = 0;
     ws->from_bitmap = 0;
     ws->keep_mode = 0;
+    ws->scans_done = 0;
   }
   for (uint32_t i = tid; i < (kArriveLines + 1) * 16; i += kScanBlock) (&ws->arrivals.line[0][0])[i] = 0ull;
   uint32_t pre[8], total;
@@ -566,7 +568,7 @@ __global__ __launch_bounds__(kScanBlock) void rank_locate_unobserved_kernel(Rank
 // in (in_new & ~cached) are counted per 64-word block and per chunk on the way, as bitmap_count_kernel would, and all in
 // all: the last workgroup to end writes both sums to totals_host.  One wavefront per chunk.  With a ticket, which that
 // workgroup writes behind the sums, a host that polls for it may go on at once, on any stream: what the refresh reads next is
-// written through to memory then (leave_done has the why).
+// written through to memory then (leave_done has the why).  Only a launch that is the placement's last one gets a ticket.
 __global__ __launch_bounds__(kBlock) void rank_combine_observed_kernel(uint32_t *counts, uint64_t nbits,
                                                                        uint64_t per_chunk, RankWs *ws,
                                                                        unsigned long long *observed,
@@ -755,27 +757,46 @@ __global__ __launch_bounds__(kBlock) void bitmap_count_diff_kernel(const unsigne
 }
 
 // one workgroup of kScanBlock threads: the counts of the chunks become their prefix
+template <bool THROUGH>
 __device__ __forceinline__ void scan_ws(BmWs *ws, uint32_t *total_host) {
+  auto put = [](auto *to, auto v) {
+    if constexpr (THROUGH) store_through(reinterpret_cast<uint64_t>(to), v);
+    else *to = v;
+  };
   uint32_t pre[8], total;
   scan_chunks(ws->base, pre, total);
   u32x4_by4 *to = reinterpret_cast<u32x4_by4 *>(ws->base) + 2 * threadIdx.x;
-  to[0] = u32x4{pre[0], pre[1], pre[2], pre[3]};
-  to[1] = u32x4{pre[4], pre[5], pre[6], pre[7]};
+  put(to, u32x4{pre[0], pre[1], pre[2], pre[3]});
+  put(to + 1, u32x4{pre[4], pre[5], pre[6], pre[7]});
   if (threadIdx.x == 0) {
-    ws->total = total;
-    ws->scanned = 1;
+    put(&ws->total, total);
+    put(&ws->scanned, 1u);
     if (total_host) *total_host = total;
   }
 }
 
 __global__ __launch_bounds__(kScanBlock) void bitmap_scan_kernel(BmWs *ws, uint32_t *total_host, const RankWs *gate) {
   if (gate && gate->keep_mode != 2) return;
-  scan_ws(ws, total_host);
+  scan_ws<false>(ws, total_host);
 }
 
 // two workspaces in one launch (one workgroup each), totals to totals_host[0] and [1]
 __global__ __launch_bounds__(kScanBlock) void bitmap_scan2_kernel(BmWs *a, BmWs *b, uint32_t *totals_host) {
-  scan_ws(blockIdx.x == 0 ? a : b, totals_host ? totals_host + blockIdx.x : (uint32_t *)nullptr);
+  scan_ws<false>(blockIdx.x == 0 ? a : b, totals_host ? totals_host + blockIdx.x : (uint32_t *)nullptr);
+}
+
+// The same behind a placement whose end the host polls for: the prefixes are the last of what the refresh reads next, so they
+// are written through and the workgroup that finishes second leaves the ticket (a ticket left by the placement itself let
+// the lists on another stream start in front of the scan).
+__global__ __launch_bounds__(kScanBlock) void bitmap_scan2_ticket_kernel(BmWs *a, BmWs *b, RankWs *placed,
+                                                                         uint32_t *ticket_host, uint32_t ticket) {
+  if (placed->from_bitmap) scan_ws<true>(blockIdx.x == 0 ? a : b, nullptr);  // else nothing was placed or counted
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores have been acknowledged
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (__hip_atomic_fetch_add(&placed->scans_done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 1u) return;
+  __threadfence_system();
+  *(volatile uint32_t *)ticket_host = ticket;
 }
 
 // The set bits of one 64-word block, a lane per word on entry (m), to out[pos0 ...] in ascending order; n_set: how
@@ -1182,13 +1203,18 @@ int ugk_rank_place_observed_ticket(uint32_t *counts_dev, uint64_t num_rows, uint
                      &ws->bm, no_gate);
   hipLaunchKernelGGL(rank_locate_unobserved_kernel, dim3(1), dim3(kScanBlock), 0, st, ws, observed, num_rows, per_chunk,
                      (unsigned long long)k, status_dev, totals_host ? totals_host + 2 : (uint32_t *)nullptr);
+  // the emit pass of longer bitmaps wants the chunk counts scanned; the ticket is left by whichever launch is the last one
+  const bool scan = cached_dev && num_rows > kSmallBits;
+  BmWs *evict_ws = static_cast<BmWs *>(evict_ws_dev), *insert_ws = static_cast<BmWs *>(insert_ws_dev);
   hipLaunchKernelGGL(rank_combine_observed_kernel, dim3(bm_grid), dim3(kBlock), 0, st, counts_dev, num_rows, per_chunk,
                      ws, observed, reinterpret_cast<unsigned long long *>(in_new_dev),
-                     reinterpret_cast<const unsigned long long *>(cached_dev), static_cast<BmWs *>(evict_ws_dev),
-                     static_cast<BmWs *>(insert_ws_dev), reset_counts, totals_host, ticket);
-  if (cached_dev && num_rows > kSmallBits)  // the emit pass of longer bitmaps wants the chunk counts scanned
-    hipLaunchKernelGGL(bitmap_scan2_kernel, dim3(2), dim3(kScanBlock), 0, st, static_cast<BmWs *>(evict_ws_dev),
-                       static_cast<BmWs *>(insert_ws_dev), (uint32_t *)nullptr);
+                     reinterpret_cast<const unsigned long long *>(cached_dev), evict_ws, insert_ws, reset_counts,
+                     totals_host, scan ? 0u : ticket);
+  if (scan && ticket)
+    hipLaunchKernelGGL(bitmap_scan2_ticket_kernel, dim3(2), dim3(kScanBlock), 0, st, evict_ws, insert_ws, ws,
+                       totals_host + 3, ticket);
+  else if (scan)
+    hipLaunchKernelGGL(bitmap_scan2_kernel, dim3(2), dim3(kScanBlock), 0, st, evict_ws, insert_ws, (uint32_t *)nullptr);
   UGK_HIP(hipGetLastError());
   return 0;
 }
