@@ -18,16 +18,17 @@ typedef __attribute__((address_space(1))) u32x4 *gout_t;
 // ---- the end of a launch a host polls for --------------------------------------------------------------------------
 // Stores that are written through the caches (system scope): once such a store has been acknowledged its bytes are in
 // memory, and not in the L2 of an XCD that is written back when the kernel has ended.  In assembler, for the language has
-// no such stores of 16 bytes; the s_nop is for the vector instruction that may overwrite the stored registers next.
+// no such stores of 16 bytes.  The s_nop: gfx940 and later want two wait states between a store of more than 8 bytes and a
+// vector instruction that overwrites its data, and the compiler, which sees to that elsewhere, does not look into assembler.
 template <typename V>
 __device__ __forceinline__ void store_through(uint64_t to, V v) {
   typedef __attribute__((address_space(1))) char *gbyte_t;
   const gbyte_t p = reinterpret_cast<gbyte_t>(to);
-  if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
-  else if constexpr (sizeof(V) == 8) asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
-  else if constexpr (sizeof(V) == 4) asm volatile("global_store_dword %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
-  else if constexpr (sizeof(V) == 2) asm volatile("global_store_short %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"((uint32_t)v) : "memory");
-  else asm volatile("global_store_byte %0, %1, off sc0 sc1\n\ts_nop 0" ::"v"(p), "v"((uint32_t)v) : "memory");
+  if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+  else if constexpr (sizeof(V) == 8) asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+  else if constexpr (sizeof(V) == 4) asm volatile("global_store_dword %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+  else if constexpr (sizeof(V) == 2) asm volatile("global_store_short %0, %1, off sc0 sc1" ::"v"(p), "v"((uint32_t)v) : "memory");
+  else asm volatile("global_store_byte %0, %1, off sc0 sc1" ::"v"(p), "v"((uint32_t)v) : "memory");
 }
 
 // how a kernel stores its rows: a template parameter, not a launch argument, for with a run-time choice the optimiser merges
