@@ -2,7 +2,10 @@
 // with which arguments, without a GPU.  This executable defines the runtime's launch calls itself, in front of those of
 // libamdhip64, and notes every launch instead of performing it; device pointers are made up and never followed.
 //
-// usage: launch_order <libugache_hip.so> <call> <number>; prints a line per launch: the kernel and its arguments
+// usage: launch_order <libugache_hip.so> place <rows>                          a placement with a ticket
+//                                       pool <id bytes> <row bytes> <ids> <samples> <max norm> <words>
+// words: 0: nobody polls, 1: words are asked for (ugk_leave_done_words).  Prints a line per launch, the kernel, its template
+// arguments, the stream and the other arguments, and how many words the call says it leaves.
 #include <cxxabi.h>
 #include <dlfcn.h>
 
@@ -13,6 +16,8 @@
 #include <map>
 #include <string>
 #include <vector>
+
+#include "ugache_hip.h"
 
 namespace {
 struct Dim3 {
@@ -29,7 +34,7 @@ std::map<const void *, std::string> &kernels() {  // registered while the librar
 }
 
 // the types between the outer parentheses of a demangled kernel
-std::vector<std::string> parameters(const std::string &name) {
+std::vector<std::string> parameters(const std::string &name, size_t *open_at) {
   std::vector<std::string> out;
   int angle = 0, depth = 0;
   size_t begin = 0, open = name.size();
@@ -42,6 +47,7 @@ std::vector<std::string> parameters(const std::string &name) {
     }
   }
   begin = open + 1;
+  *open_at = open;
   for (size_t i = begin; i < name.size(); ++i) {
     const char c = name[i];
     if (c == '(' || c == '<') ++depth;
@@ -88,10 +94,13 @@ int hipDeviceGetAttribute(int *value, int, int) {
 int hipGetLastError() { return 0; }
 int hipLaunchKernel(const void *f, Dim3, Dim3, void **args, size_t, void *stream) {
   const std::string &name = kernels()[f];
-  std::string line = name.substr(0, name.find("_kernel") + 7);
-  line = line.substr(line.rfind("::") == std::string::npos ? 0 : line.rfind("::") + 2);
-  printf("%s stream=%llx", line.c_str(), (unsigned long long)(uintptr_t)stream);
-  const std::vector<std::string> types = parameters(name);
+  const size_t end = name.find("_kernel") + 7, begin = name.rfind("::", end) == std::string::npos ? 0 : name.rfind("::", end) + 2;
+  size_t open = 0;
+  const std::vector<std::string> types = parameters(name, &open);
+  std::string templ = name.substr(end, open - end);
+  for (size_t i; (i = templ.find(' ')) != std::string::npos;) templ.erase(i, 1);
+  printf("%s %s stream=%llx", name.substr(begin, end - begin).c_str(), templ.empty() ? "<>" : templ.c_str(),
+         (unsigned long long)(uintptr_t)stream);
   for (size_t i = 0; i < types.size(); ++i) {
     unsigned long long v = 0;
     const std::string &t = types[i];
@@ -109,20 +118,38 @@ int hipLaunchKernel(const void *f, Dim3, Dim3, void **args, size_t, void *stream
 }
 
 int main(int argc, char **argv) {
-  if (argc != 4) return 2;
+  if (argc < 4) return 2;
   void *lib = dlopen(argv[1], RTLD_NOW);
   if (!lib) {
     fprintf(stderr, "%s\n", dlerror());
     return 1;
   }
-  const uint64_t number = strtoull(argv[3], nullptr, 0);
   const auto dev = [](uint64_t k) { return reinterpret_cast<void *>(0x100000000000ull + (k << 32)); };
-  if (strcmp(argv[2], "place_with_ticket") == 0) {
-    typedef int (*fn_t)(void *, uint64_t, uint64_t, void *, void *, void *, int, void *, void *, void *, void *, void *, uint32_t,
-                        void *);
-    const fn_t fn = reinterpret_cast<fn_t>(dlsym(lib, "ugk_rank_place_observed_ticket"));
-    // evict and insert workspaces at 7 and 8, the ticket is 0xabcd
-    return !fn || fn(dev(1), number, number / 2, dev(2), dev(3), dev(4), 1, dev(6), dev(7), dev(8), dev(9), dev(10), 0xabcd, dev(11));
+  const auto number = [&](int i) { return i < argc ? strtoull(argv[i], nullptr, 0) : 0ull; };
+  const std::string call = argv[2];
+  ugk_done_t done{};
+  done.words_host = static_cast<uint64_t *>(dev(20)), done.counters_dev = static_cast<uint64_t *>(dev(21)), done.tag = 1;
+  const auto ask = [&](uint64_t words) {
+    return words == 0 || reinterpret_cast<decltype(&ugk_leave_done_words)>(dlsym(lib, "ugk_leave_done_words"))(&done) == 0;
+  };
+  uint32_t *u32 = static_cast<uint32_t *>(dev(9));
+  int rc = 2;
+  if (call == "place") {  // evict and insert workspaces at 7 and 8, the ticket is 0xabcd
+    const auto fn = reinterpret_cast<decltype(&ugk_rank_place_observed_ticket)>(dlsym(lib, "ugk_rank_place_observed_ticket"));
+    rc = fn(static_cast<uint32_t *>(dev(1)), number(3), number(3) / 2, dev(2), static_cast<uint64_t *>(dev(3)),
+            static_cast<uint64_t *>(dev(4)), 1, static_cast<uint64_t *>(dev(6)), dev(7), dev(8), u32, static_cast<uint32_t *>(dev(10)),
+            0xabcd, dev(11));
+  } else if (call == "pool" && argc == 9 && ask(number(8))) {
+    ugk_table_t none{};
+    const auto run = [&](auto fn, auto *ids) {
+      return fn(none, ids, static_cast<int64_t *>(dev(2)), nullptr, number(6), number(5), 0, 4, (float)number(7), nullptr, 0, dev(3),
+                1000, dev(4), number(4), u32, nullptr, nullptr, nullptr, dev(11));
+    };
+    rc = number(3) == 4 ? run(reinterpret_cast<decltype(&ugk_extract_pool_clip_u32)>(dlsym(lib, "ugk_extract_pool_clip_u32")),
+                              static_cast<uint32_t *>(dev(1)))
+                        : run(reinterpret_cast<decltype(&ugk_extract_pool_clip_i64)>(dlsym(lib, "ugk_extract_pool_clip_i64")),
+                              static_cast<int64_t *>(dev(1)));
   }
-  return 2;
+  if (rc == 0) printf("words %u\n", done.num_words);
+  return rc;
 }

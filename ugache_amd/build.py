@@ -23,8 +23,8 @@ INCLUDE = os.path.join(ROOT, "include")
 HIP_LIB = os.path.join(PKG, "libugache_hip.so")
 HOST_LIB = os.path.join(PKG, "libcoll_cache.so")
 
-HIP_SOURCES = ["ugk_runtime.hip", "ugk_gather.hip", "ugk_table.hip", "ugk_partition.hip", "ugk_pool.hip",
-               "ugk_hotness.hip", "ugk_refresh.hip"]
+HIP_SOURCES = ["ugk_partition.hip", "ugk_pool_i64.hip", "ugk_pool.hip", "ugk_gather.hip", "ugk_refresh.hip",
+               "ugk_runtime.hip", "ugk_table.hip", "ugk_hotness.hip"]
 OBJ_DIR = os.path.join(PKG, "_build")
 
 HIPCC_FLAGS = [

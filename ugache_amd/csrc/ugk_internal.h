@@ -93,6 +93,7 @@ void preload_gather(hipStream_t stream);
 void preload_hotness(hipStream_t stream);
 void preload_partition(hipStream_t stream);
 void preload_pool(hipStream_t stream);
+void preload_pool_i64(hipStream_t stream);
 void preload_refresh(hipStream_t stream);
 void preload_table(hipStream_t stream);
 

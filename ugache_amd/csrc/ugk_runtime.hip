@@ -335,6 +335,7 @@ int ugk_preload_kernels(void) {
   ugk::preload_hotness(st);
   ugk::preload_partition(st);
   ugk::preload_pool(st);
+  ugk::preload_pool_i64(st);
   ugk::preload_refresh(st);
   ugk::preload_table(st);
   const hipError_t launched = hipGetLastError();
