@@ -1,4 +1,5 @@
 """What the compiler makes of the kernels' own assembler, on the CPU (hipcc compiles for gfx950 without a GPU)."""
+import os
 import re
 import subprocess
 
@@ -65,3 +66,25 @@ def test_a_written_through_store_leaves_its_data_as_long_as_the_compiler_does(as
     want = _wait_states_behind_the_store(assembly, kernel + "_by_compiler")
     assert _wait_states_behind_the_store(assembly, kernel + "_by_hand") >= want
     assert kernel != "store16" or want == 2  # the case there is a wait for
+
+
+@pytest.fixture(scope="module")
+def gather_kernels():
+    """name -> where the number of workgroups stands among the arguments of each kernel of ugk_gather.hip"""
+    cmd = [build.hipcc_path()] + build.HIPCC_FLAGS + ["--cuda-device-only", "-S", "-I", build.INCLUDE, "-I", build.CSRC,
+                                                      os.path.join(build.CSRC, "ugk_gather.hip"), "-o", "-"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
+    assert proc.returncode == 0, proc.stderr[-3000:]
+    found = {}
+    for meta in re.findall(r"- \.agpr_count.*?\.wavefront_size: +\d+", proc.stdout, re.S):
+        at = re.search(r"\.offset: +(\d+)\n +\.size: +4\n +\.value_kind: +hidden_block_count_x", meta)
+        found[re.search(r"\.name: +(\S+)", meta).group(1)] = int(at.group(1)) if at else None
+    return found
+
+
+def test_a_gather_nobody_polls_for_has_its_arguments_in_two_lines(gather_kernels):
+    """a launch's arguments are in host memory: the 48 bytes that only a polled launch needs pushed the number of workgroups,
+    which stands behind the kernel's own arguments, into a third line of 64 bytes"""
+    plain = {k: at for k, at in gather_kernels.items() if "Direct" in k and "StoreE2E" not in k and at is not None}
+    assert len(plain) > 20
+    assert max(plain.values()) < 128, max(plain, key=plain.get)

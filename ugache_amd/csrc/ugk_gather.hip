@@ -95,9 +95,8 @@ __device__ __forceinline__ void st_stream(V *p, V v) {
 template <typename V, int LPR, int UNROLL, Store STORE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restrict__ src, uint64_t src_rows,
                                                         V *__restrict__ out, uint64_t out_rows, uint32_t vpr,
-                                                        const uint32_t *__restrict__ counts, uint32_t group, size_t n,
-                                                        bool many_groups, uint32_t *status, uint32_t *host_mirror,
-                                                        DoneWords done) {
+                                                        const uint32_t *__restrict__ counts, uint32_t group,
+                                                        bool many_groups, size_t n, uint32_t *status, uint32_t *host_mirror, Ending<STORE> done) {
   size_t begin = 0, count = n;
   if (counts) {
     const uint32_t c = counts[group];
@@ -167,7 +166,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
           copy_key_along(done, i, ix.keys[i]);
     }
   }
-  if constexpr (STORE == kThrough) leave_done<true>(done, nullptr);
+  if constexpr (STORE == kThrough) leave_done(done, nullptr);
 }
 
 // The same for rows the lanes of gather_kernel do not fit (see flat_copy): a wavefront takes f.tile rows, one index
@@ -177,7 +176,7 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
                                                              char *__restrict__ out, uint64_t out_rows, FlatRow f,
                                                              const uint32_t *__restrict__ counts, uint32_t group,
                                                              size_t n, uint32_t *status, uint32_t *host_mirror,
-                                                             DoneWords done) {
+                                                             Ending<STORE> done) {
   size_t begin = 0, count = n;
   if (counts) {
     const uint32_t c = counts[group];
@@ -208,7 +207,7 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
       if (lane_id() < rows) copy_key_along(done, base + lane_id(), (typename Idx::key_t)s);
     }
   }
-  if constexpr (STORE == kThrough) leave_done<true>(done, nullptr);
+  if constexpr (STORE == kThrough) leave_done(done, nullptr);
 }
 
 // ... and with the output dealt out instead of the rows, for batches whose row i becomes output row i: a wavefront owns
@@ -233,7 +232,7 @@ StreamRow stream_row(size_t row_bytes, size_t n) {
 template <Store STORE, bool SHARE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                                char *__restrict__ out, StreamRow f, uint32_t *status,
-                                                               uint32_t *host_mirror, DoneWords done) {
+                                                               uint32_t *host_mirror, Ending<STORE> done) {
   static_assert(Idx::kDense, "row i goes to output row i");
   typedef __attribute__((address_space(1))) uint32_t *gword_t;
   constexpr int U = (int)(kStreamPart / (kWave * 16));
@@ -261,7 +260,9 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     }
     const unsigned long long good = __ballot(ok);
     if (good == 0ull) {
-      if (STORE == kThrough && active) copy_key_along(done, row0 + lane, (typename Idx::key_t)s);
+      if constexpr (STORE == kThrough) {
+        if (active) copy_key_along(done, row0 + lane, (typename Idx::key_t)s);
+      }
       continue;
     }
     // a row that is skipped is read where the first good one is (all lanes take part in the shuffle)
@@ -337,10 +338,11 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
         }
       }
     }
-    if (STORE == kThrough && active)
-      copy_key_along(done, row0 + lane, (typename Idx::key_t)s);  // a row in two parts: twice the same key
+    if constexpr (STORE == kThrough) {
+      if (active) copy_key_along(done, row0 + lane, (typename Idx::key_t)s);  // a row in two parts: twice the same key
+    }
   }
-  if constexpr (STORE == kThrough) leave_done<true>(done, nullptr);
+  if constexpr (STORE == kThrough) leave_done(done, nullptr);
 }
 
 // Re-expansion of duplicates inside one buffer: row i takes the bytes of its representative row.  Source and
@@ -476,7 +478,7 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
 #define UGK_GO(STORE)                                                                                                  \
   hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,            \
                      reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,   \
-                     group, n, many_groups, status, host_mirror, done)
+                     group, many_groups, n, status, host_mirror, Ending<STORE>(done))
   if (done.tag) UGK_GO(kThrough);
   else if (nt) UGK_GO(kStreaming);
   else UGK_GO(kOrdinary);
@@ -579,10 +581,10 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
   const DoneWords done = request.take(grid);
   if (done.tag)
     hipLaunchKernelGGL((gather_flat_kernel<kThrough, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,
-                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, done);
+                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<kThrough>(done));
   else
     hipLaunchKernelGGL((gather_flat_kernel<kOrdinary, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,
-                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, done);
+                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<kOrdinary>(done));
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -597,7 +599,7 @@ int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t 
   const DoneWords done = nt ? DoneWords{} : request.take(grid);
 #define UGK_GO(STORE, SHARE)                                                                                          \
   hipLaunchKernelGGL((gather_stream_kernel<STORE, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,             \
-                     (const char *)src, src_rows, (char *)out, f, status, host_mirror, done)
+                     (const char *)src, src_rows, (char *)out, f, status, host_mirror, Ending<STORE>(done))
   const bool share = row_bytes % 16 != 0;
   if (done.tag && share) UGK_GO(kThrough, true);
   else if (done.tag) UGK_GO(kThrough, false);

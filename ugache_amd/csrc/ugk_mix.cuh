@@ -36,6 +36,21 @@ __device__ __forceinline__ void store_through(uint64_t to, V v) {
 // 0.2 to 0.4 us (26,624 rows of 64 bytes 3.6 -> 4.0)
 enum Store { kOrdinary, kStreaming, kThrough };
 
+// What a kernel is told about its end: one that is polled for everything, any other where the counts of its workgroups go, if
+// anywhere.  Not more than that: the arguments are in host memory, and the line of 64 bytes that the whole of DoneWords pushed
+// the launch's own numbers into cost every launch of a plain gather (us, stream-ordered: 262,144 rows of 200 bytes 24.9 ->
+// 25.9, of 12 bytes 7.9 -> 8.2, 16,384 rows of 512 bytes 4.3 -> 5.1).
+template <Store STORE>
+struct Ending {
+  unsigned long long *words;
+  explicit Ending(const DoneWords &done) : words(done.words) {}
+  __device__ explicit Ending(unsigned long long *counts) : words(counts) {}
+};
+template <>
+struct Ending<kThrough> : DoneWords {
+  explicit Ending(const DoneWords &done) : DoneWords(done) {}
+};
+
 // A word for the host beside the rows (an error flag, a key).  The same kind of store: an ordinary one into host memory is
 // acknowledged before it is there, and the words of leave_done, which say that all of this is complete, may overtake it
 // (a lookup of four keys, one of them out of range, returned without its error that way).
@@ -52,9 +67,9 @@ __device__ __forceinline__ void copy_key_along(const DoneWords &done, uint64_t i
 
 // The last thing a workgroup does: its counts, and where a host polls the news that it has ended.  All threads call it; tot (in LDS,
 // may be NULL) holds the rows taken from the cache and all others.
-template <bool POLLED>
-__device__ __forceinline__ void leave_done(const DoneWords &done, const uint32_t *tot) {
-  if constexpr (POLLED) {
+template <Store STORE>
+__device__ __forceinline__ void leave_done(const Ending<STORE> &done, const uint32_t *tot) {
+  if constexpr (STORE == kThrough) {
     // The set of counters this launch does not use is made zero for the next one, in front of the wait: once all words are
     // there that is complete, also for a launch on another stream, which does not wait for this one to end.  (A counter
     // cleared by the workgroup that finds it complete would need a wait between that and its word.)
@@ -66,21 +81,21 @@ __device__ __forceinline__ void leave_done(const DoneWords &done, const uint32_t
   __syncthreads();
   if (threadIdx.x != 0) return;
   const uint32_t local = tot ? tot[0] : 0u, others = tot ? tot[1] : 0u;
-  if constexpr (!POLLED) {
+  if constexpr (STORE != kThrough) {
     done.words[blockIdx.x] = ((unsigned long long)others << 32) | local;
-    return;
+  } else {
+    const unsigned long long tag = (unsigned long long)done.tag << 48, mine = ((unsigned long long)others << 24) | local;
+    if (gridDim.x <= kDoneDirect) {
+      done.words[blockIdx.x] = tag | mine;
+      return;
+    }
+    const uint32_t g = blockIdx.x % kDoneFan, members = gridDim.x / kDoneFan + (g < gridDim.x % kDoneFan ? 1u : 0u);
+    const unsigned long long add = (1ull << 48) | mine;
+    unsigned long long *counter = done.counters + (done.set * kDoneFan + g) * 16;  // a line each
+    const unsigned long long sum =
+        __hip_atomic_fetch_add(counter, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
+    if ((uint32_t)(sum >> 48) == members) done.words[g] = tag | (sum & 0xffffffffffffull);
   }
-  const unsigned long long tag = (unsigned long long)done.tag << 48, mine = ((unsigned long long)others << 24) | local;
-  if (gridDim.x <= kDoneDirect) {
-    done.words[blockIdx.x] = tag | mine;
-    return;
-  }
-  const uint32_t g = blockIdx.x % kDoneFan, members = gridDim.x / kDoneFan + (g < gridDim.x % kDoneFan ? 1u : 0u);
-  const unsigned long long add = (1ull << 48) | mine;
-  unsigned long long *counter = done.counters + (done.set * kDoneFan + g) * 16;  // a line each
-  const unsigned long long sum =
-      __hip_atomic_fetch_add(counter, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
-  if ((uint32_t)(sum >> 48) == members) done.words[g] = tag | (sum & 0xffffffffffffull);
 }
 
 // ---- flat row copy -------------------------------------------------------------------------------------------------
@@ -204,14 +219,14 @@ __device__ __forceinline__ MixRow mix_resolve(const ugk_table_t &t, uint64_t key
 // result tells the last workgroup still 5 us (every workgroup ends by waiting for the round trip), and a device-scope
 // fence per workgroup 13-49 % of a whole step (each writes back and invalidates the L2 of its XCD).
 // (A launch that a host polls for waits for its stores anyway, and adds its workgroups up in a few counters: leave_done.)
-template <bool POLLED>
+template <Store STORE>
 __device__ __forceinline__ void mix_leave_counts(uint32_t *block_tot, uint32_t wave_local, uint32_t wave_host,
-                                                 const DoneWords &done) {
+                                                 const Ending<STORE> &done) {
   if (lane_id() == 0) {
     if (wave_local) atomicAdd(&block_tot[0], wave_local);
     if (wave_host) atomicAdd(&block_tot[1], wave_host);
   }
-  leave_done<POLLED>(done, block_tot);
+  leave_done(done, block_tot);
 }
 
 }  // namespace

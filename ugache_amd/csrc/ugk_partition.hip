@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
                                                              const void *__restrict__ host, uint64_t host_rows,
                                                              void *__restrict__ out, FlatRow f_row,
                                                              uint32_t *status, uint32_t *host_mirror,
-                                                             DoneWords done, ugk_stage_t stage) {
+                                                             Ending<STORE> done, ugk_stage_t stage) {
   __shared__ uint32_t block_tot[2];
   if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
   __syncthreads();
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       if (active) copy_key_along<K>(done, i, (K)key);
     }
   }
-  if (done.words) mix_leave_counts<STORE == kThrough>(block_tot, wave_local, wave_host, done);
+  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
 }
 
 // ---- dedup -----------------------------------------------------------------------------------------------
@@ -573,7 +573,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const ugk_stage_t no_stage{};
 #define UGK_GO4(L, W, NT, ST)                                                                                       \
   hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, NT, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
-                     cache, cache_rows, host, host_rows, out, f_row, status, host_mirror, done,                    \
+                     cache, cache_rows, host, host_rows, out, f_row, status, host_mirror, Ending<NT>(done),        \
                      ST ? *stage : no_stage)
 #define UGK_GO3(L, W, NT)               \
   do {                                  \

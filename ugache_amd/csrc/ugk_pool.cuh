@@ -105,7 +105,7 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
                                              uint64_t cache_rows, const u32x4 *__restrict__ host, uint64_t host_rows,
                                              u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
                                              float max_norm, uint32_t *status, uint32_t *host_mirror,
-                                             const DoneWords &done, uint32_t &wave_local,
+                                             const Ending<STORE> &done, uint32_t &wave_local,
                                              uint32_t &wave_host) {
   constexpr int RPW = kWave / LPR;  // output rows per wavefront and pass
   constexpr int EPC = PoolElem<E>::kPerChunk;
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
                                                               const u32x4 *__restrict__ host, uint64_t host_rows,
                                                               u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
                                                               float max_norm, uint32_t *status, uint32_t *host_mirror,
-                                                              DoneWords done, uint32_t keep_waves) {
+                                                              Ending<STORE> done, uint32_t keep_waves) {
   __shared__ uint32_t block_tot[2];
   if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
   __syncthreads();
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
     pool_samples<K, KIND, LPR, CH, U, E, CLIP, false, STORE>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host,
                                                              host_rows, out, vpr, combiner, bf16, max_norm, status,
                                                              host_mirror, done, wave_local, wave_host);
-  if (done.words) mix_leave_counts<STORE == kThrough>(block_tot, wave_local, wave_host, done);
+  if (done.words) mix_leave_counts(block_tot, wave_local, wave_host, done);
 }
 
 constexpr int kPoolMaxRows = 8;  // output rows a lane group may own per pass
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(kBlock) void extract_pool_rows_kernel(ugk_table_t t
     pool_short_samples<K, KIND, LPR, E, false>(t, ids, seg_off, weights, n_rows, nnz, rows_per_group, cache, cache_rows,
                                                host, host_rows, out, vpr, combiner, bf16, status, host_mirror, counts,
                                                wave_local, wave_host, seg_beg, seg_start);
-  if (counts) mix_leave_counts<false>(block_tot, wave_local, wave_host, DoneWords{counts, nullptr, nullptr, 0, 0, 0});
+  if (counts) mix_leave_counts(block_tot, wave_local, wave_host, Ending<kOrdinary>(counts));
 }
 
 template <typename K, int KIND, typename E>
@@ -601,7 +601,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   hipLaunchKernelGGL((extract_pool_kernel<K, KIND, L, CH, U, E, CLIP, MIXED, STORE>), dim3(grid), dim3(kBlock), 0, st, t, \
                      ids, seg_off, weights, n_rows, (long long)nnz, (const u32x4 *)cache, cache_rows,                  \
                      (const u32x4 *)host, host_rows, (u32x4 *)out, vpr, combiner, bf16, max_norm, status, host_mirror, \
-                     done, keep_waves)
+                     Ending<STORE>(done), keep_waves)
 #define UGK_POOL(L, CH, U, CLIP, MIXED)                                                                                \
   if (shape == L * 100 + CH * 10 + U && clip == CLIP && mixed == MIXED) {                                              \
     launched = true;                                                                                                   \
