@@ -167,7 +167,8 @@ typedef struct {
   void *keys_host;    /* pinned: a launch with words leaves its first num_keys keys there, complete as its rows are */
   uint64_t num_keys;  /* 0: none */
   uint32_t counter_set; /* 0 before the first launch, kept by the launches from then on */
-  uint32_t reserved;
+  uint32_t where_faster; /* non-zero: words only where they are there no later than a ticket kernel (ugk_stream_sync_ticket)
+                          * behind the launch, with a kernel that copies the keys if keys are wanted */
 } ugk_done_t;
 int ugk_leave_done_words(ugk_done_t *done);
 int ugk_done_wait(const ugk_done_t *done, unsigned spin_us, void *stream, uint64_t *local, uint64_t *others);

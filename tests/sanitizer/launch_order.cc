@@ -3,8 +3,10 @@
 // libamdhip64, and notes every launch instead of performing it; device pointers are made up and never followed.
 //
 // usage: launch_order <libugache_hip.so> place <rows>                          a placement with a ticket
+//                                       gather <row bytes> <rows> <words>
+//                                       mix <row bytes> <rows> <words>
 //                                       pool <id bytes> <row bytes> <ids> <samples> <max norm> <words>
-// words: 0: nobody polls, 1: words are asked for (ugk_leave_done_words).  Prints a line per launch, the kernel, its template
+// words: 0: nobody polls, 1: words are asked for (ugk_leave_done_words), 2: where they are faster, 3: and a key with them.  Prints a line per launch, the kernel, its template
 // arguments, the stream and the other arguments, and how many words the call says it leaves.
 #include <cxxabi.h>
 #include <dlfcn.h>
@@ -130,6 +132,8 @@ int main(int argc, char **argv) {
   ugk_done_t done{};
   done.words_host = static_cast<uint64_t *>(dev(20)), done.counters_dev = static_cast<uint64_t *>(dev(21)), done.tag = 1;
   const auto ask = [&](uint64_t words) {
+    done.where_faster = words >= 2;
+    if (words == 3) done.keys_host = dev(22), done.num_keys = 1;
     return words == 0 || reinterpret_cast<decltype(&ugk_leave_done_words)>(dlsym(lib, "ugk_leave_done_words"))(&done) == 0;
   };
   uint32_t *u32 = static_cast<uint32_t *>(dev(9));
@@ -139,6 +143,15 @@ int main(int argc, char **argv) {
     rc = fn(static_cast<uint32_t *>(dev(1)), number(3), number(3) / 2, dev(2), static_cast<uint64_t *>(dev(3)),
             static_cast<uint64_t *>(dev(4)), 1, static_cast<uint64_t *>(dev(6)), dev(7), dev(8), u32, static_cast<uint32_t *>(dev(10)),
             0xabcd, dev(11));
+  } else if (call == "gather" && argc == 6 && ask(number(5))) {
+    const auto fn = reinterpret_cast<decltype(&ugk_gather_direct_i64)>(dlsym(lib, "ugk_gather_direct_i64"));
+    rc = fn(dev(1), 1000, static_cast<int64_t *>(dev(2)), number(4), dev(3), number(3), 0, u32, nullptr, dev(11));
+  } else if (call == "mix" && argc == 6 && ask(number(5))) {
+    ugk_table_t flat{};
+    flat.kind = 1, flat.table = dev(4), flat.size = 1000;
+    const auto fn = reinterpret_cast<decltype(&ugk_extract_mix_i64)>(dlsym(lib, "ugk_extract_mix_i64"));
+    rc = fn(flat, static_cast<int64_t *>(dev(2)), number(4), dev(1), 1000, dev(5), 1000, dev(3), number(3), u32, nullptr, nullptr,
+            nullptr, UGK_HINT_UNKNOWN, dev(11));
   } else if (call == "pool" && argc == 9 && ask(number(8))) {
     ugk_table_t none{};
     const auto run = [&](auto fn, auto *ids) {

@@ -54,3 +54,30 @@ def test_a_pooled_lookup_nobody_polls_for_is_a_kernel_without_words(launches, id
     assert none == 0 and words > 0 and len(plain) == len(polled) == 1
     assert plain[0][0] == polled[0][0] == "extract_pool_kernel"
     assert plain[0][1] != polled[0][1]
+
+
+# (row bytes, megabytes of output, when words come, against a ticket kernel): on both sides of every line of the rules
+@pytest.mark.parametrize("call,row_bytes,mb,told", [
+    ("gather", 512, 8, "sooner"), ("gather", 64, 8, "sooner"), ("gather", 12, 8, "sooner"), ("gather", 2048, 8, "sooner"),
+    ("gather", 1040, 8, "sooner"), ("gather", 4096, 0.1, "later"), ("gather", 4096, 33, "later"), ("gather", 4096, 34, "sooner"),
+    ("gather", 8192, 8, "later"), ("gather", 200, 8, "sooner"), ("gather", 3200, 8, "sooner"), ("gather", 1204, 8, "sooner"),
+    ("gather", 193, 1, "too late"), ("gather", 193, 34, "too late"), ("gather", 98, 1, "too late"), ("gather", 15, 1, "too late"),
+    ("mix", 1024, 8, "sooner"), ("mix", 1040, 8, "later"), ("mix", 1204, 30, "later"), ("mix", 4096, 33, "later"),
+    ("mix", 4096, 34, "sooner"), ("mix", 4112, 100, "later"), ("mix", 36, 8, "sooner"),
+])
+def test_a_lookup_is_told_its_end_by_words_where_they_are_sooner(launches, call, row_bytes, mb, told):
+    rows = int(mb * 1e6 / row_bytes)
+    plain, none = launches(call, row_bytes, rows, 0)
+    done, words = launches(call, row_bytes, rows, 2)
+    assert none == 0 and (words > 0) == (told == "sooner")
+    assert (done[0][:2] == plain[0][:2]) == (words == 0)  # without words it is the launch nobody polls for
+    assert launches(call, row_bytes, rows, 1)[1] > 0  # who insists gets them
+    assert (launches(call, row_bytes, rows, 3)[1] > 0) == (told != "too late")  # keys would be copied by a kernel
+
+
+@pytest.mark.parametrize("row_bytes,bag,mb,told", [(512, 1, 67, True), (512, 1, 67.2, False), (512, 2, 68, False), (512, 3, 68, True),
+                                                   (1024, 2, 67, True), (1024, 2, 68, False), (4096, 4, 134, True)])
+def test_a_pooled_lookup_is_told_its_end_by_words_where_they_are_sooner(launches, row_bytes, bag, mb, told):
+    samples = int(mb * 1e6 / row_bytes)
+    words = [launches("pool", 8, row_bytes, samples * bag, samples, 0, how)[1] for how in range(4)]
+    assert words[0] == 0 and words[1] > 0 and (words[2] > 0) == (words[3] > 0) == told

@@ -335,6 +335,7 @@ ExtractSession::ExtractSession(std::shared_ptr<CacheContext> cache_ctx) : _cache
   UGK_CALL(ugk_stream_sync(nullptr));
   _done.words_host = _done_words->ptr<uint64_t>();
   _done.counters_dev = _done_counters->ptr<uint64_t>();
+  _done.where_faster = 1;
   _host_mirror_handle = PinnedHostAlloc(256);
   _host_mirror = _host_mirror_handle->ptr<uint32_t>();
   memset(_host_mirror, 0, 256);

@@ -467,6 +467,21 @@ unsigned gather_grid(size_t passes, unsigned max_blocks) {
   return (unsigned)(passes > 0x7fffffffull ? 0x7fffffffull : passes);
 }
 
+// Words (ugk_leave_done_words) come later than a ticket kernel behind the launch would
+//   * for rows of single bytes or pairs: a line that is written through does not come together in L2.  us, launch to end of
+//     poll, ticket / words, rows in HBM: 97 bytes 1 MB 9.9 / 10.2, 8 MB 22.8 / 27.5, 32 MB 62 / 84; 1001 bytes 1 MB 15.8 / 19.6,
+//     8 MB 18.7 / 23.8, 32 MB 36 / 54;
+//   * for rows of more than two vectors per lane: the loads of a row's next vectors come back behind the stores of the last, and
+//     those end in memory, not in L2.  4 KB x 64 8.9 / 9.6, x 250 10.0 / 10.9, x 2,000 12.8 / 13.5, x 8,000 19.6 / 20.1; 8 KB x 64
+//     10.7 / 12.8, x 1,000 15.5 / 17.9, x 4,000 20.4 / 22.6; 16 KB 14 to 29 % later.  2 KB 2 to 12 % sooner at any size.  Large
+//     outputs hide it (blocking lookups of 8,192 rows of 8 KB 30.5 / 28.5).
+// (Outputs of 6 to 10 MB, about what the wavefronts of one round copy and all written at once, are 0.1 to 0.6 us later too where
+// a launch costs the host 3 us, and 0.9 us sooner where it costs 4: words there.)
+Telling gather_tells(size_t vector_bytes, uint32_t vectors_per_row, uint32_t lanes, size_t out_bytes) {
+  if (vector_bytes < 4) return Telling::kTooLate;
+  return vectors_per_row <= 2 * lanes || out_bytes > (size_t)32 << 20 ? Telling::kSooner : Telling::kLater;
+}
+
 template <typename V, int LPR, int UNROLL, typename Idx>
 int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, uint32_t vpr,
                     const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
@@ -474,7 +489,7 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
   constexpr size_t kPerIter = (size_t)(kBlock / LPR) * UNROLL;
   const unsigned grid = gather_grid((n + kPerIter - 1) / kPerIter, max_blocks);
   const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
-  const DoneWords done = nt ? DoneWords{} : request.take(grid);
+  const DoneWords done = nt ? DoneWords{} : request.take(grid, gather_tells(sizeof(V), vpr, LPR, n * (size_t)vpr * sizeof(V)));
 #define UGK_GO(STORE)                                                                                                  \
   hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,            \
                      reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,   \
@@ -578,7 +593,7 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
   const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes, n));
   const size_t per_block = (size_t)f.tile * kWavesPerBlock;
   const unsigned grid = gather_grid((n + per_block - 1) / per_block, max_blocks);
-  const DoneWords done = request.take(grid);
+  const DoneWords done = request.take(grid, Telling::kSooner);
   if (done.tag)
     hipLaunchKernelGGL((gather_flat_kernel<kThrough, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,
                        src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<kThrough>(done));
@@ -596,7 +611,7 @@ int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t 
   const uint64_t per_block = (uint64_t)kStreamPart * kWavesPerBlock;
   const unsigned grid = gather_grid((f.total + per_block - 1) / per_block, max_blocks);
   const bool nt = nt_store_for(n * row_bytes);
-  const DoneWords done = nt ? DoneWords{} : request.take(grid);
+  const DoneWords done = nt ? DoneWords{} : request.take(grid, Telling::kSooner);
 #define UGK_GO(STORE, SHARE)                                                                                          \
   hipLaunchKernelGGL((gather_stream_kernel<STORE, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,             \
                      (const char *)src, src_rows, (char *)out, f, status, host_mirror, Ending<STORE>(done))

@@ -72,13 +72,17 @@ struct DoneWords {
 // 8.6 / 8.2 / 8.2 / 8.1 / 8.1, 8.0 and 9.4; 8 rows 6.3 against 8.5.
 constexpr uint32_t kDoneDirect = UGK_DONE_WORDS, kDoneFan = UGK_DONE_COUNTERS / 2;
 
+// When words are there, against a ticket kernel behind the launch (ugk_done_t::where_faster): sooner or at the same time, later
+// but by less than a kernel that copies keys takes, later than that.
+enum class Telling { kSooner, kLater, kTooLate };
+
 // The request of ugk_leave_done_words, if this thread has made one: the entry points that can fulfil it take it as they
 // begin, so that it never meets a later launch.
 class DoneRequest {
  public:
   DoneRequest();
   // grid: workgroups of the launch; count_limit: no counter of it reaches this, 0 where none are kept
-  DoneWords take(unsigned grid, uint64_t count_limit = 0);
+  DoneWords take(unsigned grid, Telling words, uint64_t count_limit = 0);
 
  private:
   ugk_done_t *_done;

@@ -567,7 +567,15 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const FlatRow f_row = flat_row(row_bytes, (uint32_t)kpw);
   const size_t keys_per_group = (size_t)kpw * kWavesPerBlock;
   const unsigned grid = clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u);
-  DoneWords done = nt && !flat ? DoneWords{} : request.take(grid, n);
+  // Rows of more than one vector per lane wait between their vectors, for memory where they are written through: a ticket behind
+  // the launch is there sooner than words (see gather_tells).  us, launch to end of poll, ticket / words, all
+  // rows in HBM: 1536 bytes x 40 10.7 / 12.1, x 5,200 14.5 / 15.6, x 20,800 21.4 / 21.8; 4 KB x 250 17.0 / 18.7, x 2,000 18.6 / 20.6,
+  // x 8,192 23.5 / 25.0, x 16,384 32.9 / 32.8; 8 KB 5 to 20 % later up to 64 MB.  With a tenth of the rows over the link 4 KB 5 to
+  // 10 % later up to 4 MB, 2 to 4 % sooner from 16 MB on.  Up to 1 KB words are 2 to 7 % sooner with a tenth of the rows over the
+  // link at any size; with all of them in HBM sooner too but for rows of more than 512 bytes and 4 to 16 MB, 3 to 5 % later.
+  const Telling words =
+      row_bytes <= 1024 || (row_bytes <= 4096 && n * row_bytes > (size_t)32 << 20) ? Telling::kSooner : Telling::kLater;
+  DoneWords done = nt && !flat ? DoneWords{} : request.take(grid, words, n);
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;
   const ugk_stage_t no_stage{};

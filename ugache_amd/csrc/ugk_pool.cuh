@@ -592,7 +592,14 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
   }
   const size_t rows_per_block = (size_t)(kWave / (shape / 100)) * kWavesPerBlock;
   const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
-  DoneWords done = request.take(grid, polled_nnz);
+  // Samples of one or two ids write about as much as they read, and where that is much more than the L2s hold written-through
+  // rows cost more than a ticket kernel behind the launch.  us, launch to end of poll, ticket / words, all rows in one place, one
+  // id per sample: 512 bytes 31 MB 22.7 / 22.9, 64 MB 33.6 / 34.7, 120 MB 51.5 / 54.3; 1 KB 48 MB 27.7 / 26.9, 64 MB 33.3 / 33.4,
+  // 120 MB 51.8 / 62.2; 2 KB 48 MB 10 % sooner, 123 MB 53.0 / 55.6; two ids 1 KB 67 MB 42.1 / 42.0, 134 MB 77.6 / 86.2; four ids 4 KB
+  // 134 MB 121.0 / 118.4.  (Behind a table, half of 262,144 rows of 512 bytes over the link, 353 / 344.)
+  const Telling words =
+      KIND != 0 || !upto2 || n_rows * (size_t)vpr * 16 <= (size_t)64 << 20 ? Telling::kSooner : Telling::kTooLate;
+  DoneWords done = request.take(grid, words, polled_nnz);
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;
   const bool mixed = keep_waves < kWavesPerBlock;
