@@ -84,7 +84,7 @@ void coll_cache_record_i64(int replica_id, const int64_t *key, size_t num_keys);
  * sparse layer, python_tf2/collcache_tf2/collcache_tf2/core/sparse_lookup_layer.py:196-209, with the unique done on the
  * GPU inside the call): output[u, :] = row of the u-th distinct key (in order of first claim, not sorted),
  * inverse_out[i] = which distinct key position i holds, so output[inverse_out[i], :] is the row of key[i].  output
- * (device) needs room for num_keys rows, inverse_out (device) for num_keys words.  Blocking.  Returns the number of
+ * (device) needs room for num_keys rows, inverse_out (device; key itself will do) for num_keys words.  Blocking.  Returns the number of
  * distinct keys. */
 size_t coll_cache_lookup_unique(int replica_id, const uint32_t *key, size_t num_keys, void *output,
                                 uint32_t *inverse_out, StreamHandle stream);

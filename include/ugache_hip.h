@@ -444,6 +444,7 @@ int ugk_gather_scatter_staged_u32(const void *host_dev, uint64_t host_rows, cons
  * reused as is by batches of any size up to the one it was sized for (slots are epoch-tagged, so no per-call
  * clearing; the layout inside depends on workspace_bytes only, which must therefore be the same on every call that
  * shares the workspace); epoch must be non-zero and different on every such call.  n_unique_dev must be zero on entry.
+ * The outputs do not overlap keys_dev: keys are still read when the first of them are written.
  * rep_out_dev (may be NULL): rep_out_dev[u] = index of the first occurrence that introduced unique key u.
  * n_unique_host (may be NULL): pinned host word that receives *n_unique_dev when the second kernel runs. */
 size_t ugk_dedup_workspace_bytes(size_t n);

@@ -145,6 +145,22 @@ int main(int argc, char **argv) {
         if (inverse[i] >= nu ||
             memcmp(out.data() + (size_t)inverse[i] * kDim, table + (size_t)k32[i] * kDim, kDim * sizeof(float)) != 0)
           ++bad_rows;
+      // the positions in place of the keys, and of the first half of wide ones
+      std::vector<uint32_t> both = k32;
+      const size_t nu32 = coll_cache_lookup_unique(0, both.data(), both.size(), out.data(), both.data(), nullptr);
+      for (size_t i = 0; i < k32.size(); ++i)
+        if (both[i] >= nu32 ||
+            memcmp(out.data() + (size_t)both[i] * kDim, table + (size_t)k32[i] * kDim, kDim * sizeof(float)) != 0)
+          ++bad_rows;
+      std::vector<int64_t> wide = k64;
+      uint32_t *half = reinterpret_cast<uint32_t *>(wide.data());
+      const size_t nu64 = coll_cache_lookup_unique_i64(0, wide.data(), wide.size(), out.data(), half, nullptr);
+      for (size_t i = 0; i < k32.size(); ++i) {
+        uint32_t at;
+        memcpy(&at, reinterpret_cast<char *>(wide.data()) + i * sizeof(at), sizeof(at));
+        if (at >= nu64 || memcmp(out.data() + (size_t)at * kDim, table + (size_t)k32[i] * kDim, kDim * sizeof(float)) != 0)
+          ++bad_rows;
+      }
     }
 
     // 4. the serving loop with its own background refresh thread

@@ -579,6 +579,11 @@ int dedup(const K *keys, size_t n, K *unique_out, uint32_t *inverse, uint32_t *r
           uint32_t *n_unique_host) {
   if (n == 0) return 0;
   REQUIRE(keys && unique_out && inverse && n_unique, "ugk_dedup: null pointer");
+  const auto apart = [&](const void *out, size_t bytes) {
+    return (uintptr_t)out + bytes <= (uintptr_t)keys || (uintptr_t)(keys + n) <= (uintptr_t)out;
+  };
+  REQUIRE(apart(inverse, n * sizeof(uint32_t)) && apart(unique_out, n * sizeof(K)) && apart(rep, n * sizeof(uint32_t)),
+          "ugk_dedup: an output overlaps the keys, which are still read when it is written");
   std::unordered_map<uint64_t, uint32_t> seen;
   uint32_t nu = *n_unique;
   for (size_t i = 0; i < n; ++i) {

@@ -1195,7 +1195,12 @@ size_t ExtractSession::ExtractUniqueImpl(const KeyT *nodes, size_t num_nodes, vo
   CHECK_NOTNULL(nodes);
   CHECK_NOTNULL(output);
   CHECK_NOTNULL(inverse_out);
-  const size_t nu = DedupKeys(nodes, num_nodes, inverse_out, stream);
+  // the deduplication reads keys while it writes positions: where a caller wants the positions in place of the keys they
+  // come by way of the session's buffer
+  const uintptr_t keys = (uintptr_t)nodes, out = (uintptr_t)inverse_out;
+  const bool apart = out + num_nodes * sizeof(uint32_t) <= keys || keys + num_nodes * sizeof(KeyT) <= out;
+  const size_t nu = DedupKeys(nodes, num_nodes, apart ? inverse_out : nullptr, stream);
+  if (!apart) UGK_CALL(ugk_memcpy_async(inverse_out, DedupInverse(), num_nodes * sizeof(uint32_t), stream));
   _skip_dedup = true;
   ExtractFeatImpl<KeyT>(DedupUnique<KeyT>(), nu, output, stream, task_key);  // blocks: the kernels above are done too
   _skip_dedup = false;
