@@ -145,8 +145,9 @@ int ugk_word_wait(const uint32_t *word_host, uint32_t value, unsigned spin_us, v
 /* The end of one launch polled for without a kernel behind it.  ugk_leave_done_words: the next ugk_gather_*,
  * ugk_extract_mix_* or ugk_extract_pool_* call of this thread (that one only; after a call that failed, and where none
  * comes, NULL takes the request back) makes its workgroups leave words in words_host as they end, and stores the number of
- * words in done->num_words before it returns: 0 where the launch cannot (outputs written with non-temporal stores, nothing
- * to do, counts of 2^24 and more), and the caller then waits for the stream in another way.  With words a launch leaves no
+ * words in done->num_words before it returns: 0 where the launch cannot (outputs written with non-temporal stores, gathers
+ * other than ugk_gather_direct_*, samples of mostly one id combined as a list, nothing to do, counts of 2^24 and more), and
+ * the caller then waits for the stream in another way.  With words a launch leaves no
  * group_counts_host and *num_groups_host is 0.  ugk_done_wait polls them for up to
  * spin_us microseconds before it falls back to waiting for the stream, and returns with the two group sizes of the launch
  * (0 where it keeps none; either may be NULL).  What the launch wrote is complete then, for kernels and copies on any

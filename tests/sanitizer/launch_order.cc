@@ -4,6 +4,7 @@
 //
 // usage: launch_order <libugache_hip.so> place <rows>                          a placement with a ticket
 //                                       gather <row bytes> <rows> <words>
+//                                       scatter <row bytes> <rows> <words>            and a direct gather behind it
 //                                       mix <row bytes> <rows> <words>
 //                                       pool <id bytes> <row bytes> <ids> <samples> <max norm> <words>
 // words: 0: nobody polls, 1: words are asked for (ugk_leave_done_words), 2: where they are faster, 3: and a key with them.  Prints a line per launch, the kernel, its template
@@ -146,6 +147,12 @@ int main(int argc, char **argv) {
   } else if (call == "gather" && argc == 6 && ask(number(5))) {
     const auto fn = reinterpret_cast<decltype(&ugk_gather_direct_i64)>(dlsym(lib, "ugk_gather_direct_i64"));
     rc = fn(dev(1), 1000, static_cast<int64_t *>(dev(2)), number(4), dev(3), number(3), 0, u32, nullptr, dev(11));
+  } else if (call == "scatter" && argc == 6 && ask(number(5))) {
+    const auto fn = reinterpret_cast<decltype(&ugk_gather_scatter_i64)>(dlsym(lib, "ugk_gather_scatter_i64"));
+    const auto next = reinterpret_cast<decltype(&ugk_gather_direct_i64)>(dlsym(lib, "ugk_gather_direct_i64"));
+    rc = fn(dev(1), 1000, static_cast<int64_t *>(dev(2)), static_cast<uint32_t *>(dev(4)), number(4), dev(3), 1000, number(3), 0, u32,
+            nullptr, dev(11)) ||
+         next(dev(1), 1000, static_cast<int64_t *>(dev(2)), number(4), dev(3), number(3), 0, u32, nullptr, dev(11));
   } else if (call == "mix" && argc == 6 && ask(number(5))) {
     ugk_table_t flat{};
     flat.kind = 1, flat.table = dev(4), flat.size = 1000;

@@ -81,3 +81,12 @@ def test_a_pooled_lookup_is_told_its_end_by_words_where_they_are_sooner(launches
     samples = int(mb * 1e6 / row_bytes)
     words = [launches("pool", 8, row_bytes, samples * bag, samples, 0, how)[1] for how in range(4)]
     assert words[0] == 0 and words[1] > 0 and (words[2] > 0) == (words[3] > 0) == told
+
+
+@pytest.mark.parametrize("row_bytes", [512, 404, 12, 3])
+@pytest.mark.parametrize("words", [1, 3])
+def test_a_scattering_gather_takes_the_request_and_leaves_no_words(launches, row_bytes, words):
+    """its keys are not those of its output rows, so it could not leave them; nor does the next call see the request"""
+    done, left = launches("scatter", row_bytes, 1000, words)
+    assert left == 0 and len(done) == 2
+    assert not any("Store)2" in templ for _, templ, _, _ in done)

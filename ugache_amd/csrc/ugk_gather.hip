@@ -489,13 +489,22 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
   constexpr size_t kPerIter = (size_t)(kBlock / LPR) * UNROLL;
   const unsigned grid = gather_grid((n + kPerIter - 1) / kPerIter, max_blocks);
   const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
-  const DoneWords done = nt ? DoneWords{} : request.take(grid, gather_tells(sizeof(V), vpr, LPR, n * (size_t)vpr * sizeof(V)));
+  DoneWords done{};
+  if constexpr (Idx::kDense) {
+    if (!nt) done = request.take(grid, gather_tells(sizeof(V), vpr, LPR, n * (size_t)vpr * sizeof(V)));
+  }
 #define UGK_GO(STORE)                                                                                                  \
   hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,            \
                      reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,   \
                      group, many_groups, n, status, host_mirror, Ending<STORE>(done))
-  if (done.tag) UGK_GO(kThrough);
-  else if (nt) UGK_GO(kStreaming);
+  if constexpr (Idx::kDense) {
+    if (done.tag) {
+      UGK_GO(kThrough);
+      UGK_HIP(hipGetLastError());
+      return 0;
+    }
+  }
+  if (nt) UGK_GO(kStreaming);
   else UGK_GO(kOrdinary);
 #undef UGK_GO
   UGK_HIP(hipGetLastError());
@@ -593,13 +602,19 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
   const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes, n));
   const size_t per_block = (size_t)f.tile * kWavesPerBlock;
   const unsigned grid = gather_grid((n + per_block - 1) / per_block, max_blocks);
-  const DoneWords done = request.take(grid, Telling::kSooner);
-  if (done.tag)
-    hipLaunchKernelGGL((gather_flat_kernel<kThrough, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,
-                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<kThrough>(done));
-  else
-    hipLaunchKernelGGL((gather_flat_kernel<kOrdinary, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,
-                       src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<kOrdinary>(done));
+#define UGK_GO(STORE, DONE)                                                                                            \
+  hipLaunchKernelGGL((gather_flat_kernel<STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,     \
+                     src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<STORE>(DONE))
+  if constexpr (Idx::kDense) {
+    const DoneWords done = request.take(grid, Telling::kSooner);
+    if (done.tag) {
+      UGK_GO(kThrough, done);
+      UGK_HIP(hipGetLastError());
+      return 0;
+    }
+  }
+  UGK_GO(kOrdinary, DoneWords{});
+#undef UGK_GO
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -631,7 +646,7 @@ template <typename Idx>
 int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, size_t row_bytes,
                   const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
                   uint32_t *host_mirror, void *stream) {
-  DoneRequest request;
+  DoneRequest request;  // (of which only gathers whose row i is output row i make use)
   if (n == 0) return 0;
   UGK_REQUIRE(src && out, "gather: null source or output");
   UGK_REQUIRE(status, "gather: null status word");
@@ -738,6 +753,7 @@ int ugk_gather_scatter_staged_u32(const void *host_dev, uint64_t host_rows, cons
                                   size_t row_bytes, ugk_stage_t stage, unsigned max_blocks, uint32_t *status_dev,
                                   uint32_t *staged_dev, uint32_t *rest_rows_dev, uint32_t *rest_dst_dev,
                                   uint32_t *rest_count_dev, uint32_t *done_count_dev, void *stream) {
+  DoneRequest request;
   if (n == 0) return 0;
   UGK_REQUIRE(rest_count_dev == nullptr || (rest_rows_dev && rest_dst_dev),
               "ugk_gather_scatter_staged_u32: a rest count without the two rest lists");
