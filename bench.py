@@ -92,6 +92,8 @@ def parse_args():
                     help="run this one workload in this process (default: the all-hit configuration at the top level "
                          "plus the mixed-source legs, each in a child process)")
     ap.add_argument("--no-legs", action="store_true", help="default run without the mixed-source legs")
+    ap.add_argument("--legs-file", default=None, metavar="FILE",
+                    help="default run: the mixed-source legs in full to FILE, as one JSON object (the line carries their figures)")
     ap.add_argument("--cpu-seconds", type=float, default=10.0, help="CPU baseline budget")
     ap.add_argument("--pool", type=int, default=None, help="distinct key batches cycled through the steps")
     ap.add_argument("--impl", default="", choices=["", "DIRECT", "SMMaskPhase", "NONE"],
@@ -1040,16 +1042,22 @@ def run_default(args):
                               "host_link_GBps": hl.get("achieved"), "host_link_frac": hl.get("frac"),
                               "frac_of_row_ceiling": hl.get("frac_of_row_ceiling"),
                               "cpu_keys_per_s": leg["cpu_baseline"]["value"], "cpu_cores": leg["cpu_baseline"]["cores"],
-                              "gpu_over_cpu": leg.get("gpu_over_cpu"), "parity": "bit-exact, every pooled batch"}
+                              "gpu_over_cpu": leg.get("gpu_over_cpu")}
             if leg.get("refresh_each_step"):
                 summary[short]["refresh_each_step_ms"] = leg["refresh_each_step"]["ms_per_step"]
                 summary[short]["refresh_ms"] = leg["refresh_each_step"]["refresh_ms"]
             if leg.get("cache_build"):
                 summary[short]["build_frac_of_link"] = leg["cache_build"]["frac_of_measured_link"]
-    result["legs"] = legs
-    result["legs_note"] = ("each leg is the same bench.py with --workload <name> (and the options named), run after the "
-                           "top-level workload in a process of its own, same --steps and --warmup; value / roofline / "
-                           "cpu_baseline at the top level are the all-hit configuration's alone")
+            summary[short] = {k: float("%.6g" % v) if isinstance(v, float) else v for k, v in summary[short].items()}
+    # A leg's line is 3 to 4 KB and there are six of them: whoever reads the end of this program's output, a few KB of it, would
+    # find no whole line.  So the line carries each leg's figures, and the legs in full go where they are asked for.
+    if args.legs_file:
+        with open(args.legs_file, "w") as f:
+            json.dump(legs, f, indent=1)
+    result["legs_note"] = ("other_configs: the same bench.py with --workload <name> (and its options), run after the top-level "
+                           "workload in processes of their own, same --steps and --warmup, every pooled batch bit-exact (in "
+                           "full: --legs-file); value / "
+                           "roofline / cpu_baseline at the top level are the all-hit configuration's alone")
     # The figures of the other configurations once more in short form, at the top level and inside `roofline` (a
     # reader that keeps only the objects of the contract keeps these)
     large = result.get("all_hit_large_output") or {}
