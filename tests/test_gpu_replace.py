@@ -406,9 +406,10 @@ def test_bitmap_emit_diff_writes_both_lists_as_two_emits_would(nbits, shape):
         total.free()
 
 
-# chunks of one block, of two and (beyond 2^26 bits) of more; the pass that adds the chunk counts up itself and the one
-# behind a scan
-@pytest.mark.parametrize("nbits", [1, 4096, 8192, (1 << 25) - 1, 1 << 25, (1 << 25) + 1, 1 << 26, (1 << 26) + 1])
+# chunks of one block, of two and (beyond 2^26 bits) of more; workgroups of one wavefront (up to 512 chunks), of two and of
+# sixteen, with and without one that has no chunk; the pass that adds the chunk counts up itself and the one behind a scan
+@pytest.mark.parametrize("nbits", [1, 4096, 8192, 1 << 21, (1 << 21) + 1, (1 << 21) + 4097, (1 << 24) - 4096 * 3, (1 << 25) - 1,
+                                   1 << 25, (1 << 25) + 1, 1 << 26, (1 << 26) + 1])
 @pytest.mark.parametrize("scanned", [False, True])
 def test_bitmap_lists_at_the_edges_of_the_emit_passes(nbits, scanned):
     gen = torch.Generator(device="cuda").manual_seed(nbits)

@@ -759,15 +759,16 @@ __global__ __launch_bounds__(kBlock) void bitmap_count_diff_kernel(const unsigne
 // one workgroup of kScanBlock threads: the counts of the chunks become their prefix
 template <bool THROUGH>
 __device__ __forceinline__ void scan_ws(BmWs *ws, uint32_t *total_host) {
-  auto put = [](auto *to, auto v) {
+  auto put = [](uint32_t *to, auto v) {
+    typedef decltype(v) __attribute__((aligned(4))) by4_t;
     if constexpr (THROUGH) store_through(reinterpret_cast<uint64_t>(to), v);
-    else *to = v;
+    else *reinterpret_cast<by4_t *>(to) = v;
   };
   uint32_t pre[8], total;
   scan_chunks(ws->base, pre, total);
-  u32x4_by4 *to = reinterpret_cast<u32x4_by4 *>(ws->base) + 2 * threadIdx.x;
+  uint32_t *to = ws->base + 8 * threadIdx.x;
   put(to, u32x4{pre[0], pre[1], pre[2], pre[3]});
-  put(to + 1, u32x4{pre[4], pre[5], pre[6], pre[7]});
+  put(to + 4, u32x4{pre[4], pre[5], pre[6], pre[7]});
   if (threadIdx.x == 0) {
     put(&ws->total, total);
     put(&ws->scanned, 1u);
@@ -810,6 +811,10 @@ constexpr uint32_t kEmitDense = 2 * kWave;
 __device__ __forceinline__ uint32_t set_bits_upto(unsigned long long m) {  // in the words of this lane and the ones below
   return wave_incl_sum(__popcll(m));
 }
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {  // a value that all lanes have, in scalar registers
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32)) << 32) |
+         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x);
+}
 __device__ __forceinline__ void emit_word(unsigned long long m, uint32_t incl, uint32_t n_set, uint64_t pos0, uint64_t w,
                                           int lane, uint32_t *out, uint64_t max_out) {
   const uint32_t excl = incl - __popcll(m);
@@ -823,17 +828,33 @@ __device__ __forceinline__ void emit_word(unsigned long long m, uint32_t incl, u
     }
     return;
   }
-  const uint64_t w_first = w - (uint64_t)lane;
-  const unsigned long long below = (1ull << lane) - 1ull;
-  unsigned long long todo = __ballot(m != 0ull);
-  while (todo) {  // wavefront-uniform
-    const int src = __builtin_ctzll(todo);
-    todo &= todo - 1;
-    const unsigned long long word =
-        ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(m >> 32), src) << 32) |
-        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)m, src);
-    const uint64_t pos = pos0 + (uint32_t)__builtin_amdgcn_readlane((int)excl, src) + __popcll(word & below);
-    if (((word >> lane) & 1ull) && pos < max_out) out[pos] = (uint32_t)((w_first + src) * 64 + lane);
+  if (pos0 >= max_out) return;
+  // What is the same in all lanes is in scalar registers, so that a word is two bit counts, the value and the store, and the
+  // positions of four words are worked out before the first of them is stored (unrolled further the code of a block no longer
+  // stays in the instruction cache beside the rest: lists of scattered bits 1.5 us longer).
+  const uint64_t blk_pos = uniform64(pos0), room64 = max_out - blk_pos;
+  const uint32_t room = room64 < n_set ? (uint32_t)room64 : n_set;  // entries of the block that the list has room for
+  const uint32_t w_first = (uint32_t)uniform64(w - (uint64_t)lane);
+  uint32_t *const to = out + blk_pos;
+  const unsigned long long todo = __ballot(m != 0ull);
+  constexpr int kAtOnce = 4;
+#pragma unroll 1
+  for (int src = 0; src < kWave; src += kAtOnce) {  // wavefront-uniform
+    if (((todo >> src) & ((1u << kAtOnce) - 1u)) == 0) continue;
+    unsigned long long word[kAtOnce];
+    uint32_t pos[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) {
+      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)m, src + u);
+      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(m >> 32), src + u);
+      const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)excl, src + u);
+      word[u] = ((unsigned long long)hi << 32) | lo;
+      pos[u] = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, before));
+    }
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u)
+      if (__builtin_amdgcn_inverse_ballot_w64(word[u]) && pos[u] < room)
+        to[pos[u]] = (w_first + (uint32_t)(src + u)) * 64 + (uint32_t)lane;
   }
 }
 
@@ -947,17 +968,29 @@ __global__ __launch_bounds__(kBlock) void bitmap_emit_diff_kernel(const unsigned
   }
 }
 
-// The emit pass over a bitmap of up to kSmallBits bits, whose chunks are at most kSmallBlocks blocks long: a workgroup of a
-// wavefront per chunk.  The words are asked for together with the counts of the chunks in front of the workgroup, which it adds up
-// itself where no scan has run: one round of reads, and no one-workgroup launch between the count and this one (40 M
-// bits, 72,000 rows that leave and as many that come: 7.9 us, against 5.0 for the scan and 8.0; 72,000 free slots among 4 M:
-// 11.3 against 5.7 and 9.0, and a hand-over less).  Longer chunks would make a wavefront of a dense one work long after
+// The emit pass over a bitmap of up to kSmallBits bits, whose chunks are at most kSmallBlocks blocks long: a wavefront per chunk, which
+// asks for its words together with the counts it needs to know its place, where no scan has run: one round of reads, and
+// no one-workgroup launch between the count and this one.  Longer chunks would make a wavefront of a dense one work long after
 // the others.
+// Wavefront v of workgroup b takes chunk v * grid + b, so that neighbouring chunks, which are dense together where rows or slots are
+// set in one run, are on different CUs, and adds up the counts of its strip of the chunks, v * grid and on: all of
+// them for the other wavefronts of the workgroup, those in front of its own chunk for itself.
+// us, the list alone / a scan and a wavefront per 64-word block (what it replaces) / a workgroup taking neighbouring chunks, one word at a
+// time with its positions in 64-bit vector registers: 50.5 M bits, 461,000 of them in one run 10.6 / 5.0 + 8.8 / 24.0, scattered 5.5 /
+// 5.0 + 6.3 / 5.5, 5 M in one run 15.0 / 5.0 + 12.1 / 26.0; 4 M bits, 72,000 in one run 6.2 / 5.0 + 8.0 / 10.8, scattered 4.0 / 5.0 + 3.9 /
+// 4.0, all 9.1 / 5.0 + 10.4 / 15.4; 100,000 bits, all 6.1 / 5.0 + 8.2 / 12.8; two lists out of 40 M bits, 72,000 each, scattered 6.2 /
+// 5.0 + 6.6 / 6.6, one of them a run 10.9 / 5.0 + 8.5 / 14.7, 60 M bits and 461,000 each 13.8 / 5.0 + 9.3 / 25.2.
 constexpr uint64_t kSmallBlocks = 2, kSmallBits = (uint64_t)kBmChunks * kSmallBlocks * kWave * 64;
-constexpr int kSmallBlock = 1024, kSmallWaves = kSmallBlock / kWave;
-static inline unsigned small_grid(uint64_t nbits, uint64_t per_chunk) {
-  return (unsigned)(((nbits + 63) / 64 + per_chunk * kSmallWaves - 1) / (per_chunk * kSmallWaves));
-}
+constexpr uint32_t kSmallStrip = 512, kSmallWaves = kBmChunks / kSmallStrip;
+struct SmallGrid {
+  unsigned groups, threads;
+  SmallGrid(uint64_t nbits, uint64_t per_chunk) {
+    const uint32_t chunks = (uint32_t)(((nbits + 63) / 64 + per_chunk - 1) / per_chunk);  // that hold any word
+    const uint32_t waves = (chunks + kSmallStrip - 1) / kSmallStrip;
+    groups = (chunks + waves - 1) / waves;
+    threads = waves * kWave;
+  }
+};
 struct BmList {
   const BmWs *ws;
   uint32_t *out;
@@ -965,16 +998,17 @@ struct BmList {
 };
 // sets S of one (LISTS == 1: bm_word's of a and b) or two lists (a & ~b, b & ~a); total_host (LISTS == 1): |S|
 template <int LISTS>
-__global__ __launch_bounds__(kSmallBlock) void bitmap_emit_small_kernel(const unsigned long long *a,
-                                                                        const unsigned long long *b, int flags,
-                                                                        uint64_t nbits, uint64_t per_chunk, BmList first,
-                                                                        BmList second, uint32_t *total_host) {
+__global__ __launch_bounds__(kSmallWaves * kWave) void bitmap_emit_small_kernel(const unsigned long long *a,
+                                                                                const unsigned long long *b, int flags,
+                                                                                uint64_t nbits, uint64_t per_chunk,
+                                                                                BmList first, BmList second,
+                                                                                uint32_t *total_host) {
   __shared__ uint32_t part[LISTS][kSmallWaves];
   const BmList list[2] = {first, second};
-  const int tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
+  const int lane = (int)lane_id(), wv = (int)wave_in_block(), waves = (int)(blockDim.x / kWave);
   const uint64_t n_words = (nbits + 63) / 64;
-  const uint32_t chunk0 = blockIdx.x * kSmallWaves;
-  const uint64_t w_first = (uint64_t)(chunk0 + wv) * per_chunk + lane;
+  const uint32_t strip = (uint32_t)wv * gridDim.x, chunk = strip + blockIdx.x;  // below kBmChunks
+  const uint64_t w_first = (uint64_t)chunk * per_chunk + lane;
   unsigned long long m[LISTS][kSmallBlocks];
 #pragma unroll
   for (uint64_t j = 0; j < kSmallBlocks; ++j) {
@@ -990,35 +1024,39 @@ __global__ __launch_bounds__(kSmallBlock) void bitmap_emit_small_kernel(const un
       m[1][j] = wb & ~wa & valid;
     }
   }
-  // the counts in front of the workgroup, and of its own chunks (a chunk behind the last word has a count of zero)
-  uint32_t before[LISTS], own[LISTS], scanned[LISTS];
+  // (a chunk behind the last word has a count of zero)
+  uint32_t front[LISTS], sum[LISTS], own[LISTS], scanned[LISTS], all[LISTS];
 #pragma unroll
   for (int l = 0; l < LISTS; ++l) {
     const uint32_t *counts = list[l].ws->base;
     scanned[l] = list[l].ws->scanned;
-    own[l] = counts[chunk0 + lane % kSmallWaves];
-    before[l] = 0;
+    all[l] = list[l].ws->total;
+    own[l] = counts[chunk];
+    front[l] = sum[l] = 0;
 #pragma unroll
-    for (int q = 0; q < kBmChunks / kSmallBlock; ++q) {
-      const uint32_t c = q * kSmallBlock + tid;
-      const uint32_t n = counts[c];
-      if (c < chunk0) before[l] += n;
+    for (uint32_t q = 0; q < kSmallStrip / kWave; ++q) {
+      const uint32_t c = q * kWave + lane;
+      const uint32_t n = counts[strip + min(c, gridDim.x - 1)];
+      if (c < gridDim.x) sum[l] += n;
+      if (c < blockIdx.x) front[l] += n;
     }
   }
 #pragma unroll
   for (int l = 0; l < LISTS; ++l) {
-    before[l] = wave_sum(before[l]);
-    if (lane == 0) part[l][wv] = before[l];
+    front[l] = wave_sum(front[l]);
+    sum[l] = wave_sum(sum[l]);
+    if (lane == 0) part[l][wv] = sum[l];
   }
   __syncthreads();
 #pragma unroll
   for (int l = 0; l < LISTS; ++l) {
-    // (lane q of the first sixteen: what wavefront q added up, and the count of its chunk)
-    const uint32_t front = wave_sum(lane < kSmallWaves ? part[l][lane] : 0u);
-    uint32_t pos = front + wave_sum(lane < wv ? own[l] : 0u);
-    uint32_t all = front + wave_sum(lane < kSmallWaves ? own[l] : 0u);
-    if (scanned[l]) pos = __shfl(own[l], wv), all = list[l].ws->total;
-    if (LISTS == 1 && total_host && blockIdx.x == gridDim.x - 1 && tid == 0) *total_host = all;
+    const uint32_t others = lane < waves ? part[l][lane] : 0u;
+    uint32_t pos = front[l] + wave_sum(lane < wv ? others : 0u);
+    if (scanned[l]) pos = own[l];
+    if (LISTS == 1 && total_host && blockIdx.x == 0 && wv == 0) {
+      const uint32_t total = scanned[l] ? all[l] : wave_sum(others);
+      if (lane == 0) *total_host = total;
+    }
 #pragma unroll
     for (uint64_t j = 0; j < kSmallBlocks; ++j) {
       if (__ballot(m[l][j] != 0ull) == 0ull) continue;
@@ -1281,7 +1319,8 @@ int ugk_bitmap_emit_counted(const uint64_t *a_dev, const uint64_t *b_dev, int in
   const uint64_t n_words = (nbits + 63) / 64;
   const uint64_t per_chunk = bm_words_per_chunk(n_words);
   if (nbits <= kSmallBits) {
-    hipLaunchKernelGGL((bitmap_emit_small_kernel<1>), dim3(small_grid(nbits, per_chunk)), dim3(kSmallBlock), 0, as_stream(stream),
+    const SmallGrid grid(nbits, per_chunk);
+    hipLaunchKernelGGL((bitmap_emit_small_kernel<1>), dim3(grid.groups), dim3(grid.threads), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long *>(a_dev),
                        reinterpret_cast<const unsigned long long *>(b_dev), invert_a ? kBmInvertA : 0, nbits, per_chunk,
                        BmList{static_cast<const BmWs *>(ws_dev), out_dev, max_out}, BmList{nullptr, nullptr, 0}, total_host);
@@ -1309,7 +1348,8 @@ int ugk_bitmap_emit_diff(const uint64_t *a_dev, const uint64_t *b_dev, uint64_t 
   const uint64_t n_words = (nbits + 63) / 64;
   const uint64_t per_chunk = bm_words_per_chunk(n_words);
   if (nbits <= kSmallBits) {
-    hipLaunchKernelGGL((bitmap_emit_small_kernel<2>), dim3(small_grid(nbits, per_chunk)), dim3(kSmallBlock), 0, as_stream(stream),
+    const SmallGrid grid(nbits, per_chunk);
+    hipLaunchKernelGGL((bitmap_emit_small_kernel<2>), dim3(grid.groups), dim3(grid.threads), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long *>(a_dev),
                        reinterpret_cast<const unsigned long long *>(b_dev), 0, nbits, per_chunk,
                        BmList{static_cast<const BmWs *>(ws_ab_dev), out_ab_dev, max_ab},
