@@ -89,7 +89,8 @@ __device__ __forceinline__ void st_stream(V *p, V v) {
 // 512 bytes x 65,536 15.5 / 14.7, x 262,144 45.5 / 44.8 (6.0 TB/s); 1 KB x 32,768 15.5 / 14.7, x 262,144 83.1 / 81.5; 4 KB x 2,048
 // 6.8 / 6.4, x 8,192 15.5 / 14.1, x 131,072 193 / 188; 128 bytes x 196,608 13.4 / 12.2.  A launch that is all on the chip at
 // once is no faster for it and up to 5 % slower near that size: 512 bytes x 16,384 5.8 / 5.7, x 32,768 8.5 / 9.0, x 36,000
-// 10.5 / 10.3, 64 bytes x 262,144 11.3 / 11.7, 128 bytes x 131,072 8.7 / 9.1.  Rows in flight per lane, one / two / four /
+// 10.5 / 10.3, 64 bytes x 262,144 11.3 / 11.7, 128 bytes x 131,072 8.7 / 9.1.  (Of the rows of several vectors per lane 2 KB x
+// 7,812 with skewed keys and 8 KB x 7,812, about half of one round, lose: 7.1 / 7.5 and 24.4 / 25.8.)  Rows in flight per lane, one / two / four /
 // eight, all without: 512 bytes x 65,536 15.9 / 14.7 / 15.1 / 15.5, x 524,288 91.1 / 82.4 / 82.5 / 83.5; 4 KB x 32,768 43.4 /
 // 43.4 / 51.9 / 48.4; 16 bytes x 32,768 3.8 / 4.5 / 5.8 / 9.0.
 template <typename V, int LPR, int UNROLL, Store STORE, typename Idx>
