@@ -7,8 +7,10 @@
 //                                       scatter <row bytes> <rows> <words>            and a direct gather behind it
 //                                       mix <row bytes> <rows> <words>
 //                                       pool <id bytes> <row bytes> <ids> <samples> <max norm> <words>
-// words: 0: nobody polls, 1: words are asked for (ugk_leave_done_words), 2: where they are faster, 3: and a key with them.  Prints a line per launch, the kernel, its template
-// arguments, the stream and the other arguments, and how many words the call says it leaves.
+//                                       lists <bits>                                  one out of a bitmap, two out of two
+// words: 0: nobody polls, 1: words are asked for (ugk_leave_done_words), 2: where they are faster, 3: and a key with them.
+// Prints a line per launch, the kernel, its template arguments, the stream, workgroups x threads and the other arguments, and how
+// many words the call says it leaves.
 #include <cxxabi.h>
 #include <dlfcn.h>
 
@@ -95,15 +97,15 @@ int hipDeviceGetAttribute(int *value, int, int) {
   return 0;
 }
 int hipGetLastError() { return 0; }
-int hipLaunchKernel(const void *f, Dim3, Dim3, void **args, size_t, void *stream) {
+int hipLaunchKernel(const void *f, Dim3 grid, Dim3 block, void **args, size_t, void *stream) {
   const std::string &name = kernels()[f];
   const size_t end = name.find("_kernel") + 7, begin = name.rfind("::", end) == std::string::npos ? 0 : name.rfind("::", end) + 2;
   size_t open = 0;
   const std::vector<std::string> types = parameters(name, &open);
   std::string templ = name.substr(end, open - end);
   for (size_t i; (i = templ.find(' ')) != std::string::npos;) templ.erase(i, 1);
-  printf("%s %s stream=%llx", name.substr(begin, end - begin).c_str(), templ.empty() ? "<>" : templ.c_str(),
-         (unsigned long long)(uintptr_t)stream);
+  printf("%s %s stream=%llx %ux%u", name.substr(begin, end - begin).c_str(), templ.empty() ? "<>" : templ.c_str(),
+         (unsigned long long)(uintptr_t)stream, grid.x, block.x);
   for (size_t i = 0; i < types.size(); ++i) {
     unsigned long long v = 0;
     const std::string &t = types[i];
@@ -144,6 +146,12 @@ int main(int argc, char **argv) {
     rc = fn(static_cast<uint32_t *>(dev(1)), number(3), number(3) / 2, dev(2), static_cast<uint64_t *>(dev(3)),
             static_cast<uint64_t *>(dev(4)), 1, static_cast<uint64_t *>(dev(6)), dev(7), dev(8), u32, static_cast<uint32_t *>(dev(10)),
             0xabcd, dev(11));
+  } else if (call == "lists") {
+    const auto one = reinterpret_cast<decltype(&ugk_bitmap_emit)>(dlsym(lib, "ugk_bitmap_emit"));
+    const auto two = reinterpret_cast<decltype(&ugk_bitmap_emit_diff)>(dlsym(lib, "ugk_bitmap_emit_diff"));
+    uint64_t *a = static_cast<uint64_t *>(dev(1)), *b = static_cast<uint64_t *>(dev(2));
+    rc = one(a, nullptr, 0, number(3), dev(7), u32, number(3), dev(11)) ||
+         two(a, b, number(3), dev(7), dev(8), u32, number(3), static_cast<uint32_t *>(dev(10)), number(3), dev(11));
   } else if (call == "gather" && argc == 6 && ask(number(5))) {
     const auto fn = reinterpret_cast<decltype(&ugk_gather_direct_i64)>(dlsym(lib, "ugk_gather_direct_i64"));
     rc = fn(dev(1), 1000, static_cast<int64_t *>(dev(2)), number(4), dev(3), number(3), 0, u32, nullptr, dev(11));

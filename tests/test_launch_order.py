@@ -23,7 +23,8 @@ def launches():
                              stdout=subprocess.PIPE, text=True).stdout
         *lines, (word, n) = [ln.split() for ln in out.splitlines()]
         assert word == "words"
-        return [(ln[0], ln[1], ln[2], [int(w, 16) for w in ln[3:]]) for ln in lines], int(n)
+        run.grids = [tuple(map(int, ln[3].split("x"))) for ln in lines]
+        return [(ln[0], ln[1], ln[2], [int(w, 16) for w in ln[4:]]) for ln in lines], int(n)
 
     return run
 
@@ -90,3 +91,17 @@ def test_a_scattering_gather_takes_the_request_and_leaves_no_words(launches, row
     done, left = launches("scatter", row_bytes, 1000, words)
     assert left == 0 and len(done) == 2
     assert not any("Store)2" in templ for _, templ, _, _ in done)
+
+
+@pytest.mark.parametrize("nbits", [1, 4096, 100_000, 1 << 21, (1 << 21) + 1, 4_000_000, (1 << 25) + 1, 50_500_000, 1 << 26])
+def test_lists_out_of_a_bitmap_are_dealt_out_over_the_chip(launches, nbits):
+    """a wavefront per chunk that holds any bit; set bits in one run are in a few neighbouring chunks, so there are as many
+    workgroups as chunks, or hundreds of them, and no wavefront at or beyond the 8,192 counts of a workspace"""
+    words = (nbits + 63) // 64
+    per_chunk = ((words + 8191) // 8192 + 63) // 64 * 64
+    chunks = (words + per_chunk - 1) // per_chunk
+    done, _ = launches("lists", nbits)
+    assert [kernel for kernel, _, _, _ in done] == ["bitmap_emit_small_kernel"] * 2
+    for groups, threads in launches.grids:
+        assert threads % 64 == 0 and threads <= 1024
+        assert groups >= min(chunks, 250) and chunks <= groups * (threads // 64) <= 8192
