@@ -1367,6 +1367,60 @@ def test_pooled_sample_does_not_depend_on_the_others_of_its_batch(kind, vpr):
         pin.free()
 
 
+@pytest.mark.parametrize("kind", ["none", "flat", "hash", "hash32"])
+@pytest.mark.parametrize("vpr", [1, 4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 128, 129, 256])
+def test_pooled_batch_of_few_samples_is_the_batch_of_many(kind, vpr):
+    """a sample per workgroup, per wavefront or per lane group, as the number of samples decides: the same bytes for the same
+    samples, of 0 to 300 ids (rounds of 64 and 256 ids, and tiles of rows, end inside them), and the float64 segment sums with
+    the bounds of the shapes' edges ((300 + 2) 2^-24, twice that with the sum of weights: 4e-5)"""
+    rng = np.random.default_rng(vpr)
+    nkeys, rb, probes = 2_000, vpr * 16, 70
+    pin = pinned_from(np.zeros((nkeys, rb), np.uint8))
+    cached = rng.choice(nkeys, nkeys // 2, replace=False).astype(np.int64)
+    lens = np.concatenate([rng.integers(0, 90, size=probes - 6), [0, 63, 64, 65, 257, 300]])
+    ids = np.concatenate([rng.integers(0, nkeys, size=n) for n in lens]).astype(np.int64)
+    wts = (rng.random(len(ids)) + 0.5).astype(np.float32)
+    others = 20 if vpr <= 64 else 10
+    try:
+        for dt in (np.float32, np.float16):
+            host = rng.standard_normal((nkeys, rb // np.dtype(dt).itemsize)).astype(dt)
+            pin.array[...] = host.view(np.uint8).reshape(nkeys, rb)
+            cache, f64 = host[cached].view(np.uint8).reshape(len(cached), rb).copy(), host.astype(np.float64)
+            if kind == "none":
+                mem, tb = None, hip.table(0, None, 0)
+            else:
+                mem, tb = {"flat": lambda: _make_flat(nkeys), "hash": lambda: _make_hash(len(cached))[:2],
+                           "hash32": lambda: _make_hash32(len(cached))[:2]}[kind]()
+                assert _insert(tb, cached) == 0
+            d_cache, st = to_dev(cache), dev_zeros_u32(1)
+            for combiner in (0, 1, 2):
+                seen = []
+                for more in (0, 900, 1900, 3900, 20_000 if combiner == 1 else 0):  # up to 2, 4, 8 and 16 samples per CU, and more
+                    all_ids = np.concatenate([ids, rng.integers(0, nkeys, size=more * others)]).astype(np.int64)
+                    all_w = np.concatenate([wts, np.ones(more * others, np.float32)])
+                    off = np.concatenate([[0], np.cumsum(np.concatenate([lens, np.full(more, others)]))]).astype(np.int64)
+                    out = dev_bytes((probes + more) * rb + 64, fill=0x7F)
+                    d_ids, d_off, d_w = to_dev(all_ids), to_dev(off), to_dev(all_w)
+                    hip.call("ugk_extract_pool_i64", tb, ptr(d_ids), ptr(d_off), ptr(d_w), probes + more, len(all_ids), combiner,
+                             np.dtype(dt).itemsize, ptr(d_cache), 0 if kind == "none" else len(cached), pin.ptr, nkeys, ptr(out),
+                             rb, ptr(st), None, None, None, None)
+                    assert status_value(st) == 0
+                    raw = to_np(out)
+                    assert (raw[(probes + more) * rb : (probes + more) * rb + 64] == 0x7F).all()
+                    seen.append(raw[: probes * rb].tobytes())
+                assert all(b == seen[0] for b in seen), (combiner, [b == seen[0] for b in seen])
+                got = np.frombuffer(seen[0], dt).reshape(probes, -1).astype(np.float64)
+                off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+                want = _pool_reference(f64, ids, off, wts, combiner)
+                bound = 4e-5 * _pool_reference(np.abs(f64), ids, off, wts, combiner) + 1e-30
+                if dt == np.float16:
+                    bound = bound + 2.0 ** -11 * np.abs(want) + 2.0 ** -25
+                assert (np.abs(got - want) <= bound).all(), combiner
+    finally:
+        sync()
+        pin.free()
+
+
 @pytest.mark.parametrize("rows_per_group", ["", "2", "8"])
 def test_pooled_extraction_hand_worked(rows_per_group, monkeypatch):
     if rows_per_group:

@@ -6,6 +6,7 @@
 #include <hip/hip_fp16.h>
 
 #include <cstdlib>
+#include <type_traits>
 
 #include "ugk_internal.h"
 #include "ugk_mix.cuh"
@@ -272,6 +273,166 @@ __device__ __forceinline__ void pool_samples(const ugk_table_t &t, const K *__re
   }
 }
 
+
+// A sample per workgroup, for batches of few samples with many ids each.  What such a launch takes is not bandwidth but the
+// chain of a sample: a lane group that resolves LPR ids at a time and keeps U rows on their way goes through the ids of a
+// sample of 40 in ten rounds trips to memory and three lookups, on a chip that is mostly idle.  Here 256 lanes resolve up to
+// 256 ids at once and have kFewTileBytes of rows on their way at once, whichever ids and chunks those are; the rows meet in
+// LDS, where a lane per 4-byte word adds them in the order of the ids, as pool_samples does: the same sums, bit for bit.
+constexpr uint32_t kFewTileBytes = 32768;
+template <typename E>
+__device__ __forceinline__ void pool_unpack_word(uint32_t w, float *x, bool bf16) {
+  if constexpr (sizeof(E) == 4) {
+    x[0] = __uint_as_float(w);
+  } else if (bf16) {
+    x[0] = __uint_as_float(w << 16), x[1] = __uint_as_float(w & 0xffff0000u);
+  } else {
+    x[0] = __half2float(__ushort_as_half((unsigned short)(w & 0xffffu)));
+    x[1] = __half2float(__ushort_as_half((unsigned short)(w >> 16)));
+  }
+}
+template <typename E>
+__device__ __forceinline__ uint32_t pool_pack_word(const float *x, bool bf16) {
+  if constexpr (sizeof(E) == 4) return __float_as_uint(x[0]);
+  else if (bf16) return float_to_bf16_bits(x[0]) | (float_to_bf16_bits(x[1]) << 16);
+  else return (uint32_t)__half_as_ushort(__float2half(x[0])) | ((uint32_t)__half_as_ushort(__float2half(x[1])) << 16);
+}
+
+template <typename K, int KIND, int G, typename E, Store STORE>
+__device__ __forceinline__ void pool_few_samples(const ugk_table_t &t, const K *__restrict__ ids,
+                                                 const long long *__restrict__ seg_off, const float *__restrict__ weights,
+                                                 size_t n_rows, long long nnz, const u32x4 *__restrict__ cache,
+                                                 uint64_t cache_rows, const u32x4 *__restrict__ host, uint64_t host_rows,
+                                                 u32x4 *__restrict__ out, uint32_t vpr, int combiner, bool bf16,
+                                                 uint32_t *status, uint32_t *host_mirror, const Ending<STORE> &done,
+                                                 uint32_t &wave_local, uint32_t &wave_host) {
+  constexpr int kGroups = kBlock / G;
+  constexpr uint32_t kTileChunks = kFewTileBytes / 16 / kGroups;
+  constexpr int U = kTileChunks / G;           // chunks on their way per lane
+  constexpr int EPW = sizeof(E) == 4 ? 1 : 2;  // elements per word
+  constexpr int kMaxWords = 4;                 // words of a row a lane may own: rows of up to G chunks
+  __shared__ u32x4 tiles[kGroups][kTileChunks];
+  __shared__ uint64_t rows_at[kGroups][G];  // where the id's row is read, kNoRowBit: it has none
+  __shared__ float weights_of[kGroups][G];
+  __shared__ float denominators[kGroups];
+  const uint32_t tid = threadIdx.x % G, group = threadIdx.x / G, words = vpr * 4;
+  u32x4 *tile = tiles[group];
+  uint64_t *row_at = rows_at[group];
+  float *weight = weights_of[group];
+  auto sync = [] {  // between the lanes of the group
+    if constexpr (G == kBlock) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  };
+  const uint32_t tile_rows = min(kTileChunks / vpr, (uint32_t)G);  // (8 at least)
+  const uint32_t magic = vpr > 1 ? (uint32_t)(0x100000000ull / vpr) + 1u : 0u;  // i / vpr = mulhi(i, magic) for i < kTileChunks
+  // sums of weights per sample, the order that pool_samples' shapes for rows of this length keep
+  const uint32_t parts = vpr <= 32 ? 8 : vpr <= 128 ? 32 : 64;
+  for (size_t r = (size_t)blockIdx.x * kGroups + group; r < n_rows; r += (size_t)gridDim.x * kGroups) {
+    long long beg = seg_off[r], end = seg_off[r + 1];
+    const bool bad = beg < 0 || end > nnz || end < beg;  // outside the ids: nothing is read for it, its row is zeros
+    if (tid == 0 && (bad || (r == 0 && beg != 0) || (r + 1 == n_rows && end != nnz))) {
+      atomicOr(status, UGK_ST_BAD_SEGMENT);
+      if (host_mirror) tell_host<uint32_t>(host_mirror, UGK_ST_BAD_SEGMENT);
+    }
+    if (bad) beg = end = 0;
+    float acc[kMaxWords][EPW] = {};
+    float wsum = 0.f;
+    for (long long j0 = beg; j0 < end; j0 += G) {  // the same for all lanes of the group
+      const long long j = j0 + tid;
+      const bool active = j < end;
+      const uint64_t key = active ? key_to_u64<K>(ids[j]) : 0;
+      const float w_of_id = active && weights ? weights[j] : 1.f;
+      const Found f = table_lookup<KIND>(t, key, active);
+      const MixRow row = mix_resolve(t, key, active, f, cache, cache_rows, host, host_rows, out, vpr, status, host_mirror);
+      if (done.words) {
+        wave_local += __popcll(__ballot(row.from_cache));
+        wave_host += __popcll(__ballot(active && !row.from_cache));
+      }
+      const bool use = active && row.has_row;  // a key without a row adds nothing (the launch is flagged)
+      row_at[tid] = use ? row.bits : row.bits | kNoRowBit;
+      weight[tid] = use ? w_of_id : 0.f;
+      sync();
+      const uint32_t here = (uint32_t)min((long long)G, end - j0);
+      if (combiner != 0 && tid < parts)
+        for (uint32_t i = tid; i < here; i += parts) {
+          const float w = weight[i];
+          const float wterm = combiner == 2 ? w * w : w;
+          wsum += wterm;
+        }
+      for (uint32_t i0 = 0; i0 < here; i0 += tile_rows) {
+        const uint32_t rows = min(tile_rows, here - i0), chunks = rows * vpr;
+        // (a lane past the end reads the last chunk again instead of branching around its load)
+        auto fetch = [&](auto n) {
+          u32x4 v[n()];
+          bool none[n()];
+#pragma unroll
+          for (int u = 0; u < n(); ++u) {
+            const uint32_t i = min((uint32_t)u * G + tid, chunks - 1);
+            const uint32_t q = vpr > 1 ? __umulhi(i, magic) : i;
+            const uint64_t at = row_at[i0 + q];
+            none[u] = (at & kNoRowBit) != 0;
+            v[u] = reinterpret_cast<grow_t>(at & ~(uint64_t)kNoRowBit)[i - q * vpr];
+          }
+#pragma unroll
+          for (int u = 0; u < n(); ++u) {
+            const uint32_t i = (uint32_t)u * G + tid;
+            if (i < chunks) tile[i] = none[u] ? u32x4{0, 0, 0, 0} : v[u];
+          }
+        };
+        if (chunks <= 2 * G) fetch(std::integral_constant<int, 2>{});
+        else fetch(std::integral_constant<int, U>{});
+        sync();
+#pragma unroll
+        for (int c = 0; c < kMaxWords; ++c) {
+          const uint32_t word = (uint32_t)c * G + tid;
+          if (word >= words) break;
+          const uint32_t *column = reinterpret_cast<const uint32_t *>(tile) + word;
+#pragma unroll 8
+          for (uint32_t i = 0; i < rows; ++i) {
+            float x[EPW];
+            pool_unpack_word<E>(column[i * words], x, bf16);
+#pragma unroll
+            for (int e = 0; e < EPW; ++e) acc[c][e] = fmaf(weight[i0 + i], x[e], acc[c][e]);
+          }
+        }
+        sync();  // the next rows, the next ids' rows and weights
+      }
+      if constexpr (STORE == kThrough) {
+        if (active) copy_key_along<K>(done, (uint64_t)j, (K)key);
+      }
+    }
+    float denom = 1.f;
+    if (combiner != 0) {
+      if (tid < (uint32_t)kWave) {
+        for (uint32_t d = parts / 2; d > 0; d >>= 1) wsum += __shfl_xor(wsum, d);
+        if (tid == 0) denominators[group] = combiner == 1 ? wsum : sqrtf(wsum);
+      }
+      sync();
+      denom = denominators[group];
+    }
+    uint32_t *to = reinterpret_cast<uint32_t *>(out + r * vpr);
+#pragma unroll
+    for (int c = 0; c < kMaxWords; ++c) {
+      const uint32_t word = (uint32_t)c * G + tid;
+      if (word < words) {
+        float y[EPW];
+#pragma unroll
+        for (int e = 0; e < EPW; ++e) y[e] = denom != 0.f ? acc[c][e] / denom : 0.f;  // div_no_nan
+        const uint32_t packed = pool_pack_word<E>(y, bf16);
+        if constexpr (STORE == kThrough) store_through(reinterpret_cast<uint64_t>(to + word), packed);
+        else to[word] = packed;
+      }
+    }
+    sync();  // the next sample's denominator
+  }
+}
+
+// CH 0: a sample per LPR lanes, a wavefront or the workgroup (pool_few_samples)
 template <typename K, int KIND, int LPR, int CH, int U, typename E, bool CLIP, bool MIXED, Store STORE>
 __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, const K *__restrict__ ids,
                                                               const long long *__restrict__ seg_off,
@@ -286,7 +447,10 @@ __global__ __launch_bounds__(kBlock) void extract_pool_kernel(ugk_table_t t, con
   if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
   __syncthreads();
   uint32_t wave_local = 0, wave_host = 0;
-  if (!MIXED || wave_in_block() < keep_waves)
+  if constexpr (CH == 0)
+    pool_few_samples<K, KIND, LPR, E, STORE>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host, host_rows, out, vpr,
+                                        combiner, bf16, status, host_mirror, done, wave_local, wave_host);
+  else if (!MIXED || wave_in_block() < keep_waves)
     pool_samples<K, KIND, LPR, CH, U, E, CLIP, true, STORE>(t, ids, seg_off, weights, n_rows, nnz, cache, cache_rows, host,
                                                             host_rows, out, vpr, combiner, bf16, max_norm, status,
                                                             host_mirror, done, wave_local, wave_host);
@@ -542,6 +706,33 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
     else if (upto12 && vpr < 32) shape = 842, keep_waves = 3;
     else if (nnz > rows64 * 24 && sizeof(E) == 4) shape = 1622, keep_waves = 3;
   }
+  // Launches of few samples are a sample's own time, on a chip that has wavefronts to spare: more lanes per sample, and a
+  // sample per wavefront or workgroup from 12 ids on (pool_few_samples).  us per launch, rows in HBM, uniform ids, mean:
+  //   lanes, as above / as here: 64 B 8 ids x 4,096 5.0 / 4.4, 16 ids x 8,192 7.6 / 6.4, x 16,384 10.4 / 9.6; 256 B 8 ids x 1,024
+  //     4.3 / 3.7, x 4,096 5.6 / 4.8 (x 16,384 9.1 / 8.9, 2 ids x 8,192 4.1 / 4.5); 512 B 4 ids x 1,024 5.8 / 3.8, x 4,096 6.4 / 5.0,
+  //     x 8,192 7.6 / 6.4 (x 32,768 16.8 / 17.9); 512 B 40 ids x 4,096 22.5 / 19.4, x 8,192 30.2 / 31.2; 1 KB 8 ids x 1,024 6.9 /
+  //     5.5, x 4,096 9.7 / 9.0 (x 8,192 15.3 / 15.5)
+  //   a workgroup per sample, lanes as here / this: 512 B 16 ids x 256 5.3 / 4.1, x 1,024 6.7 / 5.8, 40 ids x 64 11.4 / 5.0, x 1,024
+  //     12.2 / 8.0, 100 ids x 64 39.3 / 7.2; 1 KB 16 ids x 256 6.2 / 4.8, x 1,024 7.2 / 7.1, 40 ids x 1,024 14.4 / 11.3 (8 ids 5.5 /
+  //     5.8); 2 KB 8 ids x 256 6.5 / 5.1, x 1,024 7.7 / 7.8, 40 ids x 256 18.5 / 9.1; 4 KB 16 ids x 512 11.3 / 10.7 (x 1,024 15.4 /
+  //     16.6; of two-byte elements, whose words are two sums each, 16 ids x 64 10.2 / 9.9, 8.9 / 9.6 for 16 samples)
+  //   a wavefront per sample: 64 B 16 ids x 1,024 4.7 / 4.2, x 2,048 5.7 / 4.8, 40 ids x 4,096 11.7 / 8.7; 256 B 16 ids x 2,048 5.4 /
+  //     5.8 (two-byte 7.7 / 6.5), 40 ids x 2,048 9.8 / 8.0, x 4,096 13.0 / 11.3; 512 B 40 ids x 2,048 15.1 / 11.8
+  const uint64_t cus = (uint64_t)cu_count();
+  if (!clip) {
+    if (vpr <= 4 && !upto6 && rows64 <= cus * 64) shape = 814;
+    else if (vpr > 8 && vpr <= 16 && rows64 <= cus * 16) shape = KIND == 0 && sizeof(E) == 2 ? 1612 : 1614;
+    else if (vpr > 16 && vpr <= 32 && rows64 <= cus * 32 && (keep_waves < kWavesPerBlock || upto2))
+      shape = nnz <= rows64 * 24 ? 1622 : 1624, keep_waves = kWavesPerBlock;
+    else if (vpr > 32 && vpr <= 64 && rows64 <= cus * 16) shape = 3224;
+    const bool over24 = nnz > rows64 * 24;
+    const bool by_workgroup = rows64 <= cus * 2 ? (vpr <= 64 ? !upto12 : vpr <= 128 ? !upto6 : !upto12 && sizeof(E) == 4)
+                                                : rows64 <= cus * 4 && vpr > 16 && vpr <= 128 && !upto12;
+    const bool by_wave = vpr <= 16 ? rows64 <= cus * 16 && (over24 || (!upto12 && rows64 <= cus * 8 && (vpr <= 8 || sizeof(E) == 2)))
+                                   : vpr <= 32 && rows64 <= cus * 8 && over24;
+    if (by_workgroup) shape = kBlock * 100, keep_waves = kWavesPerBlock;
+    else if (by_wave) shape = kWave * 100, keep_waves = kWavesPerBlock;
+  }
   if (const char *forced = getenv("UGK_POOL_LPR")) {  // for sweeps; a weighted mean's last bits may vary with it
     const int v = atoi(forced);
     if (!clip && (v == 8 || v == 32 || v == 64) && vpr <= (uint32_t)v * kPoolChunks)
@@ -590,7 +781,7 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
       return 0;
     }
   }
-  const size_t rows_per_block = (size_t)(kWave / (shape / 100)) * kWavesPerBlock;
+  const size_t rows_per_block = (size_t)kBlock / (shape / 100);
   const unsigned grid = clamp_grid((n_rows + rows_per_block - 1) / rows_per_block, 0);
   // Samples of one or two ids write about as much as they read, and where that is much more than the L2s hold written-through
   // rows cost more than a ticket kernel behind the launch.  us, launch to end of poll, ticket / words, all rows in one place, one
@@ -615,6 +806,8 @@ int extract_pool_lpr(ugk_table_t t, const K *ids, const long long *seg_off, cons
     if (done.tag) UGK_POOL_GO(L, CH, U, CLIP, MIXED, kThrough);                                                        \
     else UGK_POOL_GO(L, CH, U, CLIP, MIXED, kOrdinary);                                                                \
   }
+  UGK_POOL(kBlock, 0, 0, false, false)
+  UGK_POOL(kWave, 0, 0, false, false)
   UGK_POOL(4, 1, 2, false, false)
   UGK_POOL(4, 1, 4, false, false)
   UGK_POOL(8, 1, 4, false, false)
