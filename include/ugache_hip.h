@@ -103,7 +103,7 @@ typedef struct {
 const char *ugk_last_error(void);
 /* version of this ABI; bumped on any signature change.  ugk_abi_version() is what the loaded library was built with:
  * a caller compiled against another UGK_ABI_VERSION must not go on. */
-#define UGK_ABI_VERSION 24
+#define UGK_ABI_VERSION 25
 int ugk_abi_version(void);
 
 /* ---- runtime plumbing: Device::{AllocDataSpace,FreeDataSpace,CopyDataFromTo,StreamSync,CreateStream}
@@ -170,6 +170,11 @@ typedef struct {
   uint32_t counter_set; /* 0 before the first launch, kept by the launches from then on */
   uint32_t where_faster; /* non-zero: words only where they are there no later than a ticket kernel (ugk_stream_sync_ticket)
                           * behind the launch, with a kernel that copies the keys if keys are wanted */
+  const uint32_t *count_dev; /* not NULL: of the n keys it is given the launch looks up the first *count_dev, at most n, a device
+                              * word that launches in front of it on the stream leave (the distinct keys of ugk_dedup_*), so that
+                              * the host need not wait for that number.  ugk_gather_direct_* and ugk_extract_mix_* only, with
+                              * words whatever where_faster says and without keys; a launch that cannot refuses the call.  Its
+                              * stores are not non-temporal whatever the size of the output */
 } ugk_done_t;
 int ugk_leave_done_words(ugk_done_t *done);
 int ugk_done_wait(const ugk_done_t *done, unsigned spin_us, void *stream, uint64_t *local, uint64_t *others);

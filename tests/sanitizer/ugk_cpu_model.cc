@@ -171,11 +171,15 @@ bool leave_done(uint64_t local, uint64_t others, const K *keys, size_t n) {
   return true;
 }
 
+// ugk_done_t::count_dev: how many of its keys a launch looks up
+size_t launch_count(size_t n) { return g_done && g_done->count_dev ? std::min<size_t>(n, *g_done->count_dev) : n; }
+
 template <typename K>
 int gather_direct(const void *src, uint64_t src_rows, const K *keys, const uint32_t *dst, size_t n, void *out,
                   uint64_t out_rows, size_t rb, uint32_t *status, uint32_t *mirror) {
   if (n == 0) return 0;
   REQUIRE(src && out && keys && status, "gather: null pointer");
+  if (dst == nullptr) n = launch_count(n);
   for (size_t i = 0; i < n; ++i) {
     const uint64_t s = k64(keys[i]), d = dst ? dst[i] : i;
     if (s >= src_rows || d >= out_rows) {
@@ -404,6 +408,7 @@ int extract_mix(ugk_table_t t, const K *keys, size_t n, const void *cache, uint6
   if (num_groups) *num_groups = 0;
   if (n == 0) return 0;
   REQUIRE(keys && out && status, "ugk_extract_mix: null keys, output or status");
+  n = launch_count(n);
   if (check_table(t, "ugk_extract_mix")) return 1;
   const uintptr_t align = (uintptr_t)cache | (uintptr_t)host | (uintptr_t)out | (uintptr_t)rb;
   REQUIRE(rb > 0 && (align % 16 == 0 || (!stage && align % 4 == 0 && rb >= 20)),

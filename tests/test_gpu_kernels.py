@@ -1228,6 +1228,64 @@ def test_pooled_extraction_matches_a_float64_segment_sum(kind, dim, etype, rows_
         words.free()
 
 
+# every kernel and kind of lane of the gathers, the fused one with and without a stage
+@pytest.mark.parametrize("kind,rb", [("none", 512), ("none", 64), ("none", 8192), ("none", 100), ("none", 36), ("none", 1204),
+                                     ("none", 800), ("none", 2), ("none", 1), ("flat", 512), ("flat", 100), ("hash", 64),
+                                     ("hash32", 1024), ("hash32", 36)])
+def test_launch_that_finds_its_count_on_the_device(kind, rb):
+    """ugk_done_t::count_dev: of n keys a polled launch looks up as many as a device word says, n at most; the rows behind them
+    stay as they are, the group sizes are those of the keys looked up.  Grids of one workgroup and of more than are launched"""
+    rng = np.random.default_rng(rb)
+    nkeys = 3_000
+    host = rng.integers(0, 256, size=(nkeys, rb)).astype(np.uint8)
+    cached = rng.choice(nkeys, nkeys // 2, replace=False).astype(np.int64)
+    pin, done, count = pinned_from(host), _DoneWords(), dev_zeros_u32(1)
+    done.done.where_faster = 1  # words all the same
+    words = PinnedArray((hip.lib().ugk_extract_mix_max_groups(),), np.uint64)
+    d_host, d_cache, st = to_dev(host), to_dev(host[cached].copy()), dev_zeros_u32(1)
+    if kind != "none":
+        mem, tb = {"flat": lambda: _make_flat(nkeys), "hash": lambda: _make_hash(len(cached))[:2],
+                   "hash32": lambda: _make_hash32(len(cached))[:2]}[kind]()
+        assert _insert(tb, cached) == 0
+    groups = C.c_uint32(0)
+    try:
+        for n in (5, 3_000, max(3_000, (8 << 20) // rb)):
+            keys = rng.integers(0, nkeys, size=n)
+            d_keys = to_dev(keys.astype(np.int64))
+            for have in (0, 1, n // 2 + 1, n - 1, n, n + 7):
+                count.fill_(have)
+                done.done.count_dev = ptr(count)
+                m, out = min(n, have), dev_bytes(n * rb, fill=0x7F)
+                done.ask(0)
+                if kind == "none":
+                    hip.call("ugk_gather_direct_i64", ptr(d_host), nkeys, ptr(d_keys), n, ptr(out), rb, 0, ptr(st), done.mirror.ptr, None)
+                else:
+                    hip.call("ugk_extract_mix_i64", tb, ptr(d_keys), n, ptr(d_cache), len(cached), pin.ptr, nkeys, ptr(out), rb, ptr(st),
+                             done.mirror.ptr, words.ptr, C.byref(groups), hip.HINT_UNKNOWN, None)
+                assert done.done.num_words > 0
+                local, others = C.c_uint64(), C.c_uint64()
+                hip.call("ugk_done_wait", C.byref(done.done), 1_000_000, None, C.byref(local), C.byref(others))
+                done.check_flag(0)
+                done.check_counters()
+                raw = to_np(out).reshape(n, rb)
+                assert raw[:m].tobytes() == host[keys[:m]].tobytes() and (raw[m:] == 0x7F).all(), (n, have)
+                if kind != "none":
+                    assert (local.value, others.value) == (int(np.isin(keys[:m], cached).sum()), m - int(np.isin(keys[:m], cached).sum()))
+        # refused: launches that cannot, which then do nothing
+        out, dst = dev_bytes(5 * rb, fill=0x7F), to_dev(np.arange(5, dtype=np.uint32))
+        done.ask(0)
+        with pytest.raises(RuntimeError):
+            hip.call("ugk_gather_scatter_i64", ptr(d_host), nkeys, ptr(d_keys), ptr(dst), 5, ptr(out), 5, rb, 0, ptr(st), None, None)
+        done.done.num_keys = 1
+        with pytest.raises(RuntimeError):
+            hip.call("ugk_leave_done_words", C.byref(done.done))
+        assert (to_np(out) == 0x7F).all() and status_value(st) == 0
+    finally:
+        sync()
+        pin.free()
+        words.free()
+
+
 @pytest.mark.parametrize("kind", ["none", "flat", "hash"])
 @pytest.mark.parametrize("vpr", [1, 4, 5, 8, 9, 16, 17, 24, 32, 33, 64, 65, 128, 129, 256])
 def test_pooled_extraction_at_the_edges_of_its_shapes(kind, vpr):

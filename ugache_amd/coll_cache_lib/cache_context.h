@@ -125,6 +125,13 @@ class ExtractSession {
   uint32_t *DedupInverse() const { return reinterpret_cast<uint32_t *>(_dedup_out->ptr<char>() + _dedup_cap * 8); }
   uint32_t *DedupRep() const { return DedupInverse() + _dedup_cap; }
   template <typename KeyT>
+  const uint32_t *DedupLaunch(const KeyT *nodes, size_t num_nodes, uint32_t *inverse, StreamHandle stream);
+  size_t DedupFound(size_t num_nodes) const;
+  bool CountsFromDevice(size_t num_nodes, const void *output) const;
+  template <typename KeyT>
+  size_t ExtractUniqueCounted(const KeyT *nodes, size_t num_nodes, void *output, uint32_t *inverse_out, StreamHandle stream,
+                              uint64_t task_key);
+  template <typename KeyT>
   size_t DedupKeys(const KeyT *nodes, size_t num_nodes, uint32_t *inverse, StreamHandle stream);
   bool _dedup_odd = false;  // which of the two count words the next deduplication uses
 

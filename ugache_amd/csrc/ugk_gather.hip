@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
                                                         V *__restrict__ out, uint64_t out_rows, uint32_t vpr,
                                                         const uint32_t *__restrict__ counts, uint32_t group,
                                                         bool many_groups, size_t n, uint32_t *status, uint32_t *host_mirror, Ending<STORE> done) {
-  size_t begin = 0, count = n;
+  size_t begin = 0, count = Idx::kDense ? launch_count(done, n) : n;
   if (counts) {
     const uint32_t c = counts[group];
     count = c;
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
                                                              const uint32_t *__restrict__ counts, uint32_t group,
                                                              size_t n, uint32_t *status, uint32_t *host_mirror,
                                                              Ending<STORE> done) {
-  size_t begin = 0, count = n;
+  size_t begin = 0, count = Idx::kDense ? launch_count(done, n) : n;
   if (counts) {
     const uint32_t c = counts[group];
     count = c;
@@ -242,12 +242,13 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     else *q = w;
   };
   const uint32_t lane = lane_id();
+  const uint64_t total = STORE == kThrough ? launch_count(done, f.total / f.row_bytes) * f.row_bytes : f.total;
   const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock * kStreamPart;
-  for (uint64_t begin = ((uint64_t)blockIdx.x * kWavesPerBlock + wave_in_block()) * kStreamPart; begin < f.total;
+  for (uint64_t begin = ((uint64_t)blockIdx.x * kWavesPerBlock + wave_in_block()) * kStreamPart; begin < total;
        begin += stride) {
     const uint64_t row0 = begin / f.row_bytes;
     const uint32_t off0 = (uint32_t)(begin - row0 * f.row_bytes);  // the part begins at byte off0 of row row0
-    const uint32_t bytes = (uint32_t)min((uint64_t)kStreamPart, f.total - begin);
+    const uint32_t bytes = (uint32_t)min((uint64_t)kStreamPart, total - begin);
     const uint64_t to = reinterpret_cast<uint64_t>(out) + begin;
     // lane l: where row row0 + l is read
     uint64_t s = 0, d = 0;
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     if constexpr (SHARE) {
       const uint32_t rest = bytes % 16;  // the words behind the last whole vector of the output: the end of its last row
       if (rest) {
-        const uint32_t r = (uint32_t)((f.total - 1) / f.row_bytes - row0);
+        const uint32_t r = (uint32_t)((total - 1) / f.row_bytes - row0);
         const uint32_t rlo = __shfl(lo, (int)r), rhi = __shfl(hi, (int)r);
         if (lane < rest / 4 && (rlo & kNoRowBit) == 0) {
           const uint64_t from = (((uint64_t)rhi << 32) | rlo) + f.row_bytes - rest;
@@ -488,11 +489,12 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
                     const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
                     uint32_t *host_mirror, bool nt, DoneRequest &request, hipStream_t stream) {
   constexpr size_t kPerIter = (size_t)(kBlock / LPR) * UNROLL;
-  const unsigned grid = gather_grid((n + kPerIter - 1) / kPerIter, max_blocks);
+  const unsigned grid = request.grid(gather_grid((n + kPerIter - 1) / kPerIter, max_blocks));
   const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
   DoneWords done{};
   if constexpr (Idx::kDense) {
     if (!nt) done = request.take(grid, gather_tells(sizeof(V), vpr, LPR, n * (size_t)vpr * sizeof(V)));
+    UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
   }
 #define UGK_GO(STORE)                                                                                                  \
   hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,            \
@@ -519,7 +521,8 @@ int launch_one(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t o
   // two rows in flight per lane; one was measured with streaming stores and is no better (262,144 keys of 512 bytes
   // into rotating outputs 49.3 us against 47.9 us, 1 M keys 184 against 180 us)
   return launch_unrolled<V, LPR, 2, Idx>(ix, src, src_rows, out, out_rows, vpr, counts, group, n, max_blocks, status,
-                                         host_mirror, nt_store_for(n * (size_t)vpr * sizeof(V)), request, stream);
+                                         host_mirror, !request.counted() && nt_store_for(n * (size_t)vpr * sizeof(V)), request,
+                                         stream);
 }
 
 template <typename V, typename Idx>
@@ -602,7 +605,7 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
                 uint32_t *host_mirror, DoneRequest &request, hipStream_t stream) {
   const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes, n));
   const size_t per_block = (size_t)f.tile * kWavesPerBlock;
-  const unsigned grid = gather_grid((n + per_block - 1) / per_block, max_blocks);
+  const unsigned grid = request.grid(gather_grid((n + per_block - 1) / per_block, max_blocks));
 #define UGK_GO(STORE, DONE)                                                                                            \
   hipLaunchKernelGGL((gather_flat_kernel<STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,     \
                      src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<STORE>(DONE))
@@ -613,6 +616,7 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
       UGK_HIP(hipGetLastError());
       return 0;
     }
+    UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
   }
   UGK_GO(kOrdinary, DoneWords{});
 #undef UGK_GO
@@ -625,9 +629,10 @@ int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t 
                   unsigned max_blocks, uint32_t *status, uint32_t *host_mirror, DoneRequest &request, hipStream_t stream) {
   const StreamRow f = stream_row(row_bytes, n);
   const uint64_t per_block = (uint64_t)kStreamPart * kWavesPerBlock;
-  const unsigned grid = gather_grid((f.total + per_block - 1) / per_block, max_blocks);
-  const bool nt = nt_store_for(n * row_bytes);
+  const unsigned grid = request.grid(gather_grid((f.total + per_block - 1) / per_block, max_blocks));
+  const bool nt = !request.counted() && nt_store_for(n * row_bytes);
   const DoneWords done = nt ? DoneWords{} : request.take(grid, Telling::kSooner);
+  UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
 #define UGK_GO(STORE, SHARE)                                                                                          \
   hipLaunchKernelGGL((gather_stream_kernel<STORE, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,             \
                      (const char *)src, src_rows, (char *)out, f, status, host_mirror, Ending<STORE>(done))
@@ -653,6 +658,7 @@ int launch_gather(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_
   UGK_REQUIRE(status, "gather: null status word");
   UGK_REQUIRE(row_bytes > 0 && row_bytes <= (1u << 30), "gather: row_bytes %zu out of range", row_bytes);
   UGK_REQUIRE(n <= 0xffffffffull, "gather: batch of %zu rows exceeds 2^32", n);
+  UGK_REQUIRE(Idx::kDense || !request.counted(), "gather: only ugk_gather_direct_* takes its count from the device");
   const uintptr_t align = (uintptr_t)src | (uintptr_t)out | (uintptr_t)row_bytes;
   hipStream_t st = as_stream(stream);
 #define UGK_VEC(V)                                                                                                  \

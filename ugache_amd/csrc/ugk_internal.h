@@ -59,8 +59,8 @@ bool nt_store_for(size_t out_bytes);
 // polls, and words, if there are any, are the per-workgroup counts of ugk_extract_mix_*.
 struct DoneWords {
   unsigned long long *words, *counters;
-  void *keys;         // the launch leaves its first num_keys keys here (pinned host memory)
-  uint64_t num_keys;
+  void *keys;         // the launch leaves its first num_keys keys here (pinned host memory); where num_keys is 0 and this is
+  uint64_t num_keys;  // not, it is a device word: how many of the launch's keys there are (launch_count)
   uint32_t tag;
   uint32_t set;       // which of the two sets of counters
 };
@@ -83,6 +83,10 @@ class DoneRequest {
   DoneRequest();
   // grid: workgroups of the launch; count_limit: no counter of it reaches this, 0 where none are kept
   DoneWords take(unsigned grid, Telling words, uint64_t count_limit = 0);
+  // whether the number of keys is in a device word; a launch that has not taken the request then must not go ahead
+  bool counted() const;
+  // ... and one that has leaves workgroups without keys: not more of them than keep the chip busy
+  unsigned grid(unsigned wanted) const;
 
  private:
   ugk_done_t *_done;

@@ -51,6 +51,15 @@ struct Ending<kThrough> : DoneWords {
   explicit Ending(const DoneWords &done) : DoneWords(done) {}
 };
 
+// how many of its n keys the launch looks up (ugk_done_t::count_dev)
+template <Store STORE>
+__device__ __forceinline__ size_t launch_count(const Ending<STORE> &done, size_t n) {
+  if constexpr (STORE == kThrough) {
+    if (done.num_keys == 0 && done.keys) return min(n, (size_t)*static_cast<const uint32_t *>(done.keys));
+  }
+  return n;
+}
+
 // A word for the host beside the rows (an error flag, a key).  The same kind of store: an ordinary one into host memory is
 // acknowledged before it is there, and the words of leave_done, which say that all of this is complete, may overtake it
 // (a lookup of four keys, one of them out of range, returned without its error that way).

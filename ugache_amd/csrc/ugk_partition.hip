@@ -238,6 +238,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
   __shared__ uint32_t block_tot[2];
   if (threadIdx.x < 2) block_tot[threadIdx.x] = 0;
   __syncthreads();
+  n = launch_count(done, n);
   uint32_t wave_local = 0, wave_host = 0;  // rows this wavefront took from each source (wavefront-uniform)
   const int lane = (int)lane_id();
   const size_t wave_global = (size_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
@@ -519,7 +520,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
                     DoneRequest &request, hipStream_t st) {
   // ordinary write-back stores while the output fits the memory-side cache (the consumer finds it there),
   // non-temporal beyond, or as the caller's hint says
-  const bool nt = nt_store_for(n * row_bytes);
+  const bool nt = !request.counted() && nt_store_for(n * row_bytes);
   const uint32_t vpr = (uint32_t)((row_bytes + 15) / 16);
   // Keys per wavefront.  A wavefront resolves its keys together and then copies their rows a few at a time; once its
   // first stores are out, every later load of the wavefront returns behind them, so wavefronts of one round of rows
@@ -546,15 +547,16 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const size_t slots = (size_t)cu_count() * 4 * 8;
   const int lpr = vpr <= 1 ? 1 : vpr <= 2 ? 2 : vpr <= 4 ? 4 : vpr <= 8 ? 8 : vpr <= 16 ? 16 : vpr <= 32 ? 32 : 64;
   const bool small_rows = lpr <= 8;  // rows of up to 128 bytes
+  const size_t likely = request.counted() ? n / 2 : n;  // distinct keys of n: anything between a seventh of them and all
   int kpw;
   if (KIND == 1) {
     kpw = small_rows ? 32 : 8;
-  } else if (n <= slots) {
+  } else if (likely <= slots) {
     kpw = 8;
   } else if (small_rows) {
-    kpw = n <= slots * 16 ? 32 : 64;
+    kpw = likely <= slots * 16 ? 32 : 64;
   } else {
-    kpw = n <= slots * 8 ? 16 : n <= slots * 16 ? 32 : n <= slots * 32 ? 64 : 16;
+    kpw = likely <= slots * 8 ? 16 : likely <= slots * 16 ? 32 : likely <= slots * 32 ? 64 : 16;
   }
   // UGK_MIX_KPW=8|16|32|64 forces the shape (read on every launch: the sweep that measures the rule above changes it
   // between launches); never a byte of the result depends on it
@@ -566,7 +568,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   // a wavefront copies all its rows as one run of vectors, or a row at a time where they are too long to divide by
   const FlatRow f_row = flat_row(row_bytes, (uint32_t)kpw);
   const size_t keys_per_group = (size_t)kpw * kWavesPerBlock;
-  const unsigned grid = clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u);
+  const unsigned grid = request.grid(clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u));
   // Rows of more than one vector per lane wait between their vectors, for memory where they are written through: a ticket behind
   // the launch is there sooner than words (see gather_tells).  us, launch to end of poll, ticket / words, all
   // rows in HBM: 1536 bytes x 40 10.7 / 12.1, x 5,200 14.5 / 15.6, x 20,800 21.4 / 21.8; 4 KB x 250 17.0 / 18.7, x 2,000 18.6 / 20.6,
@@ -576,6 +578,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const Telling words =
       row_bytes <= 1024 || (row_bytes <= 4096 && n * row_bytes > (size_t)32 << 20) ? Telling::kSooner : Telling::kLater;
   DoneWords done = nt && !flat ? DoneWords{} : request.take(grid, words, n);
+  UGK_REQUIRE(!request.counted(), "ugk_extract_mix: a launch that leaves no words cannot take its count from the device");
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;
   const ugk_stage_t no_stage{};

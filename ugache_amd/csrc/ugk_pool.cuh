@@ -848,6 +848,7 @@ int extract_pool(ugk_table_t t, const K *ids, const int64_t *seg_off, const floa
   DoneRequest request;
   if (num_groups) *num_groups = 0;
   if (n_rows == 0) return 0;
+  UGK_REQUIRE(!request.counted(), "ugk_extract_pool: the count of ids comes from the host");
   UGK_REQUIRE(seg_off && out && status, "ugk_extract_pool: null offsets, output or status");
   UGK_REQUIRE(max_norm >= 0.f, "ugk_extract_pool: max_norm %g is not a norm (0 = no clipping)", (double)max_norm);
   UGK_REQUIRE(nnz == 0 || ids, "ugk_extract_pool: null ids");

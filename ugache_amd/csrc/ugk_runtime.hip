@@ -2,6 +2,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 
@@ -38,15 +39,24 @@ DoneRequest::DoneRequest() : _done(g_done) { g_done = nullptr; }
 // a counter holds 16 bits of workgroups and two counts of 24 bits
 DoneWords DoneRequest::take(unsigned grid, Telling words, uint64_t count_limit) {
   if (!_done || grid / kDoneFan >= 0xffffu || count_limit >= (1u << 24)) return DoneWords{};
-  if (_done->where_faster && words != Telling::kSooner && (words == Telling::kTooLate || _done->num_keys == 0))
+  if (_done->where_faster && !counted() && words != Telling::kSooner && (words == Telling::kTooLate || _done->num_keys == 0))
     return DoneWords{};
   ugk_done_t *d = _done;
   _done = nullptr;
   d->num_words = grid <= kDoneDirect ? grid : kDoneFan;
   if (grid > kDoneDirect) d->counter_set ^= 1u;
+  void *keys = d->num_keys ? d->keys_host : const_cast<uint32_t *>(d->count_dev);
   return DoneWords{reinterpret_cast<unsigned long long *>(d->words_host),
-                   reinterpret_cast<unsigned long long *>(d->counters_dev), d->keys_host, d->num_keys, d->tag,
+                   reinterpret_cast<unsigned long long *>(d->counters_dev), keys, d->num_keys, d->tag,
                    d->counter_set & 1u};
+}
+
+bool DoneRequest::counted() const { return _done && _done->count_dev; }
+
+// The 262,144 keys of a skewed batch may be 38,000 distinct ones: of the 16,384 workgroups of a gather of 512-byte rows the
+// others would each read the count and leave, eight to a compute unit at a time.
+unsigned DoneRequest::grid(unsigned wanted) const {
+  return counted() ? std::min(wanted, (unsigned)cu_count() * 16u) : wanted;
 }
 
 int blocks_per_cu() {
@@ -286,6 +296,7 @@ int ugk_leave_done_words(ugk_done_t *done) {
     UGK_REQUIRE(done->tag > 0 && done->tag <= UGK_DONE_MAX_TAG, "ugk_leave_done_words: tag %u is not in [1, %u]", done->tag,
                 UGK_DONE_MAX_TAG);
     UGK_REQUIRE(done->keys_host || done->num_keys == 0, "ugk_leave_done_words: null buffer for the keys");
+    UGK_REQUIRE(!done->count_dev || done->num_keys == 0, "ugk_leave_done_words: keys of a launch whose count is not known");
     done->num_words = 0;
   }
   ugk::g_done = done;

@@ -47,7 +47,8 @@ class Stage(C.Structure):
 class Done(C.Structure):
     """ugk_done_t"""
     _fields_ = [("words_host", C.c_void_p), ("counters_dev", C.c_void_p), ("tag", C.c_uint32), ("num_words", C.c_uint32),
-                ("keys_host", C.c_void_p), ("num_keys", C.c_uint64), ("counter_set", C.c_uint32), ("where_faster", C.c_uint32)]
+                ("keys_host", C.c_void_p), ("num_keys", C.c_uint64), ("counter_set", C.c_uint32), ("where_faster", C.c_uint32),
+                ("count_dev", C.c_void_p)]
 
 
 class DeviceInfo(C.Structure):
