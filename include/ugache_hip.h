@@ -103,7 +103,7 @@ typedef struct {
 const char *ugk_last_error(void);
 /* version of this ABI; bumped on any signature change.  ugk_abi_version() is what the loaded library was built with:
  * a caller compiled against another UGK_ABI_VERSION must not go on. */
-#define UGK_ABI_VERSION 25
+#define UGK_ABI_VERSION 26
 int ugk_abi_version(void);
 
 /* ---- runtime plumbing: Device::{AllocDataSpace,FreeDataSpace,CopyDataFromTo,StreamSync,CreateStream}
@@ -281,6 +281,12 @@ int ugk_table_evict_release_u32(ugk_table_t t, const uint32_t *keys_dev, size_t 
                                 uint64_t nslots, uint32_t *status_dev, void *stream);
 int ugk_table_evict_release_i64(ugk_table_t t, const int64_t *keys_dev, size_t n, uint64_t *slot_bits_dev,
                                 uint64_t nslots, uint32_t *status_dev, void *stream);
+/* the same without a bitmap: slots_out_dev[i] = the cache slot keys_dev[i] held (~0 where the key is not there), for as many
+ * rows that come in */
+int ugk_table_evict_slots_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint32_t *slots_out_dev, uint32_t *status_dev,
+                              void *stream);
+int ugk_table_evict_slots_i64(ugk_table_t t, const int64_t *keys_dev, size_t n, uint32_t *slots_out_dev, uint32_t *status_dev,
+                              void *stream);
 /* LookupValCustom with SepLocOffset (cache_hashtable.cuh:420-434): loc_out/off_out per key; a miss gives
  * (fallback_loc, (uint32)key).  Either output may be NULL (OffsetOnly, cuh:396-407). */
 int ugk_table_lookup_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint32_t fallback_loc,

@@ -289,8 +289,11 @@ int table_insert(ugk_table_t t, const K *keys, const uint32_t *offs, uint32_t se
 
 template <typename K>
 int table_evict(ugk_table_t t, const K *keys, size_t n, uint32_t *status, uint64_t *slot_bits = nullptr,
-                uint64_t nslots = 0) {
+                uint64_t nslots = 0, uint32_t *slots_out = nullptr) {
+  if (slots_out) std::fill(slots_out, slots_out + n, ~0u);
+  size_t at = 0;
   auto release = [&](uint32_t slot) {
+    if (slots_out) slots_out[at] = slot;
     if (!slot_bits) return;
     if (slot >= nslots) or_status(status, UGK_ST_KEY_OUT_OF_RANGE);
     else __atomic_fetch_and(slot_bits + (slot >> 6), ~(1ull << (slot & 63)), __ATOMIC_RELAXED);
@@ -299,6 +302,7 @@ int table_evict(ugk_table_t t, const K *keys, size_t n, uint32_t *status, uint64
   if (check_table(t, "ugk_table_evict")) return 1;
   REQUIRE(keys && status, "ugk_table_evict: null pointer");
   for (size_t i = 0; i < n; ++i) {
+    at = i;
     const uint64_t key = k64(keys[i]);
     if (t.kind == 1) {
       if (key >= t.size) {
@@ -1139,6 +1143,14 @@ int ugk_table_evict_release_i64(ugk_table_t t, const int64_t *keys, size_t n, ui
                                 uint32_t *status, void *) {
   REQUIRE(n == 0 || slot_bits, "ugk_table_evict_release_i64: null slot bitmap");
   return table_evict(t, keys, n, status, slot_bits, nslots);
+}
+int ugk_table_evict_slots_u32(ugk_table_t t, const uint32_t *keys, size_t n, uint32_t *slots_out, uint32_t *status, void *) {
+  REQUIRE(n == 0 || slots_out, "ugk_table_evict_slots_u32: null list of slots");
+  return table_evict(t, keys, n, status, nullptr, 0, slots_out);
+}
+int ugk_table_evict_slots_i64(ugk_table_t t, const int64_t *keys, size_t n, uint32_t *slots_out, uint32_t *status, void *) {
+  REQUIRE(n == 0 || slots_out, "ugk_table_evict_slots_i64: null list of slots");
+  return table_evict(t, keys, n, status, nullptr, 0, slots_out);
 }
 int ugk_table_lookup_u32(ugk_table_t t, const uint32_t *keys, size_t n, uint32_t fallback_loc, uint32_t *loc_out,
                          uint32_t *off_out, void *) {

@@ -618,3 +618,47 @@ def test_evict_that_releases_the_slots(kind, kdtype):
     assert status_value(st) & hip.ST_EVICT_ABSENT
     got = np.unpackbits(to_np(bm, np.uint64)[: len(used) // 64].view(np.uint8), bitorder="little").astype(bool)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["flat", "hash", "hash32"])
+@pytest.mark.parametrize("kdtype", [np.uint32, np.int64])
+@pytest.mark.parametrize("n_gone", [1, 7, 8, 9, 6_000])
+def test_evict_that_lists_the_slots(kind, kdtype, n_gone):
+    """ugk_table_evict_slots_*: the keys leave the table and slot i of the list is the one key i held; ~0 and a flag for a key
+    that is not there, or that no table could hold"""
+    rng = np.random.default_rng(n_gone)
+    nkeys, n, nslots = 50_000, 20_000, 30_000
+    keys = rng.choice(nkeys, n, replace=False).astype(kdtype)
+    slots = rng.choice(nslots, n, replace=False).astype(np.uint32)
+    if kind == "flat":
+        mem = dev_zeros_u32(nkeys)
+        hip.call("ugk_fill_u32", ptr(mem), hip.EMPTY_U32, nkeys, None)
+        tb = hip.table(hip.TABLE_FLAT, ptr(mem), nkeys)
+    else:
+        size = getattr(hip.lib(), "ugk_hash_buckets_for" if kind == "hash" else "ugk_hash32_entries_for")(n, 0.7)
+        mem = dev_bytes(size * 16 + 128)
+        base = (ptr(mem) + 127) // 128 * 128
+        tb = hip.table(hip.TABLE_HASH if kind == "hash" else hip.TABLE_HASH32, base, size)
+        hip.call("ugk_table_init", tb, None)
+    st, wide = dev_zeros_u32(1), "i64" if kdtype == np.int64 else "u32"
+    d_keys, d_slots = to_dev(keys), to_dev(slots)
+    hip.call("ugk_table_insert_" + wide, tb, ptr(d_keys), ptr(d_slots), 0, 0, n, ptr(st), None)
+    gone = rng.choice(n, n_gone, replace=False)
+    d_gone, d_list = to_dev(keys[gone]), to_dev(np.full(n_gone + 4, 77, np.uint32))
+    hip.call("ugk_table_evict_slots_" + wide, tb, ptr(d_gone), n_gone, ptr(d_list), ptr(st), None)
+    assert status_value(st) == 0
+    got = to_np(d_list, np.uint32)
+    assert np.array_equal(got[:n_gone], slots[gone]) and got[n_gone] == 77
+    loc, off = dev_zeros_u32(n), dev_zeros_u32(n)
+    hip.call("ugk_table_lookup_" + wide, tb, ptr(d_keys), n, 9, ptr(loc), ptr(off), None)
+    stays = np.ones(n, bool)
+    stays[gone] = False
+    got_loc, got_off = to_np(loc, np.uint32)[:n], to_np(off, np.uint32)[:n]
+    assert (got_loc[stays] == 0).all() and np.array_equal(got_off[stays], slots[stays]) and (got_loc[~stays] == 9).all()
+    # again, between keys that are there: absent, and beyond every table
+    here = keys[np.flatnonzero(stays)[:2]]
+    d_mixed = to_dev(np.array([here[0], keys[gone[0]], 0xFFFFFFFE, here[1]], kdtype))
+    hip.call("ugk_table_evict_slots_" + wide, tb, ptr(d_mixed), 4, ptr(d_list), ptr(st), None)
+    assert status_value(st) != 0
+    want = [slots[np.flatnonzero(stays)[0]], 0xFFFFFFFF, 0xFFFFFFFF, slots[np.flatnonzero(stays)[1]]]
+    assert to_np(d_list, np.uint32)[:4].tolist() == want

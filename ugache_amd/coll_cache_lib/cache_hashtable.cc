@@ -240,6 +240,19 @@ TensorPtr CacheEntryManager::CompactBits(const uint64_t *a, const uint64_t *b, b
   return list;
 }
 
+TensorPtr CacheEntryManager::EvictForSlots(TensorPtr keys_to_evict, TensorPtr &buffer,
+                                           const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream) {
+  TensorPtr slots = ReuseList(buffer, kI32, keys_to_evict->NumItem(), allocator, ctx);
+  if (keys_to_evict->Type() == kI64)
+    UGK_CALL(ugk_table_evict_slots_i64(_table, keys_to_evict->CPtr<int64_t>(), keys_to_evict->NumItem(),
+                                       slots->Ptr<uint32_t>(), StatusPtr(this, stream), stream));
+  else
+    UGK_CALL(ugk_table_evict_slots_u32(RowView(), keys_to_evict->CPtr<uint32_t>(), keys_to_evict->NumItem(),
+                                       slots->Ptr<uint32_t>(), StatusPtr(this, stream), stream));
+  NoteEvicted(keys_to_evict->NumItem());
+  return slots;
+}
+
 TensorPtr CacheEntryManager::FreeSlots(size_t n, volatile uint32_t **num_free, TensorPtr &buffer,
                                        const std::function<MemHandle(size_t)> &allocator, Context ctx,
                                        StreamHandle stream) {

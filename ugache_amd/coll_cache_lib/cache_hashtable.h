@@ -83,6 +83,9 @@ class CacheEntryManager {
   // the same, and the evicted keys' slots leave the slot bitmap (SlotUsedBits) in the same launch: what LookupOffset +
   // ReturnOffset + Evict do together when the bookkeeping lives on the device
   void EvictRelease(TensorPtr keys_to_evict, StreamHandle stream);
+  /// ... and the slots the keys held, in the order of the keys
+  TensorPtr EvictForSlots(TensorPtr keys_to_evict, TensorPtr &buffer, const std::function<MemHandle(size_t)> &allocator,
+                          Context ctx, StreamHandle stream);
   // cuh:635-655 — free-list: returned offsets go to the back, reservations come from the front
   void ReturnOffset(TensorPtr new_offsets);
   TensorPtr ReserveOffsetFront(IdType num_new_insert_keys);

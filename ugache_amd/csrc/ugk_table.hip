@@ -32,30 +32,42 @@ __global__ __launch_bounds__(kBlock) void flat_insert_kernel(uint32_t *table, ui
   }
 }
 
-// slot_bits (may be null): one bit per cache slot; the bit of the slot an evicted key held is cleared on the way
-__device__ __forceinline__ void release_slot(unsigned long long *slot_bits, uint64_t nslots, uint32_t slot,
-                                             uint32_t *status) {
-  if (slot_bits == nullptr) return;
-  if (slot >= nslots) {
+// Where the slots that evicted keys held go; either may be null.
+struct SlotsOut {
+  unsigned long long *bits;  // one bit per cache slot, cleared for those
+  uint64_t nslots;
+  uint32_t *list;            // slot of the i-th key evicted, ~0 for a key that is not there
+};
+__device__ __forceinline__ void release_slot(const SlotsOut &out, size_t i, uint32_t slot, uint32_t *status) {
+  if (out.list) out.list[i] = slot;
+  if (out.bits == nullptr) return;
+  if (slot >= out.nslots) {
     atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
     return;
   }
-  atomicAnd(slot_bits + (slot >> 6), ~(1ull << (slot & 63u)));
+  atomicAnd(out.bits + (slot >> 6), ~(1ull << (slot & 63u)));
+}
+__device__ __forceinline__ void no_slot(const SlotsOut &out, size_t i) {
+  if (out.list) out.list[i] = ~0u;
 }
 
 template <typename K>
 __global__ __launch_bounds__(kBlock) void flat_evict_kernel(uint32_t *table, uint64_t nkeys, const K *keys, size_t n,
-                                                            unsigned long long *slot_bits, uint64_t nslots,
-                                                            uint32_t *status) {
+                                                            SlotsOut slots, uint32_t *status) {
   for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
     const uint64_t key = key_to_u64<K>(keys[i]);
     if (key >= nkeys) {
       atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
+      no_slot(slots, i);
       continue;
     }
     const uint32_t old = atomicExch(table + key, UGK_EMPTY_U32);
-    if (old == UGK_EMPTY_U32) atomicOr(status, UGK_ST_EVICT_ABSENT);
-    else release_slot(slot_bits, nslots, old & 0x0fffffffu, status);
+    if (old == UGK_EMPTY_U32) {
+      atomicOr(status, UGK_ST_EVICT_ABSENT);
+      no_slot(slots, i);
+    } else {
+      release_slot(slots, i, old & 0x0fffffffu, status);
+    }
   }
 }
 
@@ -160,17 +172,17 @@ __global__ __launch_bounds__(kBlock) void hash_insert_kernel(ugk_bucket_t *table
 
 template <typename K>
 __global__ __launch_bounds__(kBlock) void hash_evict_kernel(ugk_bucket_t *table, uint64_t nb, const K *keys,
-                                                            size_t n, unsigned long long *slot_bits, uint64_t nslots,
-                                                            uint32_t *status) {
+                                                            size_t n, SlotsOut slots, uint32_t *status) {
   for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) {
     const uint64_t key = key_to_u64<K>(keys[i]);
     uint64_t pos = key_is_reserved(key) ? 0 : hash_home(key, nb);
-    bool done = key_is_reserved(key);
+    bool done = key_is_reserved(key), found = false;
     if (done) atomicOr(status, UGK_ST_EVICT_ABSENT);
     for (uint64_t step = 0; step < nb && !done; ++step) {
       const uint64_t cur = load_key_relaxed(table + pos);
       if (cur == key) {
-        if (slot_bits) release_slot(slot_bits, nslots, __atomic_load_n(&table[pos].off, __ATOMIC_RELAXED), status);
+        if (slots.bits || slots.list) release_slot(slots, i, __atomic_load_n(&table[pos].off, __ATOMIC_RELAXED), status);
+        found = true;
         // either order of these two stores is safe for a concurrent lookup: it sees the key still valid (its slot
         // keeps the row until a later lookup has passed), not valid, or gone
         store_off_meta(table + pos, 0u, 0u);
@@ -184,6 +196,7 @@ __global__ __launch_bounds__(kBlock) void hash_evict_kernel(ugk_bucket_t *table,
       }
     }
     if (!done) atomicOr(status, UGK_ST_EVICT_ABSENT);
+    if (!found) no_slot(slots, i);
   }
 }
 
@@ -290,8 +303,7 @@ __global__ __launch_bounds__(kBlock) void h32_insert_kernel(ugk_table_t t, const
 // the key in it settles the walk whatever else it holds, and one without the key but with a never-used entry ends it.
 template <typename K>
 __global__ __launch_bounds__(kBlock) void h32_evict_kernel(ugk_table_t t, const K *keys, size_t n,
-                                                           unsigned long long *slot_bits, uint64_t nslots,
-                                                           uint32_t *status) {
+                                                           SlotsOut slots, uint32_t *status) {
   unsigned long long *table = reinterpret_cast<unsigned long long *>(t.table);
   const uint64_t ne = t.size;
   const int lane = (int)lane_id();
@@ -305,7 +317,10 @@ __global__ __launch_bounds__(kBlock) void h32_evict_kernel(ugk_table_t t, const 
     const uint64_t row = active ? h32_row(t, key_to_u64<K>(keys[i])) : 0;
     bool done = !active;
     if (active && row >= kH32Tomb) {  // no entry can hold it
-      if (sub == 0) atomicOr(status, UGK_ST_EVICT_ABSENT);
+      if (sub == 0) {
+        atomicOr(status, UGK_ST_EVICT_ABSENT);
+        no_slot(slots, i);
+      }
       done = true;
     }
     const uint32_t r32 = (uint32_t)row;
@@ -324,10 +339,11 @@ __global__ __launch_bounds__(kBlock) void h32_evict_kernel(ugk_table_t t, const 
       // neighbouring slots (a refresh evicts runs of rows that went in together), whose bits share a word: the lanes
       // of the wavefront that hold a found entry merge their bits per word first, one atomic per word.
       const bool mine = !done && (m0 || m1);
-      if (slot_bits) {
-        const uint32_t slot = (uint32_t)((m0 ? w0 : w1) >> 32) & 0x0fffffffu;
+      const uint32_t slot = (uint32_t)((m0 ? w0 : w1) >> 32) & 0x0fffffffu;
+      if (slots.list && mine) slots.list[i] = slot;
+      if (slots.bits) {
         bool todo = mine;
-        if (mine && slot >= nslots) {
+        if (mine && slot >= slots.nslots) {
           atomicOr(status, UGK_ST_KEY_OUT_OF_RANGE);
           todo = false;
         }
@@ -342,7 +358,7 @@ __global__ __launch_bounds__(kBlock) void h32_evict_kernel(ugk_table_t t, const 
             const int l = __ffsll(g) - 1;
             bits |= 1ull << (__shfl(slot, l) & 63u);
           }
-          if (lane == lead) atomicAnd(slot_bits + word, ~bits);
+          if (lane == lead) atomicAnd(slots.bits + word, ~bits);
           left &= ~group;
         }
       }
@@ -355,7 +371,10 @@ __global__ __launch_bounds__(kBlock) void h32_evict_kernel(ugk_table_t t, const 
           }
           done = true;
         } else if (never || ++steps > lines) {
-          if (sub == 0) atomicOr(status, UGK_ST_EVICT_ABSENT);
+          if (sub == 0) {
+            atomicOr(status, UGK_ST_EVICT_ABSENT);
+            no_slot(slots, i);
+          }
           done = true;
         } else {
           win += 16;
@@ -482,22 +501,22 @@ int table_insert(ugk_table_t t, const K *keys, const uint32_t *offs, uint32_t se
 }
 
 template <typename K>
-int table_evict(ugk_table_t t, const K *keys, size_t n, uint64_t *slot_bits_dev, uint64_t nslots, uint32_t *status,
-                void *stream) {
+int table_evict(ugk_table_t t, const K *keys, size_t n, uint64_t *slot_bits_dev, uint64_t nslots, uint32_t *slots_out_dev,
+                uint32_t *status, void *stream) {
   if (n == 0) return 0;
   if (check_table(t, "ugk_table_evict")) return 1;
   UGK_REQUIRE(keys && status, "ugk_table_evict: null keys or status");
-  unsigned long long *slot_bits = reinterpret_cast<unsigned long long *>(slot_bits_dev);
+  const SlotsOut slots{reinterpret_cast<unsigned long long *>(slot_bits_dev), nslots, slots_out_dev};
   const unsigned grid = clamp_grid((n + kBlock - 1) / kBlock, 0);
   if (t.kind == 1)
     hipLaunchKernelGGL(flat_evict_kernel<K>, dim3(grid), dim3(kBlock), 0, as_stream(stream), (uint32_t *)t.table,
-                       t.size, keys, n, slot_bits, nslots, status);
+                       t.size, keys, n, slots, status);
   else if (t.kind == 2)
     hipLaunchKernelGGL(hash_evict_kernel<K>, dim3(grid), dim3(kBlock), 0, as_stream(stream), (ugk_bucket_t *)t.table,
-                       t.size, keys, n, slot_bits, nslots, status);
+                       t.size, keys, n, slots, status);
   else
     hipLaunchKernelGGL(h32_evict_kernel<K>, dim3(clamp_grid((n + 31) / 32, 0)), dim3(kBlock), 0, as_stream(stream), t,
-                       keys, n, slot_bits, nslots, status);
+                       keys, n, slots, status);
   UGK_HIP(hipGetLastError());
   return 0;
 }
@@ -591,20 +610,30 @@ int ugk_table_insert_i64(ugk_table_t t, const int64_t *keys_dev, const uint32_t 
   return table_insert<int64_t>(t, keys_dev, offs_dev, seq_base, loc, n, status_dev, stream);
 }
 int ugk_table_evict_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint32_t *status_dev, void *stream) {
-  return table_evict<uint32_t>(t, keys_dev, n, nullptr, 0, status_dev, stream);
+  return table_evict<uint32_t>(t, keys_dev, n, nullptr, 0, nullptr, status_dev, stream);
 }
 int ugk_table_evict_i64(ugk_table_t t, const int64_t *keys_dev, size_t n, uint32_t *status_dev, void *stream) {
-  return table_evict<int64_t>(t, keys_dev, n, nullptr, 0, status_dev, stream);
+  return table_evict<int64_t>(t, keys_dev, n, nullptr, 0, nullptr, status_dev, stream);
 }
 int ugk_table_evict_release_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint64_t *slot_bits_dev,
                                 uint64_t nslots, uint32_t *status_dev, void *stream) {
   UGK_REQUIRE(n == 0 || slot_bits_dev, "ugk_table_evict_release_u32: null slot bitmap");
-  return table_evict<uint32_t>(t, keys_dev, n, slot_bits_dev, nslots, status_dev, stream);
+  return table_evict<uint32_t>(t, keys_dev, n, slot_bits_dev, nslots, nullptr, status_dev, stream);
 }
 int ugk_table_evict_release_i64(ugk_table_t t, const int64_t *keys_dev, size_t n, uint64_t *slot_bits_dev,
                                 uint64_t nslots, uint32_t *status_dev, void *stream) {
   UGK_REQUIRE(n == 0 || slot_bits_dev, "ugk_table_evict_release_i64: null slot bitmap");
-  return table_evict<int64_t>(t, keys_dev, n, slot_bits_dev, nslots, status_dev, stream);
+  return table_evict<int64_t>(t, keys_dev, n, slot_bits_dev, nslots, nullptr, status_dev, stream);
+}
+int ugk_table_evict_slots_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint32_t *slots_out_dev, uint32_t *status_dev,
+                              void *stream) {
+  UGK_REQUIRE(n == 0 || slots_out_dev, "ugk_table_evict_slots_u32: null list of slots");
+  return table_evict<uint32_t>(t, keys_dev, n, nullptr, 0, slots_out_dev, status_dev, stream);
+}
+int ugk_table_evict_slots_i64(ugk_table_t t, const int64_t *keys_dev, size_t n, uint32_t *slots_out_dev, uint32_t *status_dev,
+                              void *stream) {
+  UGK_REQUIRE(n == 0 || slots_out_dev, "ugk_table_evict_slots_i64: null list of slots");
+  return table_evict<int64_t>(t, keys_dev, n, nullptr, 0, slots_out_dev, status_dev, stream);
 }
 int ugk_table_lookup_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint32_t fallback_loc,
                          uint32_t *loc_out_dev, uint32_t *off_out_dev, void *stream) {

@@ -112,6 +112,8 @@ SIGNATURES = {
     "ugk_table_insert_i64": [Table, _vp, _vp, _u32, _u32, _sz, _vp, _vp],
     "ugk_table_evict_u32": [Table, _vp, _sz, _vp, _vp],
     "ugk_table_evict_i64": [Table, _vp, _sz, _vp, _vp],
+    "ugk_table_evict_slots_u32": [Table, _vp, _sz, _vp, _vp, _vp],
+    "ugk_table_evict_slots_i64": [Table, _vp, _sz, _vp, _vp, _vp],
     "ugk_table_evict_release_u32": [Table, _vp, _sz, _vp, _u64, _vp, _vp],
     "ugk_table_evict_release_i64": [Table, _vp, _sz, _vp, _u64, _vp, _vp],
     "ugk_table_lookup_u32": [Table, _vp, _sz, _u32, _vp, _vp, _vp],
