@@ -161,9 +161,9 @@ int main(int argc, char **argv) {
     rc = fn(dev(1), 1000, static_cast<int64_t *>(dev(2)), static_cast<uint32_t *>(dev(4)), number(4), dev(3), 1000, number(3), 0, u32,
             nullptr, dev(11)) ||
          next(dev(1), 1000, static_cast<int64_t *>(dev(2)), number(4), dev(3), number(3), 0, u32, nullptr, dev(11));
-  } else if (call == "mix" && argc == 6 && ask(number(5))) {
+  } else if (call == "mix" && argc >= 6 && ask(number(5))) {
     ugk_table_t flat{};
-    flat.kind = 1, flat.table = dev(4), flat.size = 1000;
+    flat.kind = argc > 6 ? (int32_t)number(6) : 1, flat.table = dev(4), flat.size = flat.kind == 1 ? 1000 : 1024;
     const auto fn = reinterpret_cast<decltype(&ugk_extract_mix_i64)>(dlsym(lib, "ugk_extract_mix_i64"));
     rc = fn(flat, static_cast<int64_t *>(dev(2)), number(4), dev(1), 1000, dev(5), 1000, dev(3), number(3), u32, nullptr, nullptr,
             nullptr, UGK_HINT_UNKNOWN, dev(11));

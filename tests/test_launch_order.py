@@ -76,6 +76,15 @@ def test_a_lookup_is_told_its_end_by_words_where_they_are_sooner(launches, call,
     assert (launches(call, row_bytes, rows, 3)[1] > 0) == (told != "too late")  # keys would be copied by a kernel
 
 
+# (table, row bytes, rows): a flat table's lines for rows of more than 1 KB, where a hash table has none; and a few long rows
+@pytest.mark.parametrize("kind,row_bytes,rows,sooner", [(1, 1040, 4_032, True), (1, 1040, 4_034, False), (1, 4112, 1_020, True),
+                                                        (1, 4112, 1_021, False), (3, 1040, 4_034, True), (2, 4112, 8_160, True),
+                                                        (3, 4112, 5, True), (3, 4112, 4, False), (1, 4112, 4, False), (3, 4096, 4, True)])
+def test_a_mixed_lookup_of_long_rows_is_told_its_end_by_words(launches, kind, row_bytes, rows, sooner):
+    assert (launches("mix", row_bytes, rows, 2, kind)[1] > 0) == sooner
+    assert launches("mix", row_bytes, rows, 1, kind)[1] > 0  # who insists gets them
+
+
 @pytest.mark.parametrize("row_bytes,bag,mb,told", [(512, 1, 67, True), (512, 1, 67.2, False), (512, 2, 68, False), (512, 3, 68, True),
                                                    (1024, 2, 67, True), (1024, 2, 68, False), (4096, 4, 134, True)])
 def test_a_pooled_lookup_is_told_its_end_by_words_where_they_are_sooner(launches, row_bytes, bag, mb, told):

@@ -149,12 +149,14 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
         if (no_branch) {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) v[u] = ld_stream(src + s[u] * vpr + col);
+          if constexpr (STORE == kThrough) arrived(v);
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u) put(u);
         } else {
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
             if (ok[u]) v[u] = ld_stream(src + s[u] * vpr + col);
+          arrived(v);
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
             if (ok[u]) put(u);
@@ -301,6 +303,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     u32x4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
+    if constexpr (STORE == kThrough) arrived(v);
     if constexpr (SHARE) {
       if (head) {
         const gout_t q = reinterpret_cast<gout_t>(to + end - head);

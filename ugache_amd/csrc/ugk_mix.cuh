@@ -31,6 +31,22 @@ __device__ __forceinline__ void store_through(uint64_t to, V v) {
   else asm volatile("global_store_byte %0, %1, off sc0 sc1" ::"v"(p), "v"((uint32_t)v) : "memory");
 }
 
+// Everything in v has arrived, before the first of it is stored.  One counter counts a wavefront's loads and stores, in the
+// order they were issued, and a wait names how many may still be on their way.  Stores that are written through are not in
+// the compiler's count (they are assembly), stores behind a condition may or may not have been issued: so the wait for the
+// second of four loads would be one for the first store as well, until that is in memory, and a lane's stores leave one by
+// one.  us, launch to end of poll, before / with this: gather 512 bytes x 1,024 10.8 / 10.2, 4 KB x 128 13.5 / 11.7, 8 KB x
+// 1,024 19.3 / 15.6; lookup and gather in one kernel, 512 bytes x 4,096 13.9 / 13.3, 1 KB x 4,096 15.9 / 14.7, 2 KB x 512 17.1 /
+// 14.3, 4 KB x 2,048 25.5 / 18.7; that kernel with ordinary stores and a ticket behind it 15.3 / 15.1, 16.1 / 15.6, 16.3 / 14.9,
+// 22.8 / 19.8.  (Ordinary stores of the flat and the stream copy of a plain gather: 1 to 5 % either way, left as they were.)
+template <typename V, int N>
+__device__ __forceinline__ void arrived(V (&v)[N]) {
+  if constexpr (sizeof(V) >= 4) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) asm volatile("" : "+v"(v[u]));
+  }
+}
+
 // how a kernel stores its rows: a template parameter, not a launch argument, for with a run-time choice the optimiser merges
 // an ordinary and a non-temporal store into one and the hint is lost, and the code of all of them costs a small launch
 // 0.2 to 0.4 us (26,624 rows of 64 bytes 3.6 -> 4.0)
@@ -151,7 +167,7 @@ static inline FlatRow flat_row(size_t row_bytes, uint32_t tile) {
 // Copies the rows r0 .. r0 + count - 1 of the wavefront, count <= f.tile: lane r holds where row r is read (kNoRowBit:
 // not at all) and, with DENSE false, which output row it becomes; with DENSE row r becomes output row d0 + r.  All
 // lanes call it with the same r0 and count.
-template <bool DENSE, bool THROUGH>
+template <bool DENSE, bool THROUGH, bool WAIT = THROUGH>
 __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, char *out, size_t d0, uint32_t r0,
                                           uint32_t count, const FlatRow &f) {
   constexpr int U = 4;  // vectors in flight per lane
@@ -177,6 +193,7 @@ __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, c
     u32x4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
+    if constexpr (WAIT) arrived(v);
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (ok[u]) {

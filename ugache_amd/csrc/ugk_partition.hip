@@ -188,6 +188,7 @@ __device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits,
         u32x4 v[UNROLL];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) v[u] = __builtin_nontemporal_load(p[u] + col);
+        arrived(v);
         const gout_t dst = (gout_t)out + (b0 + r0 + rg) * vpr + col;
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
@@ -265,7 +266,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       const uint64_t bits = row.has_row ? row.bits : row.bits | kNoRowBit;
       const uint32_t here = (uint32_t)min((size_t)KPW, n - b0);
       for (uint32_t r0 = 0; r0 < here; r0 += f_row.tile)
-        flat_copy<true, STORE == kThrough>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
+        flat_copy<true, STORE == kThrough, true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
     } else {
       const uint32_t vpr = f_row.chunks;
       uint64_t stage_bits = 0;
@@ -569,14 +570,16 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const FlatRow f_row = flat_row(row_bytes, (uint32_t)kpw);
   const size_t keys_per_group = (size_t)kpw * kWavesPerBlock;
   const unsigned grid = request.grid(clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u));
-  // Rows of more than one vector per lane wait between their vectors, for memory where they are written through: a ticket behind
-  // the launch is there sooner than words (see gather_tells).  us, launch to end of poll, ticket / words, all
-  // rows in HBM: 1536 bytes x 40 10.7 / 12.1, x 5,200 14.5 / 15.6, x 20,800 21.4 / 21.8; 4 KB x 250 17.0 / 18.7, x 2,000 18.6 / 20.6,
-  // x 8,192 23.5 / 25.0, x 16,384 32.9 / 32.8; 8 KB 5 to 20 % later up to 64 MB.  With a tenth of the rows over the link 4 KB 5 to
-  // 10 % later up to 4 MB, 2 to 4 % sooner from 16 MB on.  Up to 1 KB words are 2 to 7 % sooner with a tenth of the rows over the
-  // link at any size; with all of them in HBM sooner too but for rows of more than 512 bytes and 4 to 16 MB, 3 to 5 % later.
-  const Telling words =
-      row_bytes <= 1024 || (row_bytes <= 4096 && n * row_bytes > (size_t)32 << 20) ? Telling::kSooner : Telling::kLater;
+  // Words come sooner than a ticket behind the launch would, but for up to four long rows, whose wavefront waits between their
+  // vectors for memory, where they are written through (see gather_tells).  us, launch to end of poll, ticket / words, all rows
+  // in HBM, a hash table: 512 bytes x 1,024 13.2 / 12.3; 1536 bytes x 85 15.1 / 12.9, x 5,461 19.5 / 16.8; 4 KB x 4 12.6 / 12.7, x 8 15.0 /
+  // 14.3, x 2,048 20.2 / 19.0, x 16,384 36.9 / 33.4; 8 KB x 2 13.0 / 14.3, x 8 18.8 / 18.7, x 1,024 24.6 / 23.6; 32 KB x 4 34.2 / 38.8, x 64
+  // 51.4 / 50.3; a twentieth of the rows over the link: the same signs.  With a flat table rows of more than 1 KB gain up to outputs
+  // of 4 MB (1040 bytes x 252 13.4 / 12.5, x 4,032 13.9 / 13.6) and, of up to 4 KB, beyond 32 MB, and come out even between those
+  // (1040 bytes x 8,065 14.8 / 14.8, 4112 bytes x 2,040 18.8 / 18.8, 4 KB x 8,192 22.9 / 22.5).
+  const size_t out_bytes = n * row_bytes;
+  const bool even = KIND == 1 && row_bytes > 1024 && out_bytes > (size_t)4 << 20 && (row_bytes > 4096 || out_bytes <= (size_t)32 << 20);
+  const Telling words = even || (row_bytes > 4096 && n <= 4) ? Telling::kLater : Telling::kSooner;
   DoneWords done = nt && !flat ? DoneWords{} : request.take(grid, words, n);
   UGK_REQUIRE(!request.counted(), "ugk_extract_mix: a launch that leaves no words cannot take its count from the device");
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
