@@ -168,6 +168,16 @@ def test_gather_of_more_than_one_round_of_workgroups(row_bytes, n, hint):
     _gather_with_keys_that_miss(row_bytes, n, hint)
 
 
+# both sides of the lines between launches of which all wavefronts, one of four and none load past the caches: short rows of
+# whole vectors whose lines the L2s just hold, rows of 48 bytes, output and kept lines of 256 MiB
+@pytest.mark.parametrize("row_bytes,n", [(16, 180_224), (16, 180_225), (32, 458_752), (32, 458_753), (20, 300_001), (44, 9_001),
+                                         (48, 9_001), (48, 2_981_300), (512, 419_430), (512, 419_431), (500, 409_200),
+                                         (500, 409_201), (1204, 174_762), (1204, 174_763)])
+@pytest.mark.parametrize("hint", [0, 1])
+def test_gather_on_both_sides_of_what_the_caches_hold(row_bytes, n, hint):
+    _gather_with_keys_that_miss(row_bytes, n, hint)
+
+
 def test_gather_direct_empty_and_capped_grid():
     rng = np.random.default_rng(1)
     table = _rand_table(rng, 100, 512)

@@ -6,9 +6,10 @@
 //     instruction moves 64/LPR whole rows as fully coalesced segments (512-B rows: 2 rows, 128-B rows: 8);
 //   * every lane keeps UNROLL = 2 independent rows in flight (both loads issued before the first store) and the
 //     launch uses many small workgroups of one pass each (gather_kernel has the figures of one, four and eight rows);
-//   * loads carry the non-temporal hint (table rows are touched once); stores are ordinary write-back stores
-//     while the output fits the 256 MiB memory-side cache, so the consumer finds it there, and non-temporal
-//     beyond that or when the caller says its outputs do not stay there (ugk_set_output_hint);
+//   * three wavefronts of four load with the non-temporal hint (most rows of a table are touched once), the fourth
+//     without it for the rows that a batch repeats (keep_waves_for has the figures and the exceptions); stores are
+//     ordinary write-back stores while the output fits the 256 MiB memory-side cache, so the consumer finds it there, and
+//     non-temporal beyond that or when the caller says its outputs do not stay there (ugk_set_output_hint);
 //   * the grid has one workgroup per pass of rows, or is capped by the caller so a host-link gather occupies
 //     only a few CUs while the HBM gather runs next to it (then the workgroups stride over the batch);
 //   * rows of other lengths have two more kernels: gather_flat_kernel (any multiple of 4 bytes, see flat_copy) and
@@ -17,6 +18,7 @@
 //     and its row is skipped instead of faulting.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "ugk_internal.h"
 #include "ugk_mix.cuh"
@@ -74,9 +76,10 @@ struct IdxList {
   }
 };
 
-template <typename V>
-__device__ __forceinline__ V ld_stream(const V *p) {
-  return __builtin_nontemporal_load(p);
+template <bool KEEP, typename V>
+__device__ __forceinline__ V ld_row(const V *p) {
+  if constexpr (KEEP) return *p;
+  else return __builtin_nontemporal_load(p);
 }
 template <typename V>
 __device__ __forceinline__ void st_stream(V *p, V v) {
@@ -97,7 +100,7 @@ template <typename V, int LPR, int UNROLL, Store STORE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restrict__ src, uint64_t src_rows,
                                                         V *__restrict__ out, uint64_t out_rows, uint32_t vpr,
                                                         const uint32_t *__restrict__ counts, uint32_t group,
-                                                        bool many_groups, size_t n, uint32_t *status, uint32_t *host_mirror, Ending<STORE> done) {
+                                                        bool many_groups, uint8_t keep_waves, size_t n, uint32_t *status, uint32_t *host_mirror, Ending<STORE> done) {
   size_t begin = 0, count = Idx::kDense ? launch_count(done, n) : n;
   if (counts) {
     const uint32_t c = counts[group];
@@ -136,32 +139,36 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
     for (int u = 0; u < UNROLL; ++u) whole = whole && ok[u];
     // (rows of up to 64 bytes gain nothing and stay as they were)
     const bool no_branch = LPR >= 8 && (many_groups || vpr > LPR) && __ballot(!whole) == 0ull;
-    for (uint32_t c0 = 0; c0 < vpr; c0 += LPR) {
-      const uint32_t col = c0 + lane;
-      if (col < vpr) {
-        V v[UNROLL];
-        auto put = [&](int u) {
-          V *to = out + d[u] * vpr + col;
-          if constexpr (STORE == kThrough) store_through(reinterpret_cast<uint64_t>(to), v[u]);
-          else if constexpr (STORE == kStreaming) st_stream(to, v[u]);
-          else *to = v[u];
-        };
-        if (no_branch) {
-#pragma unroll
-          for (int u = 0; u < UNROLL; ++u) v[u] = ld_stream(src + s[u] * vpr + col);
-          if constexpr (STORE == kThrough) arrived(v);
-#pragma unroll
-          for (int u = 0; u < UNROLL; ++u) put(u);
-        } else {
+    // (a loop of its own for each way: in one loop the compiler makes one last store of the two arms' and lets it wait for
+    // the others, 5 % of a launch)
+    auto copy = [&](auto keep, auto branch) {
+      constexpr bool KEEP = decltype(keep)::value, BRANCH = decltype(branch)::value;
+      for (uint32_t c0 = 0; c0 < vpr; c0 += LPR) {
+        const uint32_t col = c0 + lane;
+        if (col < vpr) {
+          V v[UNROLL];
 #pragma unroll
           for (int u = 0; u < UNROLL; ++u)
-            if (ok[u]) v[u] = ld_stream(src + s[u] * vpr + col);
-          arrived(v);
+            if (!BRANCH || ok[u]) v[u] = ld_row<KEEP>(src + s[u] * vpr + col);
+          if constexpr (BRANCH || STORE == kThrough) arrived(v);
 #pragma unroll
-          for (int u = 0; u < UNROLL; ++u)
-            if (ok[u]) put(u);
+          for (int u = 0; u < UNROLL; ++u) {
+            if (BRANCH && !ok[u]) continue;
+            V *to = out + d[u] * vpr + col;
+            if constexpr (STORE == kThrough) store_through(reinterpret_cast<uint64_t>(to), v[u]);
+            else if constexpr (STORE == kStreaming) st_stream(to, v[u]);
+            else *to = v[u];
+          }
         }
       }
+    };
+    // (written through, only short rows gain, see keep_waves_for: no code for the others)
+    if ((STORE != kThrough || sizeof(V) * LPR < 64) && wave_in_block() < keep_waves) {
+      if (no_branch) copy(std::true_type{}, std::false_type{});
+      else copy(std::true_type{}, std::true_type{});
+    } else {
+      if (no_branch) copy(std::false_type{}, std::false_type{});
+      else copy(std::false_type{}, std::true_type{});
     }
     if constexpr (Idx::kDense && STORE == kThrough) {
       if (base < done.num_keys)
@@ -178,8 +185,8 @@ template <Store STORE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                              char *__restrict__ out, uint64_t out_rows, FlatRow f,
                                                              const uint32_t *__restrict__ counts, uint32_t group,
-                                                             size_t n, uint32_t *status, uint32_t *host_mirror,
-                                                             Ending<STORE> done) {
+                                                             uint8_t keep_waves, size_t n, uint32_t *status,
+                                                             uint32_t *host_mirror, Ending<STORE> done) {
   size_t begin = 0, count = Idx::kDense ? launch_count(done, n) : n;
   if (counts) {
     const uint32_t c = counts[group];
@@ -204,7 +211,11 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
       // a row that is skipped is read where the tile's first good row is
       const uint64_t at = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
       const uint64_t dummy = shfl64(at, __ffsll(good) - 1);
-      flat_copy<Idx::kDense, STORE == kThrough>(ok ? at : dummy | kNoRowBit, (uint32_t)d, out, base, 0, rows, f);
+      const uint64_t bits = ok ? at : dummy | kNoRowBit;
+      if (wave_in_block() < keep_waves)
+        flat_copy<Idx::kDense, STORE == kThrough, true>(bits, (uint32_t)d, out, base, 0, rows, f);
+      else
+        flat_copy<Idx::kDense, STORE == kThrough, false>(bits, (uint32_t)d, out, base, 0, rows, f);
     }
     if constexpr (Idx::kDense && STORE == kThrough) {
       if (lane_id() < rows) copy_key_along(done, base + lane_id(), (typename Idx::key_t)s);
@@ -235,7 +246,8 @@ StreamRow stream_row(size_t row_bytes, size_t n) {
 template <Store STORE, bool SHARE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                                char *__restrict__ out, StreamRow f, uint32_t *status,
-                                                               uint32_t *host_mirror, Ending<STORE> done) {
+                                                               uint32_t *host_mirror, Ending<STORE> done,
+                                                               uint8_t keep_waves) {
   static_assert(Idx::kDense, "row i goes to output row i");
   typedef __attribute__((address_space(1))) uint32_t *gword_t;
   constexpr int U = (int)(kStreamPart / (kWave * 16));
@@ -274,64 +286,75 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
     const uint64_t dummy = shfl64(mine, __ffsll(good) - 1);
     const uint64_t at = ok ? mine : dummy;
     const uint32_t lo = (uint32_t)at | (ok ? 0u : kNoRowBit), hi = (uint32_t)(at >> 32);
-    // the vector that row l shares with the next one is lane l's: `end` is where row l ends in the part, its last `head`
-    // bytes lie in that vector (no branch around the two loads: the ones that follow would wait for them at its end)
-    u32x4 sa{}, sb{};
-    uint32_t head = 0, end = 0, nlo = kNoRowBit;
-    if constexpr (SHARE) {
-      nlo = __shfl_down(lo, 1);
-      const uint32_t nhi = __shfl_down(hi, 1);
-      end = (lane + 1) * f.row_bytes - off0;
-      if (active && end < bytes) head = end % 16;
-      sa = __builtin_nontemporal_load(reinterpret_cast<grow_by4_t>(at + f.row_bytes - 16));
-      sb = __builtin_nontemporal_load(reinterpret_cast<grow_by4_t>(((uint64_t)nhi << 32) | (nlo & ~kNoRowBit)));
-    }
-    grow_by4_t p[U];
-    bool copy[U];
+    auto part = [&](auto keep) {
+      constexpr bool KEEP = decltype(keep)::value;
+      // the vector that row l shares with the next one is lane l's: `end` is where row l ends in the part, its last `head`
+      // bytes lie in that vector (no branch around the two loads: the ones that follow would wait for them at its end)
+      u32x4 sa{}, sb{};
+      uint32_t head = 0, end = 0, nlo = kNoRowBit;
+      if constexpr (SHARE) {
+        nlo = __shfl_down(lo, 1);
+        const uint32_t nhi = __shfl_down(hi, 1);
+        end = (lane + 1) * f.row_bytes - off0;
+        if (active && end < bytes) head = end % 16;
+        sa = __builtin_nontemporal_load(reinterpret_cast<grow_by4_t>(at + f.row_bytes - 16));
+        sb = __builtin_nontemporal_load(reinterpret_cast<grow_by4_t>(((uint64_t)nhi << 32) | (nlo & ~kNoRowBit)));
+      }
+      u32x4 v[U];
+      bool copy[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t i = (u * kWave + lane) * 16;
-      const bool in = i + 16 <= bytes;
-      const uint32_t x = off0 + (in ? i : 0u);  // a lane past the end reads the part's first vector
-      const uint32_t r = max(__umulhi(x, f.magic), x >= f.row_bytes ? 1u : 0u);
-      const uint32_t off = x - r * f.row_bytes;
-      const uint32_t rlo = __shfl(lo, (int)r), rhi = __shfl(hi, (int)r);
-      copy[u] = in && (rlo & kNoRowBit) == 0 && (!SHARE || off + 16 <= f.row_bytes);
-      p[u] = reinterpret_cast<grow_by4_t>((((uint64_t)rhi << 32) | (rlo & ~kNoRowBit)) +
-                                          (SHARE ? min(off, f.row_bytes - 16) : off));
-    }
-    u32x4 v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
-    if constexpr (STORE == kThrough) arrived(v);
-    if constexpr (SHARE) {
-      if (head) {
-        const gout_t q = reinterpret_cast<gout_t>(to + end - head);
-        const bool row_a = (lo & kNoRowBit) == 0, row_b = (nlo & kNoRowBit) == 0;
-        u32x4 w;  // the last words of sa, then the first of sb
-        w.x = head == 12 ? sa.y : head == 8 ? sa.z : sa.w;
-        w.y = head == 12 ? sa.z : head == 8 ? sa.w : sb.x;
-        w.z = head == 12 ? sa.w : head == 8 ? sb.x : sb.y;
-        w.w = head == 12 ? sb.x : head == 8 ? sb.y : sb.z;
-        if (row_a && row_b) {
-          if constexpr (STORE == kStreaming) __builtin_nontemporal_store(w, q);
-          else put(q, w);
-        } else {  // a skipped row leaves its words of the output alone
-          const gword_t q1 = reinterpret_cast<gword_t>(q);
-          if (row_a) put(q1, (uint32_t)w.x);
-          if (head > 4 ? row_a : row_b) put(q1 + 1, (uint32_t)w.y);
-          if (head > 8 ? row_a : row_b) put(q1 + 2, (uint32_t)w.z);
-          if (row_b) put(q1 + 3, (uint32_t)w.w);
+      for (int u = 0; u < U; ++u) {
+        const uint32_t i = (u * kWave + lane) * 16;
+        const bool in = i + 16 <= bytes;
+        const uint32_t x = off0 + (in ? i : 0u);  // a lane past the end reads the part's first vector
+        const uint32_t r = max(__umulhi(x, f.magic), x >= f.row_bytes ? 1u : 0u);
+        const uint32_t off = x - r * f.row_bytes;
+        const uint32_t rlo = __shfl(lo, (int)r), rhi = __shfl(hi, (int)r);
+        copy[u] = in && (rlo & kNoRowBit) == 0 && (!SHARE || off + 16 <= f.row_bytes);
+        const grow_by4_t p = reinterpret_cast<grow_by4_t>((((uint64_t)rhi << 32) | (rlo & ~kNoRowBit)) +
+                                                          (SHARE ? min(off, f.row_bytes - 16) : off));
+        if constexpr (KEEP) v[u] = *p;
+        else v[u] = __builtin_nontemporal_load(p);
+      }
+      if constexpr (STORE == kThrough) arrived(v);
+      if constexpr (STORE == kThrough && SHARE) arrived(sa), arrived(sb);
+      if constexpr (SHARE) {
+        if (head) {
+          const gout_t q = reinterpret_cast<gout_t>(to + end - head);
+          const bool row_a = (lo & kNoRowBit) == 0, row_b = (nlo & kNoRowBit) == 0;
+          u32x4 w;  // the last words of sa, then the first of sb
+          w.x = head == 12 ? sa.y : head == 8 ? sa.z : sa.w;
+          w.y = head == 12 ? sa.z : head == 8 ? sa.w : sb.x;
+          w.z = head == 12 ? sa.w : head == 8 ? sb.x : sb.y;
+          w.w = head == 12 ? sb.x : head == 8 ? sb.y : sb.z;
+          if (row_a && row_b) {
+            if constexpr (STORE == kStreaming) __builtin_nontemporal_store(w, q);
+            else put(q, w);
+          } else {  // a skipped row leaves its words of the output alone
+            const gword_t q1 = reinterpret_cast<gword_t>(q);
+            if (row_a) put(q1, (uint32_t)w.x);
+            if (head > 4 ? row_a : row_b) put(q1 + 1, (uint32_t)w.y);
+            if (head > 8 ? row_a : row_b) put(q1 + 2, (uint32_t)w.z);
+            if (row_b) put(q1 + 3, (uint32_t)w.w);
+          }
         }
       }
-    }
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (copy[u]) {
-        const gout_t q = reinterpret_cast<gout_t>(to + (u * kWave + lane) * 16);
-        if constexpr (STORE == kStreaming) __builtin_nontemporal_store(v[u], q);
-        else put(q, v[u]);
-      }
+      for (int u = 0; u < U; ++u)
+        if (copy[u]) {
+          const gout_t q = reinterpret_cast<gout_t>(to + (u * kWave + lane) * 16);
+          if constexpr (STORE == kStreaming) __builtin_nontemporal_store(v[u], q);
+          else put(q, v[u]);
+        }
+    };
+    if (STORE != kThrough && wave_in_block() < keep_waves) {
+      // (for the compiler alone, which makes one of two loads that differ in the hint, and that without it)
+      asm volatile("" ::: "memory");
+      part(std::true_type{});
+      asm volatile("" ::: "memory");
+    } else {
+      part(std::false_type{});
+    }
     if constexpr (SHARE) {
       const uint32_t rest = bytes % 16;  // the words behind the last whole vector of the output: the end of its last row
       if (rest) {
@@ -449,7 +472,7 @@ __global__ __launch_bounds__(kBlock) void gather_staged_kernel(const u32x4 *__re
       if (col < vpr) {
         u32x4 v[UNROLL];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) v[u] = ld_stream(src[u] + col);
+        for (int u = 0; u < UNROLL; ++u) v[u] = ld_row<false>(src[u] + col);
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
           if (ok[u]) out[d[u] * vpr + col] = v[u];
@@ -472,14 +495,60 @@ unsigned gather_grid(size_t passes, unsigned max_blocks) {
   return (unsigned)(passes > 0x7fffffffull ? 0x7fffffffull : passes);
 }
 
+// A caller caps the launch for rows that come over a link, and the groups other than the local one are peers and the host.
+bool over_link(const uint32_t *counts, uint32_t group, unsigned max_blocks) {
+  return max_blocks != 0 || (counts && group != UGK_LOC_LOCAL);
+}
+
+// How many of a workgroup's four wavefronts load rows the ordinary way, the others past the caches.  What a wavefront
+// loads past the caches keeps their room for the output, but a row that the batch repeats (keys are skewed, and a line
+// holds several short rows) is fetched as often as it is asked for, through the channel where its line lives.  One
+// wavefront of four is enough for the rows that come often to be found in the caches by all four, and leaves three
+// quarters of the room alone.  us, 512-byte rows in HBM, none / one / four of the wavefronts, keys uniform and
+// zipf 0.8 and 1.05: 8 MB 5.1 / 5.0 / 5.3 and 5.1 / 4.9 / 5.0 and 4.8 / 4.7 / 4.4; 64 MB 25.6 / 24.6 / 25.3 and
+// 24.9 / 24.2 / 23.7 and 25.4 / 22.4 / 19.2; 128 MB 44.8 / 43.8 / 44.7 and 45.5 / 42.7 / 42.1 and 48.8 / 41.0 / 39.0;
+// 200 MB 65.9 / 65.9 / 84.6 and 66.5 / 63.3 / 72.7; streaming stores, 290 MB 103 / 98 / 106 and 104 / 92 / 91 and
+// 96 / 87 / 86.
+//   * The output and the share of the lines that is kept have to fit the memory-side cache, or the lines push the output
+//     out (250 MB, uniform keys: 80 none, 99 one of four); a launch with streaming stores has left it to the lines.
+//   * Rows under 48 bytes, of which a line holds several: all four, at every size (32 bytes, 128 MB, uniform 113 / 108 / 106,
+//     zipf 1.05 90 / 71 / 62; 4 bytes, 64 MB 371 / 312 / 317 and 248 / 180 / 136; 40 bytes, 200 MB 182 / 199 / 173).
+//     Except that lines that come to about what the L2s hold, 32 MB, push the output out of there, the more the longer the
+//     rows: 262,144 rows of 32 bytes 8.7 / 9.1 / 9.7, of 16 bytes 8.0 / 8.5 / 8.6, of 20 bytes (flat) 9.0 / 9.0 / 9.5, of
+//     12 bytes 8.4 / 8.4 / 8.3, where 131,072 and 524,288 of them lose nothing.
+//   * Stores that are written through keep no room in the L2s, and of the rows of 48 bytes and more those come no sooner: none
+//     (512 bytes x 131,072, launch to end of poll, none / one, uniform and zipf 1.05: 30.4 / 29.6 and 27.4 / 27.8; 1204 bytes x 870
+//     10.8 / 11.1, the code for both.  16 bytes x 1,048,576 34.6 / 32.5 and 25.9 / 21.8 with all four; 36 bytes
+//     x 466,033 25.4 / 24.7 and 21.2 / 19.4, x 5,688,888 194 / 201 and 131 / 123.)
+//   * Rows over a link: none, as nothing that the chip's caches do shows beside the link (that of an uncapped gather out of
+//     host memory, which cannot be told from one out of HBM here: 16 to 1204 bytes x 0.25 to 8 MB 0.98 to 1.2 times as fast).
+constexpr size_t kMemorySideCache = 256ull << 20;
+uint8_t keep_waves_for(size_t n, size_t row_bytes, Store store, bool over_link) {
+  constexpr size_t kLine = 128;
+  if (over_link) return 0;
+  // bytes of the lines that a row touches, on the average over where it can begin
+  const size_t lines = kLine % row_bytes == 0      ? kLine
+                       : row_bytes % kLine == 0    ? row_bytes
+                       : row_bytes % 16 == 0       ? row_bytes + kLine - 16
+                                                   : row_bytes + kLine - 4;
+  if (row_bytes < 48) {
+    if (store == kThrough && row_bytes > 32 && n * (row_bytes + lines) > kMemorySideCache) return 0;
+    const bool as_l2 = n > (22ull << 20) / kLine && n <= (56ull << 20) / kLine;
+    return !as_l2 || row_bytes < 16 ? kWavesPerBlock : row_bytes % 16 == 0 ? 0 : 1;
+  }
+  if (store == kThrough) return 0;
+  return store == kStreaming || n * (row_bytes + lines / kWavesPerBlock) <= kMemorySideCache ? 1 : 0;
+}
+
 // Words (ugk_leave_done_words) come later than a ticket kernel behind the launch would
 //   * for rows of single bytes or pairs: a line that is written through does not come together in L2.  us, launch to end of
 //     poll, ticket / words, rows in HBM: 97 bytes 1 MB 9.9 / 10.2, 8 MB 22.8 / 27.5, 32 MB 62 / 84; 1001 bytes 1 MB 15.8 / 19.6,
 //     8 MB 18.7 / 23.8, 32 MB 36 / 54;
-//   * for rows of more than two vectors per lane: the loads of a row's next vectors come back behind the stores of the last, and
-//     those end in memory, not in L2.  4 KB x 64 8.9 / 9.6, x 250 10.0 / 10.9, x 2,000 12.8 / 13.5, x 8,000 19.6 / 20.1; 8 KB x 64
-//     10.7 / 12.8, x 1,000 15.5 / 17.9, x 4,000 20.4 / 22.6; 16 KB 14 to 29 % later.  2 KB 2 to 12 % sooner at any size.  Large
-//     outputs hide it (blocking lookups of 8,192 rows of 8 KB 30.5 / 28.5).
+//   * for a few rows of more than two vectors per lane: the loads of a row's next vectors come back behind the stores of the last,
+//     and those end in memory, not in L2, with nothing else to do meanwhile.  Ticket / words: 8 KB x 4 10.7 / 11.1, 16 KB x 2 11.4 /
+//     13.0, x 8 17.3 / 17.5, 32 KB x 1 14.1 / 17.7, x 16 25.9 / 26.0; with more rows they come out even or words a little sooner (4 KB x
+//     128 11.8 / 11.6, x 2,048 14.2 / 13.6; 8 KB x 64 13.5 / 13.5, x 1,024 16.3 / 15.8).  2 KB 2 to 14 % sooner at any size, as large
+//     outputs are (4 KB x 16,384 31.8 / 29.9).
 // (Outputs of 6 to 10 MB, about what the wavefronts of one round copy and all written at once, are 0.1 to 0.6 us later too where
 // a launch costs the host 3 us, and 0.9 us sooner where it costs 4: words there.)
 Telling gather_tells(size_t vector_bytes, uint32_t vectors_per_row, uint32_t lanes, size_t out_bytes) {
@@ -499,10 +568,12 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
     if (!nt) done = request.take(grid, gather_tells(sizeof(V), vpr, LPR, n * (size_t)vpr * sizeof(V)));
     UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
   }
+  const uint8_t keep_waves = keep_waves_for(n, (size_t)vpr * sizeof(V), done.tag ? kThrough : nt ? kStreaming : kOrdinary,
+                                            over_link(counts, group, max_blocks));
 #define UGK_GO(STORE)                                                                                                  \
-  hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,            \
+  hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,     \
                      reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,   \
-                     group, many_groups, n, status, host_mirror, Ending<STORE>(done))
+                     group, many_groups, keep_waves, n, status, host_mirror, Ending<STORE>(done))
   if constexpr (Idx::kDense) {
     if (done.tag) {
       UGK_GO(kThrough);
@@ -611,7 +682,9 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
   const unsigned grid = request.grid(gather_grid((n + per_block - 1) / per_block, max_blocks));
 #define UGK_GO(STORE, DONE)                                                                                            \
   hipLaunchKernelGGL((gather_flat_kernel<STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,     \
-                     src_rows, (char *)out, out_rows, f, counts, group, n, status, host_mirror, Ending<STORE>(DONE))
+                     src_rows, (char *)out, out_rows, f, counts, group,                     \
+                     keep_waves_for(n, row_bytes, STORE, over_link(counts, group, max_blocks)), n, status, host_mirror, \
+                     Ending<STORE>(DONE))
   if constexpr (Idx::kDense) {
     const DoneWords done = request.take(grid, Telling::kSooner);
     if (done.tag) {
@@ -636,9 +709,10 @@ int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t 
   const bool nt = !request.counted() && nt_store_for(n * row_bytes);
   const DoneWords done = nt ? DoneWords{} : request.take(grid, Telling::kSooner);
   UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
+  const uint8_t keep_waves = keep_waves_for(n, row_bytes, nt ? kStreaming : kOrdinary, over_link(nullptr, 0, max_blocks));
 #define UGK_GO(STORE, SHARE)                                                                                          \
   hipLaunchKernelGGL((gather_stream_kernel<STORE, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,             \
-                     (const char *)src, src_rows, (char *)out, f, status, host_mirror, Ending<STORE>(done))
+                     (const char *)src, src_rows, (char *)out, f, status, host_mirror, Ending<STORE>(done), keep_waves)
   const bool share = row_bytes % 16 != 0;
   if (done.tag && share) UGK_GO(kThrough, true);
   else if (done.tag) UGK_GO(kThrough, false);

@@ -39,12 +39,14 @@ __device__ __forceinline__ void store_through(uint64_t to, V v) {
 // 1,024 19.3 / 15.6; lookup and gather in one kernel, 512 bytes x 4,096 13.9 / 13.3, 1 KB x 4,096 15.9 / 14.7, 2 KB x 512 17.1 /
 // 14.3, 4 KB x 2,048 25.5 / 18.7; that kernel with ordinary stores and a ticket behind it 15.3 / 15.1, 16.1 / 15.6, 16.3 / 14.9,
 // 22.8 / 19.8.  (Ordinary stores of the flat and the stream copy of a plain gather: 1 to 5 % either way, left as they were.)
+template <typename V>
+__device__ __forceinline__ void arrived(V &v) {
+  if constexpr (sizeof(V) >= 4) asm volatile("" : "+v"(v));
+}
 template <typename V, int N>
 __device__ __forceinline__ void arrived(V (&v)[N]) {
-  if constexpr (sizeof(V) >= 4) {
 #pragma unroll
-    for (int u = 0; u < N; ++u) asm volatile("" : "+v"(v[u]));
-  }
+  for (int u = 0; u < N; ++u) arrived(v[u]);
 }
 
 // how a kernel stores its rows: a template parameter, not a launch argument, for with a run-time choice the optimiser merges
@@ -167,7 +169,7 @@ static inline FlatRow flat_row(size_t row_bytes, uint32_t tile) {
 // Copies the rows r0 .. r0 + count - 1 of the wavefront, count <= f.tile: lane r holds where row r is read (kNoRowBit:
 // not at all) and, with DENSE false, which output row it becomes; with DENSE row r becomes output row d0 + r.  All
 // lanes call it with the same r0 and count.
-template <bool DENSE, bool THROUGH, bool WAIT = THROUGH>
+template <bool DENSE, bool THROUGH, bool KEEP, bool WAIT = THROUGH>
 __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, char *out, size_t d0, uint32_t r0,
                                           uint32_t count, const FlatRow &f) {
   constexpr int U = 4;  // vectors in flight per lane
@@ -192,7 +194,10 @@ __device__ __forceinline__ void flat_copy(uint64_t src_bits, uint32_t dst_row, c
     }
     u32x4 v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(p[u]);
+    for (int u = 0; u < U; ++u) {
+      if constexpr (KEEP) v[u] = *p[u];
+      else v[u] = __builtin_nontemporal_load(p[u]);
+    }
     if constexpr (WAIT) arrived(v);
 #pragma unroll
     for (int u = 0; u < U; ++u)

@@ -266,7 +266,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       const uint64_t bits = row.has_row ? row.bits : row.bits | kNoRowBit;
       const uint32_t here = (uint32_t)min((size_t)KPW, n - b0);
       for (uint32_t r0 = 0; r0 < here; r0 += f_row.tile)
-        flat_copy<true, STORE == kThrough, true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
+        flat_copy<true, STORE == kThrough, false, true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
     } else {
       const uint32_t vpr = f_row.chunks;
       uint64_t stage_bits = 0;
