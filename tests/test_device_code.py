@@ -88,3 +88,21 @@ def test_a_gather_nobody_polls_for_has_its_arguments_in_two_lines(gather_kernels
     plain = {k: at for k, at in gather_kernels.items() if "Direct" in k and "StoreE2E" not in k and at is not None}
     assert len(plain) > 20
     assert max(plain.values()) < 128, max(plain, key=plain.get)
+
+
+@pytest.mark.parametrize("source,kernel,words", [("ugk_partition.hip", "dedup_resolve_kernel", 1),
+                                                 ("ugk_refresh.hip", "rank_combine_observed_kernel", 2)])
+def test_a_word_for_the_host_is_there_before_its_launch_has_ended(source, kernel, words):
+    """the host reads them once a launch behind this one tells it that all is done; what is acknowledged is in host memory only if
+    it was stored at system scope, as tell_host does (before optimisation: two seconds where the kernels take a minute)"""
+    cmd = [build.hipcc_path()] + build.HIPCC_FLAGS + ["--cuda-device-only", "-S", "-emit-llvm", "-Xclang", "-disable-llvm-passes",
+                                                      "-I", build.INCLUDE, "-I", build.CSRC, os.path.join(build.CSRC, source), "-o", "-"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
+    assert proc.returncode == 0, proc.stderr[-3000:]
+
+    def body(name):
+        return re.search(r"\ndefine [^\n]*%s.*?\n}" % name, proc.stdout, re.S).group(0)
+
+    assert len(re.findall(r"call void @\w*tell_host", body(kernel))) >= words
+    assert re.search(r"store atomic i32 [^\n]* monotonic", body(r"\w*tell_hostIj"))
+    assert "syncscope" not in body(r"\w*tell_hostIj")

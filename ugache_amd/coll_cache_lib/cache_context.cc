@@ -1234,6 +1234,8 @@ size_t ExtractSession::ExtractUniqueCounted(const KeyT *nodes, size_t num_nodes,
   }
   _done.count_dev = nullptr;
   WaitForBatch(stream);
+  // (written by a launch in front of the one that was waited for: there already, or all but)
+  UGK_CALL(ugk_word_wait(_host_mirror + kMirNumUnique, 0, RunConfig::spin_wait_us, stream));
   const double host_time = t_host.Passed();
   CheckStatusWord(stream);
   const size_t nu = DedupFound(num_nodes);

@@ -422,7 +422,9 @@ __global__ __launch_bounds__(kBlock) void dedup_resolve_kernel(size_t n, const u
                                                                uint32_t *n_unique_host, uint32_t *next_n_unique) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (next_n_unique) *next_n_unique = 0;
-    if (n_unique_host) *n_unique_host = *n_unique;
+    // (there before this launch has ended: the host may learn of that from the words of a launch behind this one, which an
+    // ordinary store, acknowledged before it is in host memory, can be overtaken by)
+    if (n_unique_host) tell_host(n_unique_host, *n_unique);
   }
   for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock)
     inverse[i] = uid_of[inverse[i]];

@@ -650,8 +650,9 @@ __global__ __launch_bounds__(kBlock) void rank_combine_observed_kernel(uint32_t 
 #pragma unroll
   for (int w = 0; w < kBlock / kWave; ++w) out_wg += leaving_of[w], in_wg += coming_of[w];
   if (!arrive(&ws->arrivals, out_wg, in_wg)) return;
-  totals_host[0] = out_wg;
-  totals_host[1] = in_wg;
+  // (there before this launch has ended: where a scan behind it leaves the ticket, an ordinary store could be overtaken by that)
+  tell_host(totals_host, out_wg);
+  tell_host(totals_host + 1, in_wg);
   if (ticket) {
     __threadfence_system();
     *(volatile uint32_t *)(totals_host + 3) = ticket;
