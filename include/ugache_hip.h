@@ -458,7 +458,7 @@ int ugk_gather_scatter_staged_u32(const void *host_dev, uint64_t host_rows, cons
  * shares the workspace); epoch must be non-zero and different on every such call.  n_unique_dev must be zero on entry.
  * The outputs do not overlap keys_dev: keys are still read when the first of them are written.
  * rep_out_dev (may be NULL): rep_out_dev[u] = index of the first occurrence that introduced unique key u.
- * n_unique_host (may be NULL): pinned host word that receives *n_unique_dev when the second kernel runs. */
+ * n_unique_host (may be NULL): pinned host word that receives *n_unique_dev as the last of the call's kernels runs. */
 size_t ugk_dedup_workspace_bytes(size_t n);
 int ugk_dedup_u32(const uint32_t *keys_dev, size_t n, void *workspace_dev, size_t workspace_bytes, uint32_t epoch,
                   uint32_t *unique_out_dev, uint32_t *inverse_out_dev, uint32_t *rep_out_dev, uint32_t *n_unique_dev,

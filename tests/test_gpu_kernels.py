@@ -2011,6 +2011,35 @@ def test_dedup_of_small_and_large_batches_sharing_one_workspace(kdtype):
                  ptr(dev_zeros_u32(n)), None, ptr(dev_zeros_u32(1)), None, None)
 
 
+# the sizes between which the keys per lane of the one workgroup change, and the first that it does not hold
+@pytest.mark.parametrize("kdtype", [np.uint32, np.int64])
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097])
+@pytest.mark.parametrize("distinct", [1, 3, 40, 1 << 31])
+def test_dedup_of_a_batch_that_one_workgroup_holds(kdtype, n, distinct):
+    """few distinct keys, many lanes after the same slots; all keys distinct, the set as full as it gets"""
+    rng = np.random.default_rng(n + distinct % 1000)
+    keys = (rng.integers(0, distinct, size=n) * 2654435761 if distinct < n else rng.choice(1 << 31, size=n, replace=False)).astype(kdtype)
+    ws_bytes = hip.lib().ugk_dedup_workspace_bytes(n)
+    ws, d_keys, found = dev_bytes(ws_bytes, fill=0), to_dev(keys), PinnedArray((1,), np.uint32)
+    try:
+        for rep in (dev_zeros_u32(n), None):
+            uniq, inv, counts = dev_bytes(n * 8, fill=0x5A), dev_zeros_u32(n), to_dev(np.array([0, 9], np.uint32))
+            hip.call("ugk_dedup_rotating", ptr(d_keys), keys.itemsize, n, ptr(ws), ws_bytes, 1 if rep is None else 2, ptr(uniq), ptr(inv),
+                     ptr(rep), ptr(counts), ptr(counts) + 4, found.ptr, None)
+            sync()
+            k, spare = to_np(counts, np.uint32)[:2]
+            u, i = to_np(uniq, kdtype), to_np(inv, np.uint32)[:n]
+            assert k == found.array[0] == len(np.unique(keys)) and spare == 0
+            assert len(np.unique(u[:k])) == k and i.max() < k and np.array_equal(u[i], keys)
+            assert (u[k:].view(np.uint8) == 0x5A).all()
+            if rep is not None:
+                r = to_np(rep, np.uint32)[:k]
+                assert np.array_equal(keys[r], u[:k]) and np.array_equal(i[r], np.arange(k))
+    finally:
+        sync()
+        found.free()
+
+
 @pytest.mark.parametrize("kdtype", [np.uint32, np.int64])
 def test_dedup_with_two_count_words_in_turn(kdtype):
     """each call finds its word at zero and leaves the other so; the number of distinct keys can be polled for, and what is

@@ -665,7 +665,7 @@ size_t ExtractSession::DrainHotness(FreqRecorder *recorder) {
 // Deduplication in front of the extraction: the distinct keys of the batch, the index of the first occurrence of
 // each (where its row is gathered to) and, per input position, which distinct key it is.  One blocking wait: the
 // host needs the number of distinct keys to size the launches that follow.
-// (DedupLaunch: without the wait; returns the device word that the number is in from the second kernel on)
+// (DedupLaunch: without the wait; returns the device word that the number is in for what is launched behind it)
 template <typename KeyT>
 const uint32_t *ExtractSession::DedupLaunch(const KeyT *nodes, size_t num_nodes, uint32_t *inverse, StreamHandle stream) {
   const size_t ws_bytes = ugk_dedup_workspace_bytes(num_nodes);
@@ -709,7 +709,7 @@ size_t ExtractSession::DedupFound(size_t num_nodes) const {
 template <typename KeyT>
 size_t ExtractSession::DedupKeys(const KeyT *nodes, size_t num_nodes, uint32_t *inverse, StreamHandle stream) {
   DedupLaunch(nodes, num_nodes, inverse, stream);
-  // the number is there as the second of the two kernels starts, which what is launched next stands behind
+  // the number is there before the last of the kernels has ended, which what is launched next stands behind
   if (RunConfig::spin_wait_us == 0) UGK_CALL(ugk_stream_sync(stream));
   else UGK_CALL(ugk_word_wait(_host_mirror + kMirNumUnique, 0, RunConfig::spin_wait_us, stream));
   return DedupFound(num_nodes);
