@@ -1093,6 +1093,39 @@ def test_extract_mix_at_every_launch_shape(kind, rb):
         mirror.free()
 
 
+# batches whose wavefronts have eight rows per lane on their way, and the first behind a flat table that have four; rows of one
+# vector per lane and of more, a last wavefront with one key and with all
+@pytest.mark.parametrize("kind,n", [("flat", 9), ("flat", 4_096), ("flat", 4_097), ("hash32", 8), ("hash32", 8_192), ("hash32", 8_193),
+                                    ("hash", 16_400)])
+@pytest.mark.parametrize("rb", [512, 1024, 1040, 4096])
+def test_extract_mix_with_eight_rows_on_their_way(kind, n, rb):
+    rng = np.random.default_rng(rb + n)
+    nkeys = 6_000
+    host = _rand_table(rng, nkeys, rb)
+    cached = rng.choice(nkeys, nkeys * 3 // 4, replace=False).astype(np.int64)
+    mem, tb = {"flat": lambda: _make_flat(nkeys), "hash": lambda: _make_hash(len(cached))[:2],
+               "hash32": lambda: _make_hash32(len(cached))[:2]}[kind]()
+    assert _insert(tb, cached) == 0
+    pin, mirror = pinned_from(host), pinned_from(np.zeros(4, np.uint32))
+    try:
+        st, d_cache = dev_zeros_u32(1), to_dev(host[cached].copy())
+        keys = rng.integers(0, nkeys, size=n).astype(np.int64)
+        bad = np.arange(n) % 509 == 7
+        d_keys, out = to_dev(np.where(bad, nkeys + 5, keys)), dev_bytes(n * rb, fill=0x3C)
+        sizes = _extract_mix("ugk_extract_mix_i64", tb, d_keys, n, d_cache, len(cached), pin, nkeys, out, rb, st, mirror,
+                             hip.HINT_UNKNOWN)
+        assert status_value(st) == hip.ST_KEY_OUT_OF_RANGE
+        n_local = int(np.isin(keys[~bad], cached).sum())
+        assert sizes == [n_local, n - n_local]
+        want = host[keys]
+        want[bad] = 0x3C
+        assert to_np(out)[: n * rb].tobytes() == want.tobytes()
+    finally:
+        sync()
+        pin.free()
+        mirror.free()
+
+
 def _pool_reference(table_f64, ids, seg_off, weights, combiner):
     """embedding_lookup_sparse in float64: weighted sum of every segment's rows, divided by the sum of the weights
     (mean) or the root of the sum of their squares (sqrtn); a zero denominator and an empty segment give a zero row"""

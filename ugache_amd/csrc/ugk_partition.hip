@@ -161,12 +161,12 @@ __global__ __launch_bounds__(kBlock) void select_keys_kernel(const K *__restrict
 // against 48.5 us).  With eight short wavefronts per SIMD the chip already overlaps one wavefront's table round trip
 // with the others' row copies, and wavefronts that stride over the batch give up the moving window of output rows
 // that workgroups started in order write.
-// the rows of one wavefront's KPW keys, lane l holding the address of key b0 + l's row
+// the rows of one wavefront's KPW keys, lane l holding the address of key b0 + l's row, ROWS of them on their way per lane
 // stage_bits (STAGE only): where the lane's row is filed as well, 0 for a row that is not
-template <int LPR, int KPW, Store STORE, bool STAGE>
+template <int LPR, int KPW, int ROWS, Store STORE, bool STAGE>
 __device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits, u32x4 *out, size_t b0, uint32_t vpr) {
   constexpr int RPW = kWave / LPR;  // rows per wavefront instruction
-  constexpr int UNROLL = (RPW * 4 <= KPW) ? 4 : (KPW / RPW);
+  constexpr int UNROLL = RPW * ROWS <= KPW ? ROWS : KPW / RPW;
   static_assert(KPW <= kWave && KPW % (RPW * UNROLL) == 0, "keys per wavefront must be whole rounds of rows");
   const int lane = (int)lane_id();
   const int sub = lane % LPR, rg = lane / LPR;
@@ -228,8 +228,16 @@ __device__ __forceinline__ uint64_t stage_claim(const ugk_stage_t &stage, const 
   return reinterpret_cast<uint64_t>(reinterpret_cast<u32x4 *>(stage.rows_dev) + h * vpr);
 }
 
+// Rows of 512 bytes and more of a wavefront with few keys: eight per lane on their way, half the rounds to memory of four.  us,
+// launch to end of poll, four / eight, a hash table, all rows in HBM and a twentieth over the link: 1 KB x 512 13.1 / 12.5 and
+// 14.8 / 14.1, x 16,384 19.5 / 18.3 and 29.2 / 28.9; 4 KB x 16 14.5 / 12.9 and 16.6 / 14.5, x 1,024 18.3 / 17.0 and 23.2 / 21.1; 512
+// bytes x 16,384 16.6 / 15.5 and 21.3 / 21.1.  Behind a flat table, which is soon looked up in, a launch that fills the chip has
+// enough of them on their way: 1 KB x 2,048 11.9 / 11.6 and 13.3 / 12.7, x 8,192 13.3 / 13.6 and 18.1 / 18.5; 4 KB x 1,024 16.3 / 15.3
+// and 21.4 / 19.1, x 4,096 18.6 / 17.7 and 26.1 / 26.5, x 16,384 31.7 / 34.2.
+constexpr int mix_rows(int lpr, int kpw) { return lpr >= 32 && kpw <= 16 && kWave / lpr * 8 <= kpw ? 8 : 4; }
+
 // LPR: lanes per row, or 0 for rows that are copied flat (flat_copy; f.tile rows at a time)
-template <typename K, int KIND, int LPR, int KPW, Store STORE, bool STAGE>
+template <typename K, int KIND, int LPR, int KPW, int ROWS, Store STORE, bool STAGE>
 __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, const K *__restrict__ keys, size_t n,
                                                              const void *__restrict__ cache, uint64_t cache_rows,
                                                              const void *__restrict__ host, uint64_t host_rows,
@@ -271,7 +279,7 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       const uint32_t vpr = f_row.chunks;
       uint64_t stage_bits = 0;
       if constexpr (STAGE) stage_bits = stage_claim(stage, row, vpr);
-      mix_copy<LPR, KPW, STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
+      mix_copy<LPR, KPW, ROWS, STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
     }
     // behind the rows: in front of them it would be in the way of the lookup
     if constexpr (STORE == kThrough) {
@@ -672,25 +680,35 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;
   const ugk_stage_t no_stage{};
-#define UGK_GO4(L, W, NT, ST)                                                                                       \
-  hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, NT, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
+#define UGK_GO4(L, W, R, NT, ST)                                                                                    \
+  hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, R, NT, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
                      cache, cache_rows, host, host_rows, out, f_row, status, host_mirror, Ending<NT>(done),        \
                      ST ? *stage : no_stage)
-#define UGK_GO3(L, W, NT)               \
-  do {                                  \
-    if (stage) UGK_GO4(L, W, NT, true); \
-    else UGK_GO4(L, W, NT, false);      \
+#define UGK_GO3(L, W, R, NT)               \
+  do {                                     \
+    if (stage) UGK_GO4(L, W, R, NT, true); \
+    else UGK_GO4(L, W, R, NT, false);      \
   } while (0)
-#define UGK_GO2(L, W)                          \
-  do {                                         \
-    if (done.tag) UGK_GO3(L, W, kThrough);     \
-    else if (nt) UGK_GO3(L, W, kStreaming);    \
-    else UGK_GO3(L, W, kOrdinary);             \
+#define UGK_ROWS(L, W, R)                         \
+  do {                                            \
+    if (done.tag) UGK_GO3(L, W, R, kThrough);     \
+    else if (nt) UGK_GO3(L, W, R, kStreaming);    \
+    else UGK_GO3(L, W, R, kOrdinary);             \
   } while (0)
-#define UGK_FLAT(W)                                   \
-  do {                                                \
-    if (done.tag) UGK_GO4(0, W, kThrough, false);     \
-    else UGK_GO4(0, W, kOrdinary, false);             \
+#define UGK_GO2(L, W)                                             \
+  do {                                                            \
+    if constexpr (KIND == 1 && mix_rows(L, W) == 8) {             \
+      if (n > 4096) {                                             \
+        UGK_ROWS(L, W, 4);                                        \
+        break;                                                    \
+      }                                                           \
+    }                                                             \
+    UGK_ROWS(L, W, mix_rows(L, W));                               \
+  } while (0)
+#define UGK_FLAT(W)                                      \
+  do {                                                   \
+    if (done.tag) UGK_GO4(0, W, 4, kThrough, false);     \
+    else UGK_GO4(0, W, 4, kOrdinary, false);             \
   } while (0)
 #define UGK_GO(L)                                   \
   do {                                              \
@@ -728,6 +746,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   else UGK_GO(64);
 #undef UGK_GO
 #undef UGK_GO2
+#undef UGK_ROWS
 #undef UGK_GO3
 #undef UGK_GO4
 #undef UGK_FLAT
