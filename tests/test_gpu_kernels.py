@@ -168,6 +168,31 @@ def test_gather_of_more_than_one_round_of_workgroups(row_bytes, n, hint):
     _gather_with_keys_that_miss(row_bytes, n, hint)
 
 
+# polled launches on both sides of the lines between those whose wavefronts all load past the caches and those of which none does
+@pytest.mark.parametrize("row_bytes,n", [(16, 180_224), (16, 180_225), (20, 9_001), (20, 300_001), (44, 1_300_000), (64, 262_144),
+                                         (64, 262_145), (200, 52_428), (200, 52_429), (512, 32_768), (512, 32_769), (800, 13_107),
+                                         (800, 13_108), (1204, 8_709), (1204, 8_710), (4096, 2_560), (4096, 4_097)])
+def test_polled_gather_on_both_sides_of_what_the_caches_hold(row_bytes, n):
+    gen = torch.Generator(device="cuda").manual_seed(row_bytes + n)
+    rows, words, done = 5_003, row_bytes // 4, _DoneWords()
+    table = torch.randint(-(1 << 31), 1 << 31, (rows, words), dtype=torch.int32, device="cuda", generator=gen)
+    keys = torch.randint(0, rows, (n,), device="cuda", generator=gen)
+    bad = torch.rand(n, device="cuda", generator=gen) < 0.01
+    q = torch.where(bad, rows, keys)
+    out, st = torch.full((n, words), 0x7E7E7E7E, dtype=torch.int32, device="cuda"), dev_zeros_u32(1)
+    sync()
+    done.ask(1_000)
+    hip.call("ugk_gather_direct_i64", ptr(table), rows, ptr(q), n, ptr(out), row_bytes, 0, ptr(st), done.mirror.ptr, None)
+    assert done.done.num_words > 0
+    hip.call("ugk_done_wait", C.byref(done.done), 1_000_000, None, None, None)
+    done.check_flag(hip.ST_KEY_OUT_OF_RANGE)
+    done.check_counters()
+    done.check_keys(to_np(q))
+    want = table[keys]
+    want[bad] = 0x7E7E7E7E
+    assert torch.equal(out, want)
+
+
 # both sides of the lines between launches of which all wavefronts, one of four and none load past the caches: short rows of
 # whole vectors whose lines the L2s just hold, rows of 48 bytes, output and kept lines of 256 MiB
 @pytest.mark.parametrize("row_bytes,n", [(16, 180_224), (16, 180_225), (32, 458_752), (32, 458_753), (20, 300_001), (44, 9_001),

@@ -76,6 +76,13 @@ struct IdxList {
   }
 };
 
+// which wavefronts load rows the ordinary way (keep_waves_for): a launch argument says, or, for a launch that is polled for and is over
+// sooner without the code of both, all of them or none
+enum Loads { kByWave, kPast, kKept };
+template <Loads LOADS>
+__device__ __forceinline__ bool keeps(uint32_t keep_waves) {
+  return LOADS == kKept || (LOADS == kByWave && wave_in_block() < keep_waves);
+}
 template <bool KEEP, typename V>
 __device__ __forceinline__ V ld_row(const V *p) {
   if constexpr (KEEP) return *p;
@@ -96,7 +103,7 @@ __device__ __forceinline__ void st_stream(V *p, V v) {
 // 7,812 with skewed keys and 8 KB x 7,812, about half of one round, lose: 7.1 / 7.5 and 24.4 / 25.8.)  Rows in flight per lane, one / two / four /
 // eight, all without: 512 bytes x 65,536 15.9 / 14.7 / 15.1 / 15.5, x 524,288 91.1 / 82.4 / 82.5 / 83.5; 4 KB x 32,768 43.4 /
 // 43.4 / 51.9 / 48.4; 16 bytes x 32,768 3.8 / 4.5 / 5.8 / 9.0.
-template <typename V, int LPR, int UNROLL, Store STORE, typename Idx>
+template <typename V, int LPR, int UNROLL, Store STORE, Loads LOADS, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restrict__ src, uint64_t src_rows,
                                                         V *__restrict__ out, uint64_t out_rows, uint32_t vpr,
                                                         const uint32_t *__restrict__ counts, uint32_t group,
@@ -162,8 +169,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
         }
       }
     };
-    // (written through, only short rows gain, see keep_waves_for: no code for the others)
-    if ((STORE != kThrough || sizeof(V) * LPR < 64) && wave_in_block() < keep_waves) {
+    if (keeps<LOADS>(keep_waves)) {
       if (no_branch) copy(std::true_type{}, std::false_type{});
       else copy(std::true_type{}, std::true_type{});
     } else {
@@ -181,7 +187,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Idx ix, const V *__restr
 
 // The same for rows the lanes of gather_kernel do not fit (see flat_copy): a wavefront takes f.tile rows, one index
 // word per lane, and copies their vectors numbered through.
-template <Store STORE, typename Idx>
+template <Store STORE, Loads LOADS, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                              char *__restrict__ out, uint64_t out_rows, FlatRow f,
                                                              const uint32_t *__restrict__ counts, uint32_t group,
@@ -212,7 +218,7 @@ __global__ __launch_bounds__(kBlock) void gather_flat_kernel(Idx ix, const char 
       const uint64_t at = reinterpret_cast<uint64_t>(src) + s * f.row_bytes;
       const uint64_t dummy = shfl64(at, __ffsll(good) - 1);
       const uint64_t bits = ok ? at : dummy | kNoRowBit;
-      if (wave_in_block() < keep_waves)
+      if (keeps<LOADS>(keep_waves))
         flat_copy<Idx::kDense, STORE == kThrough, true>(bits, (uint32_t)d, out, base, 0, rows, f);
       else
         flat_copy<Idx::kDense, STORE == kThrough, false>(bits, (uint32_t)d, out, base, 0, rows, f);
@@ -243,7 +249,7 @@ StreamRow stream_row(size_t row_bytes, size_t n) {
                    (uint64_t)n * row_bytes};
 }
 
-template <Store STORE, bool SHARE, typename Idx>
+template <Store STORE, Loads LOADS, bool SHARE, typename Idx>
 __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const char *__restrict__ src, uint64_t src_rows,
                                                                char *__restrict__ out, StreamRow f, uint32_t *status,
                                                                uint32_t *host_mirror, Ending<STORE> done,
@@ -347,7 +353,7 @@ __global__ __launch_bounds__(kBlock) void gather_stream_kernel(Idx ix, const cha
           else put(q, v[u]);
         }
     };
-    if (STORE != kThrough && wave_in_block() < keep_waves) {
+    if (keeps<LOADS>(keep_waves)) {
       // (for the compiler alone, which makes one of two loads that differ in the hint, and that without it)
       asm volatile("" ::: "memory");
       part(std::true_type{});
@@ -516,10 +522,14 @@ bool over_link(const uint32_t *counts, uint32_t group, unsigned max_blocks) {
 //     Except that lines that come to about what the L2s hold, 32 MB, push the output out of there, the more the longer the
 //     rows: 262,144 rows of 32 bytes 8.7 / 9.1 / 9.7, of 16 bytes 8.0 / 8.5 / 8.6, of 20 bytes (flat) 9.0 / 9.0 / 9.5, of
 //     12 bytes 8.4 / 8.4 / 8.3, where 131,072 and 524,288 of them lose nothing.
-//   * Stores that are written through keep no room in the L2s, and of the rows of 48 bytes and more those come no sooner: none
-//     (512 bytes x 131,072, launch to end of poll, none / one, uniform and zipf 1.05: 30.4 / 29.6 and 27.4 / 27.8; 1204 bytes x 870
-//     10.8 / 11.1, the code for both.  16 bytes x 1,048,576 34.6 / 32.5 and 25.9 / 21.8 with all four; 36 bytes
-//     x 466,033 25.4 / 24.7 and 21.2 / 19.4, x 5,688,888 194 / 201 and 131 / 123.)
+//   * Stores that are written through need no room in the L2s, and what one wavefront of four keeps there the others, reading past
+//     it, drop again: all four or none.  us, launch to end of poll, none / one / two / all, uniform and zipf 1.05 and 1.2, 512 bytes:
+//     2 MB 10.8 / 11.0 / 10.9 / 10.5 and 10.8 / 10.7 / 10.9 / 10.4 and 10.7 / 10.7 / 10.7 / 10.5; 8 MB 13.2 / 13.0 / 12.9 / 13.1 and
+//     12.4 / 12.5 / 12.4 / 11.4 and 12.5 / 12.4 / 12.4 / 11.3; 16 MB 15.7 / 15.6 / 15.4 / 15.6 and 15.1 / 15.0 / 14.8 / 13.5 and 14.9 /
+//     14.8 / 14.7 / 13.2; 32 MB 20.7 / 20.6 / 20.5 / 21.2 and 19.3 / 19.4 / 19.4 / 17.1.  All up to 16 MB, and none beyond, for what it
+//     costs uniform keys there; up to 10 MB for rows that begin inside a line (200 bytes, 12 MB, none / all 16.4 / 16.8 and, zipf
+//     1.2, 15.5 / 12.6).  Short rows: 16 bytes x 1,048,576 34.6 / 32.5 and, zipf 1.05, 25.9 / 21.8; 36 bytes x 466,033 25.4 / 24.7 and
+//     21.2 / 19.4, but x 5,688,888 194 / 201 and 131 / 123.
 //   * Rows over a link: none, as nothing that the chip's caches do shows beside the link (that of an uncapped gather out of
 //     host memory, which cannot be told from one out of HBM here: 16 to 1204 bytes x 0.25 to 8 MB 0.98 to 1.2 times as fast).
 constexpr size_t kMemorySideCache = 256ull << 20;
@@ -531,12 +541,14 @@ uint8_t keep_waves_for(size_t n, size_t row_bytes, Store store, bool over_link) 
                        : row_bytes % kLine == 0    ? row_bytes
                        : row_bytes % 16 == 0       ? row_bytes + kLine - 16
                                                    : row_bytes + kLine - 4;
-  if (row_bytes < 48) {
-    if (store == kThrough && row_bytes > 32 && n * (row_bytes + lines) > kMemorySideCache) return 0;
-    const bool as_l2 = n > (22ull << 20) / kLine && n <= (56ull << 20) / kLine;
-    return !as_l2 || row_bytes < 16 ? kWavesPerBlock : row_bytes % 16 == 0 ? 0 : 1;
+  const bool as_l2 = n > (22ull << 20) / kLine && n <= (56ull << 20) / kLine;
+  if (store == kThrough) {
+    const bool all = row_bytes >= 48  ? n * row_bytes <= (size_t)(row_bytes % 64 == 0 ? 16 : 10) << 20
+                     : row_bytes > 32 ? n * (row_bytes + lines) <= kMemorySideCache
+                                      : !as_l2 || row_bytes < 16;
+    return all ? kWavesPerBlock : 0;
   }
-  if (store == kThrough) return 0;
+  if (row_bytes < 48) return !as_l2 || row_bytes < 16 ? kWavesPerBlock : row_bytes % 16 == 0 ? 0 : 1;
   return store == kStreaming || n * (row_bytes + lines / kWavesPerBlock) <= kMemorySideCache ? 1 : 0;
 }
 
@@ -570,19 +582,20 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
   }
   const uint8_t keep_waves = keep_waves_for(n, (size_t)vpr * sizeof(V), done.tag ? kThrough : nt ? kStreaming : kOrdinary,
                                             over_link(counts, group, max_blocks));
-#define UGK_GO(STORE)                                                                                                  \
-  hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,     \
+#define UGK_GO(STORE, LOADS)                                                                                           \
+  hipLaunchKernelGGL((gather_kernel<V, LPR, UNROLL, STORE, LOADS, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,     \
                      reinterpret_cast<const V *>(src), src_rows, reinterpret_cast<V *>(out), out_rows, vpr, counts,   \
                      group, many_groups, keep_waves, n, status, host_mirror, Ending<STORE>(done))
   if constexpr (Idx::kDense) {
     if (done.tag) {
-      UGK_GO(kThrough);
+      if (keep_waves) UGK_GO(kThrough, kKept);
+      else UGK_GO(kThrough, kPast);
       UGK_HIP(hipGetLastError());
       return 0;
     }
   }
-  if (nt) UGK_GO(kStreaming);
-  else UGK_GO(kOrdinary);
+  if (nt) UGK_GO(kStreaming, kByWave);
+  else UGK_GO(kOrdinary, kByWave);
 #undef UGK_GO
   UGK_HIP(hipGetLastError());
   return 0;
@@ -680,21 +693,22 @@ int launch_flat(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t 
   const FlatRow f = flat_row(row_bytes, flat_tile(row_bytes, n));
   const size_t per_block = (size_t)f.tile * kWavesPerBlock;
   const unsigned grid = request.grid(gather_grid((n + per_block - 1) / per_block, max_blocks));
-#define UGK_GO(STORE, DONE)                                                                                            \
-  hipLaunchKernelGGL((gather_flat_kernel<STORE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix, (const char *)src,     \
-                     src_rows, (char *)out, out_rows, f, counts, group,                     \
-                     keep_waves_for(n, row_bytes, STORE, over_link(counts, group, max_blocks)), n, status, host_mirror, \
+  const bool far = over_link(counts, group, max_blocks);
+#define UGK_GO(STORE, LOADS, KEEP, DONE)                                                                               \
+  hipLaunchKernelGGL((gather_flat_kernel<STORE, LOADS, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,                 \
+                     (const char *)src, src_rows, (char *)out, out_rows, f, counts, group, KEEP, n, status, host_mirror, \
                      Ending<STORE>(DONE))
   if constexpr (Idx::kDense) {
     const DoneWords done = request.take(grid, Telling::kSooner);
     if (done.tag) {
-      UGK_GO(kThrough, done);
+      if (keep_waves_for(n, row_bytes, kThrough, far)) UGK_GO(kThrough, kKept, kWavesPerBlock, done);
+      else UGK_GO(kThrough, kPast, 0, done);
       UGK_HIP(hipGetLastError());
       return 0;
     }
     UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
   }
-  UGK_GO(kOrdinary, DoneWords{});
+  UGK_GO(kOrdinary, kByWave, keep_waves_for(n, row_bytes, kOrdinary, far), DoneWords{});
 #undef UGK_GO
   UGK_HIP(hipGetLastError());
   return 0;
@@ -709,17 +723,22 @@ int launch_stream(Idx ix, const void *src, uint64_t src_rows, void *out, size_t 
   const bool nt = !request.counted() && nt_store_for(n * row_bytes);
   const DoneWords done = nt ? DoneWords{} : request.take(grid, Telling::kSooner);
   UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
-  const uint8_t keep_waves = keep_waves_for(n, row_bytes, nt ? kStreaming : kOrdinary, over_link(nullptr, 0, max_blocks));
-#define UGK_GO(STORE, SHARE)                                                                                          \
-  hipLaunchKernelGGL((gather_stream_kernel<STORE, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,             \
+  const uint8_t keep_waves = keep_waves_for(n, row_bytes, done.tag ? kThrough : nt ? kStreaming : kOrdinary,
+                                            over_link(nullptr, 0, max_blocks));
+#define UGK_GO2(STORE, LOADS, SHARE)                                                                                  \
+  hipLaunchKernelGGL((gather_stream_kernel<STORE, LOADS, SHARE, Idx>), dim3(grid), dim3(kBlock), 0, stream, ix,      \
                      (const char *)src, src_rows, (char *)out, f, status, host_mirror, Ending<STORE>(done), keep_waves)
+#define UGK_GO(STORE, LOADS)                  \
+  do {                                        \
+    if (share) UGK_GO2(STORE, LOADS, true);   \
+    else UGK_GO2(STORE, LOADS, false);        \
+  } while (0)
   const bool share = row_bytes % 16 != 0;
-  if (done.tag && share) UGK_GO(kThrough, true);
-  else if (done.tag) UGK_GO(kThrough, false);
-  else if (nt && share) UGK_GO(kStreaming, true);
-  else if (nt) UGK_GO(kStreaming, false);
-  else if (share) UGK_GO(kOrdinary, true);
-  else UGK_GO(kOrdinary, false);
+  if (done.tag && keep_waves) UGK_GO(kThrough, kKept);
+  else if (done.tag) UGK_GO(kThrough, kPast);
+  else if (nt) UGK_GO(kStreaming, kByWave);
+  else UGK_GO(kOrdinary, kByWave);
+#undef UGK_GO2
 #undef UGK_GO
   UGK_HIP(hipGetLastError());
   return 0;
