@@ -1151,6 +1151,40 @@ def test_extract_mix_with_eight_rows_on_their_way(kind, n, rb):
         mirror.free()
 
 
+# polled launches on both sides of the line beyond which long rows are loaded past the caches (64 MiB of output), and short rows,
+# which never are
+@pytest.mark.parametrize("kind", ["flat", "hash32"])
+@pytest.mark.parametrize("rb,n", [(64, 1_048_577), (128, 524_288), (128, 524_289), (1040, 64_527), (1040, 64_528), (36, 1_900_000),
+                                  (100, 671_088), (100, 671_089)])
+def test_polled_extract_mix_on_both_sides_of_what_the_caches_hold(kind, rb, n):
+    rng = np.random.default_rng(rb)
+    nkeys, done = 6_000, _DoneWords()
+    host = _rand_table(rng, nkeys, rb)
+    cached = rng.choice(nkeys, nkeys * 19 // 20, replace=False).astype(np.int64)
+    mem, tb = _make_flat(nkeys) if kind == "flat" else _make_hash32(len(cached))[:2]
+    assert _insert(tb, cached) == 0
+    pin, words, groups = pinned_from(host), PinnedArray((hip.lib().ugk_extract_mix_max_groups(),), np.uint64), C.c_uint32(0)
+    try:
+        st, d_cache, d_host = dev_zeros_u32(1), to_dev(host[cached].copy()), to_dev(host).view(nkeys, rb)
+        keys = torch.randint(0, nkeys, (n,), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n))
+        out = dev_bytes(n * rb, fill=0x3C)
+        done.ask(500)
+        hip.call("ugk_extract_mix_i64", tb, ptr(keys), n, ptr(d_cache), len(cached), pin.ptr, nkeys, ptr(out), rb, ptr(st),
+                 done.mirror.ptr, words.ptr, C.byref(groups), hip.HINT_UNKNOWN, None)
+        assert done.done.num_words > 0
+        local, others = C.c_uint64(), C.c_uint64()
+        hip.call("ugk_done_wait", C.byref(done.done), 1_000_000, None, C.byref(local), C.byref(others))
+        done.check_flag(0)
+        done.check_keys(to_np(keys))
+        n_local = int(torch.isin(keys, to_dev(cached)).sum())
+        assert (local.value, others.value) == (n_local, n - n_local)
+        assert torch.equal(out[: n * rb].view(n, rb), d_host[keys])
+    finally:
+        sync()
+        pin.free()
+        words.free()
+
+
 def _pool_reference(table_f64, ids, seg_off, weights, combiner):
     """embedding_lookup_sparse in float64: weighted sum of every segment's rows, divided by the sum of the weights
     (mean) or the root of the sum of their squares (sqrtn); a zero denominator and an empty segment give a zero row"""

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kBlock) void select_keys_kernel(const K *__restrict
 // that workgroups started in order write.
 // the rows of one wavefront's KPW keys, lane l holding the address of key b0 + l's row, ROWS of them on their way per lane
 // stage_bits (STAGE only): where the lane's row is filed as well, 0 for a row that is not
-template <int LPR, int KPW, int ROWS, Store STORE, bool STAGE>
+template <int LPR, int KPW, int ROWS, Store STORE, bool KEEP, bool STAGE>
 __device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits, u32x4 *out, size_t b0, uint32_t vpr) {
   constexpr int RPW = kWave / LPR;  // rows per wavefront instruction
   constexpr int UNROLL = RPW * ROWS <= KPW ? ROWS : KPW / RPW;
@@ -187,7 +187,10 @@ __device__ __forceinline__ void mix_copy(const MixRow &row, uint64_t stage_bits,
       if (col < vpr) {
         u32x4 v[UNROLL];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) v[u] = __builtin_nontemporal_load(p[u] + col);
+        for (int u = 0; u < UNROLL; ++u) {
+          if constexpr (KEEP) v[u] = p[u][col];
+          else v[u] = __builtin_nontemporal_load(p[u] + col);
+        }
         arrived(v);
         const gout_t dst = (gout_t)out + (b0 + r0 + rg) * vpr + col;
 #pragma unroll
@@ -236,8 +239,15 @@ __device__ __forceinline__ uint64_t stage_claim(const ugk_stage_t &stage, const 
 // and 21.4 / 19.1, x 4,096 18.6 / 17.7 and 26.1 / 26.5, x 16,384 31.7 / 34.2.
 constexpr int mix_rows(int lpr, int kpw) { return lpr >= 32 && kpw <= 16 && kWave / lpr * 8 <= kpw ? 8 : 4; }
 
+// KEEP: rows are loaded the ordinary way instead of past the caches, where the keys that repeat find them.  Stores that are written
+// through need no room there, and with them every launch gains or loses nothing whose output leaves the lines room in the
+// memory-side cache.  us, launch to end of poll, past / kept, a fiftieth of the rows over the link, uniform keys, zipf 0.8, 1.05 and
+// 1.2: 512 bytes x 4,096 14.8 / 14.7, 13.9 / 13.7, 13.4 / 13.2 and 13.4 / 13.3, x 32,768 21.0 / 20.9, 18.6 / 17.7, 17.7 / 16.7 and 17.4 /
+// 16.3, x 131,072 40.2 / 39.7, 31.7 / 31.8, 30.2 / 29.1 and 32.4 / 25.5; 100 bytes x 671,088 82.9 / 83.0, 55.1 / 52.6, 51.6 / 43.5 and
+// 50.0 / 39.9.  Beyond 64 MB rows of more than 64 bytes lose, 512 bytes x 262,144 47.3 / 51.4 with zipf 1.05, x 400,000 72 / 77 with
+// 0.8; shorter ones gain at any size (64 bytes x 4,000,000 271 / 270, 179 / 176, 169 / 162 and 160 / 152).
 // LPR: lanes per row, or 0 for rows that are copied flat (flat_copy; f.tile rows at a time)
-template <typename K, int KIND, int LPR, int KPW, int ROWS, Store STORE, bool STAGE>
+template <typename K, int KIND, int LPR, int KPW, int ROWS, Store STORE, bool KEEP, bool STAGE>
 __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, const K *__restrict__ keys, size_t n,
                                                              const void *__restrict__ cache, uint64_t cache_rows,
                                                              const void *__restrict__ host, uint64_t host_rows,
@@ -274,12 +284,12 @@ __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, cons
       const uint64_t bits = row.has_row ? row.bits : row.bits | kNoRowBit;
       const uint32_t here = (uint32_t)min((size_t)KPW, n - b0);
       for (uint32_t r0 = 0; r0 < here; r0 += f_row.tile)
-        flat_copy<true, STORE == kThrough, false, true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
+        flat_copy<true, STORE == kThrough, KEEP, true>(bits, 0, static_cast<char *>(out), b0, r0, min(f_row.tile, here - r0), f_row);
     } else {
       const uint32_t vpr = f_row.chunks;
       uint64_t stage_bits = 0;
       if constexpr (STAGE) stage_bits = stage_claim(stage, row, vpr);
-      mix_copy<LPR, KPW, ROWS, STORE, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
+      mix_copy<LPR, KPW, ROWS, STORE, KEEP, STAGE>(row, stage_bits, static_cast<u32x4 *>(out), b0, vpr);
     }
     // behind the rows: in front of them it would be in the way of the lookup
     if constexpr (STORE == kThrough) {
@@ -680,20 +690,27 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;
   const ugk_stage_t no_stage{};
-#define UGK_GO4(L, W, R, NT, ST)                                                                                    \
-  hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, R, NT, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
+  const bool keep = row_bytes <= 64 || out_bytes <= (size_t)64 << 20;
+#define UGK_GO4(L, W, R, NT, KEEP, ST)                                                                              \
+  hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, R, NT, KEEP, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
                      cache, cache_rows, host, host_rows, out, f_row, status, host_mirror, Ending<NT>(done),        \
                      ST ? *stage : no_stage)
-#define UGK_GO3(L, W, R, NT)               \
-  do {                                     \
-    if (stage) UGK_GO4(L, W, R, NT, true); \
-    else UGK_GO4(L, W, R, NT, false);      \
+#define UGK_GO3(L, W, R, NT, KEEP)               \
+  do {                                           \
+    if (stage) UGK_GO4(L, W, R, NT, KEEP, true); \
+    else UGK_GO4(L, W, R, NT, KEEP, false);      \
   } while (0)
-#define UGK_ROWS(L, W, R)                         \
-  do {                                            \
-    if (done.tag) UGK_GO3(L, W, R, kThrough);     \
-    else if (nt) UGK_GO3(L, W, R, kStreaming);    \
-    else UGK_GO3(L, W, R, kOrdinary);             \
+#define UGK_ROWS(L, W, R)                                \
+  do {                                                   \
+    if constexpr (L > 4) {                               \
+      if (done.tag && !keep) {                           \
+        UGK_GO3(L, W, R, kThrough, false);               \
+        break;                                           \
+      }                                                  \
+    }                                                    \
+    if (done.tag) UGK_GO3(L, W, R, kThrough, true);      \
+    else if (nt) UGK_GO3(L, W, R, kStreaming, false);    \
+    else UGK_GO3(L, W, R, kOrdinary, false);             \
   } while (0)
 #define UGK_GO2(L, W)                                             \
   do {                                                            \
@@ -705,10 +722,11 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
     }                                                             \
     UGK_ROWS(L, W, mix_rows(L, W));                               \
   } while (0)
-#define UGK_FLAT(W)                                      \
-  do {                                                   \
-    if (done.tag) UGK_GO4(0, W, 4, kThrough, false);     \
-    else UGK_GO4(0, W, 4, kOrdinary, false);             \
+#define UGK_FLAT(W)                                                \
+  do {                                                             \
+    if (done.tag && keep) UGK_GO4(0, W, 4, kThrough, true, false); \
+    else if (done.tag) UGK_GO4(0, W, 4, kThrough, false, false);   \
+    else UGK_GO4(0, W, 4, kOrdinary, false, false);                \
   } while (0)
 #define UGK_GO(L)                                   \
   do {                                              \
