@@ -34,6 +34,7 @@ extern "C" {
 #define UGK_ST_EVICT_ABSENT 0x8u     /* evict of a key that is not present */
 #define UGK_ST_BAD_SEGMENT 0x10u     /* pooled extraction: offsets that leave [0, nnz], run backwards or do not span [0, nnz] */
 #define UGK_ST_PLACE_PROMISE 0x20u   /* ugk_rank_place_observed: k or more rows were observed; nothing was placed */
+#define UGK_ST_SLOT_CLASH 0x40u      /* ugk_handed_check, ugk_table_insert_handed_*: a cache slot listed twice, or one not in use */
 
 /* element code of the pooled extraction for bfloat16 rows (fp32 and fp16 are named by their size, 4 and 2) */
 #define UGK_ELEM_BF16 0x102
@@ -103,7 +104,7 @@ typedef struct {
 const char *ugk_last_error(void);
 /* version of this ABI; bumped on any signature change.  ugk_abi_version() is what the loaded library was built with:
  * a caller compiled against another UGK_ABI_VERSION must not go on. */
-#define UGK_ABI_VERSION 26
+#define UGK_ABI_VERSION 27
 int ugk_abi_version(void);
 
 /* ---- runtime plumbing: Device::{AllocDataSpace,FreeDataSpace,CopyDataFromTo,StreamSync,CreateStream}
@@ -287,6 +288,24 @@ int ugk_table_evict_slots_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n,
                               void *stream);
 int ugk_table_evict_slots_i64(ugk_table_t t, const int64_t *keys_dev, size_t n, uint32_t *slots_out_dev, uint32_t *status_dev,
                               void *stream);
+/* Slots that keys which leave hand on to as many that come in.  ugk_table_evict_handed_*: ugk_table_evict_slots_*, and stamps (a word
+ * per slot, whatever they hold) say where in the list each slot is.  ugk_handed_check, and ugk_table_insert_handed_* in the launch that
+ * gives the listed slots to other keys: UGK_ST_SLOT_CLASH is set where one of the list is listed twice or not in use (its bit in
+ * used_bits, one per slot, is clear), UGK_ST_KEY_OUT_OF_RANGE where one is not below nslots.  The list is whole and in its order. */
+typedef struct {
+  uint32_t *stamps;
+  const uint64_t *used_bits;
+  uint64_t nslots;
+} ugk_handed_t;
+int ugk_table_evict_handed_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint32_t *slots_out_dev,
+                               const ugk_handed_t *handed, uint32_t *status_dev, void *stream);
+int ugk_table_evict_handed_i64(ugk_table_t t, const int64_t *keys_dev, size_t n, uint32_t *slots_out_dev,
+                               const ugk_handed_t *handed, uint32_t *status_dev, void *stream);
+int ugk_table_insert_handed_u32(ugk_table_t t, const uint32_t *keys_dev, const uint32_t *slots_dev, uint32_t loc, size_t n,
+                                const ugk_handed_t *handed, uint32_t *status_dev, void *stream);
+int ugk_table_insert_handed_i64(ugk_table_t t, const int64_t *keys_dev, const uint32_t *slots_dev, uint32_t loc, size_t n,
+                                const ugk_handed_t *handed, uint32_t *status_dev, void *stream);
+int ugk_handed_check(const ugk_handed_t *handed, const uint32_t *slots_dev, size_t n, uint32_t *status_dev, void *stream);
 /* LookupValCustom with SepLocOffset (cache_hashtable.cuh:420-434): loc_out/off_out per key; a miss gives
  * (fallback_loc, (uint32)key).  Either output may be NULL (OffsetOnly, cuh:396-407). */
 int ugk_table_lookup_u32(ugk_table_t t, const uint32_t *keys_dev, size_t n, uint32_t fallback_loc,

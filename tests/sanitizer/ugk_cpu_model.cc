@@ -287,13 +287,41 @@ int table_insert(ugk_table_t t, const K *keys, const uint32_t *offs, uint32_t se
   return 0;
 }
 
+// the word of `key`'s entry that holds its slot (below its location, where the two share one), null where it has none
+template <typename K>
+uint32_t *slot_word(ugk_table_t t, K k) {
+  const uint64_t key = k64(k);
+  if (t.kind == 1) return key < t.size ? reinterpret_cast<uint32_t *>(t.table) + key : nullptr;
+  if (t.kind == 3) {
+    const uint64_t row = fallback_row(t, key);
+    uint64_t *w = reinterpret_cast<uint64_t *>(t.table);
+    for (uint64_t step = 0, pos = h32_home(row, t.size); step < t.size && ld(w + pos) != kH32EmptyWord; ++step) {
+      if ((uint32_t)ld(w + pos) == (uint32_t)row) return reinterpret_cast<uint32_t *>(w + pos) + 1;
+      if (++pos == t.size) pos = 0;
+    }
+    return nullptr;
+  }
+  ugk_bucket_t *b = reinterpret_cast<ugk_bucket_t *>(t.table);
+  for (uint64_t step = 0, pos = fmix64(key) % t.size; step < t.size && ld(&b[pos].key) != UGK_HASH_EMPTY; ++step) {
+    if (ld(&b[pos].key) == key) return &b[pos].off;
+    if (++pos == t.size) pos = 0;
+  }
+  return nullptr;
+}
+std::atomic<bool> g_share_a_slot{false};  // see ugk_model_share_a_slot
+
 template <typename K>
 int table_evict(ugk_table_t t, const K *keys, size_t n, uint32_t *status, uint64_t *slot_bits = nullptr,
-                uint64_t nslots = 0, uint32_t *slots_out = nullptr) {
+                uint64_t nslots = 0, uint32_t *slots_out = nullptr, uint32_t *stamps = nullptr) {
   if (slots_out) std::fill(slots_out, slots_out + n, ~0u);
+  if (slots_out && n >= 2 && g_share_a_slot.exchange(false)) {
+    uint32_t *one = slot_word(t, keys[0]), *other = slot_word(t, keys[1]);
+    if (one && other) __atomic_store_n(other, __atomic_load_n(one, __ATOMIC_RELAXED), __ATOMIC_RELAXED);
+  }
   size_t at = 0;
   auto release = [&](uint32_t slot) {
     if (slots_out) slots_out[at] = slot;
+    if (stamps && slot < nslots) stamps[slot] = (uint32_t)at;
     if (!slot_bits) return;
     if (slot >= nslots) or_status(status, UGK_ST_KEY_OUT_OF_RANGE);
     else __atomic_fetch_and(slot_bits + (slot >> 6), ~(1ull << (slot & 63)), __ATOMIC_RELAXED);
@@ -796,6 +824,7 @@ void ugk_model_reset(void) {
   g_stage_writers.clear();
   g_written.clear();
 }
+void ugk_model_share_a_slot(void) { g_share_a_slot = true; }
 void ugk_model_small_bits(size_t nbits) {
   std::lock_guard<std::mutex> g(g_rt_mu);
   g_small_bits = nbits;
@@ -1128,6 +1157,24 @@ int ugk_table_insert_i64(ugk_table_t t, const int64_t *keys, const uint32_t *off
                          size_t n, uint32_t *status, void *) {
   return table_insert(t, keys, offs, seq_base, loc, n, status);
 }
+int ugk_handed_check(const ugk_handed_t *h, const uint32_t *slots, size_t n, uint32_t *status, void *) {
+  if (n == 0) return 0;
+  REQUIRE(slots && h && h->stamps && h->used_bits, "slots that are handed on: null list, stamps or bitmap");
+  for (size_t i = 0; i < n; ++i) {
+    const uint32_t slot = slots[i];
+    if (slot >= h->nslots) or_status(status, UGK_ST_KEY_OUT_OF_RANGE);
+    else if (h->stamps[slot] != i || !(h->used_bits[slot >> 6] >> (slot & 63) & 1)) or_status(status, UGK_ST_SLOT_CLASH);
+  }
+  return 0;
+}
+int ugk_table_insert_handed_u32(ugk_table_t t, const uint32_t *keys, const uint32_t *slots, uint32_t loc, size_t n,
+                                const ugk_handed_t *handed, uint32_t *status, void *stream) {
+  return ugk_handed_check(handed, slots, n, status, stream) || table_insert(t, keys, slots, 0, loc, n, status);
+}
+int ugk_table_insert_handed_i64(ugk_table_t t, const int64_t *keys, const uint32_t *slots, uint32_t loc, size_t n,
+                                const ugk_handed_t *handed, uint32_t *status, void *stream) {
+  return ugk_handed_check(handed, slots, n, status, stream) || table_insert(t, keys, slots, 0, loc, n, status);
+}
 int ugk_table_evict_u32(ugk_table_t t, const uint32_t *keys, size_t n, uint32_t *status, void *) {
   return table_evict(t, keys, n, status);
 }
@@ -1151,6 +1198,16 @@ int ugk_table_evict_slots_u32(ugk_table_t t, const uint32_t *keys, size_t n, uin
 int ugk_table_evict_slots_i64(ugk_table_t t, const int64_t *keys, size_t n, uint32_t *slots_out, uint32_t *status, void *) {
   REQUIRE(n == 0 || slots_out, "ugk_table_evict_slots_i64: null list of slots");
   return table_evict(t, keys, n, status, nullptr, 0, slots_out);
+}
+int ugk_table_evict_handed_u32(ugk_table_t t, const uint32_t *keys, size_t n, uint32_t *slots_out, const ugk_handed_t *handed,
+                               uint32_t *status, void *) {
+  REQUIRE(n == 0 || (slots_out && handed && handed->stamps), "ugk_table_evict_handed_u32: null list of slots or stamps");
+  return n == 0 ? 0 : table_evict<uint32_t>(t, keys, n, status, nullptr, handed->nslots, slots_out, handed->stamps);
+}
+int ugk_table_evict_handed_i64(ugk_table_t t, const int64_t *keys, size_t n, uint32_t *slots_out, const ugk_handed_t *handed,
+                               uint32_t *status, void *) {
+  REQUIRE(n == 0 || (slots_out && handed && handed->stamps), "ugk_table_evict_handed_i64: null list of slots or stamps");
+  return n == 0 ? 0 : table_evict<int64_t>(t, keys, n, status, nullptr, handed->nslots, slots_out, handed->stamps);
 }
 int ugk_table_lookup_u32(ugk_table_t t, const uint32_t *keys, size_t n, uint32_t fallback_loc, uint32_t *loc_out,
                          uint32_t *off_out, void *) {

@@ -662,3 +662,54 @@ def test_evict_that_lists_the_slots(kind, kdtype, n_gone):
     assert status_value(st) != 0
     want = [slots[np.flatnonzero(stays)[0]], 0xFFFFFFFF, 0xFFFFFFFF, slots[np.flatnonzero(stays)[1]]]
     assert to_np(d_list, np.uint32)[:4].tolist() == want
+
+
+@pytest.mark.parametrize("kind", ["flat", "hash", "hash32"])
+@pytest.mark.parametrize("kdtype", [np.uint32, np.int64])
+@pytest.mark.parametrize("nslots,n", [(100, 60), (30_001, 20_000), (9_000_000, 140_003)])
+def test_slots_that_are_handed_on(kind, kdtype, nslots, n):
+    """ugk_table_evict_handed_* lists slots, ugk_table_insert_handed_* gives them to other keys and looks at them on the way, as
+    ugk_handed_check does: one that two entries name, in one wavefront or far apart, one not in use and one beyond the bitmap are
+    flagged.  What the stamps held before does not matter"""
+    rng = np.random.default_rng(nslots)
+    nkeys, n_gone = 2 * n, n // 3
+    wide = "i64" if kdtype == np.int64 else "u32"
+    keys = rng.choice(nkeys, n, replace=False).astype(kdtype)
+    coming = np.setdiff1d(np.arange(nkeys), keys)[:n_gone].astype(kdtype)
+    slots = rng.choice(nslots, n, replace=False).astype(np.uint32)
+    used = np.zeros((nslots + 63) // 64 * 64, bool)
+    used[slots] = True
+    d_keys, d_in, stamps = to_dev(keys), to_dev(coming), to_dev(rng.integers(0, n_gone, size=nslots).astype(np.uint32))
+    size = getattr(hip.lib(), "ugk_hash_buckets_for" if kind == "hash" else "ugk_hash32_entries_for")(n, 0.7)
+    mem = dev_bytes(size * 16 + 128) if kind != "flat" else dev_zeros_u32(nkeys)
+    for fault, flag in ((None, 0), (1, hip.ST_SLOT_CLASH), (n_gone - 1, hip.ST_SLOT_CLASH), ("free", hip.ST_SLOT_CLASH),
+                        ("beyond", hip.ST_KEY_OUT_OF_RANGE)):
+        mine, in_use, limit = slots.copy(), used.copy(), nslots
+        if fault == "free":
+            in_use[mine[n_gone // 2]] = False
+        elif fault == "beyond":
+            limit = int(mine[:n_gone].max())
+        elif fault:
+            mine[fault] = mine[0]
+        d_mine, d_used = to_dev(mine), to_dev(np.packbits(in_use, bitorder="little").view(np.uint64))
+        d_list, st = to_dev(np.full(n_gone + 4, 77, np.uint32)), dev_zeros_u32(1)
+        if kind == "flat":
+            hip.call("ugk_fill_u32", ptr(mem), hip.EMPTY_U32, nkeys, None)
+            tb = hip.table(hip.TABLE_FLAT, ptr(mem), nkeys)
+        else:
+            tb = hip.table(hip.TABLE_HASH if kind == "hash" else hip.TABLE_HASH32, (ptr(mem) + 127) // 128 * 128, size)
+            hip.call("ugk_table_init", tb, None)
+        handed = hip.Handed(ptr(stamps), ptr(d_used), limit)
+        hip.call("ugk_table_insert_" + wide, tb, ptr(d_keys), ptr(d_mine), 0, 0, n, ptr(st), None)
+        hip.call("ugk_table_evict_handed_" + wide, tb, ptr(d_keys), n_gone, ptr(d_list), C.byref(handed), ptr(st), None)
+        got = to_np(d_list, np.uint32)
+        assert status_value(st) == 0 and np.array_equal(got[:n_gone], mine[:n_gone]) and got[n_gone] == 77
+        hip.call("ugk_handed_check", C.byref(handed), ptr(d_list), n_gone, ptr(st), None)
+        assert status_value(st) == flag, fault
+        st.zero_()
+        hip.call("ugk_table_insert_handed_" + wide, tb, ptr(d_in), ptr(d_list), 0, n_gone, C.byref(handed), ptr(st), None)
+        assert status_value(st) == flag, fault
+        loc, off = dev_zeros_u32(n_gone), dev_zeros_u32(n_gone)
+        hip.call("ugk_table_lookup_" + wide, tb, ptr(d_in), n_gone, 9, ptr(loc), ptr(off), None)
+        assert (to_np(loc, np.uint32)[:n_gone] == 0).all() and np.array_equal(to_np(off, np.uint32)[:n_gone], mine[:n_gone])
+        assert np.array_equal(np.unpackbits(to_np(d_used, np.uint64).view(np.uint8), bitorder="little").astype(bool), in_use)

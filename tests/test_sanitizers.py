@@ -66,6 +66,15 @@ def test_host_table_between_two_vectors(drivers, table, refresh, shift):
     assert rc == 0 and out.rstrip().endswith("OK"), out[-3000:]
 
 
+@pytest.mark.parametrize("foreground", ["1", "0"])
+@pytest.mark.parametrize("table", ["FLAT", "HASH", "HASH16"])
+def test_refresh_finds_two_entries_that_name_one_slot(drivers, table, foreground):
+    """rows that come in take the slots of those that leave: a slot named twice would hold one row under two keys"""
+    rc, out = _run(drivers["asan"], table, "device", 20, DRIVER_SHARED_SLOT=foreground)
+    assert "AddressSanitizer" not in out and "runtime error" not in out, out[-6000:]
+    assert rc != 0 and "0x40" in out and "found nothing" not in out, out[-3000:]
+
+
 @pytest.mark.parametrize("refresh", ["host", "device"])
 @pytest.mark.parametrize("table", ["FLAT", "HASH", "HASH16"])
 def test_host_library_under_tsan(drivers, table, refresh):

@@ -1534,7 +1534,8 @@ void RefreshSession::WaitForOneLookup(ExtractSession *session, bool foreground, 
 }
 
 void RefreshSession::CopyRowsIntoSlots(const uint32_t *rows_dev, const uint32_t *slots_dev, size_t num_rows,
-                                       bool foreground, StreamHandle copy_stream, const ugk_stage_t *stage) {
+                                       bool handed, bool foreground, StreamHandle copy_stream,
+                                       const ugk_stage_t *stage) {
   CacheContext *ctx = _cache_ctx.get();
   auto table = ctx->_new_hash_table;
   const Context gpu_ctx = ctx->_trainer_ctx;
@@ -1556,8 +1557,13 @@ void RefreshSession::CopyRowsIntoSlots(const uint32_t *rows_dev, const uint32_t 
       UGK_CALL(ugk_stream_sync(copy_stream));
       session->WaitForLookupsInFlight(false, 20.0);
     }
-    table->PublishRows(rows, slots, n, local, __publish_ids, ctx->_eager_gpu_mem_allocator, gpu_ctx, copy_stream);
+    table->PublishRows(rows, slots, n, local, handed && foreground, __publish_ids, ctx->_eager_gpu_mem_allocator, gpu_ctx,
+                       copy_stream);
   };
+  if (handed && !foreground) {  // the list is published in parts; else the launch that publishes it looks at it as well
+    table->CheckHanded(slots_dev, num_rows, copy_stream);
+    table->CheckStatus(copy_stream, "refresh slots");
+  }
   if (foreground) {
     // Nothing runs beside a foreground refresh: one launch copies every row.  Without a stage all of them cross the host
     // link, on a capped grid: rows of 512 bytes and more cross it faster from 128 workgroups than from as many as the
@@ -1717,7 +1723,7 @@ void RefreshSession::refresh_after_solve_new(bool foreground) {
     auto insert_keys_gpu = CopyTo1DReuse(__keys_buffer, new_insert_keys, gpu_ctx, low_pri_stream);
     auto reserved_offset =
         CopyTo1DReuse(__offs_buffer, table->ReserveOffsetFront((IdType)num_insert), gpu_ctx, low_pri_stream);
-    CopyRowsIntoSlots(insert_keys_gpu->CPtr<uint32_t>(), reserved_offset->CPtr<uint32_t>(), num_insert, foreground,
+    CopyRowsIntoSlots(insert_keys_gpu->CPtr<uint32_t>(), reserved_offset->CPtr<uint32_t>(), num_insert, false, foreground,
                       low_pri_stream, stage);  // waits for the copy stream: rows copied and published
     table->CheckStatus(stream, "refresh insert");
   }
@@ -1898,11 +1904,12 @@ void RefreshSession::ApplyPlacedBits(ExtractSession *session, size_t num_cached,
     if (!hand_over) slots = table->FreeSlots(num_insert, &n_free_word, __free_slots, alloc, gpu_ctx, stream);
     if (foreground) {
       // nothing runs beside a foreground refresh: the copy goes on the refresh's own stream, behind the lists it reads
-      CopyRowsIntoSlots(insert_rows->CPtr<uint32_t>(), slots->CPtr<uint32_t>(), num_insert, true, stream, stage);
+      CopyRowsIntoSlots(insert_rows->CPtr<uint32_t>(), slots->CPtr<uint32_t>(), num_insert, hand_over, true,
+                        stream, stage);
     } else {
       UGK_CALL(ugk_stream_sync(stream));  // the lists are read on the copy stream next
-      CopyRowsIntoSlots(insert_rows->CPtr<uint32_t>(), slots->CPtr<uint32_t>(), num_insert, false, low_pri_stream,
-                        stage);
+      CopyRowsIntoSlots(insert_rows->CPtr<uint32_t>(), slots->CPtr<uint32_t>(), num_insert, hand_over, false,
+                        low_pri_stream, stage);
     }
     // the slots taken are the lowest free ones: every bit up to the last of them is set now
     if (!hand_over)
@@ -1914,7 +1921,8 @@ void RefreshSession::ApplyPlacedBits(ExtractSession *session, size_t num_cached,
   const uint32_t table_status = table->StatusAndWords(_status_handle->ptr<uint32_t>(), 9, stw, stream);
   CHECK_EQ(table_status, 0u) << "refresh on the device: table maintenance kernel reported status 0x" << std::hex
                              << table_status
-                             << " (1 key out of range, 2 table full, 4 duplicate key, 8 evict of absent key)";
+                             << " (1 key out of range, 2 table full, 4 duplicate key, 8 evict of absent key, 0x40 two "
+                                "entries name one slot)";
   CHECK_EQ(stw[0], 0u) << "refresh on the device: a listed row or slot is outside its table or bitmap (1), or the "
                           "placement found more observed rows than the host's bound allows (0x20)";
   const uint32_t from_stage = stw[8] - _rows_from_stage;

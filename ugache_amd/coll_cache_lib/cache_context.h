@@ -413,9 +413,10 @@ class RefreshSession {
  private:
   // copies the listed host rows into the listed cache slots and publishes them in the table (step 6): in one launch
   // each when in the foreground; behind running lookups in small throttled batches, every batch published as soon as
-  // it has arrived, so the hit rate climbs while the refresh runs instead of at its end
-  void CopyRowsIntoSlots(const uint32_t *rows_dev, const uint32_t *slots_dev, size_t num_rows, bool foreground,
-                         StreamHandle copy_stream, const ugk_stage_t *stage);
+  // it has arrived, so the hit rate climbs while the refresh runs instead of at its end.  handed: the
+  // slots are those of rows that left, and looked at on the way (see EvictForSlots)
+  void CopyRowsIntoSlots(const uint32_t *rows_dev, const uint32_t *slots_dev, size_t num_rows, bool handed,
+                         bool foreground, StreamHandle copy_stream, const ugk_stage_t *stage);
   TensorPtr __publish_ids;  // table keys of the rows being published (sparse ids)
   TensorPtr __keys_buffer;
   TensorPtr __offs_buffer;

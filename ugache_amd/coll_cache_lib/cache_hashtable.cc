@@ -243,14 +243,20 @@ TensorPtr CacheEntryManager::CompactBits(const uint64_t *a, const uint64_t *b, b
 TensorPtr CacheEntryManager::EvictForSlots(TensorPtr keys_to_evict, TensorPtr &buffer,
                                            const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream) {
   TensorPtr slots = ReuseList(buffer, kI32, keys_to_evict->NumItem(), allocator, ctx);
+  const ugk_handed_t handed = Handed();
   if (keys_to_evict->Type() == kI64)
-    UGK_CALL(ugk_table_evict_slots_i64(_table, keys_to_evict->CPtr<int64_t>(), keys_to_evict->NumItem(),
-                                       slots->Ptr<uint32_t>(), StatusPtr(this, stream), stream));
+    UGK_CALL(ugk_table_evict_handed_i64(_table, keys_to_evict->CPtr<int64_t>(), keys_to_evict->NumItem(), slots->Ptr<uint32_t>(),
+                                        &handed, StatusPtr(this, stream), stream));
   else
-    UGK_CALL(ugk_table_evict_slots_u32(RowView(), keys_to_evict->CPtr<uint32_t>(), keys_to_evict->NumItem(),
-                                       slots->Ptr<uint32_t>(), StatusPtr(this, stream), stream));
+    UGK_CALL(ugk_table_evict_handed_u32(RowView(), keys_to_evict->CPtr<uint32_t>(), keys_to_evict->NumItem(),
+                                        slots->Ptr<uint32_t>(), &handed, StatusPtr(this, stream), stream));
   NoteEvicted(keys_to_evict->NumItem());
   return slots;
+}
+
+void CacheEntryManager::CheckHanded(const uint32_t *slots_dev, size_t n, StreamHandle stream) {
+  const ugk_handed_t handed = Handed();
+  UGK_CALL(ugk_handed_check(&handed, slots_dev, n, StatusPtr(this, stream), stream));
 }
 
 TensorPtr CacheEntryManager::FreeSlots(size_t n, volatile uint32_t **num_free, TensorPtr &buffer,
@@ -330,17 +336,25 @@ TensorPtr CacheEntryManager::RowsToTableKeys(TensorPtr rows_dev, TensorPtr &buff
 }
 
 void CacheEntryManager::PublishRows(const uint32_t *rows_dev, const uint32_t *slots_dev, size_t n, int loc,
-                                    TensorPtr &id_buffer, const std::function<MemHandle(size_t)> &allocator,
-                                    Context ctx, StreamHandle stream) {
+                                    bool check_slots, TensorPtr &id_buffer,
+                                    const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream) {
   if (n == 0) return;
+  const ugk_handed_t handed = check_slots ? Handed() : ugk_handed_t{};
   if (RunConfig::key_map_mul == 0 || _table.kind == 3) {
-    UGK_CALL(ugk_table_insert_u32(RowView(), rows_dev, slots_dev, 0, (uint32_t)loc, n, StatusPtr(this, stream), stream));
+    if (check_slots)
+      UGK_CALL(ugk_table_insert_handed_u32(RowView(), rows_dev, slots_dev, (uint32_t)loc, n, &handed, StatusPtr(this, stream), stream));
+    else
+      UGK_CALL(ugk_table_insert_u32(RowView(), rows_dev, slots_dev, 0, (uint32_t)loc, n, StatusPtr(this, stream), stream));
     return;
   }
   TensorPtr ids = ReuseList(id_buffer, kI64, n, allocator, ctx);
   UGK_CALL(ugk_rows_to_keys(rows_dev, n, RunConfig::key_map_mul, RunConfig::key_map_mask, ids->Ptr<int64_t>(), stream));
-  UGK_CALL(ugk_table_insert_i64(_table, ids->CPtr<int64_t>(), slots_dev, 0, (uint32_t)loc, n, StatusPtr(this, stream),
-                                stream));
+  if (check_slots)
+    UGK_CALL(ugk_table_insert_handed_i64(_table, ids->CPtr<int64_t>(), slots_dev, (uint32_t)loc, n, &handed, StatusPtr(this, stream),
+                                         stream));
+  else
+    UGK_CALL(ugk_table_insert_i64(_table, ids->CPtr<int64_t>(), slots_dev, 0, (uint32_t)loc, n, StatusPtr(this, stream),
+                                  stream));
 }
 
 void CacheEntryManager::EnsureDeviceLists(const std::function<MemHandle(size_t)> &allocator, Context ctx,
@@ -351,6 +365,7 @@ void CacheEntryManager::EnsureDeviceLists(const std::function<MemHandle(size_t)>
     _dev_in_new = EagerGPUAlloc(_device_id, row_words * 8);
     _dev_scratch_bits = EagerGPUAlloc(_device_id, row_words * 8);
     _dev_slot_used = EagerGPUAlloc(_device_id, std::max<size_t>(slot_words, 1) * 8);
+    _dev_slot_stamps = EagerGPUAlloc(_device_id, std::max<size_t>(_cache_space_capacity, 1) * sizeof(uint32_t));
     _dev_rank_ws = EagerGPUAlloc(_device_id, ugk_rank_workspace_bytes());
     _dev_bm_ws = EagerGPUAlloc(_device_id, ugk_bitmap_workspace_bytes());
     _dev_bm_ws2 = EagerGPUAlloc(_device_id, ugk_bitmap_workspace_bytes());
@@ -433,7 +448,7 @@ void CacheEntryManager::CheckStatus(StreamHandle stream, const char *what) {
   UGK_CALL(ugk_memcpy_async(&st, StatusPtr(this, stream), sizeof(st), stream));
   UGK_CALL(ugk_stream_sync(stream));
   CHECK_EQ(st, 0u) << what << ": table maintenance kernel reported status 0x" << std::hex << st
-                   << " (1 key out of range, 2 table full, 4 duplicate key, 8 evict of absent key)";
+                   << " (1 key out of range, 2 table full, 4 duplicate key, 8 evict of absent key, 0x40 two entries name one slot)";
 }
 
 void CacheEntryManager::ReturnOffset(TensorPtr new_offsets) {

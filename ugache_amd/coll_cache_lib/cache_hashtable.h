@@ -83,9 +83,11 @@ class CacheEntryManager {
   // the same, and the evicted keys' slots leave the slot bitmap (SlotUsedBits) in the same launch: what LookupOffset +
   // ReturnOffset + Evict do together when the bookkeeping lives on the device
   void EvictRelease(TensorPtr keys_to_evict, StreamHandle stream);
-  /// ... and the slots the keys held, in the order of the keys
+  // ... and the slots the keys held, in the order of the keys, for as many rows that come in.  They stay in use; that no two
+  // entries named one of them is for PublishRows or CheckHanded to look at (UGK_ST_SLOT_CLASH in the status word)
   TensorPtr EvictForSlots(TensorPtr keys_to_evict, TensorPtr &buffer, const std::function<MemHandle(size_t)> &allocator,
                           Context ctx, StreamHandle stream);
+  void CheckHanded(const uint32_t *slots_dev, size_t n, StreamHandle stream);
   // cuh:635-655 — free-list: returned offsets go to the back, reservations come from the front
   void ReturnOffset(TensorPtr new_offsets);
   TensorPtr ReserveOffsetFront(IdType num_new_insert_keys);
@@ -111,6 +113,7 @@ class CacheEntryManager {
   MemHandle _dev_in_cache, _dev_in_new;  // ceil(num_total_key / 64) words each
   MemHandle _dev_scratch_bits;           // as large, scratch of the placement
   MemHandle _dev_slot_used;              // ceil(capacity / 64) words
+  MemHandle _dev_slot_stamps;            // capacity 32-bit words: where in the list of its refresh a slot was handed on
   MemHandle _dev_rank_ws, _dev_bm_ws;    // workspaces of ugk_rank_* / ugk_bitmap_*
   MemHandle _dev_bm_ws2;                 // a second one, so that two compactions can be counted before one wait
   MemHandle _dev_words;                  // pinned host words the kernels report counts in
@@ -129,6 +132,7 @@ class CacheEntryManager {
   uint64_t *InCacheBits() const { return _dev_in_cache->ptr<uint64_t>(); }
   uint64_t *InNewBits() const { return _dev_in_new->ptr<uint64_t>(); }
   uint64_t *SlotUsedBits() const { return _dev_slot_used->ptr<uint64_t>(); }
+  ugk_handed_t Handed() const { return {_dev_slot_stamps->ptr<uint32_t>(), SlotUsedBits(), _cache_space_capacity}; }
   uint32_t *DevWords() const { return _dev_words->ptr<uint32_t>(); }
   // the table as 32-bit row numbers address it: a compact table stores its keys by the row, so with sparse ids the
   // lists of rows a refresh works on need no translation into ids
@@ -179,9 +183,10 @@ class CacheEntryManager {
   // device list of host rows -> device list of table keys (the rows themselves, or their ids in sparse-id mode)
   TensorPtr RowsToTableKeys(TensorPtr rows_dev, TensorPtr &buffer, const std::function<MemHandle(size_t)> &allocator,
                             Context ctx, StreamHandle stream);
-  // InsertWithLoc for device lists of host rows and their slots (raw pointers: parts of longer lists)
-  void PublishRows(const uint32_t *rows_dev, const uint32_t *slots_dev, size_t n, int loc, TensorPtr &id_buffer,
-                   const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream);
+  // InsertWithLoc for device lists of host rows and their slots (raw pointers: parts of longer lists); check_slots: what
+  // CheckHanded does, in the same launch (the list is whole then)
+  void PublishRows(const uint32_t *rows_dev, const uint32_t *slots_dev, size_t n, int loc, bool check_slots,
+                   TensorPtr &id_buffer, const std::function<MemHandle(size_t)> &allocator, Context ctx, StreamHandle stream);
 
   // cuh:693-740 — keys of `inputs` satisfying cond, in input order (deterministic, unlike the reference's
   // thread-interleaved order)

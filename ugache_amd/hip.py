@@ -15,6 +15,7 @@ ST_DUP_KEY = 0x4
 ST_EVICT_ABSENT = 0x8
 ST_BAD_SEGMENT = 0x10
 ST_PLACE_PROMISE = 0x20
+ST_SLOT_CLASH = 0x40
 ELEM_BF16 = 0x102
 
 LOC_LOCAL = 0
@@ -49,6 +50,11 @@ class Done(C.Structure):
     _fields_ = [("words_host", C.c_void_p), ("counters_dev", C.c_void_p), ("tag", C.c_uint32), ("num_words", C.c_uint32),
                 ("keys_host", C.c_void_p), ("num_keys", C.c_uint64), ("counter_set", C.c_uint32), ("where_faster", C.c_uint32),
                 ("count_dev", C.c_void_p)]
+
+
+class Handed(C.Structure):
+    """ugk_handed_t"""
+    _fields_ = [("stamps", C.c_void_p), ("used_bits", C.c_void_p), ("nslots", C.c_uint64)]
 
 
 class DeviceInfo(C.Structure):
@@ -114,6 +120,11 @@ SIGNATURES = {
     "ugk_table_evict_i64": [Table, _vp, _sz, _vp, _vp],
     "ugk_table_evict_slots_u32": [Table, _vp, _sz, _vp, _vp, _vp],
     "ugk_table_evict_slots_i64": [Table, _vp, _sz, _vp, _vp, _vp],
+    "ugk_table_evict_handed_u32": [Table, _vp, _sz, _vp, C.POINTER(Handed), _vp, _vp],
+    "ugk_table_evict_handed_i64": [Table, _vp, _sz, _vp, C.POINTER(Handed), _vp, _vp],
+    "ugk_handed_check": [C.POINTER(Handed), _vp, _sz, _vp, _vp],
+    "ugk_table_insert_handed_u32": [Table, _vp, _vp, _u32, _sz, C.POINTER(Handed), _vp, _vp],
+    "ugk_table_insert_handed_i64": [Table, _vp, _vp, _u32, _sz, C.POINTER(Handed), _vp, _vp],
     "ugk_table_evict_release_u32": [Table, _vp, _sz, _vp, _u64, _vp, _vp],
     "ugk_table_evict_release_i64": [Table, _vp, _sz, _vp, _u64, _vp, _vp],
     "ugk_table_lookup_u32": [Table, _vp, _sz, _u32, _vp, _vp, _vp],
