@@ -14,6 +14,8 @@
 // usage: driver <FLAT|HASH> <host|device> [lookup steps per phase, default 150]
 // DRIVER_TABLE_SHIFT=n: the host table begins n bytes behind a 64-byte boundary (pooled lookups, which want whole 16-byte
 // vectors, are left out where n is no multiple of 16)
+// DRIVER_SHARED_SLOT=1|0: a refresh, in the foreground or not, of a table two entries of which name one slot
+// DRIVER_UNIQUE_ROUTES=1: only distinct-key lookups of byte rows, and which of them wait once
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
@@ -51,6 +53,53 @@ long check_rows(const float *table, const float *out, const uint32_t *keys, size
   return bad;
 }
 
+// Distinct-key lookups of byte rows out of a full cache: which of them are fetched by a launch that finds its count on the device.
+int unique_routes() {
+  struct Case {
+    size_t row_bytes, out_shift, keys;
+    bool counted;
+  };
+  const Case cases[] = {{100, 0, 100000, true}, {97, 0, 86480, true}, {97, 0, 86481, false}, {98, 0, 85599, false}, {98, 0, 500, true},
+                        {100, 4, 100000, true}, {100, 2, 83886, true}, {100, 2, 83887, false}, {100, 1, 100000, false}};
+  size_t open = 0;
+  char *table = nullptr;
+  std::mt19937_64 g(5);
+  for (const Case &c : cases) {
+    if (open != c.row_bytes) {
+      if (open) coll_cache_shutdown(), coll_cache_free_host_table(table);
+      open = c.row_bytes;
+      const char *keys[] = {"cache_percentage", "_cache_policy", "num_device", "num_global_step_per_epoch", "num_epoch",
+                            "num_total_item",   "omp_thread_num"};
+      const char *vals[] = {"1", "13", "1", "10", "1", "20000", "4"};
+      coll_cache_config(keys, vals, 7);
+      table = static_cast<char *>(coll_cache_alloc_host_table(kRows * open));
+      for (size_t i = 0; i < kRows * open; ++i) table[i] = (char)(i * 7 + i / 251);
+      coll_cache_record_init(0);
+      coll_cache_init_c(0, kRows, nullptr, nullptr, nullptr, table, /*kU8*/ 3, open, 1.0, nullptr);
+    }
+    std::vector<uint32_t> k(c.keys), inverse(c.keys);
+    for (auto &x : k) x = (uint32_t)(g() % kRows);
+    std::vector<char> out(c.keys * c.row_bytes + 64);
+    char *to = reinterpret_cast<char *>(((uintptr_t)out.data() + 15) / 16 * 16) + c.out_shift;
+    const size_t before = ugk_model_counted();
+    const size_t nu = coll_cache_lookup_unique(0, k.data(), k.size(), to, inverse.data(), nullptr);
+    for (size_t i = 0; i < k.size(); ++i)
+      if (inverse[i] >= nu || memcmp(to + (size_t)inverse[i] * open, table + (size_t)k[i] * open, open) != 0) {
+        fprintf(stderr, "rows of %zu bytes, %zu keys: wrong row\n", open, c.keys);
+        return 1;
+      }
+    if ((ugk_model_counted() > before) != c.counted) {
+      fprintf(stderr, "rows of %zu bytes at +%zu, %zu keys: the count was taken from the %s\n", open, c.out_shift, c.keys,
+              c.counted ? "host" : "device");
+      return 1;
+    }
+  }
+  coll_cache_shutdown();
+  coll_cache_free_host_table(table);
+  printf("OK\n");
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -65,6 +114,7 @@ int main(int argc, char **argv) {
   setenv("COLL_GPU_REFRESH", on_device ? "1" : "0", 1);
   setenv("SAMGRAPH_LOG_LEVEL", "warn", 0);
 
+  if (getenv("DRIVER_UNIQUE_ROUTES")) return unique_routes();
   const char *keys[] = {"cache_percentage", "_cache_policy", "num_device", "num_global_step_per_epoch", "num_epoch",
                         "num_total_item",   "omp_thread_num"};
   const char *vals[] = {"0.25", "13", "1", "10", "1", "20000", "4"};

@@ -172,7 +172,12 @@ bool leave_done(uint64_t local, uint64_t others, const K *keys, size_t n) {
 }
 
 // ugk_done_t::count_dev: how many of its keys a launch looks up
-size_t launch_count(size_t n) { return g_done && g_done->count_dev ? std::min<size_t>(n, *g_done->count_dev) : n; }
+std::atomic<size_t> g_counted{0};  // see ugk_model_counted
+size_t launch_count(size_t n) {
+  if (!g_done || !g_done->count_dev) return n;
+  ++g_counted;
+  return std::min<size_t>(n, *g_done->count_dev);
+}
 
 template <typename K>
 int gather_direct(const void *src, uint64_t src_rows, const K *keys, const uint32_t *dst, size_t n, void *out,
@@ -824,6 +829,7 @@ void ugk_model_reset(void) {
   g_stage_writers.clear();
   g_written.clear();
 }
+size_t ugk_model_counted(void) { return g_counted; }
 void ugk_model_share_a_slot(void) { g_share_a_slot = true; }
 void ugk_model_small_bits(size_t nbits) {
   std::lock_guard<std::mutex> g(g_rt_mu);

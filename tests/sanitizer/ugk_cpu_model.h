@@ -16,6 +16,8 @@ size_t ugk_model_violations(char *text, size_t capacity);
 void ugk_model_reset(void);
 // bitmaps longer than this take the passes that the kernel layer has for those of more than 2^26 bits
 void ugk_model_small_bits(size_t nbits);
+// launches so far that took their number of keys from the device (ugk_done_t::count_dev)
+size_t ugk_model_counted(void);
 // the next eviction that lists slots finds its second key's entry naming the slot of the first
 void ugk_model_share_a_slot(void);
 }

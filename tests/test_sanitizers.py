@@ -66,6 +66,14 @@ def test_host_table_between_two_vectors(drivers, table, refresh, shift):
     assert rc == 0 and out.rstrip().endswith("OK"), out[-3000:]
 
 
+def test_distinct_key_lookups_of_bytes_wait_once_up_to_8_mib(drivers):
+    """a launch that finds its count on the device leaves words, which come later than a ticket for large outputs of single bytes
+    or pairs (odd rows, odd outputs); rows of 4-byte words are fetched that way at any size"""
+    rc, out = _run(drivers["asan"], "HASH", "host", 20, DRIVER_UNIQUE_ROUTES="1")
+    assert "AddressSanitizer" not in out and "runtime error" not in out and "LeakSanitizer" not in out, out[-6000:]
+    assert rc == 0 and out.rstrip().endswith("OK"), out[-3000:]
+
+
 @pytest.mark.parametrize("foreground", ["1", "0"])
 @pytest.mark.parametrize("table", ["FLAT", "HASH", "HASH16"])
 def test_refresh_finds_two_entries_that_name_one_slot(drivers, table, foreground):

@@ -1198,16 +1198,23 @@ void ExtractSession::ExtractFeatAsyncImpl(const KeyT *nodes, size_t num_nodes, v
 // (ugk_done_t::count_dev), so that the call waits once, at its end: a launch that leaves words, of whose keys nothing else is to be
 // made.  With the wait for the number in between,
 // before / now, lookup and the gather back by position: 262,144 keys of 512 bytes, a quarter cached, 709 / 703 us, 6,396 keys of
-// 256 bytes 56 / 49, 2,457 of 400 bytes all in HBM 42 / 35, 77,720 of 256 bytes 73 / 66.
+// 256 bytes 56 / 49, 2,457 of 400 bytes all in HBM 42 / 35, 77,720 of 256 bytes 73 / 66.  The launch leaves words where a ticket would
+// come sooner as well, which the wait that is saved makes up for: rows of 8 KB, a full cache, 64 KB of them 24.8 / 20.1, 32 MB
+// 39.3 / 33.5, and half of them cached 31.5 / 27.7 and 97 / 89.  But not for rows or outputs of single bytes or pairs beyond 8 MiB
+// (us of a lookup, uniform keys that were not looked up before): 97 bytes 1 MB 34.1 / 29.8, 8 MB 55.9 / 54.4, 16 MB 84 / 87, 32 MB
+// 115 / 125, 128 MB 318 / 373; 1002 bytes 8 MB 36.9 / 35.7, 16 MB 43.7 / 43.6, 32 MB 53 / 57; 6 bytes 8 MB 162 / 163, 32 MB 480 / 504.
 bool ExtractSession::CountsFromDevice(size_t num_nodes, const void *output) const {
   CacheContext *ctx = _cache_ctx.get();
   if (RunConfig::spin_wait_us == 0 || RunConfig::kernel_events || _hot_counts) return false;
   if (num_nodes >= ((size_t)1 << 24) || num_nodes * ctx->_row_bytes > ((size_t)256 << 20) || _out_hint == UGK_OUTPUT_STREAMS)
     return false;  // counts that words cannot hold; outputs that may be written with non-temporal stores
-  return ctx->IsDirectMapping() ||
-         (RunConfig::concurrent_link_impl == kDirectNoGroup && GetEnv("COLL_SKIP_LOCAL") != "1" &&
-          FusedTakes(ctx->_device_cache_data[ctx->_local_location_id], ctx->_device_cache_data[ctx->_cpu_location_id], output,
-                     ctx->_row_bytes));
+  if (ctx->IsDirectMapping()) {
+    const uintptr_t align = (uintptr_t)ctx->_device_cache_data[0] | (uintptr_t)output | (uintptr_t)ctx->_row_bytes;
+    return align % 4 == 0 || num_nodes * ctx->_row_bytes <= ((size_t)8 << 20);
+  }
+  return RunConfig::concurrent_link_impl == kDirectNoGroup && GetEnv("COLL_SKIP_LOCAL") != "1" &&
+         FusedTakes(ctx->_device_cache_data[ctx->_local_location_id], ctx->_device_cache_data[ctx->_cpu_location_id], output,
+                    ctx->_row_bytes);
 }
 
 template <typename KeyT>
