@@ -22,7 +22,7 @@ ORC = Oracle()
 
 if torch.cuda.is_available():
     import collcache.torch as co
-    from collcache.common import _basics, kLogL1FeatureBytes, kLogL1MissBytes, kLogL2CacheCopyTime
+    from collcache.common import _basics, kLogL1FeatureBytes, kLogL1MissBytes, kLogL2CacheCopyTime, kLogL3CacheCombineCacheTime
 
 
 def zipf_ranks(rng, n, space, s):
@@ -1940,6 +1940,30 @@ def test_lookups_stay_exact_while_the_device_refreshes_under_them(table_kind, st
     out = co.coll_torch_lookup_key_t_val_ret(0, torch.from_numpy(keys).cuda(), False)
     assert out.cpu().numpy().tobytes() == ORC.gather(table, keys).tobytes()
     assert _basics.last_group_offset(0)[1] == int(np.isin(keys, got).sum())
+
+
+@pytest.mark.parametrize("pct", [0.4, 1.0])
+def test_logged_combine_time_of_distinct_keys_is_that_of_their_rows(pct):
+    """the deduplication in front of them is not in it: 900,000 keys of 3,000 rows of 16 bytes, whose rows take a few microseconds
+    of the call and whose deduplication most of it"""
+    rng = np.random.default_rng(4)
+    n_item, n = 3_000, 900_000
+    co.config(make_config(n_item, pct))
+    co.coll_cache_record_init(0)
+    co.coll_torch_record(0, torch.from_numpy(rng.integers(0, n_item, size=20_000)))
+    emb = co.coll_torch_create_emb_shm(0, n_item, 4, torch.float32)
+    table = fill_table(emb, rng)
+    co.coll_torch_init_t(0, 0, emb, pct)
+    keys = torch.from_numpy(rng.integers(0, n_item, size=n)).cuda()
+    shares = []
+    for step in range(8):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        rows, inverse = co.coll_torch_lookup_unique(0, keys)
+        shares.append(_basics.step_value(step, kLogL3CacheCombineCacheTime) / (time.perf_counter() - t0))
+    assert rows[inverse.long()].cpu().numpy().tobytes() == table[keys.cpu().numpy()].tobytes()
+    assert 0 < sorted(shares)[2] < 0.5, shares
+
 
 
 @pytest.mark.parametrize("pct,table_kind", [(1.0, "FLAT"), (0.0, "FLAT"), (0.25, "FLAT"), (0.25, "HASH")])

