@@ -57,6 +57,13 @@ def test_a_pooled_lookup_nobody_polls_for_is_a_kernel_without_words(launches, id
     assert plain[0][1] != polled[0][1]
 
 
+@pytest.mark.parametrize("row_bytes", [16, 20, 32])
+def test_a_polled_gather_of_short_rows_is_one_kernel_at_every_size(launches, row_bytes):
+    """its stores need no room in the L2s, so that as many lines as those hold are no reason to read past them"""
+    seen = {launches("gather", row_bytes, rows, 1)[0][0][:2] for rows in (170_000, 180_224, 180_225, 262_144, 458_752, 458_753, 900_000)}
+    assert len(seen) == 1
+
+
 # (row bytes, megabytes of output, when words come, against a ticket kernel): on both sides of every line of the rules
 @pytest.mark.parametrize("call,row_bytes,mb,told", [
     ("gather", 512, 8, "sooner"), ("gather", 64, 8, "sooner"), ("gather", 12, 8, "sooner"), ("gather", 2048, 8, "sooner"),

@@ -519,17 +519,24 @@ bool over_link(const uint32_t *counts, uint32_t group, unsigned max_blocks) {
 //     out (250 MB, uniform keys: 80 none, 99 one of four); a launch with streaming stores has left it to the lines.
 //   * Rows under 48 bytes, of which a line holds several: all four, at every size (32 bytes, 128 MB, uniform 113 / 108 / 106,
 //     zipf 1.05 90 / 71 / 62; 4 bytes, 64 MB 371 / 312 / 317 and 248 / 180 / 136; 40 bytes, 200 MB 182 / 199 / 173).
-//     Except that lines that come to about what the L2s hold, 32 MB, push the output out of there, the more the longer the
-//     rows: 262,144 rows of 32 bytes 8.7 / 9.1 / 9.7, of 16 bytes 8.0 / 8.5 / 8.6, of 20 bytes (flat) 9.0 / 9.0 / 9.5, of
-//     12 bytes 8.4 / 8.4 / 8.3, where 131,072 and 524,288 of them lose nothing.
+//     Except that lines that come to about what the L2s hold, 32 MB, push the output out of there, for rows of 16 bytes and
+//     more: one of four, by which uniform keys lose nothing and skewed ones gain half.  Keys that were not looked up before,
+//     16 bytes, uniform, zipf 0.8 and 1.05: 131,072 5.4 / 5.4 / 5.4, 5.2 / 5.0 / 4.8 and 4.6 / 4.3 / 4.2; 180,224 6.8 / 6.9 / 6.6, 6.6 /
+//     6.2 / 6.1 and 5.5 / 5.2 / 4.6; 262,144 8.2 / 8.3 / 8.6, 7.8 / 7.6 / 7.7 and 6.1 / 5.9 / 5.4; 393,216 10.9 / 11.2 / 11.4, 10.3 / 9.9 /
+//     10.5 and 7.6 / 7.0 / 6.4; 458,752 12.9 / 13.0 / 13.1, 12.1 / 12.2 / 12.1 and 9.0 / 8.1 / 7.5; 700,000 19.0 / 18.7 / 18.1, 17.9 / 17.1 /
+//     16.4 and 13.0 / 11.7 / 10.4.  32 bytes: 180,224 6.8 / 6.7 / 7.0 and 6.6 / 6.6 / 6.4; 262,144 9.1 / 8.9 / 9.4 and 8.6 / 8.4 / 8.8; 320,000
+//     10.3 / 10.2 / 10.7 and 9.7 / 9.6 / 10.0; 458,752 14.5 / 14.1 / 13.9 and 13.2 / 13.2 / 12.6.  20 bytes (flat): 180,224 7.1 / 7.0 / 7.0;
+//     262,144 8.9 / 8.9 / 9.4; 393,216 12.3 / 12.7 / 12.4; 458,752 14.3 / 14.2 / 14.0.  12 bytes: 262,144 8.1 / 8.1 / 8.4, 458,752 13.4 /
+//     13.3 / 12.9.
 //   * Stores that are written through need no room in the L2s, and what one wavefront of four keeps there the others, reading past
-//     it, drop again: all four or none.  us, launch to end of poll, none / one / two / all, uniform and zipf 1.05 and 1.2, 512 bytes:
-//     2 MB 10.8 / 11.0 / 10.9 / 10.5 and 10.8 / 10.7 / 10.9 / 10.4 and 10.7 / 10.7 / 10.7 / 10.5; 8 MB 13.2 / 13.0 / 12.9 / 13.1 and
-//     12.4 / 12.5 / 12.4 / 11.4 and 12.5 / 12.4 / 12.4 / 11.3; 16 MB 15.7 / 15.6 / 15.4 / 15.6 and 15.1 / 15.0 / 14.8 / 13.5 and 14.9 /
-//     14.8 / 14.7 / 13.2; 32 MB 20.7 / 20.6 / 20.5 / 21.2 and 19.3 / 19.4 / 19.4 / 17.1.  All up to 16 MB, and none beyond, for what it
-//     costs uniform keys there; up to 10 MB for rows that begin inside a line (200 bytes, 12 MB, none / all 16.4 / 16.8 and, zipf
-//     1.2, 15.5 / 12.6).  Short rows: 16 bytes x 1,048,576 34.6 / 32.5 and, zipf 1.05, 25.9 / 21.8; 36 bytes x 466,033 25.4 / 24.7 and
-//     21.2 / 19.4, but x 5,688,888 194 / 201 and 131 / 123.
+//     it, drop again: all four or none.  us, launch to end of poll, keys that were not looked up before, none / all, uniform, zipf
+//     0.8, 1.05 and 1.2: 512 bytes 64 KB 9.4 / 9.5, 9.5 / 9.4, 9.5 / 9.3 and 9.4 / 9.3; 1 MB 10.1 / 10.2, 10.1 / 10.2, 10.0 / 9.9 and 10.0 /
+//     9.7; 8 MB 12.7 / 12.9, 12.7 / 12.6, 12.2 / 11.8 and 12.2 / 11.0; 16 MB 15.3 / 15.5, 15.3 / 15.2, 14.7 / 14.2 and 14.6 / 12.7; 128 bytes
+//     8 MB 13.4 / 13.4, 13.3 / 13.1, 12.8 / 12.5 and 12.8 / 11.6; 4 KB 64 KB 9.9 / 10.3, 10.2 / 10.0, 10.1 / 9.6 and 10.0 / 10.1; 2 MB 12.4 / 12.5,
+//     12.5 / 12.5, 12.3 / 12.2 and 12.1 / 11.3.  (Uniform keys pay 1 %.)  Beyond 16 MB uniform keys pay 2 to 3 %, 32 MB 20.7 / 21.2: none
+//     there; up to 10 MB for rows that begin inside a line (200 bytes, 10 MB 15.8 / 15.9, 15.7 / 15.5, 14.8 / 14.5 and 14.5 / 13.3).  Short
+//     rows: 16 bytes x 262,144 16.2 / 16.3, 15.9 / 15.7 and 14.1 / 13.0, x 1,048,576 31.9 / 32.0 and, zipf 1.05, 23.8 / 20.0; 32 bytes x
+//     262,144 17.1 / 17.3, 16.6 / 16.7 and 15.2 / 14.3; 36 bytes x 466,033 24.8 / 24.9 and 21.1 / 19.3, but x 5,688,888 194 / 201.
 //   * Rows over a link: none, as nothing that the chip's caches do shows beside the link (that of an uncapped gather out of
 //     host memory, which cannot be told from one out of HBM here: 16 to 1204 bytes x 0.25 to 8 MB 0.98 to 1.2 times as fast).
 constexpr size_t kMemorySideCache = 256ull << 20;
@@ -541,14 +548,13 @@ uint8_t keep_waves_for(size_t n, size_t row_bytes, Store store, bool over_link) 
                        : row_bytes % kLine == 0    ? row_bytes
                        : row_bytes % 16 == 0       ? row_bytes + kLine - 16
                                                    : row_bytes + kLine - 4;
-  const bool as_l2 = n > (22ull << 20) / kLine && n <= (56ull << 20) / kLine;
   if (store == kThrough) {
-    const bool all = row_bytes >= 48  ? n * row_bytes <= (size_t)(row_bytes % 64 == 0 ? 16 : 10) << 20
-                     : row_bytes > 32 ? n * (row_bytes + lines) <= kMemorySideCache
-                                      : !as_l2 || row_bytes < 16;
+    const bool all = row_bytes >= 48 ? n * row_bytes <= (size_t)(row_bytes % 64 == 0 ? 16 : 10) << 20
+                                     : row_bytes <= 32 || n * (row_bytes + lines) <= kMemorySideCache;
     return all ? kWavesPerBlock : 0;
   }
-  if (row_bytes < 48) return !as_l2 || row_bytes < 16 ? kWavesPerBlock : row_bytes % 16 == 0 ? 0 : 1;
+  const bool as_l2 = n > (22ull << 20) / kLine && n <= (56ull << 20) / kLine;
+  if (row_bytes < 48) return !as_l2 || row_bytes < 16 ? kWavesPerBlock : 1;
   return store == kStreaming || n * (row_bytes + lines / kWavesPerBlock) <= kMemorySideCache ? 1 : 0;
 }
 
