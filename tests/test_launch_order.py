@@ -57,6 +57,16 @@ def test_a_pooled_lookup_nobody_polls_for_is_a_kernel_without_words(launches, id
     assert plain[0][1] != polled[0][1]
 
 
+# (table, row bytes, keys): eight rows of a lane on their way in small launches of long rows, four in the others
+@pytest.mark.parametrize("kind,row_bytes,n,rows", [(3, 512, 8_192, 4), (3, 1024, 8_192, 8), (3, 512, 8_193, 8), (3, 512, 65_536, 8),
+                                                   (3, 512, 65_537, 4), (3, 512, 262_145, 4), (3, 1024, 400_000, 4), (2, 4096, 65_536, 8),
+                                                   (2, 4096, 270_000, 4), (1, 1024, 4_096, 8), (1, 1024, 4_097, 4)])
+@pytest.mark.parametrize("words", [0, 1])
+def test_rows_on_their_way_in_a_mixed_lookup(launches, kind, row_bytes, n, rows, words):
+    templ = launches("mix", row_bytes, n, words, kind)[0][0][1].strip("<>").split(",")
+    assert templ[1] == str(kind) and int(templ[4]) == rows, templ
+
+
 @pytest.mark.parametrize("row_bytes", [16, 20, 32])
 def test_a_polled_gather_of_short_rows_is_one_kernel_at_every_size(launches, row_bytes):
     """its stores need no room in the L2s, so that as many lines as those hold are no reason to read past them"""

@@ -236,7 +236,11 @@ __device__ __forceinline__ uint64_t stage_claim(const ugk_stage_t &stage, const 
 // 14.8 / 14.1, x 16,384 19.5 / 18.3 and 29.2 / 28.9; 4 KB x 16 14.5 / 12.9 and 16.6 / 14.5, x 1,024 18.3 / 17.0 and 23.2 / 21.1; 512
 // bytes x 16,384 16.6 / 15.5 and 21.3 / 21.1.  Behind a flat table, which is soon looked up in, a launch that fills the chip has
 // enough of them on their way: 1 KB x 2,048 11.9 / 11.6 and 13.3 / 12.7, x 8,192 13.3 / 13.6 and 18.1 / 18.5; 4 KB x 1,024 16.3 / 15.3
-// and 21.4 / 19.1, x 4,096 18.6 / 17.7 and 26.1 / 26.5, x 16,384 31.7 / 34.2.
+// and 21.4 / 19.1, x 4,096 18.6 / 17.7 and 26.1 / 26.5, x 16,384 31.7 / 34.2: up to 4,096 keys there.  Behind a hash table up to the
+// 65,536 of the first arm of the rule that gives 16 keys (512 bytes x 32,768 20.3 / 19.8, x 65,536 24.3 / 24.5; 2 KB x 16,384 24.8 / 24.0),
+// not beyond 262,144, where they are 16 again (uniform keys and zipf 1.05, a five-hundredth over the link: 512 bytes x 400,000 77.4 /
+// 77.9 and 64.9 / 66.3, x 524,000 111.6 / 112.1 and 79.9 / 82.2; with streaming stores, x 1,040,000, 199.8 / 200.7 and 187.5 / 184.6; 1 KB x
+// 520,000 204.7 / 205.6 and 178.0 / 174.4).
 constexpr int mix_rows(int lpr, int kpw) { return lpr >= 32 && kpw <= 16 && kWave / lpr * 8 <= kpw ? 8 : 4; }
 
 // KEEP: rows are loaded the ordinary way instead of past the caches, where the keys that repeat find them.  Stores that are written
@@ -653,7 +657,9 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const size_t slots = (size_t)cu_count() * 4 * 8;
   const int lpr = vpr <= 1 ? 1 : vpr <= 2 ? 2 : vpr <= 4 ? 4 : vpr <= 8 ? 8 : vpr <= 16 ? 16 : vpr <= 32 ? 32 : 64;
   const bool small_rows = lpr <= 8;  // rows of up to 128 bytes
-  const size_t likely = request.counted() ? n / 2 : n;  // distinct keys of n: anything between a seventh of them and all
+  // of n keys whose number is in a device word, the distinct ones of a batch, any number may be there: half of them is a guess for
+  // the shape (a skewed batch of 262,144 has 38,000, a uniform one all but 7,000)
+  const size_t likely = request.counted() ? n / 2 : n;
   int kpw;
   if (KIND == 1) {
     kpw = small_rows ? 32 : 8;
@@ -690,6 +696,7 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;
   const ugk_stage_t no_stage{};
+  const bool few = KIND == 1 ? n <= 4096 : likely <= slots * 8;
   const bool keep = row_bytes <= 64 || out_bytes <= (size_t)64 << 20;
 #define UGK_GO4(L, W, R, NT, KEEP, ST)                                                                              \
   hipLaunchKernelGGL((extract_mix_kernel<K, KIND, L, W, R, NT, KEEP, ST>), dim3(grid), dim3(kBlock), 0, st, t, keys, n,     \
@@ -714,8 +721,8 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   } while (0)
 #define UGK_GO2(L, W)                                             \
   do {                                                            \
-    if constexpr (KIND == 1 && mix_rows(L, W) == 8) {             \
-      if (n > 4096) {                                             \
+    if constexpr (mix_rows(L, W) == 8 && (KIND == 1 || W == 16)) { \
+      if (!few) {                                                 \
         UGK_ROWS(L, W, 4);                                        \
         break;                                                    \
       }                                                           \
