@@ -558,22 +558,16 @@ uint8_t keep_waves_for(size_t n, size_t row_bytes, Store store, bool over_link) 
   return store == kStreaming || n * (row_bytes + lines / kWavesPerBlock) <= kMemorySideCache ? 1 : 0;
 }
 
-// Words (ugk_leave_done_words) come later than a ticket kernel behind the launch would
-//   * for rows of single bytes or pairs: a line that is written through does not come together in L2.  us, launch to end of
-//     poll, ticket / words, rows in HBM: 97 bytes 1 MB 9.9 / 10.2, 8 MB 22.8 / 27.5, 32 MB 62 / 84; 1001 bytes 1 MB 15.8 / 19.6,
-//     8 MB 18.7 / 23.8, 32 MB 36 / 54;
-//   * for a few rows of more than two vectors per lane: the loads of a row's next vectors come back behind the stores of the last,
-//     and those end in memory, not in L2, with nothing else to do meanwhile.  Ticket / words: 8 KB x 4 10.7 / 11.1, 16 KB x 2 11.4 /
-//     13.0, x 8 17.3 / 17.5, 32 KB x 1 14.1 / 17.7, x 16 25.9 / 26.0; with more rows they come out even or words a little sooner (4 KB x
-//     128 11.8 / 11.6, x 2,048 14.2 / 13.6; 8 KB x 64 13.5 / 13.5, x 1,024 16.3 / 15.8).  2 KB 2 to 14 % sooner at any size, as large
-//     outputs are (4 KB x 16,384 31.8 / 29.9).
+// Words (ugk_leave_done_words) come sooner than a ticket kernel behind the launch would, but for rows of single bytes or pairs: a
+// line that is written through does not come together in L2.  us, launch to end of poll, ticket / words, rows in HBM: 97 bytes 1 MB
+// 9.9 / 10.2, 8 MB 22.8 / 27.5, 32 MB 62 / 84; 1001 bytes 1 MB 15.8 / 19.6, 8 MB 18.7 / 23.8, 32 MB 36 / 54.
+// Long rows, of more than two vectors per lane, whose next loads come back behind the stores of the last: keys that were not looked
+// up before, uniform: 4 KB x 1 11.4 / 9.5, x 16 11.8 / 10.8, x 512 13.1 / 12.5, x 8,192 21.7 / 20.8; 8 KB x 8 12.8 / 12.7, x 64 14.8 / 13.9, x
+// 1,024 17.1 / 16.2; 16 KB x 4 15.6 / 15.7, x 64 18.9 / 18.1; 32 KB x 2 20.6 / 21.3, x 8 26.0 / 26.0, x 64 27.2 / 26.9, x 1,024 35.1 / 33.3;
+// zipf 1.05 sooner by 3 to 15 %.  (Lookups of such rows through the library, 32 KB to 16 MB of them, all in HBM, 0.6 of them and none:
+// 4 to 31, 1 to 19 and 1 to 12 % sooner than with a ticket, which batches that were looked up before had seemed to favour.)
 // (Outputs of 6 to 10 MB, about what the wavefronts of one round copy and all written at once, are 0.1 to 0.6 us later too where
 // a launch costs the host 3 us, and 0.9 us sooner where it costs 4: words there.)
-Telling gather_tells(size_t vector_bytes, uint32_t vectors_per_row, uint32_t lanes, size_t out_bytes) {
-  if (vector_bytes < 4) return Telling::kTooLate;
-  return vectors_per_row <= 2 * lanes || out_bytes > (size_t)32 << 20 ? Telling::kSooner : Telling::kLater;
-}
-
 template <typename V, int LPR, int UNROLL, typename Idx>
 int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint64_t out_rows, uint32_t vpr,
                     const uint32_t *counts, uint32_t group, size_t n, unsigned max_blocks, uint32_t *status,
@@ -583,7 +577,7 @@ int launch_unrolled(Idx ix, const void *src, uint64_t src_rows, void *out, uint6
   const bool many_groups = grid > (unsigned)cu_count() * 8u;  // more than 32 wavefronts per CU
   DoneWords done{};
   if constexpr (Idx::kDense) {
-    if (!nt) done = request.take(grid, gather_tells(sizeof(V), vpr, LPR, n * (size_t)vpr * sizeof(V)));
+    if (!nt) done = request.take(grid, sizeof(V) < 4 ? Telling::kTooLate : Telling::kSooner);
     UGK_REQUIRE(!request.counted(), "gather: a launch that leaves no words cannot take its count from the device");
   }
   const uint8_t keep_waves = keep_waves_for(n, (size_t)vpr * sizeof(V), done.tag ? kThrough : nt ? kStreaming : kOrdinary,

@@ -72,9 +72,9 @@ struct DoneWords {
 // 8.6 / 8.2 / 8.2 / 8.1 / 8.1, 8.0 and 9.4; 8 rows 6.3 against 8.5.
 constexpr uint32_t kDoneDirect = UGK_DONE_WORDS, kDoneFan = UGK_DONE_COUNTERS / 2;
 
-// When words are there, against a ticket kernel behind the launch (ugk_done_t::where_faster): sooner or at the same time, later
-// but by less than a kernel that copies keys takes, later than that.
-enum class Telling { kSooner, kLater, kTooLate };
+// When words are there, against a ticket kernel behind the launch (ugk_done_t::where_faster): sooner or at the same time, or later by
+// more than a kernel that copies keys takes.
+enum class Telling { kSooner, kTooLate };
 
 // The request of ugk_leave_done_words, if this thread has made one: the entry points that can fulfil it take it as they
 // begin, so that it never meets a later launch.

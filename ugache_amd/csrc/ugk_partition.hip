@@ -244,12 +244,17 @@ __device__ __forceinline__ uint64_t stage_claim(const ugk_stage_t &stage, const 
 constexpr int mix_rows(int lpr, int kpw) { return lpr >= 32 && kpw <= 16 && kWave / lpr * 8 <= kpw ? 8 : 4; }
 
 // KEEP: rows are loaded the ordinary way instead of past the caches, where the keys that repeat find them.  Stores that are written
-// through need no room there, and with them every launch gains or loses nothing whose output leaves the lines room in the
-// memory-side cache.  us, launch to end of poll, past / kept, a fiftieth of the rows over the link, uniform keys, zipf 0.8, 1.05 and
-// 1.2: 512 bytes x 4,096 14.8 / 14.7, 13.9 / 13.7, 13.4 / 13.2 and 13.4 / 13.3, x 32,768 21.0 / 20.9, 18.6 / 17.7, 17.7 / 16.7 and 17.4 /
-// 16.3, x 131,072 40.2 / 39.7, 31.7 / 31.8, 30.2 / 29.1 and 32.4 / 25.5; 100 bytes x 671,088 82.9 / 83.0, 55.1 / 52.6, 51.6 / 43.5 and
-// 50.0 / 39.9.  Beyond 64 MB rows of more than 64 bytes lose, 512 bytes x 262,144 47.3 / 51.4 with zipf 1.05, x 400,000 72 / 77 with
-// 0.8; shorter ones gain at any size (64 bytes x 4,000,000 271 / 270, 179 / 176, 169 / 162 and 160 / 152).
+// through need no room there, and a table that is cached in part is one whose keys are skewed: uniform ones pay 1 to 2 % for what
+// zipf 1.2 gains 5 to 25 % by.  us, launch to end of poll, past / kept, keys that were not looked up before, a five-hundredth of the
+// rows over the link, uniform, zipf 0.8, 1.05 and 1.2: 512 bytes x 128 11.1 / 11.2, 10.8 / 10.8, 10.6 / 10.4 and 10.5 / 10.3; x 4,096 13.6 /
+// 13.9, 13.3 / 13.4, 12.8 / 12.8 and 12.6 / 12.5; x 32,768 18.6 / 19.0, 18.0 / 18.3, 17.1 / 17.0 and 16.8 / 15.8; x 65,536 23.6 / 23.8, 22.6 /
+// 22.8, 21.3 / 21.6 and 21.7 / 18.5; x 131,072 32.8 / 33.0, 31.5 / 31.1, 29.3 / 31.0 and 30.6 / 25.0; 1204 bytes x 27,869 25.5 / 25.8, 24.4 /
+// 24.6, 23.5 / 23.9 and 23.8 / 19.6; 100 bytes x 20,971 16.4 / 16.8, 16.0 / 16.1, 15.0 / 15.3 and 14.8 / 14.8, x 671,088 60.8 / 64.0, 58.1 /
+// 56.6, 51.5 / 50.0 and 48.9 / 44.6.  With a fiftieth over the link, which then bounds the launch, 1 % either way.  Beyond 64 MB rows
+// of more than 64 bytes lose (512 bytes x 262,144 53.5 / 54.6, 51.0 / 50.6, 46.4 / 50.1 and 49.0 / 46.4; 100 bytes x 1,342,177 112 / 127 and
+// 101 / 104); shorter ones, of which a line holds several, go on (64 bytes x 2,097,152 117 / 123, 107.5 / 107.9, 92.1 / 89.9 and 87.0 /
+// 81.0).  Distinct keys repeat nothing within a launch; what the launch before has kept of the same rows makes them even (512
+// bytes, 0.25 to 134 MB, uniform and zipf 1.2, 0.99 to 1.02 times as fast).
 // LPR: lanes per row, or 0 for rows that are copied flat (flat_copy; f.tile rows at a time)
 template <typename K, int KIND, int LPR, int KPW, int ROWS, Store STORE, bool KEEP, bool STAGE>
 __global__ __launch_bounds__(kBlock) void extract_mix_kernel(ugk_table_t t, const K *__restrict__ keys, size_t n,
@@ -681,17 +686,14 @@ int extract_mix_lpr(ugk_table_t t, const K *keys, size_t n, const void *cache, u
   const FlatRow f_row = flat_row(row_bytes, (uint32_t)kpw);
   const size_t keys_per_group = (size_t)kpw * kWavesPerBlock;
   const unsigned grid = request.grid(clamp_grid((n + keys_per_group - 1) / keys_per_group, mostly_host ? 128u : 0u));
-  // Words come sooner than a ticket behind the launch would, but for up to four long rows, whose wavefront waits between their
-  // vectors for memory, where they are written through (see gather_tells).  us, launch to end of poll, ticket / words, all rows
-  // in HBM, a hash table: 512 bytes x 1,024 13.2 / 12.3; 1536 bytes x 85 15.1 / 12.9, x 5,461 19.5 / 16.8; 4 KB x 4 12.6 / 12.7, x 8 15.0 /
-  // 14.3, x 2,048 20.2 / 19.0, x 16,384 36.9 / 33.4; 8 KB x 2 13.0 / 14.3, x 8 18.8 / 18.7, x 1,024 24.6 / 23.6; 32 KB x 4 34.2 / 38.8, x 64
-  // 51.4 / 50.3; a twentieth of the rows over the link: the same signs.  With a flat table rows of more than 1 KB gain up to outputs
-  // of 4 MB (1040 bytes x 252 13.4 / 12.5, x 4,032 13.9 / 13.6) and, of up to 4 KB, beyond 32 MB, and come out even between those
-  // (1040 bytes x 8,065 14.8 / 14.8, 4112 bytes x 2,040 18.8 / 18.8, 4 KB x 8,192 22.9 / 22.5).
+  // Words come sooner than a ticket behind the launch would.  us, launch to end of poll, ticket / words, keys that were not looked up
+  // before, uniform, a five-hundredth over the link, a hash table: 512 bytes x 1 11.7 / 9.7, x 1,024 14.6 / 13.4, x 16,384 18.4 / 17.4; 1536
+  // bytes x 64 13.5 / 12.6, x 4,096 17.2 / 16.6; 4112 bytes x 1 12.6 / 11.6, x 1,024 20.3 / 19.7; 8 KB x 8 15.5 / 15.8, x 1,024 26.7 / 25.6; 32 KB
+  // x 2 25.4 / 27.0, x 8 33.3 / 34.9, x 64 45.7 / 45.5, x 4,096 78.4 / 75.7; a flat table: 1040 bytes x 4,032 15.0 / 14.5, x 16,384 19.2 / 18.9;
+  // 4112 bytes x 1,024 19.8 / 18.9, x 4,096 22.3 / 21.3; 8 KB x 4,096 30.1 / 27.6; 32 KB x 8 32.7 / 34.3.  Zipf 1.05 sooner everywhere but
+  // for one row of 32 KB, by up to 14 %.
   const size_t out_bytes = n * row_bytes;
-  const bool even = KIND == 1 && row_bytes > 1024 && out_bytes > (size_t)4 << 20 && (row_bytes > 4096 || out_bytes <= (size_t)32 << 20);
-  const Telling words = even || (row_bytes > 4096 && n <= 4) ? Telling::kLater : Telling::kSooner;
-  DoneWords done = nt && !flat ? DoneWords{} : request.take(grid, words, n);
+  DoneWords done = nt && !flat ? DoneWords{} : request.take(grid, Telling::kSooner, n);
   UGK_REQUIRE(!request.counted(), "ugk_extract_mix: a launch that leaves no words cannot take its count from the device");
   if (!done.tag) done.words = reinterpret_cast<unsigned long long *>(counts);
   if (num_groups) *num_groups = done.tag ? 0 : grid;

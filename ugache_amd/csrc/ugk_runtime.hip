@@ -39,8 +39,7 @@ DoneRequest::DoneRequest() : _done(g_done) { g_done = nullptr; }
 // a counter holds 16 bits of workgroups and two counts of 24 bits
 DoneWords DoneRequest::take(unsigned grid, Telling words, uint64_t count_limit) {
   if (!_done || grid / kDoneFan >= 0xffffu || count_limit >= (1u << 24)) return DoneWords{};
-  if (_done->where_faster && !counted() && words != Telling::kSooner && (words == Telling::kTooLate || _done->num_keys == 0))
-    return DoneWords{};
+  if (_done->where_faster && !counted() && words == Telling::kTooLate) return DoneWords{};
   ugk_done_t *d = _done;
   _done = nullptr;
   d->num_words = grid <= kDoneDirect ? grid : kDoneFan;
