@@ -91,6 +91,7 @@ def test_a_gather_nobody_polls_for_has_its_arguments_in_two_lines(gather_kernels
 
 
 @pytest.mark.parametrize("source,kernel,words", [("ugk_partition.hip", "dedup_resolve_kernel", 1),
+                                                 ("ugk_partition.hip", "dedup_small_kernel", 1),
                                                  ("ugk_refresh.hip", "rank_combine_observed_kernel", 2)])
 def test_a_word_for_the_host_is_there_before_its_launch_has_ended(source, kernel, words):
     """the host reads them once a launch behind this one tells it that all is done; what is acknowledged is in host memory only if

@@ -1330,7 +1330,7 @@ def test_pooled_extraction_matches_a_float64_segment_sum(kind, dim, etype, rows_
         words.free()
 
 
-# every kernel and kind of lane of the gathers, the fused one with and without a stage
+# every kernel and kind of lane of the gathers, the fused one (with a stage: test_staged_launch_that_finds_its_count_on_the_device)
 @pytest.mark.parametrize("kind,rb", [("none", 512), ("none", 64), ("none", 8192), ("none", 100), ("none", 36), ("none", 1204),
                                      ("none", 800), ("none", 2), ("none", 1), ("flat", 512), ("flat", 100), ("hash", 64),
                                      ("hash32", 1024), ("hash32", 36)])
@@ -1756,6 +1756,58 @@ def _fmix64(x):
     x *= np.uint64(0xC4CEB9FE1A85EC53)
     x ^= x >> np.uint64(33)
     return x
+
+
+@pytest.mark.parametrize("kind", ["flat", "hash", "hash32"])
+@pytest.mark.parametrize("rb", [64, 128, 512])
+def test_staged_launch_that_finds_its_count_on_the_device(kind, rb):
+    """ugk_done_t::count_dev with a stage, as a distinct-key lookup of a cache with one has it: rows and group sizes are those of the
+    keys in front of the count, and of their host rows alone some are filed"""
+    rng = np.random.default_rng(rb)
+    nkeys, entries = 12_000, 2048
+    host = _rand_table(rng, nkeys, rb)
+    cached = rng.choice(nkeys, nkeys // 2, replace=False).astype(np.int64)
+    mem, tb = {"flat": lambda: _make_flat(nkeys), "hash": lambda: _make_hash(len(cached))[:2],
+               "hash32": lambda: _make_hash32(len(cached))[:2]}[kind]()
+    assert _insert(tb, cached) == 0
+    is_cached = np.zeros(nkeys, bool)
+    is_cached[cached] = True
+    pin, done, count = pinned_from(host), _DoneWords(), dev_zeros_u32(1)
+    words, groups = PinnedArray((hip.lib().ugk_extract_mix_max_groups(),), np.uint64), C.c_uint32(0)
+    try:
+        d_cache, st = to_dev(host[cached].copy()), dev_zeros_u32(1)
+        for n in (700, 11_000):
+            keys = rng.permutation(nkeys)[:n].astype(np.int64)  # each once: a row behind the count is none in front of it
+            d_keys = to_dev(keys)
+            for have in (0, 1, n // 2 + 1, n, n + 7):
+                count.fill_(have)
+                done.done.count_dev = ptr(count)
+                m, out = min(n, have), dev_bytes(n * rb, fill=0x7F)
+                stage_rows, owner = dev_bytes(entries * rb, fill=0xEE), to_dev(np.zeros(entries, np.uint64))
+                done.ask(0)
+                hip.call("ugk_extract_mix_staged_i64", tb, ptr(d_keys), n, ptr(d_cache), len(cached), pin.ptr, nkeys, ptr(out), rb,
+                         ptr(st), done.mirror.ptr, words.ptr, C.byref(groups), hip.HINT_UNKNOWN,
+                         hip.Stage(ptr(stage_rows), ptr(owner), entries - 1, 5, 0), None)
+                assert done.done.num_words > 0
+                local, others = C.c_uint64(), C.c_uint64()
+                hip.call("ugk_done_wait", C.byref(done.done), 1_000_000, None, C.byref(local), C.byref(others))
+                done.check_flag(0)
+                done.check_counters()
+                raw = to_np(out).reshape(n, rb)
+                assert raw[:m].tobytes() == host[keys[:m]].tobytes() and (raw[m:] == 0x7F).all(), (n, have)
+                missed = keys[:m][~is_cached[keys[:m]]]
+                assert (local.value, others.value) == (m - len(missed), len(missed))
+                own = to_np(owner, np.uint64)[:entries]
+                filled = np.flatnonzero(own)
+                assert (own[filled] >> np.uint64(32) == 5).all() and (len(filled) > 0) == (len(missed) > 0)
+                rows = (own[filled] & np.uint64(0xFFFFFFFF)).astype(np.int64)
+                assert np.isin(rows, missed).all(), (n, have)
+                got = to_np(stage_rows)[: entries * rb].reshape(entries, rb)
+                assert np.array_equal(got[filled], host[rows]) and (np.delete(got, filled, axis=0) == 0xEE).all()
+    finally:
+        sync()
+        pin.free()
+        words.free()
 
 
 @pytest.mark.parametrize("kind", ["flat", "hash", "hash32"])
