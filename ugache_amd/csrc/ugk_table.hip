@@ -19,9 +19,9 @@ __global__ __launch_bounds__(kBlock) void hash_init_kernel(ugk_bucket_t *table, 
 // Slots that rows which leave hand on to rows that come in: that every listed one is in use, and listed once (two entries of a
 // table that name one slot would go on as one row under two keys).  The eviction has left in stamps[slot] where in the list the slot
 // is: of two places one finds the other's.  Plain stores, and loads that are on their way with the probes': two steps of a lookup
-// and a refresh of 72,000 rows 738 us without, 739 to 743 with, a refresh of 462,000 rows over 50 M slots 267 and 277.  (Marks in a bitmap, 72,000 atomics on the few thousand lines of 4 M bits,
-// took 20 us where the eviction looks at them, 8 where it leaves them for a count, 5 to 7 beside the insert; sets in LDS, by
-// workgroups that each read the whole list, 5 to 10.)
+// and a refresh of 72,000 rows 738 us without, 739 to 743 with, a refresh of 462,000 rows over 50 M slots 267 and 277.  (Marks in a
+// bitmap, 72,000 atomics on the few thousand lines of 4 M bits, took 20 us where the eviction looks at them, 8 where it leaves them
+// for a count, 5 to 7 beside the insert; sets in LDS, by workgroups that each read the whole list, 5 to 10.)
 struct SlotsCheck {
   const uint32_t *stamps;          // null: nothing is checked
   const unsigned long long *used;  // one bit per slot
